@@ -5,113 +5,112 @@ namespace sage {
 
 // ---------------------------------------------------------------------------------------------
 // Variable-length plan: block offsets per sequence and the cost-ordered tile list.
-// One workgroup; sequences are few (tens to thousands), tiles up to total_q/128 + nseq.
+//
+// Tiles are listed in cost TIERS of kTierCost cost units (eight causal q-tiles of 256 rows when the unit is 64 keys),
+// most expensive tier first; inside a tier sequence by sequence, and inside a sequence the heavier q-tiles first.
+// Consecutive entries of the list run at the same time (eight of them per XCD when an XCD holds one KV head), and q-tiles
+// of one sequence walk the same K/V tiles from tile 0 on at about the same pace: one fetches a tile into the XCD's L2, the
+// others hit it there.  Ordered by cost alone, neighbours in the list belong to different sequences and share nothing.
+//
+// One workgroup, bound by the latency of its dependent steps.  The cost of a q-tile does not decrease with its index, so the
+// tiles of a sequence in one tier are a contiguous range with ends in closed form, and no tile is ever visited to be counted:
+// one wavefront owns a tier, a lane a sequence, and a wavefront scan gives every sequence its place in the tier's part of the
+// list.  (A histogram over all tiles, with one pass of the whole workgroup and four barriers per sequence, took 82 us for
+// 96 sequences of 16..1024 rows and 30 us for 16 of 512..32768; this takes 6 and 9.)
 // ---------------------------------------------------------------------------------------------
-constexpr int kCostBins = 2048;
+constexpr int kCostMax = 2047, kTierCost = 32, kTiers = (kCostMax + 1) / kTierCost;
+constexpr int kPlanThreads = 1024, kPlanWaves = kPlanThreads / 64, kPlanSeqsLds = 4096;
+static_assert(kTiers == 64, "one lane per tier in the scan over the tiers");
 
-__global__ void __launch_bounds__(1024) varlen_plan_kernel(const int32_t* cu_q, const int32_t* cu_k, int nseq, int total_q,
-                                                           int blkq, int blkk, int bm, int bn, int causal, int32_t* plan) {
-  const SagePlanLayout L = plan_layout(nseq, total_q);
-  int32_t* cu_qblk = plan + L.cu_qblk;
-  int32_t* cu_kblk = plan + L.cu_kblk;
-  int32_t* cu_panel = plan + L.cu_panel;
-  int32_t* tiles = plan + L.tiles;
-  __shared__ int hist[kCostBins];
-  __shared__ int start[kCostBins];
-  const int tid = threadIdx.x;
-  for (int i = tid; i < kCostBins; i += blockDim.x) hist[i] = 0;
-  if (tid == 0) {
-    int aq = 0, ak = 0, ap = 0;
-    for (int i = 0; i < nseq; i++) {
-      cu_qblk[i] = aq; cu_kblk[i] = ak; cu_panel[i] = ap;
-      int lq = cu_q[i + 1] - cu_q[i], lk = cu_k[i + 1] - cu_k[i];
-      aq += (lq + blkq - 1) / blkq; ak += (lk + blkk - 1) / blkk; ap += (lk + kPanelRows - 1) / kPanelRows;
-    }
-    cu_qblk[nseq] = aq; cu_kblk[nseq] = ak; cu_panel[nseq] = ap;
-  }
-  __syncthreads();
-  auto cost_of = [&](int lq, int lk, int qt) {
-    int kv_end = causal ? min(lk, (qt + 1) * bm) : lk;
-    int c = (kv_end + bn - 1) / bn;
-    return min(c, kCostBins - 1);
-  };
-  // pass 1: histogram of tile costs
-  for (int i = 0; i < nseq; i++) {
-    int lq = cu_q[i + 1] - cu_q[i], lk = cu_k[i + 1] - cu_k[i];
-    int nqt = (lq + bm - 1) / bm;
-    for (int qt = tid; qt < nqt; qt += blockDim.x) atomicAdd(&hist[cost_of(lq, lk, qt)], 1);
-  }
-  __syncthreads();
-  // start[c] = number of tiles in more expensive bins: an exclusive scan over the bins in descending cost
-  // order, two bins per thread, wavefront scans combined through LDS.
-  {
-    static_assert(kCostBins == 2048, "two bins per thread of a 1024-thread workgroup");
-    __shared__ int wave_total[16];
-    const int c0 = kCostBins - 1 - 2 * tid, c1 = c0 - 1;   // this thread's bins, the more expensive one first
-    const int h0 = hist[c0], h1 = hist[c1];
-    int incl = h0 + h1;
-    const int lane = tid & 63, wv = tid >> 6;
+__device__ inline int wave_inclusive_scan(int x) {
+  const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += up;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(x, d, 64);
+    if (lane >= d) x += up;
+  }
+  return x;
+}
+
+__global__ void __launch_bounds__(kPlanThreads) varlen_plan_kernel(const int32_t* cu_q, const int32_t* cu_k, int nseq, int total_q,
+                                                                   int blkq, int blkk, int bm, int bn, int causal, int32_t* plan) {
+  const SagePlanLayout L = plan_layout(nseq, total_q);
+  int32_t* tiles = plan + L.tiles;
+  __shared__ int2 len_lds[kPlanSeqsLds];   // (query rows, keys) of the first sequences; the rest is read again where needed
+  __shared__ int tier_total[kTiers], tier_start[kTiers], longest;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  if (tid == 0) longest = 0;
+  __syncthreads();
+  auto lengths_in_memory = [&](int i) { return make_int2(cu_q[i + 1] - cu_q[i], cu_k[i + 1] - cu_k[i]); };
+  {
+    int most = 0;
+    for (int i = tid; i < nseq; i += kPlanThreads) {
+      const int2 n = lengths_in_memory(i);
+      if (i < kPlanSeqsLds) len_lds[i] = n;
+      most = max(most, causal ? min(n.y, (n.x + bm - 1) / bm * bm) : n.y);
     }
-    if (lane == 63) wave_total[wv] = incl;
-    __syncthreads();
-    int before = 0;
-    for (int i = 0; i < wv; i++) before += wave_total[i];
-    const int excl = before + incl - (h0 + h1);
-    start[c0] = excl;
-    start[c1] = excl + h0;
-    if (tid == 1023) plan[L.ntiles] = before + incl;
+    atomicMax(&longest, most);
   }
   __syncthreads();
-  // pass 2: place tiles.  Few sequences (the usual case): cost TIERS of kTierCost cost units (eight causal q-tiles of
-  // 256 rows when the unit is 64 keys), most expensive tier first;
-  // inside a tier sequence by sequence, and inside a sequence the heavier q-tiles first.  Consecutive entries of the
-  // list run at the same time (eight of them per XCD when an XCD holds one KV head), and q-tiles of one sequence
-  // walk the same K/V tiles from tile 0 on at about the same pace: one fetches a tile into the XCD's L2, the others
-  // hit it there.  Ordered by cost alone, neighbours in the list belong to different sequences and share nothing.
-  // The q-tiles of a sequence that fall into one tier are a contiguous range (cost does not decrease with the tile
-  // index), so a tile's place is the tier's fill level plus its distance from the heaviest tile of that range.
-  constexpr int kTierCost = 32, kTiers = kCostBins / kTierCost, kMaxTieredSeqs = 64;
-  if (nseq <= kMaxTieredSeqs) {
-    __shared__ int tier_fill[kTiers], tier_max[kTiers], tier_cnt[kTiers];
-    if (tid == 0) {
-      int before = 0;
-      for (int t = kTiers - 1; t >= 0; t--) {
-        tier_fill[t] = before;
-        for (int c = 0; c < kTierCost; c++) before += hist[t * kTierCost + c];
-      }
+  auto lengths = [&](int i) { return i < kPlanSeqsLds ? len_lds[i] : lengths_in_memory(i); };
+  const int top_tier = min((longest + bn - 1) / bn, kCostMax) / kTierCost;   // the tiers above it are empty
+  // First q-tile of a sequence whose tier is at least t: its cost, in units of bn keys, has to reach t * kTierCost.
+  auto first_tile = [&](int2 n, int nqt, int t) {
+    const int keys = bn * (t * kTierCost - 1) + 1;
+    return t == 0 ? 0 : n.y < keys ? nqt : causal ? min(nqt, (keys + bm - 1) / bm - 1) : 0;
+  };
+
+  // block offsets: three running sums over the sequences, one wavefront each (the last ones: tiers start at the first)
+  if (w >= kPlanWaves - 3) {
+    const int which = kPlanWaves - 1 - w;
+    int32_t* dst = plan + (which == 0 ? L.cu_qblk : which == 1 ? L.cu_kblk : L.cu_panel);
+    const int unit = which == 0 ? blkq : which == 1 ? blkk : kPanelRows;
+    int before = 0;
+    for (int i0 = 0; i0 < nseq; i0 += 64) {
+      const int i = i0 + lane;
+      const int2 n = i < nseq ? lengths(i) : make_int2(0, 0);
+      const int blocks = ((which == 0 ? n.x : n.y) + unit - 1) / unit;
+      const int upto = before + wave_inclusive_scan(blocks);
+      if (i < nseq) dst[i] = upto - blocks;
+      before = __shfl(upto, 63, 64);
     }
-    for (int i = 0; i < nseq; i++) {
-      const int lq = cu_q[i + 1] - cu_q[i], lk = cu_k[i + 1] - cu_k[i];
-      const int nqt = (lq + bm - 1) / bm;
-      for (int t = tid; t < kTiers; t += blockDim.x) { tier_max[t] = -1; tier_cnt[t] = 0; }
-      __syncthreads();
-      for (int qt = tid; qt < nqt; qt += blockDim.x) {
-        const int t = cost_of(lq, lk, qt) / kTierCost;
-        atomicMax(&tier_max[t], qt);
-        atomicAdd(&tier_cnt[t], 1);
-      }
-      __syncthreads();
-      for (int qt = tid; qt < nqt; qt += blockDim.x) {
-        const int t = cost_of(lq, lk, qt) / kTierCost;
-        tiles[tier_fill[t] + tier_max[t] - qt] = (i << 16) | qt;
-      }
-      __syncthreads();
-      for (int t = tid; t < kTiers; t += blockDim.x) tier_fill[t] += tier_cnt[t];
-      __syncthreads();
-    }
-    return;
+    if (lane == 0) dst[nseq] = before;
   }
-  // Many sequences: most expensive cost bins first, in whatever order the tiles of a bin arrive.
-  for (int i = 0; i < nseq; i++) {
-    int lq = cu_q[i + 1] - cu_q[i], lk = cu_k[i + 1] - cu_k[i];
-    int nqt = (lq + bm - 1) / bm;
-    for (int qt = tid; qt < nqt; qt += blockDim.x) {
-      int pos = atomicAdd(&start[cost_of(lq, lk, qt)], 1);
-      tiles[pos] = (i << 16) | qt;
+  // tiles per tier
+  for (int t = w; t < kTiers; t += kPlanWaves) {
+    int count = 0;
+    if (t <= top_tier) {
+      for (int i = lane; i < nseq; i += 64) {
+        const int2 n = lengths(i);
+        const int nqt = (n.x + bm - 1) / bm;
+        count += (t == kTiers - 1 ? nqt : first_tile(n, nqt, t + 1)) - first_tile(n, nqt, t);
+      }
+      count = __shfl(wave_inclusive_scan(count), 63, 64);
+    }
+    if (lane == 0) tier_total[t] = count;
+  }
+  __syncthreads();
+  if (w == 0) {   // where each tier starts in the list: lane l takes tier kTiers - 1 - l
+    const int t = kTiers - 1 - lane, upto = wave_inclusive_scan(tier_total[t]);
+    tier_start[t] = upto - tier_total[t];
+    if (lane == 63) plan[L.ntiles] = upto;
+  }
+  __syncthreads();
+  for (int t = w; t <= top_tier; t += kPlanWaves) {
+    if (tier_total[t] == 0) continue;
+    int before = tier_start[t];
+    for (int i0 = 0; i0 < nseq; i0 += 64) {
+      const int i = i0 + lane;
+      int lo = 0, hi = 0;   // this sequence's q-tiles in the tier: lo .. hi - 1
+      if (i < nseq) {
+        const int2 n = lengths(i);
+        const int nqt = (n.x + bm - 1) / bm;
+        lo = first_tile(n, nqt, t);
+        hi = t == kTiers - 1 ? nqt : first_tile(n, nqt, t + 1);
+      }
+      const int upto = before + wave_inclusive_scan(hi - lo);
+      for (int qt = lo; qt < hi; qt++) tiles[upto - 1 - (qt - lo)] = (i << 16) | qt;
+      before = __shfl(upto, 63, 64);
     }
   }
 }
@@ -171,7 +170,7 @@ hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, 
 
 hipError_t launch_varlen_plan(const int32_t* cu_q, const int32_t* cu_k, int nseq, int total_q, int blkq, int blkk, int bm,
                               int bn, int causal, int32_t* plan, hipStream_t st) {
-  varlen_plan_kernel<<<1, 1024, 0, st>>>(cu_q, cu_k, nseq, total_q, blkq, blkk, bm, bn, causal, plan);
+  varlen_plan_kernel<<<1, kPlanThreads, 0, st>>>(cu_q, cu_k, nseq, total_q, blkq, blkk, bm, bn, causal, plan);
   return hipGetLastError();
 }
 

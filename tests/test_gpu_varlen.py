@@ -67,6 +67,32 @@ def test_plan_orders_tiles_by_cost_tier_then_sequence_and_covers_every_tile():
     assert p[offs[2]:offs[2] + 7].tolist() == np.concatenate([[0], np.cumsum([(L + 127) // 128 for L in lens])]).tolist()
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("nseq,longest", [(1, 70000), (63, 3000), (64, 300), (65, 5000), (200, 1), (4097, 700), (5000, 40)])
+def test_plan_for_many_sequences_and_every_tier(nseq, longest, causal):
+    """Around the scheduler's chunk of 64 sequences, beyond the 4096 whose lengths it keeps in LDS, with empty sequences, with
+    other key than query lengths and with costs over the last tier's start (64 x 2016 keys): list and block offsets exact."""
+    rng = np.random.default_rng(nseq + longest)
+    lq = rng.integers(0, longest + 1, nseq)
+    lk = rng.integers(0, longest + 1, nseq)
+    lq[0] = longest
+    lk[0] = 135000 if nseq == 1 else 1
+    cuq, cuk = (np.concatenate([[0], np.cumsum(x)]).astype(np.int32) for x in (lq, lk))
+    plan, offs = sa.varlen_plan(torch.from_numpy(cuq).to(DEV), torch.from_numpy(cuk).to(DEV), int(cuq[-1]), 64, 16, is_causal=causal)
+    p = plan.cpu().numpy()
+    for off, x, unit in ((offs[0], lq, 64), (offs[1], lk, 16), (offs[2], lk, 128)):
+        assert np.array_equal(p[off:off + nseq + 1], np.concatenate([[0], np.cumsum((x + unit - 1) // unit)]))
+    want = []
+    for i in range(nseq):
+        for t in range((lq[i] + 255) // 256):
+            cost = min(((min(lk[i], (t + 1) * 256) if causal else lk[i]) + 63) // 64, 2047)
+            want.append((-(cost // 32), i, -t))
+    want.sort()
+    n = int(p[offs[3]])
+    got = [(int(t) >> 16, int(t) & 0xFFFF) for t in p[offs[4]:offs[4] + n]]
+    assert got == [(i, -t) for _, i, t in want]
+
+
 def test_config4_full_size_sequences_are_independent():
     """BASELINE config 4 at its full size (16 packed sequences of 512..32768 rows, Hq32/Hkv8, D128 bf16 causal, FP8
     P.V): the packed call reproduces, bit for bit, a stand-alone call on each of three of its sequences (shortest,
