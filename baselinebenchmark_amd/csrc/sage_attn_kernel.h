@@ -124,8 +124,14 @@ constexpr int attn_tile_lds_bytes() {
   constexpr int qstage = attn_tile_lead<PV, CAUSAL>() * BN * D + NW * 32 * D * 2;
   return (QF && qstage > tiles) ? qstage : tiles;
 }
-template <int D, int NW, int BN, int PV, bool CAUSAL, bool QF>
-constexpr int attn_lds_bytes() { return attn_tile_lds_bytes<D, NW, BN, PV, CAUSAL, QF>() + (PV ? D * 4 : 0); }
+// Kernels that follow a packed mask (MASK == 3) keep their list of visible tiles and the mask bits of the tiles in flight
+// behind that: four slots, because group 1 still reads the bits of tile j - 1 in period j while those of tile j + 1 (FP16
+// P.V) or j + 2 (FP8 P.V) arrive.
+constexpr int kMaskSlots = 4;
+template <int D, int NW, int BN, int PV, bool CAUSAL, bool QF, int MASK>
+constexpr int attn_lds_bytes() {
+  return attn_tile_lds_bytes<D, NW, BN, PV, CAUSAL, QF>() + (PV ? D * 4 : 0) + (MASK == 3 ? kMaskSlots * kMaskTileBytes + kMaskMaxTiles * 4 : 0);
+}
 
 // Timing build (-DSAGE_TIMING=1, not the shipped library): every wavefront stamps eight points of its
 // tile on the constant-rate 100 MHz counter and adds the seven intervals to per-class sums (class 0 =
@@ -153,7 +159,9 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 #define SAGE_T(k, x) do { } while (0)
 #endif
 // MASK: 0 none, 1 boolean keep-mask (bytes), 2 additive fp32 bias in base-2 score units
-// (sageattention_triton.py:92-105), both [B, Hq, Sq, Skv] with element strides.
+// (sageattention_triton.py:92-105), both [B, Hq, Sq, Skv] with element strides; 3 = a boolean mask in the packed form of
+// mask_pack_kernel (sage_common.h): the workgroup walks only the tiles in which one of its rows sees a key, a wavefront
+// skips the tiles in which none of its own 32 rows does, and the bits of a tile arrive like a K tile does.
 // KSUB: K scale blocks per 32 keys (1 for blocks of 32/64/128 keys, 2 for blocks of 16 keys); 3 = four interleaved scales per
 // block of 32/64/128 keys, scale t for the keys n of the block with (n % 8) / 2 == t (two of them reach every lane).
 // QF: the kernel reads fp16/bf16 Q and quantises its own tile (same arithmetic as quant_int8_kernel).
@@ -317,7 +325,32 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   const int row0 = qt * BM + w * 32;   // first query row of this wavefront
   const int my_row = row0 + m;
   const int kv_end = CAUSAL ? min(Lk, qt * BM + BM) : Lk;
-  const int ntiles = (kv_end + BN - 1) / BN;
+  constexpr bool LISTED = MASK == 3;
+  uint8_t* mask_lds = smem + attn_tile_lds_bytes<D, NW, BN, PV, CAUSAL, QF>() + (PV ? D * 4 : 0);
+  int* tile_list = reinterpret_cast<int*>(mask_lds + kMaskSlots * kMaskTileBytes);
+  int ntiles = (kv_end + BN - 1) / BN;
+  const uint8_t* mask_bits = nullptr;
+  if constexpr (LISTED) {
+    // The tiles this workgroup has to visit, in order: tile index | the visibility classes of its eight 32-row groups << 16.
+    // Every wavefront writes the same list (and reads back only what it wrote itself), so no barrier is needed.
+    const int64_t qtile = (int64_t)(b * a.mask_pb + hq_idx * a.mask_ph) * a.mask_nqt + (a.mask_nqt > 1 ? qt : 0);
+    const u16* cls = a.mask_cls + qtile * a.mask_ntk;
+    mask_bits = a.mask_bits + qtile * a.mask_ntk * kMaskTileBytes;
+    int n = 0;
+    for (int t0 = 0; t0 < a.mask_ntk; t0 += 64) {
+      const int t = t0 + lane;
+      const int c = t < a.mask_ntk ? cls[t] : 0;
+      const unsigned long long on = __builtin_amdgcn_ballot_w64(c != 0);
+      if (c != 0) tile_list[n + __popcll(on & ((1ull << lane) - 1))] = t | (c << 16);
+      n += __popcll(on);
+    }
+    ntiles = n;
+  }
+  auto list_entry = [&](int j) { return __builtin_amdgcn_readfirstlane(tile_list[min(j, ntiles - 1)]); };
+  // key tile that period j works on
+  auto tile_at = [&](int j) { return LISTED ? list_entry(j) & 0xffff : j; };
+  // packed mask: what this wavefront's rows see of it (0 nothing, 1 some keys, 2 every key)
+  auto sees = [&](int j) { return row0 < Lq ? (list_entry(j) >> (16 + 2 * w)) & 3 : 0; };
   const int wave_end = (row0 < Lq) ? (CAUSAL ? min(Lk, row0 + 32) : Lk) : 0;
   const int wave_ntiles = (wave_end + BN - 1) / BN;
 
@@ -353,8 +386,14 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   for (int i = 0; i < VPIECES; i++) voffv[i] = (i * NW + wl) * 1024 + lane * 16;
   const int ktile_bytes = BN * (int)a.k_sn;
   // dw is a multiple of 4, so the rows move by a multiple of 16 and keep their swizzle: only the uniform offset changes.
-  auto load_k = [&](int j, int dw) {
-    uint8_t* dst = kslot(j) + dw * 1024;
+  [[maybe_unused]] const __amdgpu_buffer_rsrc_t mrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)mask_bits, 0, 0x7fffffff, 0x00020000);
+  auto mslot = [&](int j) { return mask_lds + (j % kMaskSlots) * kMaskTileBytes; };
+  auto load_k = [&](int period, int dw) {
+    uint8_t* dst = kslot(period) + dw * 1024;
+    const int j = tile_at(period);
+    // (the mask bits of the tile: four 1 KB pieces, one each for the wavefronts of group 0)
+    if constexpr (LISTED)
+      if (dw == 0) dma16(mrsrc, wl * 1024 + lane * 16, j * kMaskTileBytes, mslot(period) + wl * 1024);
     if (j * BN + BN <= Lk) {
       const int uo = j * ktile_bytes + dw * (64 / CPR) * (int)a.k_sn;
 #pragma unroll
@@ -370,7 +409,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   auto load_v = [&](int j, int dw) {
     uint8_t* dst = vslot(j) + dw * 1024;
 #pragma unroll
-    for (int i = 0; i < VPIECES; i++) dma16(vrsrc, voffv[i], j * VBYTES + dw * 1024, dst + (i * NW + wl) * 1024);
+    for (int i = 0; i < VPIECES; i++) dma16(vrsrc, voffv[i], tile_at(j) * VBYTES + dw * 1024, dst + (i * NW + wl) * 1024);
   };
 
   // The K tiles of the lead are requested before anything waits on memory, and the per-channel V scales of the epilogue
@@ -558,7 +597,8 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   auto subof = [](int r) { return KSUB == 2 ? r / 8 : KSUB == 3 ? (r >> 1) & 1 : 0; };
   auto sci = [&](int nt, int r) { return (SUBS * nt + subof(r)) / GPS; };
   // K scale i of tile j as this lane needs it (before the Q scale is multiplied in)
-  auto kscale_at = [&](int j, int i) -> float {
+  auto kscale_at = [&](int period, int i) -> float {
+    const int j = tile_at(period);
     if constexpr (KSUB == 3) {
       const int blk = min((j * BN + 32 * (i >> 1)) >> a.blkk_shift, nkblk - 1);
       const float lo = ksc[blk * 4 + (i & 1)], hi = ksc[blk * 4 + 2 + (i & 1)];
@@ -609,13 +649,56 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
 
   auto rowmax = [&](int j) {
     const int n0 = j * BN;
+    if constexpr (LISTED) {
+      // Scores as in the explicit-mask variants below, the keep-mask one bit per score: bit 16 * (nt % 2) + r of word
+      // nt / 2 belongs to register r of 32-key group nt (keys past the end have no bit set).
+      const uint2 mb = *reinterpret_cast<const uint2*>(mslot(j) + (w * 32 + m) * 16 + 8 * h);
+      mloc = kNegInf;
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) {
+        int word = (int)(nt < 2 ? mb.x : mb.y);
+        asm volatile("" : "+v"(word));   // one 32-key group after the other: with all of them in flight the scores spill
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int sv = as_i((as_f(acc[nt][r]) - kBiasF) * sc[sci(nt, r)]);
+          const int keep = (word << (31 - 16 * (nt & 1) - r)) >> 31;
+          acc[nt][r] = (sv & keep) | (as_i(kNegInf) & ~keep);
+          mloc = fmaxf(mloc, as_f(acc[nt][r]));
+        }
+      }
+      return;
+    }
     if constexpr (MASK != 0) {
       // Explicit mask: the accumulators become scores (scale applied, bias removed), the mask is
       // applied element by element, and the maximum is taken over floats.
+      // (unit key stride and a whole tile: the four keys of a register quad in one load)
+      typedef unsigned keep4 __attribute__((aligned(1)));
+      typedef float bias4 __attribute__((ext_vector_type(4), aligned(4)));
+      const bool wide = a.m_sn == 1 && n0 + BN <= Lk;
       const int64_t mrow = (int64_t)b * a.m_sb + (int64_t)hq_idx * a.m_sh + (int64_t)min(my_row, Lq - 1) * a.m_sm;
       mloc = kNegInf;
 #pragma unroll
       for (int nt = 0; nt < NT; nt++) {
+        if (wide) {
+#pragma unroll
+          for (int q4 = 0; q4 < 4; q4++) {
+            const int64_t mi = mrow + n0 + 32 * nt + 8 * q4 + 4 * h;
+            unsigned keep = 0;
+            bias4 bias = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (MASK == 1) keep = *reinterpret_cast<const keep4*>(reinterpret_cast<const uint8_t*>(a.mask) + mi);
+            else bias = *reinterpret_cast<const bias4*>(reinterpret_cast<const float*>(a.mask) + mi);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const int r = 4 * q4 + i;
+              float sv = (as_f(acc[nt][r]) - kBiasF) * sc[sci(nt, r)];
+              if constexpr (MASK == 1) sv = (keep >> (8 * i)) & 0xff ? sv : kNegInf;
+              else sv = __builtin_fmaf(bias[i], a.mask_mult, sv);
+              acc[nt][r] = as_i(sv);
+              mloc = fmaxf(mloc, sv);
+            }
+          }
+          continue;
+        }
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int n = n0 + 32 * nt + 8 * (r / 4) + 4 * h + (r % 4);
@@ -910,10 +993,18 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   SAGE_T(3, qreg[0]);   // Q operand ready
   if (ntiles > 0) {
     const int grp = (w >> GSH) & 1;
-    const int wnt = wave_ntiles;
-    auto mfma_phase = [&](int j) {
-      if (j >= 1 && j - 1 < wnt) pv(j - 1);
-      if (j < wnt) { qk(j); rowmax(j); }
+    // does this wavefront work on the tile of period j?
+    auto mine = [&](int j) { return LISTED ? j < ntiles && sees(j) != 0 : j < wave_ntiles; };
+    // (a skipped tile's softmax would have fetched the next tile's K scales)
+    auto skip = [&](int j) { if constexpr (LISTED) load_scales(j + 1); };
+    bool on_prev = false;
+    auto worked = [&](int j) { return LISTED ? on_prev : j >= 1 && j - 1 < wave_ntiles; };   // ... and on that of period j - 1?
+    // (the scores of a skipped tile hold nothing: said so, they need no registers across the period)
+    auto forget_scores = [&]() {
+      if constexpr (LISTED) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) asm volatile("" : "=v"(acc[nt]));
+      }
     };
     load_scales(0);
     auto even_barrier = [&](int j, int in_flight) {
@@ -923,9 +1014,9 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       if (j == 0) sage_ts[4] = __builtin_amdgcn_s_memrealtime();   // first K tile landed, all wavefronts arrived
 #endif
     };
-    const int first_in_flight = (LEAD == 2 && ntiles > 1) ? KPIECES : 0;   // the second K tile, requested in the prologue
+    const int first_in_flight = (LEAD == 2 && ntiles > 1) ? KPIECES + (LISTED && w < PARTNER_DW) : 0;   // the second K tile, requested in the prologue
     constexpr int PARTNER = PARTNER_DW;
-    constexpr int NK = 2 * KPIECES, NV = 2 * VPIECES;   // requests per K / V tile of the wavefront that issues for its SIMD pair
+    constexpr int NK = 2 * KPIECES + LISTED, NV = 2 * VPIECES;   // requests per K / V tile of the wavefront that issues for its SIMD pair
     // Tile requests of period j, issued by one wavefront for both wavefronts of its SIMD pair: K(j+LEAD) and
     // V(j+LEAD-1), LEAD periods before their first use (a tile that has to come from HBM takes longer than one
     // period), into the slots whose last readers finished a barrier ago; with LEAD = 2, V(0) goes first in
@@ -973,13 +1064,16 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
           even_barrier(j, issuer_in_flight(j));
           SAGE_PH(0);
           if (LEAD == 2 && j == 0) first_value_tile();   // V(0) has one period only: ahead of the first Q.K^T, not after it
-          if (j >= 1 && j - 1 < wnt) pv(j - 1);
-          if (j < wnt) qk(j);
+          const bool on = mine(j);
+          if (worked(j)) pv(j - 1);
+          if (on) qk(j);
+          else forget_scores();
           request_tiles(j, false);
           SAGE_PH(1);
           odd_barrier();
           SAGE_PH(2);
-          if (j < wnt) { rowmax(j); softmax(j); }
+          if (on) { rowmax(j); softmax(j); } else skip(j);
+          on_prev = on;
         }
       } else {
         for (int j = 0; j <= ntiles; j++) {
@@ -988,13 +1082,16 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
           even_barrier(j, j == 0 ? first_in_flight : (V_BY_GROUP1 && j < ntiles ? NV : 0));
           SAGE_PH(0);
           if (V_BY_GROUP1 && j + 1 < ntiles) { load_v(j + 1, 0); load_v(j + 1, PARTNER); }
-          if (j >= 1 && j - 1 < wnt) { rowmax(j - 1); softmax(j - 1); }
+          const bool on = mine(j);
+          if (worked(j)) { rowmax(j - 1); softmax(j - 1); } else if (j >= 1) skip(j - 1);
           SAGE_PH(1);
           odd_barrier();
           SAGE_PH(2);
           if (SPLIT_REQ && j < ntiles) load_v(j, PARTNER);   // V(j) of the pair's second wavefront: LEAD is 1 here
-          if (j >= 1 && j - 1 < wnt) pv(j - 1);
-          if (j < wnt) qk(j);
+          if (worked(j)) pv(j - 1);
+          if (on) qk(j);
+          else forget_scores();
+          on_prev = on;
         }
       }
     } else if (grp == 0) {
@@ -1002,18 +1099,27 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       // the period are issued here, by the group whose matrix phase has slack, after its P.V.
       for (int j = 0; j <= ntiles; j++) {
         even_barrier(j, issuer_in_flight(j));
-        if (j >= 1 && j - 1 < wnt) pv(j - 1);
+        const bool on = mine(j);
+        if (worked(j)) pv(j - 1);
         request_tiles(j);
-        if (j < wnt) { qk(j); rowmax(j); }
+        if (on) { qk(j); rowmax(j); }
+        else forget_scores();
         lds_barrier();
-        if (j < wnt) softmax(j);
+        if (on) softmax(j);
+        else skip(j);
+        on_prev = on;
       }
     } else {
       for (int j = 0; j <= ntiles; j++) {
         even_barrier(j, j == 0 ? first_in_flight : 0);
-        if (j >= 1 && j - 1 < wnt) softmax(j - 1);
+        const bool on = mine(j);
+        if (worked(j)) softmax(j - 1);
+        else if (j >= 1) skip(j - 1);
         lds_barrier();
-        mfma_phase(j);
+        if (worked(j)) pv(j - 1);
+        if (on) { qk(j); rowmax(j); }
+        else forget_scores();
+        on_prev = on;
       }
     }
   }
@@ -1120,7 +1226,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
 
 template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1>
 static hipError_t launch_one(const AttnArgs& a, int grid, hipStream_t st) {
-  constexpr int smem = attn_lds_bytes<D, NW, BN, PV, CAUSAL, QF>();
+  constexpr int smem = attn_lds_bytes<D, NW, BN, PV, CAUSAL, QF, MASK>();
   auto kern = attn_kernel<D, NW, BN, PV, CAUSAL, MSUM, MASK, KSUB, QF, KW>;
   // More than 64 KB of dynamic LDS has to be allowed once per kernel and device.
   constexpr int kMaxDevices = 64;

@@ -71,6 +71,36 @@ __host__ __device__ inline SagePlanLayout plan_layout(int nseq, int total_q) {
 }
 
 // ---------------------------------------------------------------------------------------------
+// Packed boolean mask: one bit per (query row, key), in the order in which the attention kernel's accumulators hold the
+// scores, and one visibility class per 32 query rows and key tile.
+//   bits: [plane][q-tile of 256 rows][tile of 128 keys][row][h = 0, 1] -> 64 bits; bit 16 * nt + r is key
+//         32 * nt + 8 * (r / 4) + 4 * h + r % 4 of the tile (0 past the last key and in rows past the last one)
+//   classes: uint16 [plane][q-tile][tile], two bits per group of 32 rows: 0 no key visible, 1 some, 2 all of them
+// A plane is one distinct [Sq, Skv] slice of the mask (broadcast batches and heads share one); a mask that is the same
+// for every query row has one q-tile, whatever Sq is.
+// ---------------------------------------------------------------------------------------------
+constexpr int kMaskRows = 256, kMaskKeys = 128, kMaskTileBytes = kMaskRows * kMaskKeys / 8;
+constexpr int kMaskMaxTiles = 2048;   // key tiles the attention kernel's tile list has room for
+struct MaskPlanes {
+  int planes, nqt, ntk;   // distinct slices, q-tiles and key tiles of each
+  int pb, ph;             // plane of (batch b, head h) = b * pb + h * ph
+  int64_t bits_bytes, total_bytes;
+};
+inline MaskPlanes mask_planes(int B, int Hq, int Sq, int Skv, int64_t m_sb, int64_t m_sh, int64_t m_sm) {
+  MaskPlanes p;
+  const int heads = m_sh ? Hq : 1;
+  p.planes = (m_sb ? B : 1) * heads;
+  p.pb = m_sb ? heads : 0;
+  p.ph = m_sh ? 1 : 0;
+  p.nqt = m_sm ? (Sq + kMaskRows - 1) / kMaskRows : 1;
+  p.ntk = (Skv + kMaskKeys - 1) / kMaskKeys;
+  const int64_t tiles = (int64_t)p.planes * p.nqt * p.ntk;
+  p.bits_bytes = tiles * kMaskTileBytes;
+  p.total_bytes = p.bits_bytes + (tiles * 2 + 255) / 256 * 256;
+  return p;
+}
+
+// ---------------------------------------------------------------------------------------------
 // dtype helpers (bf16 handled as raw bits: widening is a shift, narrowing is RNE).
 // ---------------------------------------------------------------------------------------------
 __device__ inline float bf16_to_f32(u16 v) { return __builtin_bit_cast(float, (uint32_t)v << 16); }

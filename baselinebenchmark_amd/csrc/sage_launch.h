@@ -104,6 +104,9 @@ struct AttnArgs {
   const void* mask;
   int mask_kind;
   int64_t m_sb, m_sh, m_sm, m_sn;
+  const uint8_t* mask_bits; // packed boolean mask (sage_common.h) or null: taken instead of `mask`
+  const u16* mask_cls;
+  int mask_pb, mask_ph, mask_nqt, mask_ntk;
   float mask_mult;          // additive masks are scaled by this before they are added
   const float* lse_offset;  // added to LSE2 per query row (same layout as lse) or null
   // fused Q quantisation: fp16/bf16 Q with the strides of q (q and qs are then unused)
@@ -124,11 +127,16 @@ hipError_t launch_prep_v(const PrepVArgs& a, int dtype, int pv, int max_panels, 
 hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dtype, int pv, int nk, int nv, int smooth,
                                 void* km_out, float* vscale_out, hipStream_t st);
 
+// Packs a boolean mask [B, Hq, Sq, Skv] with element strides into the form of sage_common.h.
+hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,
+                            int Skv, uint8_t* bits, u16* cls, hipStream_t st);
+
 AttnConfig attn_config(int D, int pv, bool packed);
 // Fills in the launch constants of the tile decode from the dimensions already in `a` (B, Hq, Hkv, nqt, cu_q).
 void finish_attn_args(AttnArgs& a, bool causal);
 hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_masked(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
+hipError_t launch_attn_packed_mask(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_qfused(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_k16(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_kinterleaved(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);

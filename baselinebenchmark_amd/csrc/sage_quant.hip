@@ -474,6 +474,60 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
 }
 
 // ---------------------------------------------------------------------------------------------
+// Boolean mask -> bits and visibility classes (layout in sage_common.h).  One workgroup per (key tile, q-tile, plane): the
+// mask's bytes are read once, 16 per lane and eight lanes per row where keys are contiguous, and leave as one bit each.
+// ---------------------------------------------------------------------------------------------
+__device__ inline unsigned nonzero_bytes(unsigned x) {   // bit i: byte i of x is not zero
+  const unsigned t = ((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) >> 7) & 0x01010101u;
+  return (t * 0x10204080u) >> 28;
+}
+
+__global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn,
+                                                        MaskPlanes p, int Sq, int Skv, uint8_t* bits, u16* cls) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4), aligned(1)));
+  __shared__ __align__(16) uint8_t packed[kMaskTileBytes];
+  __shared__ unsigned wave_cls[4];
+  const int tile = blockIdx.x, qt = blockIdx.y, tid = threadIdx.x;
+  const int heads = p.ph ? (p.pb ? p.pb : p.planes) : 1;   // planes of one batch entry
+  const int b = blockIdx.z / heads, hd = blockIdx.z - b * heads;
+  const uint8_t* base = mask + (int64_t)b * m_sb + (int64_t)hd * m_sh;
+  const int rows = m_sm ? min(kMaskRows, Sq - qt * kMaskRows) : kMaskRows;   // (rows that all read the same row are all valid)
+  const int c = tid & 7, k0 = tile * kMaskKeys + 16 * c;   // this lane's 16 keys of the rows tid / 8 + 32 * i
+  const bool wide = m_sn == 1 && k0 + 16 <= Skv;
+#pragma unroll
+  for (int i = 0; i < kMaskRows / 32; i++) {
+    const int r = tid / 8 + 32 * i;
+    unsigned x[4] = {0, 0, 0, 0};   // 16 keys as 4 x 4 bytes
+    if (r < rows && k0 < Skv) {
+      const uint8_t* src = base + (int64_t)(qt * kMaskRows + r) * m_sm + (int64_t)k0 * m_sn;
+      if (wide) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(src);
+        x[0] = v[0]; x[1] = v[1]; x[2] = v[2]; x[3] = v[3];
+      } else {
+        for (int e = 0; e < 16; e++)
+          if (k0 + e < Skv && src[e * m_sn]) x[e >> 2] |= 1u << (8 * (e & 3));
+      }
+    }
+    // keys 0-3 and 8-11 belong to lane half 0, the others to lane half 1
+    packed[r * 16 + c] = (uint8_t)(nonzero_bytes(x[0]) | (nonzero_bytes(x[2]) << 4));
+    packed[r * 16 + 8 + c] = (uint8_t)(nonzero_bytes(x[1]) | (nonzero_bytes(x[3]) << 4));
+  }
+  __syncthreads();
+  const uint4 row = reinterpret_cast<const uint4*>(packed)[tid];
+  const int64_t t = ((int64_t)blockIdx.z * p.nqt + qt) * p.ntk + tile;
+  reinterpret_cast<uint4*>(bits + t * kMaskTileBytes)[tid] = row;
+  const unsigned long long any = __builtin_amdgcn_ballot_w64((row.x | row.y | row.z | row.w) != 0);
+  const unsigned long long gap = __builtin_amdgcn_ballot_w64(tid < rows && (row.x & row.y & row.z & row.w) != 0xffffffffu);
+  if ((tid & 63) == 0) {
+    const unsigned lo = (unsigned)any == 0 ? 0 : (unsigned)gap == 0 ? 2 : 1;
+    const unsigned hi = (any >> 32) == 0 ? 0 : (gap >> 32) == 0 ? 2 : 1;
+    wave_cls[tid >> 6] = (lo | (hi << 2)) << (4 * (tid >> 6));
+  }
+  __syncthreads();
+  if (tid == 0) cls[t] = (u16)(wave_cls[0] | wave_cls[1] | wave_cls[2] | wave_cls[3]);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Host-side launchers (called from the C ABI in sage_api.hip).
 // ---------------------------------------------------------------------------------------------
 hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_blocks, hipStream_t st) {
@@ -482,6 +536,12 @@ hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_blocks, hipS
   else if (dtype == 0 && a.D == 128) quant_int8_kernel<0, 128><<<grid, block, 0, st>>>(a);
   else if (dtype == 1 && a.D == 64) quant_int8_kernel<1, 64><<<grid, block, 0, st>>>(a);
   else quant_int8_kernel<1, 128><<<grid, block, 0, st>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,
+                            int Skv, uint8_t* bits, u16* cls, hipStream_t st) {
+  mask_pack_kernel<<<dim3(p.ntk, p.nqt, p.planes), dim3(256), 0, st>>>(mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, cls);
   return hipGetLastError();
 }
 

@@ -429,11 +429,13 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
     lse = torch.empty((B, Hq, Sq), device=q.device, dtype=torch.float32) if return_lse else None
     ws_bytes = lib().sage_sageattn_workspace_bytes_for(B, Hq, Hkv, Sq, Skv, D, BLKQ | qflag, BLKK | kflag, pv, 0, 0, 0,
                                                        int(bool(smooth_k)), int(bool(return_lse)), int(attn_mask is not None))
-    ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
     if attn_mask is not None:
         if is_causal:
             raise NotImplementedError("attn_mask cannot be combined with is_causal")
         m, kind, ms = _mask_args(attn_mask, B, Hq, Sq, Skv, q.device)
+        ws_bytes += lib().sage_sageattn_mask_bytes(B, Hq, Sq, Skv, kind, ms[0], ms[1], ms[2])
+    ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
+    if attn_mask is not None:
         check(lib().sage_sageattn_masked(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(ws), ws_bytes,
                                          B, Hq, Hkv, Sq, Skv, D, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
                                          _dt(q.dtype), BLKQ | qflag, BLKK | kflag, float(D ** -0.5 if sm_scale is None else sm_scale),

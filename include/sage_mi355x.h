@@ -264,7 +264,11 @@ int sage_sageattn(const void* q, const void* k, const void* v, void* out, float*
  * softmax(sm_scale * q.k^T + mask) at :171-178: here the additive mask is in NATURAL-log units on top
  * of sm_scale * q.k^T (it is multiplied by log2(e) internally); boolean masks as in
  * sage_attn_fwd_masked.  attn_mask == NULL makes it identical to sage_sageattn.
+ * A workspace that is larger than sage_sageattn_workspace_bytes_for by sage_sageattn_mask_bytes lets the call pack a boolean
+ * mask into bits first (one per row and key, for each distinct slice of the mask): the attention then skips the key tiles
+ * that no row of a q-tile sees.  Same results, bit for bit; 0 = nothing to gain (additive masks, more than 262144 keys).
  */
+size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, int64_t m_sb, int64_t m_sh, int64_t m_sm);
 int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out, float* lse,
                          void* workspace, size_t workspace_bytes,
                          int B, int Hq, int Hkv, int Sq, int Skv, int D,

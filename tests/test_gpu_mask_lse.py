@@ -219,3 +219,51 @@ def test_sageattn_lse_correction_causal_gqa_nhd_bf16():
     assert (lse.cpu().double() - torch.logsumexp(scores, dim=-1)).abs().max().item() < 1e-1
     ref = oa.sdpa_fp32(q, k, v, "NHD", True)
     assert oa.metrics(out.cpu().float(), ref)["cosine"] >= 0.999
+
+
+def _direct_masked_call(q, k, v, mask, layout, pv, blkq, blkk, out, lse, extra):
+    """sage_sageattn_masked with exactly the workspace that the call needs (``extra`` more bytes): with none the mask is read
+    where it lies, by the variants that take any strides."""
+    import ctypes
+    from baselinebenchmark_amd import _cabi
+    lib = _cabi.lib()
+    lay = (lambda t: (*t.shape, *t.stride()[:3])) if layout == "HND" else (lambda t: (t.shape[0], t.shape[2], t.shape[1], t.shape[3], t.stride(0), t.stride(2), t.stride(1)))
+    B, Hq, Sq, D, *qst = lay(q)
+    _, Hkv, Skv, _, *kst = lay(k)
+    pvm = _cabi.PV_FP8 if pv == "fp8" else _cabi.PV_FP16
+    need = lib.sage_sageattn_workspace_bytes_for(B, Hq, Hkv, Sq, Skv, D, blkq, blkk, pvm, 0, 0, 0, 1, 1, 1) + extra
+    ws = torch.empty(need, device=q.device, dtype=torch.uint8)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    m = mask.expand(B, Hq, Sq, Skv)
+    return lib.sage_sageattn_masked(P(q), P(k), P(v), P(out), P(lse), P(ws), need, B, Hq, Hkv, Sq, Skv, D, *qst, *kst, *lay(v)[4:],
+                                    *lay(out)[4:], _cabi.DT_BF16 if q.dtype == torch.bfloat16 else _cabi.DT_F16, blkq, blkk, D ** -0.5, 0, 1, pvm,
+                                    None, None, 0, 0, P(m), 1, *m.stride(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+
+# sizes around the edges of the 256-row q-tile, the 32-row group and the 128-key tile; strides of every kind
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("kind", ["per_head", "documents", "padding", "last_key_only", "nothing", "everything", "transposed", "every_other_key"])
+@pytest.mark.parametrize("shape", [(2, 4, 2, 257, 385, 64, 64), (1, 2, 2, 513, 128, 128, 16), (3, 2, 1, 31, 1029, 128, 128), (1, 1, 1, 1, 1, 64, 32)])
+def test_packed_boolean_mask_equals_the_mask_read_in_place(shape, kind, pv):
+    B, Hq, Hkv, Sq, Skv, D, blkk = shape
+    g = torch.Generator().manual_seed(5 + Sq + Skv)
+    q, k, v = (randn("HND", B, h, n, D, torch.float16, g).to(DEV) for h, n in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    if kind == "per_head":
+        mask = (torch.rand((B, Hq, Sq, Skv), generator=g) > 0.7).to(DEV)
+    elif kind == "documents":
+        mask = ((torch.arange(Sq)[:, None] // 100) == (torch.arange(Skv)[None] // 100))[None, None].expand(B, 1, Sq, Skv).contiguous().to(DEV)
+    elif kind == "padding":
+        mask = (torch.arange(Skv)[None] < torch.tensor([Skv - 7 * i for i in range(B)])[:, None])[:, None, None].to(DEV)
+    elif kind == "last_key_only":
+        mask = (torch.arange(Skv) == Skv - 1)[None, None, None].to(DEV)
+    elif kind == "transposed":
+        mask = (torch.rand((B, 1, Skv, Sq), generator=g) > 0.5).to(DEV).transpose(-1, -2)
+    elif kind == "every_other_key":
+        mask = (torch.rand((1, Hq, Sq, 2 * Skv), generator=g) > 0.5).to(DEV)[..., ::2]
+    else:
+        mask = torch.full((1, 1, Sq, Skv), kind == "everything", device=DEV)
+    out, lse = sa.sageattn(q, k, v, attn_mask=mask, pv_mode=pv, BLKK=blkk, return_lse=True)
+    want, want_lse = torch.empty_like(out), torch.empty_like(lse)
+    assert _direct_masked_call(q, k, v, mask, "HND", pv, 128, blkk, want, want_lse, 0) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(lse, want_lse * 0.6931471805599453)
