@@ -413,6 +413,16 @@ size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, i
   return mask_can_be_packed(p, Sq, Skv, mask_kind) ? (size_t)p.total_bytes : 0;
 }
 
+// Few query rows per KV head over keys that do not fit the one-launch pre-pass: sage_attn_few.hip.  Calls that the general
+// path refuses, slices of 2 GiB and more (32-bit row offsets) and rows that overlap are left to that path.
+static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, int64_t rows, int Sq, int Skv, int D,
+                          int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
+  const int64_t limit = 0x7fffffff;
+  return !varlen && !short_keys && !is_causal && !mask && pv_mode == SAGE_PV_FP16 && rows <= kFewRows && blk_groups(blkq) == 1 &&
+         blk_groups(blkk) == 1 && q && k && v && out && k_sn >= D && v_sn >= D && (int64_t)Sq * q_sn * 2 < limit &&
+         ((int64_t)Skv + 128) * k_sn * 2 < limit && ((int64_t)Skv + 128) * v_sn * 2 < limit;
+}
+
 int sage_sageattn(const void* q, const void* k, const void* v, void* out, float* lse, void* workspace, size_t workspace_bytes,
                   int B, int Hq, int Hkv, int Sq, int Skv, int D, int64_t q_sb, int64_t q_sh, int64_t q_sn, int64_t k_sb,
                   int64_t k_sh, int64_t k_sn, int64_t v_sb, int64_t v_sh, int64_t v_sn, int64_t o_sb, int64_t o_sh,
@@ -486,6 +496,29 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   const int64_t rereads = (Skv + blk_rows(blkk) - 1) / blk_rows(blkk) + (Skv + kPanelRows - 1) / kPanelRows;
   const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && k_elements <= kSmallPrepassElements &&
                              k_elements * rereads <= kSmallPrepassReads;
+  const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
+  if (few_rows_path(varlen, no_keys || small_prepass, is_causal, attn_mask, pv_mode, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
+                    out, q_sn, k_sn, v_sn)) {
+    if (int rc2 = check_stride16("q", q_sb, q_sh, q_sn, 2, q)) return rc2;
+    if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;
+    if (int rc2 = check_stride16("v", v_sb, v_sh, v_sn, 2, v)) return rc2;
+    if (int rc2 = check_stride16("out", o_sb, o_sh, o_sn, 2, out)) return rc2;
+    if (smooth_k) {
+      rc = sage_k_mean(k, km, stat, stat_bytes, B, Hkv, Skv, D, k_sb, k_sh, k_sn, dtype, nullptr, stream);
+      if (rc) return rc;
+    }
+    FewArgs f;
+    memset(&f, 0, sizeof(f));
+    f.q = (const u16*)q; f.k = (const u16*)k; f.v = (const u16*)v; f.km = smooth_k ? (const u16*)km : nullptr;
+    f.out = (u16*)out; f.lse = lse; f.part = (float*)panels;   // (no panels here: their region holds the partial results)
+    f.B = B; f.Hq = Hq; f.Hkv = Hkv; f.Sq = Sq; f.Skv = Skv;
+    f.q_sb = q_sb; f.q_sh = q_sh; f.q_sn = q_sn; f.k_sb = k_sb; f.k_sh = k_sh; f.k_sn = k_sn;
+    f.v_sb = v_sb; f.v_sh = v_sh; f.v_sn = v_sn; f.o_sb = o_sb; f.o_sh = o_sh; f.o_sn = o_sn;
+    f.blkq_shift = ilog2(blkq); f.blkk_shift = ilog2(blkk); f.q_mult = q_mult;
+    hipError_t e = launch_attn_few(f, dtype, D, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "sage_sageattn(few rows)");
+    return SAGE_OK;
+  }
   if (small_prepass) {
     if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;
     if (int rc2 = check_stride16("v", v_sb, v_sh, v_sn, 2, v)) return rc2;
@@ -524,7 +557,6 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   }
   // Q is quantised by the attention kernel itself (each q-tile exactly where it is consumed) unless a
   // feature needs the standalone pass: an explicit mask or the LSE correction.
-  const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
   const bool fuse_q = !attn_mask && !lse_off && blk_groups(blkq) == 1;   // (interleaved scales: standalone pass too)
   if (!fuse_q) {
     rc = quant_impl(q, q_i8, q_scale, nullptr, B, Hq, Sq, D, q_sb, q_sh, q_sn, qi_sb, qi_sh, qi_sn, 0, 0, blkq, q_mult, dtype,

@@ -1,0 +1,377 @@
+// Attention of a few query rows over a long history (token generation): FP16 P.V, no mask, at most kFewRows rows per KV head
+// counting all query heads that share it.
+//
+// Bound by the bytes of K and V.  The tiled kernel gives a q-tile of 256 rows to every query head, so one row per head leaves
+// 1/256 of its matrix work useful, puts B * Hq workgroups on 256 compute units and walks the whole history in each; in
+// front of it K is written as an INT8 copy and V as panels, and both are read back by every query head.  Here
+//   * the rows of the query heads of a KV head are the columns of one 16x16 tile (two above 16 rows), so K and V are read once
+//     per KV head, from the caller's tensors: K is smoothed and quantised in registers with the quantiser's own arithmetic,
+//     V is converted in registers, nothing is written back;
+//   * the keys are cut into `nsplit` ranges of whole 128-key tiles, one workgroup each, so that a few (batch, KV head) pairs
+//     fill the chip; a second small kernel merges the ranges' (O, m, l);
+//   * a wavefront owns 32 keys of a tile, so nothing but the maximum of scale blocks of 64 and 128 keys crosses wavefronts.
+// The order of the channels inside the Q.K^T contraction and of the keys inside the P.V one is free as long as both operands
+// agree: K fragments take the channels as whole 64-byte pieces of a row arrive, V fragments the keys as the 16x16 score tile
+// holds them, so neither the scores nor V go through LDS.
+// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 52.4 us
+// (this kernel 34 us = 3.9 TB/s of K and V, half of it vector arithmetic of the quantisation; K mean 15, merge 4); 8 rows: 170.8
+// -> 58.5; 8 x 32/8 heads, 4 rows, 16384 keys: 431.9 -> 158.9; 16 x 24 heads, 4096 keys: 452.4 -> 223.8; 1 x 2 heads, 32768
+// keys: 435.3 -> 53.2; 1 x 8/2 heads, 2048 keys: 47.1 -> 33.7.
+#include "sage_launch.h"
+
+#pragma clang fp contract(off)
+
+namespace sage {
+namespace {
+
+constexpr float kNegInfFew = -__builtin_inff();
+constexpr float kMInitFew = -1.0e30f;
+constexpr float kTauFew = 8.0f;   // the running maximum moves when it grew by more than this: probabilities stay below 2^8
+
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+
+__device__ inline float xor16_32_max(float x) {
+  x = fmaxf(x, __shfl_xor(x, 16));
+  return fmaxf(x, __shfl_xor(x, 32));
+}
+__device__ inline float xor16_32_sum(float x) {
+  x += __shfl_xor(x, 16);
+  return x + __shfl_xor(x, 32);
+}
+
+// q = trunc(x / scale + 0.5 sgn(x)) of sixteen values, as quant_int8_kernel computes it.
+template <class Quotient>
+__device__ __forceinline__ v4i pack16(const float (&x)[16], Quotient quotient) {
+  uint32_t packed[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    float z = quotient(x[i]);
+    z = z + __builtin_copysignf(0.5f, z);
+    packed[i >> 2] |= (uint32_t)((int)z & 0xff) << (8 * (i & 3));
+  }
+  return v4i{(int)packed[0], (int)packed[1], (int)packed[2], (int)packed[3]};
+}
+
+// True where the reciprocal with one correction step is the correctly rounded quotient (div_by_uniform).
+__device__ inline bool reciprocal_is_exact(float scale) {
+  return (__builtin_bit_cast(uint32_t, scale) & 0x7fffffu) != 0x7fffffu && scale < 1.0e30f;
+}
+
+template <int DT, int D, int MT>
+__global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
+  constexpr int LK = D / 32;   // 16-byte pieces of a K row per lane: piece i holds the channels 32 i + 8 (lane / 16) ..+7
+  constexpr int KS = D / 64;   // contraction steps of Q.K^T
+  constexpr int CV = D / 16;   // channels of V per lane
+  constexpr int LDO = D + 4;   // floats per row of the merge buffer
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int split = blockIdx.x, bh = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv;
+  const int G = a.Hq / a.Hkv, rows = G * a.Sq, L = a.Skv;
+  __shared__ float row_amax[16 * MT];
+  __shared__ float block_amax[2][4];
+  __shared__ float wave_m[4][16 * MT], wave_l[4][16 * MT];
+  __shared__ __align__(16) float merged[16 * MT * LDO];
+
+  // K and V through bounded buffers: rows past the end read as zeros
+  const __amdgpu_buffer_rsrc_t krsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(a.k + (int64_t)b * a.k_sb + (int64_t)kvh * a.k_sh), 0,
+                                                                         ((L - 1) * (int)a.k_sn + D) * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(a.v + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_sh), 0,
+                                                                         ((L - 1) * (int)a.v_sn + D) * 2, 0x00020000);
+  const int ntiles = (L + 127) >> 7;
+  const int t0 = split * a.tiles_per_split, t1 = min(ntiles, t0 + a.tiles_per_split);
+  v4u kraw[2][LK];
+  auto load_k = [&](int tile) {
+    const int off = ((tile * 128 + 32 * w + m) * (int)a.k_sn + 8 * g) * 2;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int i = 0; i < LK; i++) kraw[t][i] = __builtin_amdgcn_raw_buffer_load_b128(krsrc, off + t * 16 * (int)a.k_sn * 2 + 64 * i, 0, 0);
+  };
+  if (t0 < t1) load_k(t0);
+
+  float kmf[LK][8];
+  if (a.km) {
+    const u16* kp = a.km + ((int64_t)b * a.Hkv + kvh) * D + 8 * g;
+#pragma unroll
+    for (int i = 0; i < LK; i++) {
+      const v4u raw = *reinterpret_cast<const v4u*>(kp + 32 * i);
+#pragma unroll
+      for (int e = 0; e < 8; e++) kmf[i][e] = to_f32<DT>((u16)(raw[e >> 1] >> (16 * (e & 1))));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < LK; i++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) kmf[i][e] = 0.f;
+  }
+
+  // ---- Q: row r of the tile is query row r % Sq of the group's head r / Sq; a scale per BLKQ rows of a head ----
+  v4i qreg[MT][KS];
+  float qscale[MT], dot[MT];
+  {
+    float x[MT][KS][16];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
+      const u16* qp = a.q + (int64_t)b * a.q_sb + (int64_t)(kvh * G + head) * a.q_sh + (int64_t)s * a.q_sn + 8 * g;
+      float amax = 0.f, sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < LK; i++) {
+        const v4u raw = *reinterpret_cast<const v4u*>(qp + 32 * i);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float v = to_f32<DT>((u16)(raw[e >> 1] >> (16 * (e & 1)))) * a.q_mult;
+          x[mt][i >> 1][8 * (i & 1) + e] = v;
+          amax = fmaxf(amax, fabsf(v));
+          sum = __builtin_fmaf(v, kmf[i][e], sum);
+        }
+      }
+      amax = xor16_32_max(amax);
+      dot[mt] = xor16_32_sum(sum);   // what K smoothing takes from every logit of the row
+      if (w == 0 && g == 0) row_amax[16 * mt + m] = amax;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
+      const int s0 = s >> a.blkq_shift << a.blkq_shift, s1 = min(a.Sq, s0 + (1 << a.blkq_shift));
+      float amax = 0.f;
+      for (int i = s0; i < s1; i++) amax = fmaxf(amax, row_amax[head * a.Sq + i]);
+      const float scale = fmaxf(amax / 127.0f, kScaleFloor), rcp = 1.0f / scale;
+      qscale[mt] = scale;
+      if (__builtin_amdgcn_ballot_w64(!reciprocal_is_exact(scale)) == 0) {
+#pragma unroll
+        for (int s = 0; s < KS; s++) qreg[mt][s] = pack16(x[mt][s], [&](float v) { return div_by_uniform(v, scale, rcp); });
+      } else {
+#pragma unroll
+        for (int s = 0; s < KS; s++) qreg[mt][s] = pack16(x[mt][s], [&](float v) { return v / scale; });
+      }
+    }
+  }
+
+  v4f o[MT][CV];
+  float m_used[MT], lsum[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    m_used[mt] = kMInitFew;
+    lsum[mt] = 0.f;
+#pragma unroll
+    for (int i = 0; i < CV; i++) o[mt][i] = v4f{0.f, 0.f, 0.f, 0.f};
+  }
+
+  for (int tile = t0; tile < t1; tile++) {
+    const int n0 = tile * 128 + 32 * w;
+    // V rows 16 t + 4 g + r of the 32 keys, CV channels each: the keys whose scores this lane will hold
+    uint32_t vraw[2][4][CV / 2];
+    {
+      const int off = ((n0 + 4 * g) * (int)a.v_sn + CV * m) * 2;
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int at = off + (16 * t + r) * (int)a.v_sn * 2;
+          if constexpr (D == 128) {
+            const v4u x = __builtin_amdgcn_raw_buffer_load_b128(vrsrc, at, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) vraw[t][r][i] = x[i];
+          } else {
+            const v2u x = __builtin_amdgcn_raw_buffer_load_b64(vrsrc, at, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 2; i++) vraw[t][r][i] = x[i];
+          }
+        }
+    }
+    // ---- K: subtract the mean in the input type, block maxima, quantise ----
+    float amax[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const bool gone = n0 + 16 * t + m >= L;
+      float mx = 0.f;
+#pragma unroll
+      for (int i = 0; i < LK; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t x = kraw[t][i][e];
+          const u16 lo = from_f32<DT>(to_f32<DT>((u16)x) - kmf[i][2 * e]), hi = from_f32<DT>(to_f32<DT>((u16)(x >> 16)) - kmf[i][2 * e + 1]);
+          kraw[t][i][e] = gone ? 0u : (uint32_t)lo | ((uint32_t)hi << 16);
+          mx = fmaxf(mx, fmaxf(fabsf(to_f32<DT>(lo)), fabsf(to_f32<DT>(hi))));
+        }
+      amax[t] = wave_max(gone ? 0.f : mx);
+    }
+    if (a.blkk_shift >= 5) amax[0] = amax[1] = fmaxf(amax[0], amax[1]);
+    if (a.blkk_shift >= 6) {
+      // (two sets in turn: a wavefront writes the next tile's while a slower one still reads this tile's)
+      if (lane == 0) block_amax[tile & 1][w] = amax[0];
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (loads in flight stay in flight)
+      const float* p = block_amax[tile & 1];
+      const float pair = fmaxf(p[w & ~1], p[w | 1]);
+      amax[0] = amax[1] = a.blkk_shift == 6 ? pair : fmaxf(pair, fmaxf(p[(w & ~1) ^ 2], p[(w | 1) ^ 2]));
+    }
+    float kscale[2];
+    v4i kreg[2][KS];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const float scale = fmaxf(amax[t] / 127.0f, kScaleFloor), rcp = 1.0f / scale;
+      kscale[t] = scale;
+      const bool fast = __builtin_amdgcn_ballot_w64(!reciprocal_is_exact(scale)) == 0;
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        float x[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) x[e] = to_f32<DT>((u16)(kraw[t][2 * s + (e >> 3)][(e & 7) >> 1] >> (16 * (e & 1))));
+        if (fast) kreg[t][s] = pack16(x, [&](float v) { return div_by_uniform(v, scale, rcp); });
+        else kreg[t][s] = pack16(x, [&](float v) { return v / scale; });
+      }
+    }
+    if (tile + 1 < t1) load_k(tile + 1);
+
+    // ---- scores (lane: query row m, keys 16 t + 4 g + r), probabilities ----
+    v8h p[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      float sv[8], mx = kNegInfFew;
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        v4i acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < KS; s++) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kreg[t][s], qreg[mt][s], acc, 0, 0, 0);
+        const float sc = qscale[mt] * kscale[t];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float v = (float)acc[r] * sc;
+          sv[4 * t + r] = n0 + 16 * t + 4 * g + r < L ? v : kNegInfFew;
+          mx = fmaxf(mx, sv[4 * t + r]);
+        }
+      }
+      mx = xor16_32_max(mx);
+      if (__builtin_amdgcn_ballot_w64(mx > m_used[mt] + kTauFew) != 0) {
+        const float m_new = fmaxf(m_used[mt], mx), alpha = __builtin_amdgcn_exp2f(m_used[mt] - m_new);
+        lsum[mt] *= alpha;
+#pragma unroll
+        for (int i = 0; i < CV; i++) o[mt][i] *= alpha;
+        m_used[mt] = m_new;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float e = __builtin_amdgcn_exp2f(sv[j] - m_used[mt]);
+        lsum[mt] += e;
+        p[mt][j] = (_Float16)e;
+      }
+    }
+    // ---- O^T += V^T . P^T: matrix row c of product i is channel CV c + i ----
+#pragma unroll
+    for (int i = 0; i < CV; i++) {
+      v8h vf;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const u16 bits = (u16)(vraw[j >> 2][j & 3][i >> 1] >> (16 * (i & 1)));
+        vf[j] = DT == 0 ? __builtin_bit_cast(_Float16, bits) : (_Float16)bf16_to_f32(bits);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) o[mt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[mt], o[mt][i], 0, 0, 0);
+    }
+  }
+
+  // ---- the four wavefronts' parts into one, in their order ----
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    lsum[mt] = xor16_32_sum(lsum[mt]);
+    if (g == 0) {
+      wave_m[w][16 * mt + m] = m_used[mt];
+      wave_l[w][16 * mt + m] = lsum[mt];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    const int r = 16 * mt + m;
+    const float top = fmaxf(fmaxf(wave_m[0][r], wave_m[1][r]), fmaxf(wave_m[2][r], wave_m[3][r]));
+    const float f = __builtin_amdgcn_exp2f(m_used[mt] - top);
+#pragma unroll
+    for (int i = 0; i < CV; i++) o[mt][i] *= f;
+  }
+  for (int turn = 0; turn < 4; turn++) {
+    if (w == turn) {
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          float* dst = merged + (16 * mt + m) * LDO + CV * (4 * g + r);
+#pragma unroll
+          for (int i = 0; i < CV; i += 4) {
+            float4 v = make_float4(o[mt][i][r], o[mt][i + 1][r], o[mt][i + 2][r], o[mt][i + 3][r]);
+            if (turn) {
+              const float4 u = *reinterpret_cast<const float4*>(dst + i);
+              v = make_float4(u.x + v.x, u.y + v.y, u.z + v.z, u.w + v.w);
+            }
+            *reinterpret_cast<float4*>(dst + i) = v;
+          }
+        }
+    }
+    __syncthreads();
+  }
+  float* part = a.part + ((int64_t)bh * a.nsplit + split) * few_part_floats(rows, D);
+  for (int i = tid; i < rows * (D / 4); i += 256) {
+    const int r = i / (D / 4), c = i - r * (D / 4);
+    reinterpret_cast<float4*>(part)[i] = *reinterpret_cast<const float4*>(merged + r * LDO + 4 * c);
+  }
+  float* meta = part + rows * D;   // m, l and the smoothing term of every row
+  if (tid < rows) {
+    const float top = fmaxf(fmaxf(wave_m[0][tid], wave_m[1][tid]), fmaxf(wave_m[2][tid], wave_m[3][tid]));
+    float l = 0.f;
+    for (int i = 0; i < 4; i++) l += wave_l[i][tid] * __builtin_amdgcn_exp2f(wave_m[i][tid] - top);
+    meta[tid] = top;
+    meta[rows + tid] = l;
+  }
+  if (w == 0 && g == 0) {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+      if (16 * mt + m < rows) meta[2 * rows + 16 * mt + m] = dot[mt];
+  }
+}
+
+// One workgroup of D lanes per (row, batch x KV head): out = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s.
+// A few kilobytes per row out of the L2: bound by the latency of its two rounds of loads.
+template <int DT>
+__global__ void __launch_bounds__(128) attn_few_merge_kernel(FewArgs a, int D) {
+  const int r = blockIdx.x, bh = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv, d = threadIdx.x;
+  const int G = a.Hq / a.Hkv, rows = G * a.Sq, hq = kvh * G + r / a.Sq, s = r % a.Sq;
+  const int64_t stride = few_part_floats(rows, D);
+  const float* part = a.part + (int64_t)bh * a.nsplit * stride;
+  const float* meta = part + rows * D + r;
+  float top = kMInitFew;
+#pragma unroll 8
+  for (int i = 0; i < a.nsplit; i++) top = fmaxf(top, meta[i * stride]);
+  float l = 0.f, acc = 0.f;
+#pragma unroll 8
+  for (int i = 0; i < a.nsplit; i++) {
+    const float f = __builtin_amdgcn_exp2f(meta[i * stride] - top);
+    l = __builtin_fmaf(meta[i * stride + rows], f, l);
+    acc = __builtin_fmaf(part[i * stride + r * D + d], f, acc);
+  }
+  a.out[(int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + d] = from_f32<DT>(acc * (l > 0.f ? 1.0f / l : 0.f));
+  if (a.lse && d == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km ? meta[2 * rows] : 0.f) : kNegInfFew;
+}
+
+}  // namespace
+
+hipError_t launch_attn_few(FewArgs a, int dtype, int D, hipStream_t st) {
+  const int rows = a.Hq / a.Hkv * a.Sq, ntiles = (a.Skv + 127) / 128, pairs = a.B * a.Hkv;
+  // Two workgroups of four wavefronts per compute unit, no range shorter than one tile.
+  const int want = (kFewWorkgroups + pairs - 1) / pairs;
+  a.tiles_per_split = (ntiles + want - 1) / want;
+  a.nsplit = (ntiles + a.tiles_per_split - 1) / a.tiles_per_split;
+  const dim3 grid(a.nsplit, pairs), block(256);
+#define SAGE_FEW(DT, DD) (rows > 16 ? attn_few_kernel<DT, DD, 2><<<grid, block, 0, st>>>(a) : attn_few_kernel<DT, DD, 1><<<grid, block, 0, st>>>(a))
+  if (dtype == 0) { if (D == 64) SAGE_FEW(0, 64); else SAGE_FEW(0, 128); }
+  else { if (D == 64) SAGE_FEW(1, 64); else SAGE_FEW(1, 128); }
+#undef SAGE_FEW
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (dtype == 0) attn_few_merge_kernel<0><<<dim3(rows, pairs), dim3(D), 0, st>>>(a, D);
+  else attn_few_merge_kernel<1><<<dim3(rows, pairs), dim3(D), 0, st>>>(a, D);
+  return hipGetLastError();
+}
+
+}  // namespace sage

@@ -1,0 +1,68 @@
+"""A few query rows over a long history (csrc/sage_attn_few.hip) against the same formula in 64 bits on the INT8 operands of the
+public quantiser: rows per KV head around the 16-row tile and at the limit, keys around the 128-key tile and the range split,
+every K block size (a maximum per 16 keys, per wavefront, across two and four of them), both layouts, with and without K
+smoothing and LSE; and the first row count past the limit, which the tiled kernel takes."""
+import math
+
+import pytest
+import torch
+
+import baselinebenchmark_amd as sa
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, layout, BLKQ, BLKK, smooth):
+    km = sa.k_mean(k, layout) if smooth else None
+    q8, qs, k8, ks = (t.cpu().double() for t in sa.per_block_int8(q, k, km=km, BLKQ=BLKQ, BLKK=BLKK, tensor_layout=layout))
+    q, v = q.cpu().double(), v.cpu().half().double()
+    if layout == "NHD":
+        q8, k8, q, v = (t.transpose(1, 2) for t in (q8, k8, q, v))
+    rep = q8.shape[1] // k8.shape[1]
+    rows = lambda s, blk, n: s.repeat_interleave(blk, -1)[..., :n, None]  # noqa: E731
+    s2 = (q8 * rows(qs, BLKQ, q8.shape[2])) @ (k8 * rows(ks, BLKK, k8.shape[2])).repeat_interleave(rep, 1).transpose(-1, -2)
+    out = torch.softmax(s2 * math.log(2.0), -1) @ v.repeat_interleave(rep, 1)
+    lse = torch.logsumexp(s2 * math.log(2.0), -1)
+    if smooth:
+        lse = lse + (q * km.cpu().double().reshape(q.shape[0], -1, 1, q.shape[-1]).repeat_interleave(rep, 1)).sum(-1) * q.shape[-1] ** -0.5
+    return (out.transpose(1, 2) if layout == "NHD" else out), lse
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,BLKQ,BLKK,layout,smooth", [
+    (1, 1, 1, 1, 1025, 128, 64, "HND", True),      # one row, one key past a tile
+    (3, 8, 2, 4, 1152, 128, 128, "NHD", True),     # 16 rows: one whole tile; whole 128-key tiles
+    (2, 17, 1, 1, 2111, 64, 32, "HND", True),      # 17 rows: the second tile holds one
+    (1, 8, 4, 16, 1537, 16, 16, "NHD", False),     # 32 rows, the limit; 16-row and 16-key blocks, no smoothing
+    (2, 2, 2, 29, 1300, 16, 64, "HND", True),      # two Q blocks per head, the last one ragged
+    (64, 8, 8, 2, 1100, 32, 128, "HND", True),     # one range per (batch, head), ragged last tile
+    (1, 4, 1, 8, 70001, 128, 64, "HND", True),     # many ranges of several tiles
+    (1, 3, 1, 11, 1200, 128, 64, "NHD", True),     # 33 rows: past the limit
+])
+def test_few_rows_match_the_formula(dtype, D, B, Hq, Hkv, Sq, Skv, BLKQ, BLKK, layout, smooth):
+    g = torch.Generator().manual_seed(Skv + D)
+    shape = lambda H, L: (B, L, H, D) if layout == "NHD" else (B, H, L, D)  # noqa: E731
+    q, k, v = (torch.randn(shape(H, L), generator=g) for H, L in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    k = k + 2.0 * torch.randn((D,), generator=g)
+    q, k, v = (t.to(dtype).cuda() for t in (q * 2.0, k, v))
+    out, lse = sa.sageattn(q, k, v, tensor_layout=layout, smooth_k=smooth, pv_mode="fp16", BLKQ=BLKQ, BLKK=BLKK, return_lse=True)
+    plain = sa.sageattn(q, k, v, tensor_layout=layout, smooth_k=smooth, pv_mode="fp16", BLKQ=BLKQ, BLKK=BLKK)
+    want, want_lse = _reference(q, k, v, layout, BLKQ, BLKK, smooth)
+    # P is rounded to 11 bits, the output to 11 (float16) or 8 (bfloat16): a few half ulps of a row's own size
+    unit = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    rms = want.pow(2).mean().sqrt()
+    for got in (out, plain):
+        err = (got.cpu().double() - want).abs()
+        assert float((err / (want.abs() + rms)).max()) < 2 * unit + 4 * 2.0 ** -11
+    # fp32 sums of D products and of Skv probabilities
+    assert float((lse.cpu().double() - want_lse).abs().max()) < 2e-5 * max(1.0, float(want_lse.abs().max()))
+
+
+def test_equal_scores_average_v():
+    """Nothing of what lies past the last key of a ragged tile reaches the sums."""
+    g = torch.Generator().manual_seed(5)
+    k, v = (torch.randn((1, 2, 1500, 128), generator=g).half().cuda() for _ in range(2))
+    flat = sa.sageattn(torch.zeros((1, 8, 2, 128)).half().cuda(), k, v, pv_mode="fp16").cpu().double()
+    mean = v.cpu().double().mean(2, keepdim=True).repeat_interleave(4, 1)
+    assert float((flat - mean).abs().max()) < 2.0 ** -11 * float(mean.abs().max()) + 1e-6   # the output's rounding, fp32 sums
