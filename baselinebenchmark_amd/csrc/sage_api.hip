@@ -346,6 +346,12 @@ constexpr int64_t kSmallPrepassElements = (int64_t)4 << 20;
 // of 1024 rows, head_dim 128, K blocks of 64) 70 / 81; 302 M (the same with K blocks of 16) 68.7 / 54.2, and 8 x 8 heads of
 // 1024 rows at head_dim 64 with K blocks of 16, also 302 M, 88.9 / 50.1.
 constexpr int64_t kSmallPrepassReads = (int64_t)128 << 20;
+// A few query rows (sage_attn_few.hip) take four launches, 28-29 us end to end whatever the keys in this range; behind the
+// one-launch pre-pass the tiled kernel takes two, and longer with the keys of a head and with the re-reads.  bf16, K blocks of 64,
+// tiled / few rows: 1 x 8 heads of 768 keys, head_dim 128, 26.3 / 28.7 us, of 1024 keys 30.3 / 28.3; by re-reads, 4 x 8 heads
+// of 512 keys, head_dim 128 (25 M) 25.9 / 29.1; 16 x 8 of 512, head_dim 64 (50 M) 33.0 / 28.6; 4 x 8 of 768 (57 M) 34.7 / 28.4;
+// 8 x 8 of 1024, head_dim 64 (101 M) 47.7 / 28.3.
+constexpr int64_t kFewMinHeadElements = 896 * 128, kFewMinReads = (int64_t)32 << 20;
 struct E2EWorkspace {
   size_t q_i8, k_i8, q_scale, k_scale, km, v_scale, panels, stat, plan, lse_off, total;
   int64_t qs_sh, ks_sh, panel_sh;
@@ -413,7 +419,7 @@ size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, i
   return mask_can_be_packed(p, Sq, Skv, mask_kind) ? (size_t)p.total_bytes : 0;
 }
 
-// Few query rows per KV head over keys that do not fit the one-launch pre-pass: sage_attn_few.hip.  Calls that the general
+// Few query rows per KV head over a long history: sage_attn_few.hip.  Calls that the general
 // path refuses, slices of 2 GiB and more (32-bit row offsets) and rows that overlap are left to that path.
 static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, int64_t rows, int Sq, int Skv, int D,
                           int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
@@ -496,8 +502,9 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   const int64_t rereads = (Skv + blk_rows(blkk) - 1) / blk_rows(blkk) + (Skv + kPanelRows - 1) / kPanelRows;
   const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && k_elements <= kSmallPrepassElements &&
                              k_elements * rereads <= kSmallPrepassReads;
+  const bool short_keys = no_keys || (small_prepass && (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
-  if (few_rows_path(varlen, no_keys || small_prepass, is_causal, attn_mask, pv_mode, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
+  if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
                     out, q_sn, k_sn, v_sn)) {
     if (int rc2 = check_stride16("q", q_sb, q_sh, q_sn, 2, q)) return rc2;
     if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;

@@ -38,6 +38,8 @@ def _reference(q, k, v, layout, BLKQ, BLKK, smooth):
     (2, 2, 2, 29, 1300, 16, 64, "HND", True),      # two Q blocks per head, the last one ragged
     (64, 8, 8, 2, 1100, 32, 128, "HND", True),     # one range per (batch, head), ragged last tile
     (1, 4, 1, 8, 70001, 128, 64, "HND", True),     # many ranges of several tiles
+    (1, 4, 2, 3, 900, 128, 64, "HND", True),       # the fewest keys at head_dim 128, one-launch pre-pass at 64
+    (16, 8, 8, 1, 515, 128, 64, "NHD", True),      # by the pre-pass's re-reads
     (1, 3, 1, 11, 1200, 128, 64, "NHD", True),     # 33 rows: past the limit
 ])
 def test_few_rows_match_the_formula(dtype, D, B, Hq, Hkv, Sq, Skv, BLKQ, BLKK, layout, smooth):
