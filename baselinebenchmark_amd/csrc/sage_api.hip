@@ -207,6 +207,7 @@ struct QRawArg {   // fp16/bf16 Q to be quantised by the attention kernel itself
   const void* ptr = nullptr;
   int dtype = 0;
   float mult = 1.0f;
+  const void* dot_km = nullptr;   // K mean [B, Hkv, D] in q's type: its product with each scaled row is added to the row's LSE
 };
 
 struct MaskArg {
@@ -275,7 +276,7 @@ int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const floa
   a.mask_bits = mask.bits; a.mask_cls = mask.cls;
   a.mask_pb = mask.planes.pb; a.mask_ph = mask.planes.ph; a.mask_nqt = mask.planes.nqt; a.mask_ntk = mask.planes.ntk;
   a.mask_mult = mask.mult; a.lse_offset = lse_offset;
-  a.q_raw = qraw.ptr; a.q_is_bf16 = qraw.dtype == SAGE_DT_BF16; a.q_mult = qraw.mult;
+  a.q_raw = qraw.ptr; a.q_is_bf16 = qraw.dtype == SAGE_DT_BF16; a.q_mult = qraw.mult; a.q_dot_km = (const u16*)qraw.dot_km;
   int64_t grid;
   if (packed) {
     SagePlanLayout L = plan_layout(B, total_q);
@@ -553,18 +554,22 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
                          (int64_t)Hkv * D, D, blkk, 1.0f, dtype, cu_seqlens_k, cu_kblk, w.ks_sh, stream);
     if (rc) return rc;
   }
+  // Q is quantised by the attention kernel itself (each q-tile exactly where it is consumed) unless a feature needs the
+  // standalone pass: an explicit mask or interleaved scales.
+  // (LSE of smoothed keys with K blocks of 16 keys or interleaved K scales: stand-alone pass)
+  const bool want_dot = lse && smooth_k;
+  const bool fuse_q = !attn_mask && blk_groups(blkq) == 1 && !(want_dot && (blk_rows(blkk) == 16 || blk_groups(blkk) != 1));
   // With K smoothing every logit of a query row loses q . k_mean; the softmax does not notice but the
-  // log-sum-exp does, so when LSE is requested the Q quantiser also emits that dot product (in the
-  // base-2 units of the scaled Q) and the attention kernel adds it back.
+  // log-sum-exp does, so when LSE is requested whoever quantises Q also forms that dot product (in the
+  // base-2 units of the scaled Q) and the attention kernel adds it back.  In the attention kernel's prologue it costs one
+  // multiply-add per element; the pass over Q that it saves took 14 of the 243 us of a call on 32 heads of 4096 rows.
+  // (The workspace keeps room for that pass: its size is part of what callers have computed.)
   RowDot dot;
   float* lse_off = nullptr;
-  if (lse && smooth_k) {
+  if (want_dot && !fuse_q) {
     lse_off = (float*)(ws + w.lse_off);
     dot.vec = km; dot.out = lse_off; dot.sb = (int64_t)Hkv * D; dot.sh = D; dot.group = Hq / Hkv; dot.total = total_q;
   }
-  // Q is quantised by the attention kernel itself (each q-tile exactly where it is consumed) unless a
-  // feature needs the standalone pass: an explicit mask or the LSE correction.
-  const bool fuse_q = !attn_mask && !lse_off && blk_groups(blkq) == 1;   // (interleaved scales: standalone pass too)
   if (!fuse_q) {
     rc = quant_impl(q, q_i8, q_scale, nullptr, B, Hq, Sq, D, q_sb, q_sh, q_sn, qi_sb, qi_sh, qi_sn, 0, 0, blkq, q_mult, dtype,
                     cu_seqlens_q, cu_qblk, w.qs_sh, dot, stream);
@@ -576,7 +581,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     if (rc) return rc;
   }
   QRawArg qr;
-  if (fuse_q) { qr.ptr = q; qr.dtype = dtype; qr.mult = q_mult; }
+  if (fuse_q) { qr.ptr = q; qr.dtype = dtype; qr.mult = q_mult; qr.dot_km = want_dot ? km : nullptr; }
   MaskArg m;
   if (attn_mask) {
     // sageattn's additive mask is in natural-log units on top of sm_scale * q.k (test_sage_attention_mate.py:171-176)

@@ -165,10 +165,12 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 // KSUB: K scale blocks per 32 keys (1 for blocks of 32/64/128 keys, 2 for blocks of 16 keys); 3 = four interleaved scales per
 // block of 32/64/128 keys, scale t for the keys n of the block with (n % 8) / 2 == t (two of them reach every lane).
 // QF: the kernel reads fp16/bf16 Q and quantises its own tile (same arithmetic as quant_int8_kernel).
+// DOT (with QF): the kernel also forms the product of its scaled rows with the K mean, for the LSE of smoothed keys.  Variants of
+// their own: as a run-time branch in all FP16 kernels of head_dim 128 it cost calls without LSE 1 % (96 packed prompts).
 // KW (with KSUB == 1): 32-key groups that are known to share a K scale -- 1 for any block size from 32 keys on (every group
 // looks its scale up), 2 for blocks of 64 keys and more, 4 for blocks of 128: the row maximum then runs one integer chain
 // per scale and the per-scale constants of the softmax are computed once (a tenth of the vector instructions of a tile).
-template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1>
+template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
 __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   constexpr int GSH = SAGE_GSH;   // which bit of the wavefront index picks the group
   static_assert(NW == (2 << GSH), "the two groups pair wavefront w with w + NW/2");
@@ -194,6 +196,9 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   // the end of group 0's matrix phase; FP16 kernels of head_dim 64 keep the row maximum in the matrix phase (their
   // softmax, with its exponentials, is the longer one there: moving it measured -3 %, against +1 % at head_dim 128).
   constexpr bool VECMAX = PV == 1 || D == 128;
+
+  static_assert(!DOT || (QF && !MSUM), "DOT belongs to the kernels that quantise their own Q and return LSE");
+  [[maybe_unused]] __shared__ float row_dot[DOT ? BM : 1];
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
@@ -481,6 +486,16 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // for K.  Only this wavefront reads its region, so its own vmcnt wait is all the ordering needed.
     constexpr int QUPR = D * 2 / 16, QRPP = 64 / QUPR, QPIECES = 32 * D * 2 / 1024;
     uint8_t* qstage = smem + LEAD * KBYTES + w * (32 * D * 2);
+    // LSE of smoothed keys: the K mean of this head, whose product with the scaled row every logit of the row has lost.
+    // Requested ahead of the rows themselves, which complete after it.
+    [[maybe_unused]] v4u kmr[KS][2];
+    if constexpr (DOT) {
+      const u16* kp = a.q_dot_km + ((int64_t)b * a.Hkv + kvh) * D + 16 * h;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) kmr[ks][e] = *reinterpret_cast<const v4u*>(kp + 32 * ks + 8 * e);
+    }
     {
       const __amdgpu_buffer_rsrc_t qrsrc =
           __builtin_amdgcn_make_buffer_rsrc((void*)(reinterpret_cast<const u16*>(a.q_raw) + qoff), 0, 0x7fffffff, 0x00020000);
@@ -501,6 +516,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     }
     float x[KS][16];
     float amax = 0.f;
+    [[maybe_unused]] float dot = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
       uint4 raw[2];
@@ -513,6 +529,17 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
         x[ks][i] = (a.q_is_bf16 ? bf16_to_f32(e[i]) : f16_to_f32(e[i])) * a.q_mult;
         amax = fmaxf(amax, fabsf(x[ks][i]));
       }
+      if constexpr (DOT) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const u16 bits = (u16)(kmr[ks][i >> 3][(i & 7) >> 1] >> (16 * (i & 1)));
+          dot = __builtin_fmaf(x[ks][i], a.q_is_bf16 ? bf16_to_f32(bits) : f16_to_f32(bits), dot);
+        }
+      }
+    }
+    if constexpr (DOT) {
+      dot = xchg32_sum(dot);
+      if (h == 0) row_dot[w * 32 + m] = dot;   // read again by this very lane, in the epilogue
     }
     // Scale blocks of 16 rows: the lanes of a DPP row hold 16 consecutive query rows (one column half each),
     // the other column half sits 32 lanes away.  Larger blocks span the wavefront (and its neighbours, below).
@@ -1139,7 +1166,8 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   if (my_row < Lq) {
     if (a.lse && h == 0) {
       // lse_offset: what K smoothing removed from every logit of this row (q . k_mean, base-2 units)
-      const float shift = a.lse_offset ? a.lse_offset[lseoff + my_row] : 0.f;
+      float shift = a.lse_offset ? a.lse_offset[lseoff + my_row] : 0.f;
+      if constexpr (DOT) shift = row_dot[w * 32 + m];
       a.lse[lseoff + my_row] = lsum > 0.f ? m_used + __builtin_amdgcn_logf(lsum) - PSHIFT + shift : kNegInf;
     }
   }
@@ -1224,10 +1252,10 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
 }
 
 
-template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1>
+template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
 static hipError_t launch_one(const AttnArgs& a, int grid, hipStream_t st) {
   constexpr int smem = attn_lds_bytes<D, NW, BN, PV, CAUSAL, QF, MASK>();
-  auto kern = attn_kernel<D, NW, BN, PV, CAUSAL, MSUM, MASK, KSUB, QF, KW>;
+  auto kern = attn_kernel<D, NW, BN, PV, CAUSAL, MSUM, MASK, KSUB, QF, KW, DOT>;
   // More than 64 KB of dynamic LDS has to be allowed once per kernel and device.
   constexpr int kMaxDevices = 64;
   static std::atomic<bool> attr_done[kMaxDevices] = {};   // (two host threads may make the first call at once: setting it twice is harmless)

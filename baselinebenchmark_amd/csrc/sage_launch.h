@@ -134,6 +134,7 @@ struct AttnArgs {
   const void* q_raw;
   int q_is_bf16;
   float q_mult;
+  const u16* q_dot_km;      // K mean [B, Hkv, D] (packed: [nseq, Hkv, D]) in the type of q, or null: its product with the scaled row joins the row's LSE2
 };
 
 struct AttnConfig { int nw, bn; };

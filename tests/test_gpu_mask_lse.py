@@ -267,3 +267,27 @@ def test_packed_boolean_mask_equals_the_mask_read_in_place(shape, kind, pv):
     assert _direct_masked_call(q, k, v, mask, "HND", pv, 128, blkk, want, want_lse, 0) == 0
     torch.cuda.synchronize()
     assert torch.equal(out, want) and torch.equal(lse, want_lse * 0.6931471805599453)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("BLKQ,BLKK,causal", [(16, 32, False), (32, 64, True), (64, 128, False), (128, 64, True), (128, 16, False)])
+def test_lse_of_smoothed_keys_from_the_attention_prologue(dtype, D, pv, BLKQ, BLKK, causal):
+    """LSE against the formula in 64 bits on the quantiser's own INT8 operands plus q . k_mean: grouped heads, rows that end
+    inside a wavefront and a q-tile, every K scale granularity that takes its own kernel (blocks of 16: the stand-alone Q pass)."""
+    g = torch.Generator().manual_seed(D + BLKK)
+    B, Hq, Hkv, Sq, Skv = 2, 6, 2, 333, 301
+    q, k, v = (torch.randn((B, H, L, D), generator=g).to(dtype).cuda() for H, L in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    k = k + (3.0 * torch.randn((1, Hkv, 1, D), generator=g)).to(dtype).cuda()
+    _, lse = sa.sageattn(q, k, v, is_causal=causal, pv_mode=pv, BLKQ=BLKQ, BLKK=BLKK, return_lse=True)
+    km = sa.k_mean(k)
+    q8, qs, k8, ks = (t.cpu().double() for t in sa.per_block_int8(q, k, km=km, BLKQ=BLKQ, BLKK=BLKK))
+    qd = q8 * qs.repeat_interleave(BLKQ, -1)[..., :Sq, None]
+    kd = (k8 * ks.repeat_interleave(BLKK, -1)[..., :Skv, None]).repeat_interleave(Hq // Hkv, 1)
+    s = qd @ kd.transpose(-1, -2) * 0.6931471805599453
+    if causal:
+        s = s.masked_fill(torch.arange(Skv)[None] > torch.arange(Sq)[:, None], float("-inf"))
+    want = torch.logsumexp(s, -1) + (q.cpu().double() * km.cpu().double().reshape(B, Hkv, 1, D).repeat_interleave(Hq // Hkv, 1)).sum(-1) * D ** -0.5
+    # fp32 sums of D products and of at most Skv probabilities
+    assert float((lse.cpu().double() - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
