@@ -421,12 +421,14 @@ size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, i
 }
 
 // Few query rows per KV head over a long history: sage_attn_few.hip.  Calls that the general
-// path refuses, slices of 2 GiB and more (32-bit row offsets) and rows that overlap are left to that path.
-static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, int64_t rows, int Sq, int Skv, int D,
-                          int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
+// path refuses (its pre-passes have the batch and the heads on grid axes of 65535), slices of 2 GiB and more (32-bit row offsets),
+// rows that overlap and grids of 2^31 threads and more are left to that path.
+static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, int B, int Hkv, int64_t rows, int Sq, int Skv,
+                          int D, int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
   const int64_t limit = 0x7fffffff;
   return !varlen && !short_keys && !is_causal && !mask && pv_mode == SAGE_PV_FP16 && rows <= kFewRows && blk_groups(blkq) == 1 &&
-         blk_groups(blkk) == 1 && q && k && v && out && k_sn >= D && v_sn >= D && (int64_t)Sq * q_sn * 2 < limit &&
+         blk_groups(blkk) == 1 && B <= 65535 && Hkv <= 65535 && ((int64_t)B * Hkv + kFewWorkgroups) * 256 <= limit &&
+         q && k && v && out && k_sn >= D && v_sn >= D && (int64_t)Sq * q_sn * 2 < limit &&
          ((int64_t)Skv + 128) * k_sn * 2 < limit && ((int64_t)Skv + 128) * v_sn * 2 < limit;
 }
 
@@ -505,7 +507,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
                              k_elements * rereads <= kSmallPrepassReads;
   const bool short_keys = no_keys || (small_prepass && (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
-  if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
+  if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, B, Hkv, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
                     out, q_sn, k_sn, v_sn)) {
     if (int rc2 = check_stride16("q", q_sb, q_sh, q_sn, 2, q)) return rc2;
     if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;

@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
-  const int split = blockIdx.x, bh = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv;
+  const int bh = (int)fastdiv(blockIdx.x, a.div_nsplit), split = blockIdx.x - bh * a.nsplit, b = bh / a.Hkv, kvh = bh - b * a.Hkv;
   const int G = a.Hq / a.Hkv, rows = G * a.Sq, L = a.Skv;
   __shared__ float row_amax[16 * MT];
   __shared__ float block_amax[2][4];
@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 // A few kilobytes per row out of the L2: bound by the latency of its two rounds of loads.
 template <int DT>
 __global__ void __launch_bounds__(128) attn_few_merge_kernel(FewArgs a, int D) {
-  const int r = blockIdx.x, bh = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv, d = threadIdx.x;
+  const int bh = blockIdx.x, r = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv, d = threadIdx.x;
   const int G = a.Hq / a.Hkv, rows = G * a.Sq, hq = kvh * G + r / a.Sq, s = r % a.Sq;
   const int64_t stride = few_part_floats(rows, D);
   const float* part = a.part + (int64_t)bh * a.nsplit * stride;
@@ -362,15 +362,18 @@ hipError_t launch_attn_few(FewArgs a, int dtype, int D, hipStream_t st) {
   const int want = (kFewWorkgroups + pairs - 1) / pairs;
   a.tiles_per_split = (ntiles + want - 1) / want;
   a.nsplit = (ntiles + a.tiles_per_split - 1) / a.tiles_per_split;
-  const dim3 grid(a.nsplit, pairs), block(256);
+  a.div_nsplit = make_fastdiv(a.nsplit);
+  // The pairs go on x, the one grid axis that is not limited to 65535.  In the main kernel the ranges of a pair stay neighbours:
+  // with the pairs next to each other instead, 4 x 32/8 heads of 8192 keys took 50.9 us instead of 49.2.
+  const dim3 grid(pairs * a.nsplit), block(256);
 #define SAGE_FEW(DT, DD) (rows > 16 ? attn_few_kernel<DT, DD, 2><<<grid, block, 0, st>>>(a) : attn_few_kernel<DT, DD, 1><<<grid, block, 0, st>>>(a))
   if (dtype == 0) { if (D == 64) SAGE_FEW(0, 64); else SAGE_FEW(0, 128); }
   else { if (D == 64) SAGE_FEW(1, 64); else SAGE_FEW(1, 128); }
 #undef SAGE_FEW
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (dtype == 0) attn_few_merge_kernel<0><<<dim3(rows, pairs), dim3(D), 0, st>>>(a, D);
-  else attn_few_merge_kernel<1><<<dim3(rows, pairs), dim3(D), 0, st>>>(a, D);
+  if (dtype == 0) attn_few_merge_kernel<0><<<dim3(pairs, rows), dim3(D), 0, st>>>(a, D);
+  else attn_few_merge_kernel<1><<<dim3(pairs, rows), dim3(D), 0, st>>>(a, D);
   return hipGetLastError();
 }
 

@@ -46,27 +46,6 @@ struct PrepVArgs {
   int64_t panel_sh;
 };
 
-// Few query rows over a long history (sage_attn_few.hip).  `part` holds nsplit partial results per (batch, KV head): O [rows, D],
-// m [rows], l [rows], smoothing term [rows], rounded up to 16 bytes.
-// The row limit is two 16-column score tiles: at head_dim 128 the output of a third would not fit the registers.  At the limit
-// (4 x 32 heads, 16 rows, 4096 keys) a call takes 86.4 us here and 173.0 with the tiled kernel.
-constexpr int kFewRows = 32;          // query rows per KV head, over all query heads of its group
-constexpr int kFewWorkgroups = 512;   // two per compute unit, what the registers allow at once
-struct FewArgs {
-  const u16 *q, *k, *v, *km;   // km: [B, Hkv, D] or null
-  u16* out;
-  float *lse, *part;
-  int B, Hq, Hkv, Sq, Skv;
-  int64_t q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, v_sb, v_sh, v_sn, o_sb, o_sh, o_sn;
-  int blkq_shift, blkk_shift;
-  float q_mult;
-  int nsplit, tiles_per_split;   // filled in by launch_attn_few
-};
-__host__ __device__ inline int64_t few_part_floats(int rows, int D) { return (int64_t)rows * D + (3 * rows + 3) / 4 * 4; }
-// (at most one partial result per 128 keys: 32 rows of 524 bytes at head_dim 128, against the 32 KiB of an FP16 V panel)
-static_assert((kFewRows * 128 + 3 * kFewRows) * 4 <= 128 * 128 * 2 && (kFewRows * 64 + 3 * kFewRows) * 4 <= 128 * 64 * 2, "partials fit the panel region");
-hipError_t launch_attn_few(FewArgs a, int dtype, int D, hipStream_t st);
-
 // Division of a 32-bit unsigned number by a launch constant as a multiply-high and two shifts (exact for every 32-bit
 // dividend): the tile decode of the attention kernel divides the workgroup index by head counts that are no powers of
 // two, and a true integer division is some twenty dependent instructions on this hardware, paid by every workgroup
@@ -87,6 +66,28 @@ __device__ inline uint32_t fastdiv(uint32_t n, const FastDiv& f) {
   const uint32_t t = __umulhi(f.mul, n);
   return (t + ((n - t) >> f.sh1)) >> f.sh2;
 }
+
+// Few query rows over a long history (sage_attn_few.hip).  `part` holds nsplit partial results per (batch, KV head): O [rows, D],
+// m [rows], l [rows], smoothing term [rows], rounded up to 16 bytes.
+// The row limit is two 16-column score tiles: at head_dim 128 the output of a third would not fit the registers.  At the limit
+// (4 x 32 heads, 16 rows, 4096 keys) a call takes 86.4 us here and 173.0 with the tiled kernel.
+constexpr int kFewRows = 32;          // query rows per KV head, over all query heads of its group
+constexpr int kFewWorkgroups = 512;   // two per compute unit, what the registers allow at once
+struct FewArgs {
+  const u16 *q, *k, *v, *km;   // km: [B, Hkv, D] or null
+  u16* out;
+  float *lse, *part;
+  int B, Hq, Hkv, Sq, Skv;
+  int64_t q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, v_sb, v_sh, v_sn, o_sb, o_sh, o_sn;
+  int blkq_shift, blkk_shift;
+  float q_mult;
+  int nsplit, tiles_per_split;   // filled in by launch_attn_few, like the next one
+  FastDiv div_nsplit;
+};
+__host__ __device__ inline int64_t few_part_floats(int rows, int D) { return (int64_t)rows * D + (3 * rows + 3) / 4 * 4; }
+// (at most one partial result per 128 keys: 32 rows of 524 bytes at head_dim 128, against the 32 KiB of an FP16 V panel)
+static_assert((kFewRows * 128 + 3 * kFewRows) * 4 <= 128 * 128 * 2 && (kFewRows * 64 + 3 * kFewRows) * 4 <= 128 * 64 * 2, "partials fit the panel region");
+hipError_t launch_attn_few(FewArgs a, int dtype, int D, hipStream_t st);
 
 struct AttnArgs {
   const int8_t* q;

@@ -61,6 +61,24 @@ def test_few_rows_match_the_formula(dtype, D, B, Hq, Hkv, Sq, Skv, BLKQ, BLKK, l
     assert float((lse.cpu().double() - want_lse).abs().max()) < 2e-5 * max(1.0, float(want_lse.abs().max()))
 
 
+@pytest.mark.parametrize("smooth", [True, False])
+def test_more_batch_entries_and_heads_than_a_grid_axis_of_65535(smooth):
+    """Short attentions in great number (B * Hkv = 65552, one more head than the limit would hold): every entry like the same
+    entry in a batch of its own size below the limit."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q, k, v = (torch.randn((4097, 16, n, 64), generator=g, device="cuda", dtype=torch.bfloat16) for n in (2, 16, 16))
+    kw = dict(smooth_k=smooth, pv_mode="fp16", return_lse=True)
+    out, lse = sa.sageattn(q, k, v, **kw)
+    for part in (slice(0, 2048), slice(2048, 4097)):
+        o, l = sa.sageattn(q[part], k[part], v[part], **kw)
+        assert torch.equal(out[part], o) and torch.equal(lse[part], l)
+    few = slice(4095, 4097)   # the two entries around the limit, against the formula
+    want, want_lse = _reference(q[few], k[few], v[few], "HND", 128, 64, smooth)
+    rms = want.pow(2).mean().sqrt()
+    assert float(((out[few].cpu().double() - want).abs() / (want.abs() + rms)).max()) < 2 * 2.0 ** -8 + 4 * 2.0 ** -11
+    assert float((lse[few].cpu().double() - want_lse).abs().max()) < 2e-5 * max(1.0, float(want_lse.abs().max()))
+
+
 def test_equal_scores_average_v():
     """Nothing of what lies past the last key of a ragged tile reaches the sums."""
     g = torch.Generator().manual_seed(5)
