@@ -126,9 +126,6 @@ struct AttnArgs {
   const void* mask;
   int mask_kind;
   int64_t m_sb, m_sh, m_sm, m_sn;
-  const uint8_t* mask_bits; // packed boolean mask (sage_common.h) or null: taken instead of `mask`
-  const u16* mask_cls;
-  int mask_pb, mask_ph, mask_nqt, mask_ntk;
   float mask_mult;          // additive masks are scaled by this before they are added
   const float* lse_offset;  // added to LSE2 per query row (same layout as lse) or null
   // fused Q quantisation: fp16/bf16 Q with the strides of q (q and qs are then unused)
@@ -136,6 +133,9 @@ struct AttnArgs {
   int q_is_bf16;
   float q_mult;
   const u16* q_dot_km;      // K mean [B, Hkv, D] (packed: [nseq, Hkv, D]) in the type of q, or null: its product with the scaled row joins the row's LSE2
+  const uint8_t* mask_bits; // packed boolean mask (sage_common.h) or null: taken instead of `mask`
+  const u16* mask_cls;
+  int mask_pb, mask_ph, mask_nqt, mask_ntk;
 };
 
 struct AttnConfig { int nw, bn; };
