@@ -161,7 +161,8 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 // MASK: 0 none, 1 boolean keep-mask (bytes), 2 additive fp32 bias in base-2 score units
 // (sageattention_triton.py:92-105), both [B, Hq, Sq, Skv] with element strides; 3 = a boolean mask in the packed form of
 // mask_pack_kernel (sage_common.h): the workgroup walks only the tiles in which one of its rows sees a key, a wavefront
-// skips the tiles in which none of its own 32 rows does, and the bits of a tile arrive like a K tile does.
+// skips the tiles in which none of its own 32 rows does, and the bits of a tile arrive like a K tile does; 4 and 5 = 1 and 2 for
+// masks whose keys are contiguous.
 // KSUB: K scale blocks per 32 keys (1 for blocks of 32/64/128 keys, 2 for blocks of 16 keys); 3 = four interleaved scales per
 // block of 32/64/128 keys, scale t for the keys n of the block with (n % 8) / 2 == t (two of them reach every lane).
 // QF: the kernel reads fp16/bf16 Q and quantises its own tile (same arithmetic as quant_int8_kernel).
@@ -698,47 +699,84 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     if constexpr (MASK != 0) {
       // Explicit mask: the accumulators become scores (scale applied, bias removed), the mask is
       // applied element by element, and the maximum is taken over floats.
-      // (unit key stride and a whole tile: the four keys of a register quad in one load)
+      // (WIDE, contiguous keys: in a whole tile the four keys of a register quad in one load.  Kernels of their own: as a choice
+      // at run time it cost the other strides up to three times the call, see launch_attn_masked)
+      constexpr bool KEEP = MASK == 1 || MASK == 4, WIDE = MASK >= 4;
       typedef unsigned keep4 __attribute__((aligned(1)));
       typedef float bias4 __attribute__((ext_vector_type(4), aligned(4)));
-      const bool wide = a.m_sn == 1 && n0 + BN <= Lk;
-      const int64_t mrow = (int64_t)b * a.m_sb + (int64_t)hq_idx * a.m_sh + (int64_t)min(my_row, Lq - 1) * a.m_sm;
+      typedef typename std::conditional<KEEP, uint8_t, float>::type mask_t;
+      const mask_t* mrow = reinterpret_cast<const mask_t*>(a.mask) + (int64_t)b * a.m_sb + (int64_t)hq_idx * a.m_sh + (int64_t)min(my_row, Lq - 1) * a.m_sm;
       mloc = kNegInf;
+      // (the bias comes off first, exactly: the product of the biased value would have to cancel against a
+      // rounded bias * scale, an error of half an ulp of that product -- 1e-3 at large scales)
+      auto apply = [&](int nt, int r, unsigned keep, float add, bool there) {
+        float sv = (as_f(acc[nt][r]) - kBiasF) * sc[sci(nt, r)];
+        if constexpr (KEEP) sv = keep ? sv : kNegInf;
+        else sv = __builtin_fmaf(add, a.mask_mult, sv);
+        if (!there) sv = kNegInf;
+        acc[nt][r] = as_i(sv);
+        mloc = fmaxf(mloc, sv);
+      };
+      if constexpr (WIDE) {
+        const bool whole = n0 + BN <= Lk;
+        // The loads of WB groups in flight at once.  FP8 P.V of head_dim 128 has no registers to spare and leaves the order to the
+        // compiler (batches of one or two groups spill there: 92 -> 97 us on 2 x 16 heads of 1500 rows, an additive mask per head;
+        // the other kernels gain 4 to 10 % over that order).
+        constexpr bool BATCH = !(D == 128 && PV == 1);
+        constexpr int WB = BATCH ? 2 : 1;
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
-        if (wide) {
+        for (int b0 = 0; b0 < NT; b0 += WB) {
+          if (whole) {   // (asked for every batch: around all of them it lets their loads spill the scores)
+            typename std::conditional<KEEP, unsigned, bias4>::type mv[WB][4];
 #pragma unroll
-          for (int q4 = 0; q4 < 4; q4++) {
-            const int64_t mi = mrow + n0 + 32 * nt + 8 * q4 + 4 * h;
-            unsigned keep = 0;
-            bias4 bias = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (MASK == 1) keep = *reinterpret_cast<const keep4*>(reinterpret_cast<const uint8_t*>(a.mask) + mi);
-            else bias = *reinterpret_cast<const bias4*>(reinterpret_cast<const float*>(a.mask) + mi);
+            for (int i = 0; i < WB; i++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const int r = 4 * q4 + i;
-              float sv = (as_f(acc[nt][r]) - kBiasF) * sc[sci(nt, r)];
-              if constexpr (MASK == 1) sv = (keep >> (8 * i)) & 0xff ? sv : kNegInf;
-              else sv = __builtin_fmaf(bias[i], a.mask_mult, sv);
-              acc[nt][r] = as_i(sv);
-              mloc = fmaxf(mloc, sv);
-            }
+              for (int q4 = 0; q4 < 4; q4++) {
+                const mask_t* p = mrow + n0 + 32 * (b0 + i) + 8 * q4 + 4 * h;
+                if constexpr (KEEP) mv[i][q4] = *reinterpret_cast<const keep4*>(p);
+                else mv[i][q4] = *reinterpret_cast<const bias4*>(p);
+              }
+            if constexpr (BATCH) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < WB; i++)
+#pragma unroll
+              for (int r = 0; r < 16; r++) {
+                if constexpr (KEEP) apply(b0 + i, r, (mv[i][r / 4] >> (8 * (r % 4))) & 0xff, 0.f, true);
+                else apply(b0 + i, r, 0, mv[i][r / 4][r % 4], true);
+              }
+            if constexpr (BATCH) __builtin_amdgcn_sched_barrier(0);
+            continue;
           }
-          continue;
-        }
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int n = n0 + 32 * nt + 8 * (r / 4) + 4 * h + (r % 4);
-          // (the bias comes off first, exactly: the product of the biased value would have to cancel against a
-          // rounded bias * scale, an error of half an ulp of that product -- 1e-3 at large scales)
-          float sv = (as_f(acc[nt][r]) - kBiasF) * sc[sci(nt, r)];
-          const int64_t mi = mrow + (int64_t)min(n, Lk - 1) * a.m_sn;
-          if constexpr (MASK == 1) sv = reinterpret_cast<const uint8_t*>(a.mask)[mi] ? sv : kNegInf;
-          else sv = __builtin_fmaf(reinterpret_cast<const float*>(a.mask)[mi], a.mask_mult, sv);
-          if (n >= Lk) sv = kNegInf;
-          acc[nt][r] = as_i(sv);
-          mloc = fmaxf(mloc, sv);
+          for (int i = 0; i < WB; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+              const int n = n0 + 32 * (b0 + i) + 8 * (r / 4) + 4 * h + (r % 4);
+              const mask_t mv = mrow[min(n, Lk - 1)];
+              apply(b0 + i, r, (unsigned)mv, (float)mv, n < Lk);
+            }
         }
+        return;
+      }
+      // Other strides: one load per score, those of MB 32-key groups in flight at once, as many as the registers hold without a
+      // spill.  Left to the compiler they went one by one or spilled (2 x 16 heads of 1500 rows, transposed mask, additive /
+      // boolean, now and then: head_dim 64 FP16 P.V 82 / 274 -> 72 / 78 us, FP8 83 / 82 -> 76 / 76; 128 FP16 282 / 341 -> 101 / 101,
+      // FP8 110 / 108 -> 91 / 90.  MB = 1 at head_dim 64: 88 / 84; MB = 2 at 128, FP8: 99 / 102).
+      constexpr int MB = D == 64 ? 2 : 1;
+#pragma unroll
+      for (int b0 = 0; b0 < NT; b0 += MB) {
+        mask_t mv[MB][16];
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) mv[i][r] = mrow[(int64_t)min(n0 + 32 * (b0 + i) + 8 * (r / 4) + 4 * h + (r % 4), Lk - 1) * a.m_sn];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++)
+            apply(b0 + i, r, (unsigned)mv[i][r], (float)mv[i][r], n0 + 32 * (b0 + i) + 8 * (r / 4) + 4 * h + (r % 4) < Lk);
+        __builtin_amdgcn_sched_barrier(0);
       }
       return;
     }

@@ -159,6 +159,7 @@ AttnConfig attn_config(int D, int pv, bool packed);
 void finish_attn_args(AttnArgs& a, bool causal);
 hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_masked(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
+hipError_t launch_attn_masked_wide(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_packed_mask(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_qfused(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_k16(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);

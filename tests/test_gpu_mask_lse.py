@@ -291,3 +291,26 @@ def test_lse_of_smoothed_keys_from_the_attention_prologue(dtype, D, pv, BLKQ, BL
     want = torch.logsumexp(s, -1) + (q.cpu().double() * km.cpu().double().reshape(B, Hkv, 1, D).repeat_interleave(Hq // Hkv, 1)).sum(-1) * D ** -0.5
     # fp32 sums of D products and of at most Skv probabilities
     assert float((lse.cpu().double() - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("additive", [False, True])
+@pytest.mark.parametrize("Sq,Skv,D,BLKK", [(70, 127, 64, 64), (257, 128, 128, 128), (300, 129, 64, 16), (33, 385, 128, 32)])
+def test_mask_strides_reach_the_same_result(pv, additive, Sq, Skv, D, BLKK):
+    """Masks read in place: with contiguous keys (kernels of their own from one whole 128-key tile on) and with every other
+    stride, the same bits."""
+    g = torch.Generator().manual_seed(Sq + Skv)
+    B, Hq, Hkv = 2, 4, 2
+    q, k, v = (randn("HND", B, h, n, D, torch.float16, g).to(DEV) for h, n in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    q8, qs, k8, ks = sa.per_block_int8(q, k, BLKK=BLKK)
+    make = lambda *s: (torch.randn(s, generator=g) if additive else torch.rand(s, generator=g) > 0.4).to(DEV)  # noqa: E731
+    masks = {"transposed": make(B, 1, Skv, Sq).transpose(-1, -2), "every other key": make(1, Hq, Sq, 2 * Skv)[..., ::2],
+             "rows of one value": make(B, Hq, Sq, 1).expand(B, Hq, Sq, Skv), "rows at odd offsets": make(1, 1, Sq, Skv + 1)[..., 1:],
+             "one row for all": make(B, 1, 1, Skv)}
+    for name, mask in masks.items():
+        got = sa.forward(q8, k8, v, qs, ks, attn_mask=mask, pv_mode=pv, BLKK=BLKK, return_lse=True)
+        dense = mask.expand(B, Hq, Sq, Skv).contiguous()
+        strided = dense.transpose(-1, -2).contiguous().transpose(-1, -2)
+        for other in (dense, strided):
+            want = sa.forward(q8, k8, v, qs, ks, attn_mask=other, pv_mode=pv, BLKK=BLKK, return_lse=True)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), name
