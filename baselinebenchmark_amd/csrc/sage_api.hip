@@ -408,16 +408,23 @@ size_t sage_sageattn_workspace_bytes_for(int B, int Hq, int Hkv, int Sq, int Skv
 }
 
 // A boolean mask is packed into bits when the workspace has room for them behind what the call needs anyway, the grid
-// and the kernel's tile list can hold its tiles.  (2 x 16 heads of 1500 rows, head_dim 64, about four documents per row: the
-// whole call 228.7 us with the mask read in place -- 64 byte loads per lane and tile, every tile visited -- 83.0 us packed.)
-static bool mask_can_be_packed(const MaskPlanes& p, int Sq, int Skv, int mask_kind) {
-  return mask_kind == SAGE_MASK_BOOL && Sq > 0 && Skv > 0 && p.ntk <= kMaskMaxTiles && p.nqt <= 65535 && p.planes <= 65535;
+// and the kernel's tile list can hold its tiles, and the pass pays: the packing is one more launch, 3 to 6 us, and saves up to
+// half the time of every key tile that a q-tile visits and all of those it does not see.  Three key tiles are enough (one head of
+// 500 rows and 500 keys, head_dim 64, FP16 P.V, about four documents: 35.4 us packed, 36.9 read in place; 4 heads of 800: 35.6 / 63.0;
+// two tiles, 2 x 16 heads of 500 rows, 200 keys: 30.3 / 27.2), or tiles for two rounds of the chip (4 x 32 heads of 1000 rows and
+// 128 keys, 512 tile visits: 32.9 / 34.8; of 2000 rows and 77 keys, 1024: 55 / 71).  In place, keys that are not contiguous are no
+// slower than others, packed they are: five key tiles there, or twice the visits (128 rows, 500 keys, four tiles, transposed, FP8 P.V:
+// 40.6 / 36.2; 4 heads of 800: 45.9 / 48.1).
+static int64_t mask_tile_visits(const MaskPlanes& p, int B, int Hq, int Sq) { return (int64_t)B * Hq * ((Sq + kMaskRows - 1) / kMaskRows) * p.ntk; }
+static bool mask_can_be_packed(const MaskPlanes& p, int B, int Hq, int Sq, int Skv, int mask_kind) {
+  return mask_kind == SAGE_MASK_BOOL && Sq > 0 && Skv > 0 && p.ntk <= kMaskMaxTiles && p.nqt <= 65535 && p.planes <= 65535 &&
+         (p.ntk >= 3 || mask_tile_visits(p, B, Hq, Sq) >= 512);
 }
 
 size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, int64_t m_sb, int64_t m_sh, int64_t m_sm) {
   if (B <= 0 || Hq <= 0) return 0;
   const MaskPlanes p = mask_planes(B, Hq, Sq, Skv, m_sb, m_sh, m_sm);
-  return mask_can_be_packed(p, Sq, Skv, mask_kind) ? (size_t)p.total_bytes : 0;
+  return mask_can_be_packed(p, B, Hq, Sq, Skv, mask_kind) ? (size_t)p.total_bytes : 0;
 }
 
 // Few query rows per KV head over a long history: sage_attn_few.hip.  Calls that the general
@@ -589,7 +596,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     // sageattn's additive mask is in natural-log units on top of sm_scale * q.k (test_sage_attention_mate.py:171-176)
     m.ptr = attn_mask; m.kind = mask_kind; m.sb = m_sb; m.sh = m_sh; m.sm = m_sm; m.sn = m_sn; m.mult = 1.44269504f;
     const MaskPlanes p = mask_planes(B, Hq, Sq, Skv, m_sb, m_sh, m_sm);
-    if (!varlen && !is_causal && mask_can_be_packed(p, Sq, Skv, mask_kind) && workspace_bytes - w.total >= (size_t)p.total_bytes) {
+    const bool pays = m_sn == 1 || p.ntk >= 5 || mask_tile_visits(p, B, Hq, Sq) >= 1024;
+    if (!varlen && !is_causal && pays && mask_can_be_packed(p, B, Hq, Sq, Skv, mask_kind) && workspace_bytes - w.total >= (size_t)p.total_bytes) {
       uint8_t* bits = ws + w.total;
       m.planes = p; m.bits = bits; m.cls = (const u16*)(bits + p.bits_bytes);
       hipError_t e = launch_mask_pack((const uint8_t*)attn_mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, (u16*)(bits + p.bits_bytes),

@@ -266,7 +266,9 @@ int sage_sageattn(const void* q, const void* k, const void* v, void* out, float*
  * sage_attn_fwd_masked.  attn_mask == NULL makes it identical to sage_sageattn.
  * A workspace that is larger than sage_sageattn_workspace_bytes_for by sage_sageattn_mask_bytes lets the call pack a boolean
  * mask into bits first (one per row and key, for each distinct slice of the mask): the attention then skips the key tiles
- * that no row of a q-tile sees.  Same results, bit for bit; 0 = nothing to gain (additive masks, more than 262144 keys).
+ * that no row of a q-tile sees.  With finite V the results are the same, bit for bit; an infinity or NaN in V at a key that a row
+ * may not see reaches that row's output as 0 * V = NaN where its tile is visited, and not where it is skipped (as above the
+ * diagonal of a causal call).  0 = nothing to gain: additive masks, more than 262144 keys, calls too small to pay for the pass.
  */
 size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, int64_t m_sb, int64_t m_sh, int64_t m_sm);
 int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out, float* lse,

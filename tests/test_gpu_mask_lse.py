@@ -314,3 +314,57 @@ def test_mask_strides_reach_the_same_result(pv, additive, Sq, Skv, D, BLKK):
         for other in (dense, strided):
             want = sa.forward(q8, k8, v, qs, ks, attn_mask=other, pv_mode=pv, BLKK=BLKK, return_lse=True)
             assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), name
+
+
+# around the packing's chunks of 16 keys and batches of rows, the second chunk of 64 key tiles of the tile list, and every K scale kind
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,BLKQ,BLKK,groups", [
+    (8, 64, 8, 3, 5, 64, 128, 64, (1, 1)),        # fewer keys than one load of the packing
+    (2, 256, 32, 40, 16, 64, 128, 32, (1, 1)),    # exactly one
+    (1, 2, 1, 300, 257, 64, 128, 64, (1, 1)),     # one key past it, two q-tiles
+    (1, 2, 2, 129, 399, 128, 32, 64, (8, 4)),     # interleaved scales; a row past half a q-tile
+    (1, 2, 1, 257, 641, 64, 128, 16, (1, 1)),     # five key tiles and one key
+    (1, 1, 1, 256, 8300, 64, 128, 128, (1, 1)),   # 65 key tiles
+])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+def test_packed_mask_is_taken_and_changes_no_bit(B, Hq, Hkv, Sq, Skv, D, BLKQ, BLKK, groups, pv):
+    lib = __import__("baselinebenchmark_amd._cabi", fromlist=["lib"]).lib()
+    g = torch.Generator().manual_seed(Skv)
+    q, k, v = (randn("HND", B, h, n, D, torch.bfloat16, g).to(DEV) for h, n in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    flags = (sa.sageattention.BLK_INTERLEAVE8 if groups[0] == 8 else 0, sa.sageattention.BLK_INTERLEAVE4 if groups[1] == 4 else 0)
+    rows = torch.arange(Sq)[:, None]
+    masks = {"random": torch.rand((B, 1, Sq, Skv), generator=g) > 0.5,
+             "band": ((torch.arange(Skv)[None] - rows * Skv // Sq).abs() < 70)[None, None],
+             "far tiles": ((torch.arange(Skv)[None] >= Skv - 3) | (torch.arange(Skv)[None] == rows % 2))[None, None],
+             "padding": (torch.arange(Skv) < max(1, Skv - 9))[None, None, None]}
+    for name, mask in masks.items():
+        mask = mask.to(DEV)
+        m = mask.expand(B, Hq, Sq, Skv)
+        extra = lib.sage_sageattn_mask_bytes(B, Hq, Sq, Skv, 1, *m.stride()[:3])
+        assert extra > 0, name
+        outs = [torch.empty_like(q) for _ in range(2)]
+        lses = [torch.empty((B, Hq, Sq), device=DEV) for _ in range(2)]
+        for out, lse, room in zip(outs, lses, (extra, 0)):   # packed, and read in place for want of room
+            assert _direct_masked_call(q, k, v, mask, "HND", pv, BLKQ | flags[0], BLKK | flags[1], out, lse, room) == 0
+        out, lse = sa.sageattn(q, k, v, attn_mask=mask, pv_mode=pv, BLKQ=BLKQ, BLKK=BLKK, q_interleave=groups[0], k_interleave=groups[1],
+                               return_lse=True)
+        assert torch.equal(out, outs[0]) and torch.equal(lse, lses[0] * 0.6931471805599453), name
+        assert torch.equal(outs[0], outs[1]) and torch.equal(lses[0], lses[1]), name
+
+
+def test_masks_that_are_not_packed():
+    """More key tiles than the tile list holds, and calls too small for the pass: no room asked for, the mask is read in place."""
+    lib = __import__("baselinebenchmark_amd._cabi", fromlist=["lib"]).lib()
+    assert lib.sage_sageattn_mask_bytes(2, 16, 500, 200, 1, 100000, 0, 200) == 0
+    assert lib.sage_sageattn_mask_bytes(1, 2, 500, 500, 2, 250000, 0, 500) == 0   # additive
+    Skv = 128 * 2048 + 1
+    assert lib.sage_sageattn_mask_bytes(1, 1, 1, Skv - 1, 1, 0, 0, 0) > 0
+    assert lib.sage_sageattn_mask_bytes(1, 1, 1, Skv, 1, 0, 0, 0) == 0
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn((1, 1, n, 64), generator=g, device=DEV, dtype=torch.float16) for n in (2, Skv, Skv))
+    keep = torch.zeros((1, 1, 1, Skv), dtype=torch.bool, device=DEV)
+    keep[..., [0, 129, 70001, Skv - 1]] = True
+    seen = keep.flatten().nonzero().flatten()
+    out = sa.sageattn(q, k, v, attn_mask=keep, smooth_k=False)
+    want = torch.softmax((q.double() @ k[:, :, seen].double().transpose(-1, -2)) / 8.0, -1) @ v[:, :, seen].double()
+    # INT8 logits: half a step of 1/127 of the largest |k| and |q| in every product, as in the other comparisons with plain attention
+    assert torch.nn.functional.cosine_similarity(out.double().flatten(), want.flatten(), dim=0) > 0.999
