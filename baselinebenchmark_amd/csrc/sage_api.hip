@@ -353,6 +353,11 @@ constexpr int64_t kSmallPrepassReads = (int64_t)128 << 20;
 // of 512 keys, head_dim 128 (25 M) 25.9 / 29.1; 16 x 8 of 512, head_dim 64 (50 M) 33.0 / 28.6; 4 x 8 of 768 (57 M) 34.7 / 28.4;
 // 8 x 8 of 1024, head_dim 64 (101 M) 47.7 / 28.3.
 constexpr int64_t kFewMinHeadElements = 896 * 128, kFewMinReads = (int64_t)32 << 20;
+// ... and with few keys, in great number: the FP32 results of a KV head's rows are written and read again, the tiled kernel with one
+// query head per KV head launches no more workgroups, and at head_dim 128 it wins where those bytes outweigh K and V.  16384 heads,
+// bf16, tiled / few rows: 24 rows, 16 keys 729 / 725 us; 28 rows, 16 keys 733 / 782, 48 keys 814 / 803; 32 rows, 16 keys 743 / 846,
+// 64 keys 846 / 878, 80 keys 925 / 897.  (At head_dim 64, 32 rows, 32 keys 513 / 461; two query heads per KV head: few rows always.)
+bool few_rows_outweigh_keys(int64_t rows, int Sq, int Skv, int D) { return D == 128 && rows == Sq && Skv < 8 * (rows - 22); }
 struct E2EWorkspace {
   size_t q_i8, k_i8, q_scale, k_scale, km, v_scale, panels, stat, plan, lse_off, total;
   int64_t qs_sh, ks_sh, panel_sh;
@@ -433,7 +438,7 @@ size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, i
 static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, int B, int Hkv, int64_t rows, int Sq, int Skv,
                           int D, int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
   const int64_t limit = 0x7fffffff;
-  return !varlen && !short_keys && !is_causal && !mask && pv_mode == SAGE_PV_FP16 && rows <= kFewRows && blk_groups(blkq) == 1 &&
+  return !varlen && !short_keys && !is_causal && !mask && pv_mode == SAGE_PV_FP16 && rows <= kFewRows && !few_rows_outweigh_keys(rows, Sq, Skv, D) && blk_groups(blkq) == 1 &&
          blk_groups(blkk) == 1 && B <= 65535 && Hkv <= 65535 && ((int64_t)B * Hkv + kFewWorkgroups) * 256 <= limit &&
          q && k && v && out && k_sn >= D && v_sn >= D && (int64_t)Sq * q_sn * 2 < limit &&
          ((int64_t)Skv + 128) * k_sn * 2 < limit && ((int64_t)Skv + 128) * v_sn * 2 < limit;

@@ -86,3 +86,18 @@ def test_equal_scores_average_v():
     flat = sa.sageattn(torch.zeros((1, 8, 2, 128)).half().cuda(), k, v, pv_mode="fp16").cpu().double()
     mean = v.cpu().double().mean(2, keepdim=True).repeat_interleave(4, 1)
     assert float((flat - mean).abs().max()) < 2.0 ** -11 * float(mean.abs().max()) + 1e-6   # the output's rounding, fp32 sums
+
+
+@pytest.mark.parametrize("Sq,Skv", [(22, 3), (23, 7), (23, 8), (28, 47), (28, 48), (32, 79), (32, 80)])
+def test_many_heads_of_few_keys(Sq, Skv):
+    """Both sides of the line between the two kernels where K and V are short (one query head per KV head, head_dim 128)."""
+    g = torch.Generator().manual_seed(Sq + Skv)
+    B, H = 4 + (1 << 22) // (32 * Skv * 128), 32   # more elements of K than the one-launch pre-pass takes
+    q, k, v = (torch.randn((2, H, n, 128), generator=g).to(torch.bfloat16).cuda() for n in (Sq, Skv, Skv))
+    many = lambda t: t.repeat((B + 1) // 2, 1, 1, 1)  # noqa: E731
+    out, lse = sa.sageattn(many(q), many(k), many(v), pv_mode="fp16", return_lse=True)
+    want, want_lse = _reference(q, k, v, "HND", 128, 64, True)
+    rms = want.pow(2).mean().sqrt()
+    for i in (0, out.shape[0] // 4 * 2, out.shape[0] - 2):
+        assert float(((out[i:i + 2].cpu().double() - want).abs() / (want.abs() + rms)).max()) < 2 * 2.0 ** -8 + 4 * 2.0 ** -11
+        assert float((lse[i:i + 2].cpu().double() - want_lse).abs().max()) < 2e-5 * max(1.0, float(want_lse.abs().max()))
