@@ -16,7 +16,7 @@ namespace sage {
 // tiles of a sequence in one tier are a contiguous range with ends in closed form, and no tile is ever visited to be counted:
 // one wavefront owns a tier, a lane a sequence, and a wavefront scan gives every sequence its place in the tier's part of the
 // list.  (A histogram over all tiles, with one pass of the whole workgroup and four barriers per sequence, took 82 us for
-// 96 sequences of 16..1024 rows and 30 us for 16 of 512..32768; this takes 6 and 9.)
+// 96 sequences of 16..1024 rows and 30 us for 16 of 512..32768; this takes 9 and 10.)
 // ---------------------------------------------------------------------------------------------
 constexpr int kCostMax = 2047, kTierCost = 32, kTiers = (kCostMax + 1) / kTierCost;
 constexpr int kPlanThreads = 1024, kPlanWaves = kPlanThreads / 64, kPlanSeqsLds = 4096;
@@ -109,7 +109,17 @@ __global__ void __launch_bounds__(kPlanThreads) varlen_plan_kernel(const int32_t
         hi = t == kTiers - 1 ? nqt : first_tile(n, nqt, t + 1);
       }
       const int upto = before + wave_inclusive_scan(hi - lo);
-      for (int qt = lo; qt < hi; qt++) tiles[upto - 1 - (qt - lo)] = (i << 16) | qt;
+      // A lane writes its own sequence's q-tiles; those of a few long sequences (non-causal, or past the last tier's start) the
+      // whole wavefront, one after the other: 1 M rows, one sequence, took 137 us with one lane, 14 like this.  (Many long ones
+      // keep as many lanes busy by themselves: 100 of 17000 rows and 300 keys 12.8 us, one after the other 23.)
+      unsigned long long todo = __builtin_amdgcn_ballot_w64(hi - lo > 64);
+      if (__popcll(todo) > 16) todo = 0;
+      if (!(todo >> lane & 1))
+        for (int qt = lo; qt < hi; qt++) tiles[upto - 1 - (qt - lo)] = (i << 16) | qt;
+      for (; todo; todo &= todo - 1) {
+        const int src = __builtin_ctzll(todo), first = __shfl(lo, src, 64), end = __shfl(hi, src, 64), last = __shfl(upto, src, 64) - 1;
+        for (int qt = first + lane; qt < end; qt += 64) tiles[last - (qt - first)] = ((i0 + src) << 16) | qt;
+      }
       before = __shfl(upto, 63, 64);
     }
   }

@@ -93,6 +93,21 @@ def test_plan_for_many_sequences_and_every_tier(nseq, longest, causal):
     assert got == [(i, -t) for _, i, t in want]
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens", [[64 * 256 + 1], [5, 65 * 256, 0, 64 * 256, 129 * 256 - 7, 300], [65 * 256] * 16 + [40] * 50, [65 * 256] * 17 + [40]])
+def test_plan_of_long_sequences(lens, causal):
+    """Sequences whose q-tiles a wavefront lists together (more than 64 of a tier, at most 16 of them in its chunk) among short ones."""
+    lq = np.array(lens)
+    for lk in (lq, np.full_like(lq, 77)):
+        cuq, cuk = (np.concatenate([[0], np.cumsum(x)]).astype(np.int32) for x in (lq, lk))
+        plan, offs = sa.varlen_plan(torch.from_numpy(cuq).to(DEV), torch.from_numpy(cuk).to(DEV), int(cuq[-1]), 128, 64, is_causal=causal)
+        p = plan.cpu().numpy()
+        want = sorted((-(min(((min(lk[i], (t + 1) * 256) if causal else lk[i]) + 63) // 64, 2047) // 32), i, -t)
+                      for i in range(len(lq)) for t in range((lq[i] + 255) // 256))
+        got = [(int(t) >> 16, int(t) & 0xFFFF) for t in p[offs[4]:offs[4] + int(p[offs[3]])]]
+        assert got == [(i, -t) for _, i, t in want]
+
+
 def test_config4_full_size_sequences_are_independent():
     """BASELINE config 4 at its full size (16 packed sequences of 512..32768 rows, Hq32/Hkv8, D128 bf16 causal, FP8
     P.V): the packed call reproduces, bit for bit, a stand-alone call on each of three of its sequences (shortest,
