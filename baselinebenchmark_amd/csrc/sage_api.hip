@@ -215,7 +215,7 @@ struct MaskArg {
   int kind = 0;
   int64_t sb = 0, sh = 0, sm = 0, sn = 0;
   const uint8_t* bits = nullptr;   // packed form of a boolean mask (with `planes`), taken instead of ptr
-  const u16* cls = nullptr;
+  const uint8_t* seen = nullptr;
   MaskPlanes planes = {};
   float mult = 1.0f;   // additive masks are multiplied by this (1 for base-2 units, log2(e) for natural units)
 };
@@ -273,7 +273,7 @@ int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const floa
   a.out_bf16 = out_dtype == SAGE_DT_BF16;
   a.nqt = (Sq + BM - 1) / BM;
   a.mask = mask.ptr; a.mask_kind = mask.kind; a.m_sb = mask.sb; a.m_sh = mask.sh; a.m_sm = mask.sm; a.m_sn = mask.sn;
-  a.mask_bits = mask.bits; a.mask_cls = mask.cls;
+  a.mask_bits = mask.bits; a.mask_seen = mask.seen;
   a.mask_pb = mask.planes.pb; a.mask_ph = mask.planes.ph; a.mask_nqt = mask.planes.nqt; a.mask_ntk = mask.planes.ntk;
   a.mask_mult = mask.mult; a.lse_offset = lse_offset;
   a.q_raw = qraw.ptr; a.q_is_bf16 = qraw.dtype == SAGE_DT_BF16; a.q_mult = qraw.mult; a.q_dot_km = (const u16*)qraw.dot_km;
@@ -604,8 +604,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     const bool pays = m_sn == 1 || p.ntk >= 5 || mask_tile_visits(p, B, Hq, Sq) >= 1024;
     if (!varlen && !is_causal && pays && mask_can_be_packed(p, B, Hq, Sq, Skv, mask_kind) && workspace_bytes - w.total >= (size_t)p.total_bytes) {
       uint8_t* bits = ws + w.total;
-      m.planes = p; m.bits = bits; m.cls = (const u16*)(bits + p.bits_bytes);
-      hipError_t e = launch_mask_pack((const uint8_t*)attn_mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, (u16*)(bits + p.bits_bytes),
+      m.planes = p; m.bits = bits; m.seen = bits + p.bits_bytes;
+      hipError_t e = launch_mask_pack((const uint8_t*)attn_mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, bits + p.bits_bytes,
                                       (hipStream_t)stream);
       if (e != hipSuccess) return hip_fail(e, "sage_sageattn(mask)");
     }

@@ -337,15 +337,15 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   int ntiles = (kv_end + BN - 1) / BN;
   const uint8_t* mask_bits = nullptr;
   if constexpr (LISTED) {
-    // The tiles this workgroup has to visit, in order: tile index | the visibility classes of its eight 32-row groups << 16.
+    // The tiles this workgroup has to visit, in order: tile index | which of its eight 32-row groups see it << 16.
     // Every wavefront writes the same list (and reads back only what it wrote itself), so no barrier is needed.
     const int64_t qtile = (int64_t)(b * a.mask_pb + hq_idx * a.mask_ph) * a.mask_nqt + (a.mask_nqt > 1 ? qt : 0);
-    const u16* cls = a.mask_cls + qtile * a.mask_ntk;
+    const uint8_t* seen = a.mask_seen + qtile * a.mask_ntk;
     mask_bits = a.mask_bits + qtile * a.mask_ntk * kMaskTileBytes;
     int n = 0;
     for (int t0 = 0; t0 < a.mask_ntk; t0 += 64) {
       const int t = t0 + lane;
-      const int c = t < a.mask_ntk ? cls[t] : 0;
+      const int c = t < a.mask_ntk ? seen[t] : 0;
       const unsigned long long on = __builtin_amdgcn_ballot_w64(c != 0);
       if (c != 0) tile_list[n + __popcll(on & ((1ull << lane) - 1))] = t | (c << 16);
       n += __popcll(on);
@@ -355,8 +355,8 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   auto list_entry = [&](int j) { return __builtin_amdgcn_readfirstlane(tile_list[min(j, ntiles - 1)]); };
   // key tile that period j works on
   auto tile_at = [&](int j) { return LISTED ? list_entry(j) & 0xffff : j; };
-  // packed mask: what this wavefront's rows see of it (0 nothing, 1 some keys, 2 every key)
-  auto sees = [&](int j) { return row0 < Lq ? (list_entry(j) >> (16 + 2 * w)) & 3 : 0; };
+  // packed mask: does a row of this wavefront see some key of it?
+  auto sees = [&](int j) { return row0 < Lq && ((list_entry(j) >> (16 + w)) & 1); };
   const int wave_end = (row0 < Lq) ? (CAUSAL ? min(Lk, row0 + 32) : Lk) : 0;
   const int wave_ntiles = (wave_end + BN - 1) / BN;
 
@@ -1062,7 +1062,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // their tile count at every use: as a flag that is computed first and carried through the period, the condition cost the
     // FP16 P.V ones of head_dim 64 1 % (8 heads of 1024 rows: 28.8 instead of 28.4 us).
     [[maybe_unused]] bool on = false, on_prev = false;
-    auto enter = [&](int j) { if constexpr (LISTED) { on_prev = on; on = j < ntiles && sees(j) != 0; } };
+    auto enter = [&](int j) { if constexpr (LISTED) { on_prev = on; on = j < ntiles && sees(j); } };
     auto if_on = [&](int j, auto work, auto otherwise) {
       if constexpr (LISTED) { if (on) work(); else otherwise(); }
       else if (j < wave_ntiles) work();

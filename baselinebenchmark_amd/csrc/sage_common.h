@@ -72,10 +72,10 @@ __host__ __device__ inline SagePlanLayout plan_layout(int nseq, int total_q) {
 
 // ---------------------------------------------------------------------------------------------
 // Packed boolean mask: one bit per (query row, key), in the order in which the attention kernel's accumulators hold the
-// scores, and one visibility class per 32 query rows and key tile.
+// scores, and one visibility bit per 32 query rows and key tile.
 //   bits: [plane][q-tile of 256 rows][tile of 128 keys][row][h = 0, 1] -> 64 bits; bit 16 * nt + r is key
 //         32 * nt + 8 * (r / 4) + 4 * h + r % 4 of the tile (0 past the last key and in rows past the last one)
-//   classes: uint16 [plane][q-tile][tile], two bits per group of 32 rows: 0 no key visible, 1 some, 2 all of them
+//   seen: uint8 [plane][q-tile][tile], bit g: some row of the q-tile's 32-row group g sees some key of the tile
 // A plane is one distinct [Sq, Skv] slice of the mask (broadcast batches and heads share one); a mask that is the same
 // for every query row has one q-tile, whatever Sq is.
 // ---------------------------------------------------------------------------------------------
@@ -96,7 +96,7 @@ inline MaskPlanes mask_planes(int B, int Hq, int Sq, int Skv, int64_t m_sb, int6
   p.ntk = (Skv + kMaskKeys - 1) / kMaskKeys;
   const int64_t tiles = (int64_t)p.planes * p.nqt * p.ntk;
   p.bits_bytes = tiles * kMaskTileBytes;
-  p.total_bytes = p.bits_bytes + (tiles * 2 + 255) / 256 * 256;
+  p.total_bytes = p.bits_bytes + (tiles + 255) / 256 * 256;
   return p;
 }
 

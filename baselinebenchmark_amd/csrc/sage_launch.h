@@ -134,7 +134,7 @@ struct AttnArgs {
   float q_mult;
   const u16* q_dot_km;      // K mean [B, Hkv, D] (packed: [nseq, Hkv, D]) in the type of q, or null: its product with the scaled row joins the row's LSE2
   const uint8_t* mask_bits; // packed boolean mask (sage_common.h) or null: taken instead of `mask`
-  const u16* mask_cls;
+  const uint8_t* mask_seen;
   int mask_pb, mask_ph, mask_nqt, mask_ntk;
 };
 
@@ -152,7 +152,7 @@ hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dt
 
 // Packs a boolean mask [B, Hq, Sq, Skv] with element strides into the form of sage_common.h.
 hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,
-                            int Skv, uint8_t* bits, u16* cls, hipStream_t st);
+                            int Skv, uint8_t* bits, uint8_t* seen, hipStream_t st);
 
 AttnConfig attn_config(int D, int pv, bool packed);
 // Fills in the launch constants of the tile decode from the dimensions already in `a` (B, Hq, Hkv, nqt, cu_q).

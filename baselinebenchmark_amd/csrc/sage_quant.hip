@@ -474,7 +474,7 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
 }
 
 // ---------------------------------------------------------------------------------------------
-// Boolean mask -> bits and visibility classes (layout in sage_common.h).  One workgroup per (key tile, q-tile, plane): the
+// Boolean mask -> bits and visibility (layout in sage_common.h).  One workgroup per (key tile, q-tile, plane): the
 // mask's bytes are read once, 16 per lane and eight lanes per row where keys are contiguous, and leave as one bit each.
 // ---------------------------------------------------------------------------------------------
 __device__ inline unsigned nonzero_bytes(unsigned x) {   // bit i: byte i of x is not zero
@@ -483,10 +483,10 @@ __device__ inline unsigned nonzero_bytes(unsigned x) {   // bit i: byte i of x i
 }
 
 __global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn,
-                                                        MaskPlanes p, int Sq, int Skv, uint8_t* bits, u16* cls) {
+                                                        MaskPlanes p, int Sq, int Skv, uint8_t* bits, uint8_t* seen) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4), aligned(1)));
   __shared__ __align__(16) uint8_t packed[kMaskTileBytes];
-  __shared__ unsigned wave_cls[4];
+  __shared__ unsigned wave_seen[4];
   const int tile = blockIdx.x, qt = blockIdx.y, tid = threadIdx.x;
   const int heads = p.ph ? (p.pb ? p.pb : p.planes) : 1;   // planes of one batch entry
   const int b = blockIdx.z / heads, hd = blockIdx.z - b * heads;
@@ -537,14 +537,9 @@ __global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int
   const int64_t t = ((int64_t)blockIdx.z * p.nqt + qt) * p.ntk + tile;
   reinterpret_cast<uint4*>(bits + t * kMaskTileBytes)[tid] = row;
   const unsigned long long any = __builtin_amdgcn_ballot_w64((row.x | row.y | row.z | row.w) != 0);
-  const unsigned long long gap = __builtin_amdgcn_ballot_w64(tid < rows && (row.x & row.y & row.z & row.w) != 0xffffffffu);
-  if ((tid & 63) == 0) {
-    const unsigned lo = (unsigned)any == 0 ? 0 : (unsigned)gap == 0 ? 2 : 1;
-    const unsigned hi = (any >> 32) == 0 ? 0 : (gap >> 32) == 0 ? 2 : 1;
-    wave_cls[tid >> 6] = (lo | (hi << 2)) << (4 * (tid >> 6));
-  }
+  if ((tid & 63) == 0) wave_seen[tid >> 6] = ((unsigned)any != 0 ? 1 : 0) | ((any >> 32) != 0 ? 2 : 0);
   __syncthreads();
-  if (tid == 0) cls[t] = (u16)(wave_cls[0] | wave_cls[1] | wave_cls[2] | wave_cls[3]);
+  if (tid == 0) seen[t] = (uint8_t)(wave_seen[0] | wave_seen[1] << 2 | wave_seen[2] << 4 | wave_seen[3] << 6);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -560,8 +555,8 @@ hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_blocks, hipS
 }
 
 hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,
-                            int Skv, uint8_t* bits, u16* cls, hipStream_t st) {
-  mask_pack_kernel<<<dim3(p.ntk, p.nqt, p.planes), dim3(256), 0, st>>>(mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, cls);
+                            int Skv, uint8_t* bits, uint8_t* seen, hipStream_t st) {
+  mask_pack_kernel<<<dim3(p.ntk, p.nqt, p.planes), dim3(256), 0, st>>>(mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, seen);
   return hipGetLastError();
 }
 
