@@ -362,9 +362,11 @@ struct E2EWorkspace {
   size_t q_i8, k_i8, q_scale, k_scale, km, v_scale, panels, stat, plan, lse_off, total;
   int64_t qs_sh, ks_sh, panel_sh;
 };
-// What a call needs beyond K, V and their statistics: the INT8 copy of Q with its scales (only when Q is quantised by the
-// stand-alone pass: an explicit mask, the LSE correction of K smoothing, interleaved Q scales) and the per-row LSE
-// correction term (only when LSE is returned from smoothed keys).
+// What a call's workspace holds beyond K, V and their statistics: the INT8 copy of Q with its scales (calls that may quantise Q by
+// the stand-alone pass: an explicit mask, the LSE correction of K smoothing, interleaved Q scales) and the per-row LSE
+// correction term (LSE of smoothed keys).  LSE calls with K blocks of 32 keys and more form that term in the attention kernel and
+// leave both untouched; the size they ask for stays, so that what the built-in scratch array takes and refuses does not
+// move with the kernel a call happens to use.
 bool needs_q_pass(int blkq, int has_mask, int want_lse, int smooth_k) {
   return has_mask || (want_lse && smooth_k) || blk_groups(blkq) != 1;
 }

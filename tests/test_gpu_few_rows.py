@@ -8,6 +8,8 @@ import pytest
 import torch
 
 import baselinebenchmark_amd as sa
+from baselinebenchmark_amd import _cabi
+from tests.helpers import sageattn_cabi
 
 pytestmark = pytest.mark.gpu
 
@@ -101,3 +103,71 @@ def test_many_heads_of_few_keys(Sq, Skv):
     for i in (0, out.shape[0] // 4 * 2, out.shape[0] - 2):
         assert float(((out[i:i + 2].cpu().double() - want).abs() / (want.abs() + rms)).max()) < 2 * 2.0 ** -8 + 4 * 2.0 ** -11
         assert float((lse[i:i + 2].cpu().double() - want_lse).abs().max()) < 2e-5 * max(1.0, float(want_lse.abs().max()))
+
+
+def _inputs(seed, B, Hq, Hkv, Sq, Skv, D, dtype):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn((B, H, L, D), generator=g) for H, L in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    return tuple(t.to(dtype).cuda() for t in (q, k + 2.0 * torch.randn((D,), generator=g), v))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("smooth", [True, False])
+@pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("-inf")), ("v", float("nan")), ("k", float("inf")), ("k", float("nan")),
+                                         ("q", float("inf")), ("q", float("nan"))])
+def test_infinities_and_nan_reach_what_they_reach_in_the_tiled_kernel(dtype, smooth, where, value):
+    """The rows of a call with 40 of them per head (the tiled kernel), the first two alone (this one): the same elements are
+    NaN, +inf and -inf, in the outputs and the LSE, and none outside the batch entry and KV head that holds the value."""
+    q, k, v = _inputs(11, 2, 8, 2, 40, 1100, 128, dtype)
+    if where == "q":
+        q[0, 5, 1, 3] = value
+    else:
+        {"k": k, "v": v}[where][0, 1, 1099, 3] = value
+    kw = dict(smooth_k=smooth, pv_mode="fp16", BLKQ=16, return_lse=True)
+    tiled = sa.sageattn(q, k, v, **kw)
+    few = sa.sageattn(q[:, :, :2].contiguous(), k, v, **kw)
+    for t, f in zip(tiled, few):
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(t[:, :, :2]), kind(f)), kind
+        assert torch.isfinite(f[1]).all() and torch.isfinite(f[0, :4]).all()
+    if where == "v" or not math.isnan(value):   # (INT8 holds no NaN: the quantiser makes it 0)
+        assert not torch.isfinite(few[0][0, 4:]).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,Hkv,Sq,Skv", [(32, 1, 1, 1025), (2, 2, 32, 2047), (64, 2, 1, 16500), (8, 8, 1, 1100)])
+def test_partial_results_stay_inside_the_workspace(D, Hq, Hkv, Sq, Skv):
+    """The partial results lie where the V panels of other calls do: with exactly the workspace that the call asks for, nothing
+    behind it is written, and the built-in scratch array gives the same bits."""
+    q, k, v = _inputs(Skv, 1, Hq, Hkv, Sq, Skv, D, torch.bfloat16)
+    need = _cabi.lib().sage_sageattn_workspace_bytes_for(1, Hq, Hkv, Sq, Skv, D, 128, 64, _cabi.PV_FP16, 0, 0, 0, 1, 0, 0)
+    ws = torch.full((need + 65536,), 0xA5, device="cuda", dtype=torch.uint8)
+    outs = [torch.full_like(q, float("nan")) for _ in range(2)]
+    assert sageattn_cabi(q, k, v, outs[0], workspace=ws[:need]) == 0, _cabi.lib().sage_last_error().decode()
+    assert sageattn_cabi(q, k, v, outs[1], static=True) == 0, _cabi.lib().sage_last_error().decode()
+    torch.cuda.synchronize()
+    assert bool((ws[need:] == 0xA5).all())
+    assert torch.isfinite(outs[0].float()).all() and torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0], sa.sageattn(q, k, v, pv_mode="fp16"))
+
+
+def test_captured_call_replays_like_eager():
+    shape = (2, 8, 2, 3, 1700, 128, torch.bfloat16)
+    q, k, v = _inputs(1, *shape)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        sa.sageattn(q, k, v, pv_mode="fp16")
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = sa.sageattn(q, k, v, pv_mode="fp16")
+    for seed in (2, 3, 4):
+        fresh = _inputs(seed, *shape)
+        eager = sa.sageattn(*fresh, pv_mode="fp16")   # the program's own eager work between replays
+        torch.cuda.synchronize()
+        for t, n in zip((q, k, v), fresh):
+            t.copy_(n)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), seed
