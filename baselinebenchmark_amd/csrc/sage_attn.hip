@@ -11,6 +11,9 @@ namespace sage {
 // Consecutive entries of the list run at the same time (eight of them per XCD when an XCD holds one KV head), and q-tiles
 // of one sequence walk the same K/V tiles from tile 0 on at about the same pace: one fetches a tile into the XCD's L2, the
 // others hit it there.  Ordered by cost alone, neighbours in the list belong to different sequences and share nothing.
+// (Attention kernel, 32/8 heads, causal, by cost alone / by tiers: 70 sequences of 500..8000 rows 10.67 / 10.06 ms, 80 of 16..1991 1.13 /
+// 1.10.  The price is the last round of the chip: below 2048 keys all q-tiles are one tier, and a long prompt that the batch ends
+// with starts last -- 127 of 64 rows and one of 2000 176 / 182 us, 500 of 100 and one of 1990 over 8 heads 165 / 189.)
 //
 // One workgroup, bound by the latency of its dependent steps.  The cost of a q-tile does not decrease with its index, so the
 // tiles of a sequence in one tier are a contiguous range with ends in closed form, and no tile is ever visited to be counted:
