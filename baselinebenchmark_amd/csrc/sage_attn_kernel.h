@@ -1060,16 +1060,20 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     const int grp = (w >> GSH) & 1;
     // Work of this wavefront on the tile of period j, and on that of period j - 1, if it sees them.  Unlisted kernels branch on
     // their tile count at every use: as a flag that is computed first and carried through the period, the condition cost the
-    // FP16 P.V ones of head_dim 64 1 % (8 heads of 1024 rows: 28.8 instead of 28.4 us).
+    // FP16 P.V ones of head_dim 64 1 % (8 heads of 1024 rows: 28.8 instead of 28.4 us; 2 of 20000, 128-key scales: 268 / 260).  Causal
+    // ones on ready INT8 operands with 128-key scales are the exception (2 heads of 20000 rows: 228 us carried, 232 at every use).
+    constexpr bool CARRIED = LISTED || (PV == 0 && CAUSAL && !QF && KW == 4);
     [[maybe_unused]] bool on = false, on_prev = false;
-    auto enter = [&](int j) { if constexpr (LISTED) { on_prev = on; on = j < ntiles && sees(j); } };
+    auto enter = [&](int j) { if constexpr (CARRIED) { on_prev = on; on = LISTED ? j < ntiles && sees(j) : j < wave_ntiles; } };
     auto if_on = [&](int j, auto work, auto otherwise) {
-      if constexpr (LISTED) { if (on) work(); else otherwise(); }
-      else if (j < wave_ntiles) work();
+      if constexpr (!CARRIED) { if (j < wave_ntiles) work(); }
+      else if (on) work();
+      else if constexpr (LISTED) otherwise();
     };
     auto if_was_on = [&](int j, auto work, auto otherwise) {
-      if constexpr (LISTED) { if (on_prev) work(); else if (j >= 1) otherwise(); }
-      else if (j >= 1 && j - 1 < wave_ntiles) work();
+      if constexpr (!CARRIED) { if (j >= 1 && j - 1 < wave_ntiles) work(); }
+      else if (LISTED ? on_prev : j >= 1 && j - 1 < wave_ntiles) work();
+      else if constexpr (LISTED) { if (j >= 1) otherwise(); }
     };
     auto nothing = [] {};
     // (the scores of a skipped tile hold nothing: said so, they need no registers across the period)
