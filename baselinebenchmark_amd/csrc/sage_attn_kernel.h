@@ -760,9 +760,10 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       }
       // Other strides: one load per score, those of MB 32-key groups in flight at once, as many as the registers hold without a
       // spill.  Left to the compiler they went one by one or spilled (2 x 16 heads of 1500 rows, transposed mask, additive /
-      // boolean, now and then: head_dim 64 FP16 P.V 82 / 274 -> 72 / 78 us, FP8 83 / 82 -> 76 / 76; 128 FP16 282 / 341 -> 101 / 101,
-      // FP8 110 / 108 -> 91 / 90.  MB = 1 at head_dim 64: 88 / 84; MB = 2 at 128, FP8: 99 / 102).
-      constexpr int MB = D == 64 ? 2 : 1;
+      // boolean, now and then: head_dim 64 FP16 P.V 82 / 274 -> 72 / 78 us, FP8 83 / 82 -> 82 / 79; 128 FP16 282 / 341 -> 101 / 101,
+      // FP8 110 / 108 -> 91 / 90.  MB = 1 at head_dim 64, FP16: 88 / 84; MB = 2 at 128, FP8: 99 / 102; at 64, FP8: 76 / 76, but a
+      // call on 200 rows and 200 keys 24.2 to 25.8 instead of 23.6).
+      constexpr int MB = D == 64 && PV == 0 ? 2 : 1;
 #pragma unroll
       for (int b0 = 0; b0 < NT; b0 += MB) {
         mask_t mv[MB][16];
