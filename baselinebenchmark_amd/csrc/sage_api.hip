@@ -101,11 +101,11 @@ int quant_impl(const void* x, int8_t* out, float* scale, const void* km, int B, 
   a.x = (const u16*)x; a.out = out; a.scale = scale; a.km = (const u16*)km;
   a.B = B; a.H = H; a.L = L; a.D = D;
   a.x_sb = x_sb; a.x_sh = x_sh; a.x_sn = x_sn; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
-  a.km_sb = km_sb; a.km_sh = km_sh; a.blk = blk; a.groups = groups; a.mult = mult;
+  a.km_sb = km_sb; a.km_sh = km_sh; a.blk = blk; a.blk_shift = ilog2(blk); a.groups = groups; a.mult = mult;
   a.cu_seqlens = cu_seqlens; a.cu_blocks = cu_blocks; a.scale_sh = scale_sh;
   a.dotv = (const u16*)dot.vec; a.dot_out = dot.out; a.dv_sb = dot.sb; a.dv_sh = dot.sh; a.dv_group = dot.group;
   a.dot_total = dot.total;
-  hipError_t e = launch_quant_int8(a, dtype, (L + blk - 1) / blk, (hipStream_t)stream);
+  hipError_t e = launch_quant_int8(a, dtype, L, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "sage_quant_int8");
   return SAGE_OK;
 }
@@ -552,14 +552,12 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     qa.x = (const u16*)k; qa.out = k_i8; qa.scale = k_scale; qa.km = nullptr;
     qa.B = B; qa.H = Hkv; qa.L = Skv; qa.D = D;
     qa.x_sb = k_sb; qa.x_sh = k_sh; qa.x_sn = k_sn; qa.o_sb = ki_sb; qa.o_sh = ki_sh; qa.o_sn = ki_sn;
-    qa.blk = kb; qa.groups = blk_groups(blkk); qa.mult = 1.0f; qa.dv_group = 1;
+    qa.blk = kb; qa.blk_shift = ilog2(kb); qa.groups = blk_groups(blkk); qa.mult = 1.0f; qa.dv_group = 1;
     PrepVArgs va;
     memset(&va, 0, sizeof(va));
     va.v = (const u16*)v; va.panels = (uint8_t*)panels; va.vscale = v_scale; va.B = B; va.H = Hkv; va.L = Skv; va.D = D;
     va.v_sb = v_sb; va.v_sh = v_sh; va.v_sn = v_sn;
-    hipError_t e = launch_prepass_small(qa, va, dtype, pv_mode == SAGE_PV_FP8, (Skv + kb - 1) / kb,
-                                        (Skv + SAGE_PANEL_ROWS - 1) / SAGE_PANEL_ROWS, smooth_k != 0, km, v_scale,
-                                        (hipStream_t)stream);
+    hipError_t e = launch_prepass_small(qa, va, dtype, pv_mode == SAGE_PV_FP8, smooth_k != 0, km, v_scale, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sage_sageattn(pre-pass)");
   } else {
     if (smooth_k) {

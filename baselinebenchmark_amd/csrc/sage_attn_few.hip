@@ -39,22 +39,11 @@ __device__ inline float xor16_32_sum(float x) {
   return x + __shfl_xor(x, 32);
 }
 
-// q = trunc(x / scale + 0.5 sgn(x)) of sixteen values, as quant_int8_kernel computes it.
 template <class Quotient>
 __device__ __forceinline__ v4i pack16(const float (&x)[16], Quotient quotient) {
-  uint32_t packed[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < 16; i++) {
-    float z = quotient(x[i]);
-    z = z + __builtin_copysignf(0.5f, z);
-    packed[i >> 2] |= (uint32_t)((int)z & 0xff) << (8 * (i & 3));
-  }
+  uint32_t packed[4];
+  pack_codes(x, packed, quotient);
   return v4i{(int)packed[0], (int)packed[1], (int)packed[2], (int)packed[3]};
-}
-
-// True where the reciprocal with one correction step is the correctly rounded quotient (div_by_uniform).
-__device__ inline bool reciprocal_is_exact(float scale) {
-  return (__builtin_bit_cast(uint32_t, scale) & 0x7fffffu) != 0x7fffffu && scale < 1.0e30f;
 }
 
 template <int DT, int D, int MT>
@@ -144,8 +133,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 #pragma unroll
         for (int s = 0; s < KS; s++) qreg[mt][s] = pack16(x[mt][s], [&](float v) { return div_by_uniform(v, scale, rcp); });
       } else {
+        const double wide = 1.0 / (double)scale;
 #pragma unroll
-        for (int s = 0; s < KS; s++) qreg[mt][s] = pack16(x[mt][s], [&](float v) { return v / scale; });
+        for (int s = 0; s < KS; s++) qreg[mt][s] = pack16(x[mt][s], [&](float v) { return div_by_any(v, wide); });
       }
     }
   }
@@ -192,10 +182,12 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
       for (int i = 0; i < LK; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const uint32_t x = kraw[t][i][e];
-          const u16 lo = from_f32<DT>(to_f32<DT>((u16)x) - kmf[i][2 * e]), hi = from_f32<DT>(to_f32<DT>((u16)(x >> 16)) - kmf[i][2 * e + 1]);
-          kraw[t][i][e] = gone ? 0u : (uint32_t)lo | ((uint32_t)hi << 16);
-          mx = fmaxf(mx, fmaxf(fabsf(to_f32<DT>(lo)), fabsf(to_f32<DT>(hi))));
+          float lo, hi;
+          unpack2<DT>(kraw[t][i][e], lo, hi);
+          const uint32_t x = pack2<DT>(lo - kmf[i][2 * e], hi - kmf[i][2 * e + 1]);
+          kraw[t][i][e] = gone ? 0u : x;
+          unpack2<DT>(x, lo, hi);
+          mx = fmaxf(mx, fmaxf(fabsf(lo), fabsf(hi)));
         }
       amax[t] = wave_max(gone ? 0.f : mx);
     }
@@ -221,7 +213,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; e++) x[e] = to_f32<DT>((u16)(kraw[t][2 * s + (e >> 3)][(e & 7) >> 1] >> (16 * (e & 1))));
         if (fast) kreg[t][s] = pack16(x, [&](float v) { return div_by_uniform(v, scale, rcp); });
-        else kreg[t][s] = pack16(x, [&](float v) { return v / scale; });
+        else kreg[t][s] = pack16(x, [&, wide = 1.0 / (double)scale](float v) { return div_by_any(v, wide); });
       }
     }
     if (tile + 1 < t1) load_k(tile + 1);

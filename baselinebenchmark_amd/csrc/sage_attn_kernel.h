@@ -41,6 +41,7 @@
 #include "sage_launch.h"
 #include <atomic>
 #include <cstdlib>
+#include <type_traits>
 // Tuning constants of the matrix phase (measured: one more or one fewer fragment ahead is within +-1 %).
 #define SAGE_KPF 4   // K fragments read ahead of the Q.K^T MFMA that consumes them
 #define SAGE_VPF 3   // V fragment pairs read ahead of the P.V MFMA that consumes them
@@ -518,26 +519,37 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     float x[KS][16];
     float amax = 0.f;
     [[maybe_unused]] float dot = 0.f;
+    // (one copy per input type: the type is uniform, and widening both ways and selecting per element is three instructions for one)
+    auto read_rows = [&](auto type) __attribute__((always_inline)) {
+      constexpr int DT = decltype(type)::value;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      uint4 raw[2];
+      for (int ks = 0; ks < KS; ks++) {
+        uint4 raw[2];
 #pragma unroll
-      for (int e = 0; e < 2; e++)
-        raw[e] = *reinterpret_cast<const uint4*>(qstage + m * (D * 2) + 16 * ((4 * ks + 2 * h + e) ^ (m & (QUPR - 1))));
-      const u16* e = reinterpret_cast<const u16*>(raw);
+        for (int e = 0; e < 2; e++)
+          raw[e] = *reinterpret_cast<const uint4*>(qstage + m * (D * 2) + 16 * ((4 * ks + 2 * h + e) ^ (m & (QUPR - 1))));
+        const uint32_t* x2 = reinterpret_cast<const uint32_t*>(raw);
 #pragma unroll
-      for (int i = 0; i < 16; i++) {
-        x[ks][i] = (a.q_is_bf16 ? bf16_to_f32(e[i]) : f16_to_f32(e[i])) * a.q_mult;
-        amax = fmaxf(amax, fabsf(x[ks][i]));
-      }
-      if constexpr (DOT) {
+        for (int i = 0; i < 8; i++) {
+          float lo, hi;
+          unpack2<DT>(x2[i], lo, hi);
+          x[ks][2 * i] = lo * a.q_mult;
+          x[ks][2 * i + 1] = hi * a.q_mult;
+          amax = fmaxf(amax, fmaxf(fabsf(x[ks][2 * i]), fabsf(x[ks][2 * i + 1])));
+        }
+        if constexpr (DOT) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-          const u16 bits = (u16)(kmr[ks][i >> 3][(i & 7) >> 1] >> (16 * (i & 1)));
-          dot = __builtin_fmaf(x[ks][i], a.q_is_bf16 ? bf16_to_f32(bits) : f16_to_f32(bits), dot);
+          for (int i = 0; i < 8; i++) {
+            float lo, hi;
+            unpack2<DT>(kmr[ks][i >> 2][i & 3], lo, hi);
+            dot = __builtin_fmaf(x[ks][2 * i], lo, dot);
+            dot = __builtin_fmaf(x[ks][2 * i + 1], hi, dot);
+          }
         }
       }
-    }
+    };
+    if (a.q_is_bf16) read_rows(std::integral_constant<int, 1>());
+    else read_rows(std::integral_constant<int, 0>());
     if constexpr (DOT) {
       dot = xchg32_sum(dot);
       if (h == 0) row_dot[w * 32 + m] = dot;   // read again by this very lane, in the epilogue
@@ -556,25 +568,20 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     }
     const float scale = fmaxf(amax / 127.0f, kScaleFloor);
     const float rcp = 1.0f / scale;
-    const uint32_t sbits = __builtin_bit_cast(uint32_t, scale);
-    const bool fast = ((sbits & 0x7fffffu) != 0x7fffffu) && scale < 1.0e30f;
     // (one uniform branch around the whole tile, not one per element: the two quotients are the same numbers)
     auto quantise_rows = [&](auto quotient) __attribute__((always_inline)) {
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
-        uint32_t packed[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-          float z = quotient(x[ks][i]);
-          z = z + __builtin_copysignf(0.5f, z);
-          int qv = (int)z;
-          packed[i >> 2] |= (uint32_t)(qv & 0xff) << (8 * (i & 3));
-        }
+        uint32_t packed[4];
+        pack_codes(x[ks], packed, quotient);
         qreg[ks] = v4i{(int)packed[0], (int)packed[1], (int)packed[2], (int)packed[3]};
       }
     };
-    if (fast) quantise_rows([&](float v) { return div_by_uniform(v, scale, rcp); });
-    else quantise_rows([&](float v) { return v / scale; });
+    if (reciprocal_is_exact(scale)) quantise_rows([&](float v) { return div_by_uniform(v, scale, rcp); });
+    else {
+      const double wide = 1.0 / (double)scale;
+      quantise_rows([&](float v) { return div_by_any(v, wide); });
+    }
     qscale = scale;
   }
 

@@ -16,6 +16,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef unsigned short u16;
 
 constexpr int kWave = 64;
@@ -119,6 +120,19 @@ __device__ inline u16 from_f32(float f) {
   if constexpr (DT == 1) return f32_to_bf16(f);
   else return f32_to_f16(f);
 }
+// Two values narrowed into one dword by one instruction (v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32, both round to nearest even).
+template <int DT>
+__device__ inline uint32_t pack2(float lo, float hi) {
+  const v2f v = {lo, hi};
+  if constexpr (DT == 1) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2bf));
+  else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, v2h));
+}
+// Both halves of a dword widened.
+template <int DT>
+__device__ inline void unpack2(uint32_t x, float& lo, float& hi) {
+  if constexpr (DT == 1) { lo = __builtin_bit_cast(float, x << 16); hi = __builtin_bit_cast(float, x & 0xffff0000u); }
+  else { lo = f16_to_f32((u16)x); hi = f16_to_f32((u16)(x >> 16)); }
+}
 
 // ---------------------------------------------------------------------------------------------
 // Streaming accesses of the pre-pass kernels: every byte of an operand is touched once per pass and not again before
@@ -171,11 +185,40 @@ constexpr float kScaleFloor = 1.0e-12f;
 // Correctly rounded x / s for a wavefront-uniform divisor whose reciprocal r = RN(1/s) is given.
 // q0 = RN(x*r) is within 1 ulp of x/s; e = x - q0*s is exact in one FMA; RN(q0 + e*r) is then
 // the correctly rounded quotient (Markstein's correction step), provided s's significand is not
-// all ones and nothing under/overflows; the caller falls back to a true division otherwise.
+// all ones and nothing under/overflows; the caller takes div_by_any otherwise.
 __device__ inline float div_by_uniform(float x, float s, float r) {
   float q0 = x * r;
   float e = __builtin_fmaf(-q0, s, x);
   return __builtin_fmaf(e, r, q0);
+}
+// True where that holds for the divisor s.
+__device__ inline bool reciprocal_is_exact(float s) {
+  return (__builtin_bit_cast(uint32_t, s) & 0x7fffffu) != 0x7fffffu && s < 1.0e30f;
+}
+// The same quotient for any divisor, given r = RN(1/s) in binary64: x * r is off by less than 2^-51 of itself, and a quotient of
+// two 24-bit significands that is no binary32 number keeps 2^-49 of itself away from every point where binary32 rounding changes.
+// (Three instructions an element; inlined true divisions were a tenth of the attention kernels' code, nearly never run.)
+__device__ inline float div_by_any(float x, double r) { return (float)((double)x * r); }
+
+// INT8 codes of N quotients (a multiple of four): q = trunc(z + 0.5 sgn(z)), four to a dword.  |z| <= 127.5, so the low byte of the
+// converted integer is the code, and three byte permutes gather four of them (masks and shifts took twice the instructions).
+template <int N, class Quotient>
+__device__ __forceinline__ void pack_codes(const float (&x)[N], uint32_t (&packed)[N / 4], Quotient quotient) {
+#pragma unroll
+  for (int i = 0; i < N; i += 4) {
+    int q[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      // For |x| so small that the residual of the correction step is subnormal the quotient is
+      // below 1e-13 in magnitude (scale >= 1e-12): whatever its last bits, it rounds to 0.
+      float z = quotient(x[i + e]);
+      z = z + __builtin_copysignf(0.5f, z);   // +0.5 for z >= 0 (incl. -0: -0.5 + -0 = -0.5 -> 0), else -0.5
+      q[e] = (int)z;   // truncation toward zero
+    }
+    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)q[1], (uint32_t)q[0], 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)q[3], (uint32_t)q[2], 0x0c0c0400u);
+    packed[i / 4] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+  }
 }
 
 

@@ -11,7 +11,7 @@ struct QuantArgs {
   const u16* km;
   int B, H, L, D;
   int64_t x_sb, x_sh, x_sn, o_sb, o_sh, o_sn, km_sb, km_sh;
-  int blk;
+  int blk, blk_shift;   // rows per scale block and their log2
   int groups;   // scales per block: 1; 8 (scale g covers the rows r of the block with r % 8 == g); 4 ((r % 8) / 2 == g); fixed-length only
   float mult;
   const int32_t* cu_seqlens;
@@ -140,15 +140,15 @@ struct AttnArgs {
 
 struct AttnConfig { int nw, bn; };
 
-hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_blocks, hipStream_t st);
+hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_rows, hipStream_t st);
 int colstat_chunks(int L);
 hipError_t launch_k_mean(const ColStatArgs& a, int dtype, void* km, hipStream_t st);
 hipError_t launch_v_scale(const ColStatArgs& a, int dtype, float* vscale, hipStream_t st);
 hipError_t launch_prep_v(const PrepVArgs& a, int dtype, int pv, int max_panels, hipStream_t st);
-// Short fixed-length sequences: K mean + K quantiser + V scale + V panels in one launch (nk K tiles and nv V panels per
-// (batch, kv-head); km_out / vscale_out take the statistics; qa.km is ignored and must be null).
-hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dtype, int pv, int nk, int nv, int smooth,
-                                void* km_out, float* vscale_out, hipStream_t st);
+// Short fixed-length sequences: K mean + K quantiser + V scale + V panels in one launch (km_out / vscale_out take the statistics;
+// qa.km is ignored and must be null).
+hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dtype, int pv, int smooth, void* km_out,
+                                float* vscale_out, hipStream_t st);
 
 // Packs a boolean mask [B, Hq, Sq, Skv] with element strides into the form of sage_common.h.
 hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,

@@ -14,19 +14,30 @@
 
 namespace sage {
 
-// One workgroup (256 lanes) quantises one [blk, D] tile held entirely in registers:
-// pass 1 converts and reduces |x| to the tile maximum, pass 2 divides and rounds.
-// A lane owns 16 consecutive channels of a row (two 128-bit loads, one 128-bit store).
+// Geometry of the quantiser: a workgroup of 256 lanes takes quant_rows(D, blk) consecutive rows of one (batch, head), whole scale
+// blocks of them, and a wavefront quant_passes(D, blk) times quant_wave_rows(D) neighbouring ones, never more than a scale block: the
+// maximum of a block crosses wavefronts only where the block does, and no lane is idle at any block size.
+// Bound by HBM (3 bytes per element) with the vector ALU close behind it: some 12 instructions per element, 19 when the differences
+// were narrowed one by one, widened twice and packed by masks and shifts.  bf16, K mean subtracted, head_dim 128, one kernel: 4 x 32
+// heads of 4096 rows, blocks of 64: 52.0 -> 40.8 us (201 MB, 4.9 TB/s); blocks of 16, 2 x 16 heads of 4096 rows, where a block a
+// workgroup left half the lanes idle: 24.5 -> 13.1.
+__host__ __device__ constexpr int quant_wave_rows(int D) { return 64 / (D / 16); }   // rows of a pass of a wavefront
+__host__ __device__ constexpr int quant_passes(int D, int blk) { return D == 128 ? (blk == 128 ? 4 : 2) : (blk >= 64 ? 2 : 1); }
+__host__ __device__ constexpr int quant_rows(int D, int blk) { return 4 * quant_passes(D, blk) * quant_wave_rows(D); }
+
+// Quantises the rows chunk * quant_rows(D, blk) .. of (batch b, head h), which stay in registers, as floats, between the abs-max and
+// the rounding.  A lane owns 16 consecutive channels of a row (two 128-bit loads, one 128-bit store); all its loads are issued
+// before anything waits for one.
 // (km_lds: the K mean of this (batch, head) in LDS, D values in the input dtype, instead of a.km in global memory:
 // the fused pre-pass of short sequences computes it in the same workgroup.)
 // UNIT: the multiplier is 1 (every K call; x * 1.0f is x, so leaving the product out changes no bit).
-template <int DT, int D, bool UNIT = false>
-__device__ __forceinline__ void quant_int8_tile(const QuantArgs& a, const int blkid, const int h, const int b, const u16* km_lds) {
-  constexpr int TPR = D / 16;       // lanes per row
-  constexpr int RPP = 256 / TPR;    // rows per pass
-  constexpr int MAXP = 128 / RPP;   // passes for the largest tile (128 rows)
-  const int tid = threadIdx.x;
-  const int tr = tid / TPR, tc = tid % TPR;
+template <int DT, int D, int NP, bool UNIT>
+__device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int chunk, const int h, const int b, const u16* km_lds) {
+  constexpr int TPR = D / 16;                  // lanes per row
+  constexpr int RW = quant_wave_rows(D);       // rows per pass of a wavefront
+  constexpr int WROWS = NP * RW;               // rows of a wavefront
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tr = lane / TPR, tc = lane % TPR;
 
   int L = a.L;
   int64_t xbase, obase, sidx, dbase;
@@ -36,142 +47,144 @@ __device__ __forceinline__ void quant_int8_tile(const QuantArgs& a, const int bl
     dbase = (int64_t)h * a.dot_total + s0;
     xbase = (int64_t)s0 * a.x_sn + (int64_t)h * a.x_sh;
     obase = (int64_t)s0 * a.o_sn + (int64_t)h * a.o_sh;
-    sidx = (int64_t)h * a.scale_sh + a.cu_blocks[b] + blkid;
+    sidx = (int64_t)h * a.scale_sh + a.cu_blocks[b];
   } else {
     xbase = (int64_t)b * a.x_sb + (int64_t)h * a.x_sh;
     obase = (int64_t)b * a.o_sb + (int64_t)h * a.o_sh;
-    sidx = (((int64_t)b * a.H + h) * ((L + a.blk - 1) / a.blk) + blkid) * a.groups;
+    sidx = (((int64_t)b * a.H + h) * ((L + a.blk - 1) >> a.blk_shift)) * a.groups;
     dbase = ((int64_t)b * a.H + h) * L;
   }
-  const int n0 = blkid * a.blk;
+  const int n0 = chunk * 4 * WROWS;
   if (n0 >= L) return;
-  const int rows = min(a.blk, L - n0);
+  const int wrow = n0 + w * WROWS, row = wrow + tr;   // first row of the wavefront, of this lane
 
-  float kmv[16];
-  const bool has_km = a.km != nullptr || km_lds != nullptr;
-  if (km_lds) {
+  // (rows past the end read the last one again: no branch between the loads)
+  uint4 raw[NP][2];
 #pragma unroll
-    for (int i = 0; i < 16; i++) kmv[i] = to_f32<DT>(km_lds[tc * 16 + i]);
-  } else if (has_km) {
-    const uint4* kp = reinterpret_cast<const uint4*>(a.km + (int64_t)b * a.km_sb + (int64_t)h * a.km_sh + tc * 16);
-    uint4 raw2[2] = {kp[0], kp[1]};
-    const u16* p = reinterpret_cast<const u16*>(raw2);
-#pragma unroll
-    for (int i = 0; i < 16; i++) kmv[i] = to_f32<DT>(p[i]);
+  for (int p = 0; p < NP; p++) {
+    const u16* src = a.x + xbase + (int64_t)min(row + p * RW, L - 1) * a.x_sn + tc * 16;
+    raw[p][0] = load_stream16(src);
+    raw[p][1] = load_stream16(src + 8);
   }
   // k - km is rounded to the input dtype (quant_per_block.py:53-54: the subtraction happens in torch, in
-  // the tensor's dtype) once, while loading; both passes then see the rounded difference.
-  auto smoothed = [&](u16 bits, int i) { return has_km ? from_f32<DT>(to_f32<DT>(bits) - kmv[i]) : bits; };
-  auto value = [&](u16 bits) { return UNIT ? to_f32<DT>(bits) : to_f32<DT>(bits) * a.mult; };   // the fp32 value that is quantised
-
-  // Optional side output: the dot product of every (scaled) row with a per-(batch, kv-head) vector.
-  // The one-call pipeline uses it with the K mean to return the LSE of the unsmoothed logits.
-  const bool has_dot = a.dot_out != nullptr;
-  float dvv[16];
-  if (has_dot) {
-    const uint4* dp = reinterpret_cast<const uint4*>(a.dotv + (int64_t)b * a.dv_sb + (int64_t)(h / a.dv_group) * a.dv_sh + tc * 16);
-    uint4 raw2[2] = {dp[0], dp[1]};
-    const u16* p = reinterpret_cast<const u16*>(raw2);
+  // the tensor's dtype); both passes then see the rounded difference.
+  if (a.km != nullptr || km_lds != nullptr) {
+    uint4 kmr[2];
+    if (km_lds) {
+      kmr[0] = *reinterpret_cast<const uint4*>(km_lds + tc * 16);
+      kmr[1] = *reinterpret_cast<const uint4*>(km_lds + tc * 16 + 8);
+    } else {
+      const uint4* kp = reinterpret_cast<const uint4*>(a.km + (int64_t)b * a.km_sb + (int64_t)h * a.km_sh + tc * 16);
+      kmr[0] = kp[0];
+      kmr[1] = kp[1];
+    }
+    const uint32_t* km2 = reinterpret_cast<const uint32_t*>(kmr);
 #pragma unroll
-    for (int i = 0; i < 16; i++) dvv[i] = to_f32<DT>(p[i]);
-  }
-
-  uint4 raw[MAXP][2];
-  float amax = 0.f;
+    for (int i = 0; i < 8; i++) {
+      float mlo, mhi;
+      unpack2<DT>(km2[i], mlo, mhi);
 #pragma unroll
-  for (int p = 0; p < MAXP; p++) {
-    int r = p * RPP + tr;
-    raw[p][0] = raw[p][1] = make_uint4(0, 0, 0, 0);
-    float dsum = 0.f;
-    if (r < rows) {
-      const u16* src = a.x + xbase + (int64_t)(n0 + r) * a.x_sn + tc * 16;
-      raw[p][0] = load_stream16(src);
-      raw[p][1] = load_stream16(src + 8);
-      if (has_km) {
-        const u16* e = reinterpret_cast<const u16*>(raw[p]);
-        uint32_t d[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) d[i] = (uint32_t)smoothed(e[2 * i], 2 * i) | ((uint32_t)smoothed(e[2 * i + 1], 2 * i + 1) << 16);
-        raw[p][0] = make_uint4(d[0], d[1], d[2], d[3]);
-        raw[p][1] = make_uint4(d[4], d[5], d[6], d[7]);
-      }
-      const u16* e = reinterpret_cast<const u16*>(raw[p]);
-#pragma unroll
-      for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(value(e[i])));
-      if (has_dot) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) dsum = __builtin_fmaf(value(e[i]), dvv[i], dsum);
+      for (int p = 0; p < NP; p++) {
+        uint32_t* x2 = reinterpret_cast<uint32_t*>(raw[p]);
+        float lo, hi;
+        unpack2<DT>(x2[i], lo, hi);
+        x2[i] = pack2<DT>(lo - mlo, hi - mhi);
       }
     }
-    if (has_dot) {   // uniform branch; the TPR lanes of a row are neighbours inside one wavefront
+  }
+  float x[NP][16];   // the fp32 values that are quantised
+  float amax = 0.f;
 #pragma unroll
-      for (int o = 1; o < TPR; o <<= 1) dsum += __shfl_xor(dsum, o);
-      if (r < rows && tc == 0) a.dot_out[dbase + n0 + r] = dsum;
+  for (int p = 0; p < NP; p++) {
+    const uint32_t* x2 = reinterpret_cast<const uint32_t*>(raw[p]);
+    float mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      unpack2<DT>(x2[i], x[p][2 * i], x[p][2 * i + 1]);
+      if constexpr (!UNIT) { x[p][2 * i] *= a.mult; x[p][2 * i + 1] *= a.mult; }
+      mx = fmaxf(mx, fmaxf(fabsf(x[p][2 * i]), fabsf(x[p][2 * i + 1])));
+    }
+    amax = fmaxf(amax, row + p * RW < L ? mx : 0.f);
+  }
+  // Optional side output: the dot product of every (scaled) row with a per-(batch, kv-head) vector.
+  // The one-call pipeline uses it with the K mean to return the LSE of the unsmoothed logits.
+  if (a.dot_out != nullptr) {
+    const uint4* dp = reinterpret_cast<const uint4*>(a.dotv + (int64_t)b * a.dv_sb + (int64_t)(h / a.dv_group) * a.dv_sh + tc * 16);
+    const uint4 raw2[2] = {dp[0], dp[1]};
+    const uint32_t* d2 = reinterpret_cast<const uint32_t*>(raw2);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      float dsum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        float lo, hi;
+        unpack2<DT>(d2[i], lo, hi);
+        dsum = __builtin_fmaf(x[p][2 * i], lo, dsum);
+        dsum = __builtin_fmaf(x[p][2 * i + 1], hi, dsum);
+      }
+#pragma unroll
+      for (int o = 1; o < TPR; o <<= 1) dsum += __shfl_xor(dsum, o);   // the TPR lanes of a row are neighbours
+      if (row + p * RW < L && tc == 0) a.dot_out[dbase + row + p * RW] = dsum;
     }
   }
   __shared__ float wmax[4];
-  __shared__ int gmax[8];
+  __shared__ int gmax[4][8];
+  const int wpb = a.blk / WROWS;               // wavefronts per scale block (1, 2 or 4)
+  const int blk_first = w & ~(wpb - 1);        // first wavefront of this one's block
+  const int blkid = wrow >> a.blk_shift;
+  const bool block_there = blkid << a.blk_shift < L;
   if (a.groups == 1) {
     amax = wave_max(amax);
-    if ((tid & 63) == 0) wmax[tid >> 6] = amax;
-    __syncthreads();
-    amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    if (wpb > 1) {
+      if (lane == 0) wmax[w] = amax;
+      __syncthreads();
+      for (int i = 0; i < wpb; i++) amax = fmaxf(amax, wmax[blk_first + i]);
+    }
   } else {
     // Interleaved scales per block (eight: group = row % 8; four: group = (row % 8) / 2): every row this lane holds has
-    // the same index modulo 8 (the passes are RPP rows apart, a multiple of 8), so the lane belongs to one group.
-    // Maximum over the lanes of a row, then over the rows of the group through LDS (the values are non-negative
+    // the same index modulo 8 (a wavefront's rows start at a multiple of 8 and its passes are RW rows apart), so the lane belongs
+    // to one group.  Maximum over the lanes of a row, then over the rows of the group through LDS (the values are non-negative
     // floats: their bit patterns order like integers).
-    static_assert(RPP % 8 == 0, "a lane's rows must share their index modulo 8");
-    if (tid < 8) gmax[tid] = 0;
+    static_assert(RW % 8 == 0 && WROWS % 8 == 0, "a lane's rows must share their index modulo 8");
+    if (threadIdx.x < 32) gmax[threadIdx.x >> 3][threadIdx.x & 7] = 0;
     __syncthreads();
 #pragma unroll
     for (int o = 1; o < TPR; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
     const int gid = a.groups == 8 ? (tr & 7) : ((tr & 7) >> 1);
-    if (tc == 0) atomicMax(&gmax[gid], __builtin_bit_cast(int, amax));
+    if (tc == 0) atomicMax(&gmax[blk_first][gid], __builtin_bit_cast(int, amax));
     __syncthreads();
-    amax = __builtin_bit_cast(float, gmax[gid]);
+    amax = __builtin_bit_cast(float, gmax[blk_first][gid]);
   }
   const float scale = fmaxf(amax / 127.0f, kScaleFloor);
-  if (a.groups == 1) { if (tid == 0) a.scale[sidx] = scale; }
-  else if (tc == 0 && tr < a.groups) a.scale[sidx + tr] = fmaxf(__builtin_bit_cast(float, gmax[tr]) / 127.0f, kScaleFloor);   // group tr's scale
+  if (w == blk_first && block_there) {
+    if (a.groups == 1) { if (lane == 0) a.scale[sidx + blkid] = scale; }
+    else if (lane < a.groups) a.scale[sidx + (int64_t)blkid * a.groups + lane] = fmaxf(__builtin_bit_cast(float, gmax[blk_first][lane]) / 127.0f, kScaleFloor);
+  }
 
   const float rcp = 1.0f / scale;
-  // The fast correction-step division needs: significand of scale not all ones, and scale and rcp
-  // comfortably normal.  |quotient| <= 127.5, scale >= 1e-12.
-  const uint32_t sbits = __builtin_bit_cast(uint32_t, scale);
-  const bool fast = ((sbits & 0x7fffffu) != 0x7fffffu) && scale < 1.0e30f;
-
-  // One wavefront-uniform branch around the whole second pass, not one per element (the scale is uniform over the tile,
-  // or, with interleaved scales, over a lane group: if any lane of the wavefront needs the true division, all take it --
+  // One wavefront-uniform branch around the whole second pass, not one per element (the scale is uniform over the wavefront,
+  // or, with interleaved scales, over a lane group: if any lane of the wavefront needs the general division, all take it --
   // where the correction step applies, the two quotients are the same numbers).
   auto quantise_rows = [&](auto quotient) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 0; p < MAXP; p++) {
-      int r = p * RPP + tr;
-      if (r < rows) {
-        const u16* e = reinterpret_cast<const u16*>(raw[p]);
-        uint32_t packed[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-          // For |x| so small that the residual of the correction step is subnormal the quotient is
-          // below 1e-13 in magnitude (scale >= 1e-12): whatever its last bits, it rounds to 0.
-          float z = quotient(value(e[i]));
-          z = z + __builtin_copysignf(0.5f, z);   // +0.5 for z >= 0 (incl. -0: -0.5 + -0 = -0.5 -> 0), else -0.5
-          int q = (int)z;  // truncation toward zero
-          packed[i >> 2] |= (uint32_t)(q & 0xff) << (8 * (i & 3));
-        }
-        store_stream16(a.out + obase + (int64_t)(n0 + r) * a.o_sn + tc * 16, make_uint4(packed[0], packed[1], packed[2], packed[3]));
-      }
+    for (int p = 0; p < NP; p++) {
+      uint32_t packed[4];
+      pack_codes(x[p], packed, quotient);
+      if (row + p * RW < L)
+        store_stream16(a.out + obase + (int64_t)(row + p * RW) * a.o_sn + tc * 16, make_uint4(packed[0], packed[1], packed[2], packed[3]));
     }
   };
-  if (__builtin_amdgcn_ballot_w64(!fast) == 0) quantise_rows([&](float x) { return div_by_uniform(x, scale, rcp); });
-  else quantise_rows([&](float x) { return x / scale; });
+  if (__builtin_amdgcn_ballot_w64(!reciprocal_is_exact(scale)) == 0) quantise_rows([&](float v) { return div_by_uniform(v, scale, rcp); });
+  else {
+    const double wide = 1.0 / (double)scale;
+    quantise_rows([&](float v) { return div_by_any(v, wide); });
+  }
 }
 
-template <int DT, int D>
+template <int DT, int D, int NP>
 __global__ void __launch_bounds__(256) quant_int8_kernel(QuantArgs a) {
-  if (a.mult == 1.0f) quant_int8_tile<DT, D, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
-  else quant_int8_tile<DT, D, false>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
+  if (a.mult == 1.0f) quant_int8_rows<DT, D, NP, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
+  else quant_int8_rows<DT, D, NP, false>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -397,14 +410,14 @@ __global__ void __launch_bounds__(256) prep_v_kernel(PrepVArgs a) {
 // (batch, head): affordable while the sequence is short and the reads hit the L2; six dependent launches of a few
 // microseconds each become one.
 // ---------------------------------------------------------------------------------------------
-template <int DT, int D, int PV>
+template <int DT, int D, int PV, int NP>
 __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVArgs va, int nk, int smooth, u16* km_out,
                                                             float* vscale_out) {
   constexpr int TPR = D / 8, RPP = 256 / TPR;
   const int h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, tr = tid / TPR, tc = tid % TPR;
   __shared__ double red[RPP][D];
-  __shared__ u16 km_l[D];
+  __shared__ __align__(16) u16 km_l[D];
   __shared__ float vs_l[D];
   if ((int)blockIdx.x < nk) {
     if (smooth) {
@@ -440,7 +453,7 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
       }
       __syncthreads();
     }
-    quant_int8_tile<DT, D, true>(qa, blockIdx.x, h, b, smooth ? km_l : nullptr);   // (K: the multiplier is 1)
+    quant_int8_rows<DT, D, NP, true>(qa, blockIdx.x, h, b, smooth ? km_l : nullptr);   // (K: the multiplier is 1)
   } else {
     const int pidx = blockIdx.x - nk;
     if constexpr (PV == 1) {
@@ -545,12 +558,19 @@ __global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int
 // ---------------------------------------------------------------------------------------------
 // Host-side launchers (called from the C ABI in sage_api.hip).
 // ---------------------------------------------------------------------------------------------
-hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_blocks, hipStream_t st) {
-  dim3 grid(max_blocks, a.H, a.B), block(256);
-  if (dtype == 0 && a.D == 64) quant_int8_kernel<0, 64><<<grid, block, 0, st>>>(a);
-  else if (dtype == 0 && a.D == 128) quant_int8_kernel<0, 128><<<grid, block, 0, st>>>(a);
-  else if (dtype == 1 && a.D == 64) quant_int8_kernel<1, 64><<<grid, block, 0, st>>>(a);
-  else quant_int8_kernel<1, 128><<<grid, block, 0, st>>>(a);
+hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_rows, hipStream_t st) {
+  const int rows = quant_rows(a.D, a.blk);
+  dim3 grid((max_rows + rows - 1) / rows, a.H, a.B), block(256);
+#define SAGE_QUANT(DT, DD, NP) quant_int8_kernel<DT, DD, NP><<<grid, block, 0, st>>>(a)
+#define SAGE_QUANT_D(DT) \
+  do { \
+    if (a.D == 64) { if (quant_passes(64, a.blk) == 1) SAGE_QUANT(DT, 64, 1); else SAGE_QUANT(DT, 64, 2); } \
+    else { if (quant_passes(128, a.blk) == 2) SAGE_QUANT(DT, 128, 2); else SAGE_QUANT(DT, 128, 4); } \
+  } while (0)
+  if (dtype == 0) SAGE_QUANT_D(0);
+  else SAGE_QUANT_D(1);
+#undef SAGE_QUANT_D
+#undef SAGE_QUANT
   return hipGetLastError();
 }
 
@@ -591,18 +611,21 @@ hipError_t launch_v_scale(const ColStatArgs& a, int dtype, float* vscale, hipStr
   return hipGetLastError();
 }
 
-hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dtype, int pv, int nk, int nv, int smooth,
-                                void* km_out, float* vscale_out, hipStream_t st) {
+hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dtype, int pv, int smooth, void* km_out,
+                                float* vscale_out, hipStream_t st) {
+  const int rows = quant_rows(qa.D, qa.blk);
+  const int nk = (qa.L + rows - 1) / rows, nv = (va.L + kPanelRows - 1) / kPanelRows;
   if (nk + nv == 0 || qa.B == 0 || qa.H == 0) return hipSuccess;
   dim3 grid(nk + nv, qa.H, qa.B), block(256);
-#define SAGE_PREPASS(DT, DD, PVV) prepass_small_kernel<DT, DD, PVV><<<grid, block, 0, st>>>(qa, va, nk, smooth, (u16*)km_out, vscale_out)
-  if (dtype == 0) {
-    if (qa.D == 64) { if (pv) SAGE_PREPASS(0, 64, 1); else SAGE_PREPASS(0, 64, 0); }
-    else { if (pv) SAGE_PREPASS(0, 128, 1); else SAGE_PREPASS(0, 128, 0); }
-  } else {
-    if (qa.D == 64) { if (pv) SAGE_PREPASS(1, 64, 1); else SAGE_PREPASS(1, 64, 0); }
-    else { if (pv) SAGE_PREPASS(1, 128, 1); else SAGE_PREPASS(1, 128, 0); }
-  }
+#define SAGE_PREPASS(DT, DD, PVV, NP) prepass_small_kernel<DT, DD, PVV, NP><<<grid, block, 0, st>>>(qa, va, nk, smooth, (u16*)km_out, vscale_out)
+#define SAGE_PREPASS_D(DT, PVV) \
+  do { \
+    if (qa.D == 64) { if (quant_passes(64, qa.blk) == 1) SAGE_PREPASS(DT, 64, PVV, 1); else SAGE_PREPASS(DT, 64, PVV, 2); } \
+    else { if (quant_passes(128, qa.blk) == 2) SAGE_PREPASS(DT, 128, PVV, 2); else SAGE_PREPASS(DT, 128, PVV, 4); } \
+  } while (0)
+  if (dtype == 0) { if (pv) SAGE_PREPASS_D(0, 1); else SAGE_PREPASS_D(0, 0); }
+  else { if (pv) SAGE_PREPASS_D(1, 1); else SAGE_PREPASS_D(1, 0); }
+#undef SAGE_PREPASS_D
 #undef SAGE_PREPASS
   return hipGetLastError();
 }
