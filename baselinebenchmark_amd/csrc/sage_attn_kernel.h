@@ -1250,25 +1250,29 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
             f[i] = o[dt][4 * q4 + i] * inv;
             if constexpr (PV == 1) f[i] *= vs_lds[d + i];
           }
-          u16 hv[4];
-#pragma unroll
-          for (int i = 0; i < 4; i++) hv[i] = to_out(f[i]);
-          uint2 pkd = make_uint2((uint32_t)hv[0] | ((uint32_t)hv[1] << 16), (uint32_t)hv[2] | ((uint32_t)hv[3] << 16));
+          const uint2 pkd = make_uint2(to_out(f[0], f[1]), to_out(f[2], f[3]));
           const int u = 4 * dt + q4;    // 16-byte unit of the row; h picks its half
           *reinterpret_cast<uint2*>(stage + em * (D * 2) + ((u ^ (em & (UPR - 1))) * 16) + 8 * eh) = pkd;
         }
       }
     };
-    if (a.out_bf16) normalise_and_stage([](float x) { return f32_to_bf16(x); });
-    else normalise_and_stage([](float x) { return f32_to_f16(x); });
+    if (a.out_bf16) normalise_and_stage([](float lo, float hi) { return pack2<1>(lo, hi); });
+    else normalise_and_stage([](float lo, float hi) { return pack2<0>(lo, hi); });
+    // (every row is read back before the first is stored: with tile loads in this kernel the compiler guards each LDS read by a
+    // wait for all memory traffic, and one read per store made every store wait for the one before it -- 0.6 us a workgroup)
     const int k16 = el % UPR, rsub = el / UPR;
+    v4u val[32 / RPI];
 #pragma unroll
     for (int i = 0; i < 32 / RPI; i++) {
       const int r = i * RPI + rsub;
-      const uint4 val = *reinterpret_cast<const uint4*>(stage + r * (D * 2) + ((k16 ^ (r & (UPR - 1))) * 16));
-      if (row0 + r < Lq)
-        *reinterpret_cast<uint4*>(reinterpret_cast<u16*>(a.out) + ooff + (int64_t)(row0 + r) * a.o_sn + k16 * 8) = val;
+      val[i] = *reinterpret_cast<const v4u*>(stage + r * (D * 2) + ((k16 ^ (r & (UPR - 1))) * 16));
     }
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; i++) asm volatile("" : "+v"(val[i]));   // (read here, not behind the row checks)
+    u16* dst = reinterpret_cast<u16*>(a.out) + ooff + (int64_t)(row0 + rsub) * a.o_sn + k16 * 8;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; i++)
+      if (row0 + i * RPI + rsub < Lq) *reinterpret_cast<v4u*>(dst + (int64_t)(i * RPI) * a.o_sn) = val[i];
   }
 #ifdef SAGE_TIMING
   sage_ts[6] = __builtin_amdgcn_s_memrealtime();   // stores issued
