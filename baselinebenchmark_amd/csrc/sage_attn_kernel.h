@@ -97,6 +97,19 @@ __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// 16 bytes per lane from N LDS addresses, waited for.  In assembly because the compiler guards an LDS read with a wait for ALL
+// outstanding global -> LDS loads of the wavefront: where the data is already there, and younger loads are not wanted yet.
+__device__ inline unsigned lds_address(const void* p) { return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
+__device__ inline void lds_read4(v4u (&x)[4], unsigned a0, unsigned a1, unsigned a2, unsigned a3) {
+  asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]) : "v"(a0), "v"(a1), "v"(a2), "v"(a3) : "memory");
+}
+__device__ inline v4f lds_read1(unsigned a) {
+  v4f x;
+  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(x) : "v"(a) : "memory");
+  return x;
+}
+
 // 16-byte-chunk swizzle of a K row in LDS: consecutive rows read the same logical chunk from
 // different bank groups (64 banks x 4 bytes = 256 bytes per bank row).
 template <int D>
@@ -481,7 +494,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // (16 rows = half a wavefront; 32, 64 or 128 rows = 1, 2 or 4 wavefronts), q = trunc(x32 / scale + 0.5 sgn).  Rows past the
     // end repeat the last row, which belongs to the same (last) scale block or to none.
 #pragma clang fp contract(off)
-    __shared__ float q_block_amax[NW];
+    __shared__ __align__(16) float q_block_amax[NW];
     // The raw rows of this wavefront come in through LDS (1 KB per instruction, whole rows, into a region
     // that no tile uses before the first barrier of the main loop) instead of 32-byte pieces of 32 rows
     // per instruction.  16-byte units of a row are XOR-swizzled with the row index, on the global side as
@@ -519,20 +532,24 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     float x[KS][16];
     float amax = 0.f;
     [[maybe_unused]] float dot = 0.f;
+    // (the K tile requested behind the rows is still on its way)
+    v4u qraw[KS / 2][4];
+    {
+      const unsigned at = lds_address(qstage) + m * (D * 2);
+      auto unit = [&](int u) { return at + 16 * ((u + 2 * h) ^ (m & (QUPR - 1))); };
+#pragma unroll
+      for (int k2 = 0; k2 < KS / 2; k2++) lds_read4(qraw[k2], unit(8 * k2), unit(8 * k2 + 1), unit(8 * k2 + 4), unit(8 * k2 + 5));
+    }
     // (one copy per input type: the type is uniform, and widening both ways and selecting per element is three instructions for one)
     auto read_rows = [&](auto type) __attribute__((always_inline)) {
       constexpr int DT = decltype(type)::value;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
-        uint4 raw[2];
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-          raw[e] = *reinterpret_cast<const uint4*>(qstage + m * (D * 2) + 16 * ((4 * ks + 2 * h + e) ^ (m & (QUPR - 1))));
-        const uint32_t* x2 = reinterpret_cast<const uint32_t*>(raw);
+        const v4u raw[2] = {qraw[ks >> 1][2 * (ks & 1)], qraw[ks >> 1][2 * (ks & 1) + 1]};
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           float lo, hi;
-          unpack2<DT>(x2[i], lo, hi);
+          unpack2<DT>(raw[i >> 2][i & 3], lo, hi);
           x[ks][2 * i] = lo * a.q_mult;
           x[ks][2 * i + 1] = hi * a.q_mult;
           amax = fmaxf(amax, fmaxf(fabsf(x[ks][2 * i]), fabsf(x[ks][2 * i + 1])));
@@ -561,10 +578,12 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     SAGE_T(2, amax);   // the raw Q rows have arrived
     const int wpb = a.blkq >> 5;   // wavefronts per scale block
     if (wpb > 1) {
+      static_assert(NW == 8, "a scale block of 128 rows is one half of the wavefronts");
       if (lane == 0) q_block_amax[w] = amax;
-      __syncthreads();
-      const int w0 = w & ~(wpb - 1);
-      for (int i = 0; i < wpb; i++) amax = fmaxf(amax, q_block_amax[w0 + i]);
+      lds_barrier();
+      const v4f half = lds_read1(lds_address(q_block_amax) + 16 * (w >> 2));
+      const float lo = fmaxf(half[0], half[1]), hi = fmaxf(half[2], half[3]);
+      amax = wpb == 4 ? fmaxf(lo, hi) : (w & 2) ? hi : lo;
     }
     const float scale = fmaxf(amax / 127.0f, kScaleFloor);
     const float rcp = 1.0f / scale;
