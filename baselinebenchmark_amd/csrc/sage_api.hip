@@ -79,10 +79,11 @@ struct RowDot {   // optional side output of the quantiser (see QuantArgs)
   int group = 1, total = 0;
 };
 
-int quant_impl(const void* x, int8_t* out, float* scale, const void* km, int B, int H, int L, int D, int64_t x_sb,
+// Checks a quantiser call and fills in its arguments; a.out stays null where there is nothing to do.
+int quant_args(QuantArgs& a, const void* x, int8_t* out, float* scale, const void* km, int B, int H, int L, int D, int64_t x_sb,
                int64_t x_sh, int64_t x_sn, int64_t o_sb, int64_t o_sh, int64_t o_sn, int64_t km_sb, int64_t km_sh, int blk,
-               float mult, int dtype, const int32_t* cu_seqlens, const int32_t* cu_blocks, int64_t scale_sh,
-               const RowDot& dot, sage_stream_t stream) {
+               float mult, int dtype, const int32_t* cu_seqlens, const int32_t* cu_blocks, int64_t scale_sh, const RowDot& dot) {
+  memset(&a, 0, sizeof(a));
   if (int rc = check_common(B, H, L, D, dtype)) return rc;
   const int groups = blk_groups(blk);
   blk = blk_rows(blk);
@@ -96,8 +97,6 @@ int quant_impl(const void* x, int8_t* out, float* scale, const void* km, int B, 
   if (int rc = check_stride16("x", x_sb, x_sh, x_sn, 2, x)) return rc;
   if (int rc = check_stride16("out", o_sb, o_sh, o_sn, 1, out)) return rc;
   if (km && int(check_stride16("km", km_sb, km_sh, 0, 2, km))) return SAGE_EINVAL;
-  QuantArgs a;
-  memset(&a, 0, sizeof(a));
   a.x = (const u16*)x; a.out = out; a.scale = scale; a.km = (const u16*)km;
   a.B = B; a.H = H; a.L = L; a.D = D;
   a.x_sb = x_sb; a.x_sh = x_sh; a.x_sn = x_sn; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
@@ -105,8 +104,6 @@ int quant_impl(const void* x, int8_t* out, float* scale, const void* km, int B, 
   a.cu_seqlens = cu_seqlens; a.cu_blocks = cu_blocks; a.scale_sh = scale_sh;
   a.dotv = (const u16*)dot.vec; a.dot_out = dot.out; a.dv_sb = dot.sb; a.dv_sh = dot.sh; a.dv_group = dot.group;
   a.dot_total = dot.total;
-  hipError_t e = launch_quant_int8(a, dtype, L, (hipStream_t)stream);
-  if (e != hipSuccess) return hip_fail(e, "sage_quant_int8");
   return SAGE_OK;
 }
 }  // namespace
@@ -117,8 +114,13 @@ int sage_quant_int8(const void* x, int8_t* out, float* scale, const void* km, in
                     int64_t x_sh, int64_t x_sn, int64_t o_sb, int64_t o_sh, int64_t o_sn, int64_t km_sb, int64_t km_sh,
                     int blk, float mult, int dtype, const int32_t* cu_seqlens, const int32_t* cu_blocks,
                     int64_t scale_sh, sage_stream_t stream) {
-  return quant_impl(x, out, scale, km, B, H, L, D, x_sb, x_sh, x_sn, o_sb, o_sh, o_sn, km_sb, km_sh, blk, mult, dtype,
-                    cu_seqlens, cu_blocks, scale_sh, RowDot(), stream);
+  QuantArgs a;
+  if (int rc = quant_args(a, x, out, scale, km, B, H, L, D, x_sb, x_sh, x_sn, o_sb, o_sh, o_sn, km_sb, km_sh, blk, mult, dtype,
+                          cu_seqlens, cu_blocks, scale_sh, RowDot())) return rc;
+  if (!a.out) return SAGE_OK;
+  hipError_t e = launch_quant_int8(a, dtype, L, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "sage_quant_int8");
+  return SAGE_OK;
 }
 
 size_t sage_k_mean_workspace_bytes(int B, int H, int L, int D) {
@@ -173,6 +175,7 @@ int sage_prep_v(const void* v, void* panels, float* v_scale, void* workspace, si
     if (e != hipSuccess) return hip_fail(e, "sage_prep_v(scale)");
   }
   PrepVArgs a;
+  memset(&a, 0, sizeof(a));
   a.v = (const u16*)v; a.panels = (uint8_t*)panels; a.vscale = v_scale; a.B = B; a.H = H; a.L = L; a.D = D;
   a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn; a.cu_seqlens = cu_seqlens; a.cu_panels = cu_panels; a.panel_sh = panel_sh;
   hipError_t e = launch_prep_v(a, dtype, pv_mode, (L + SAGE_PANEL_ROWS - 1) / SAGE_PANEL_ROWS, st);
@@ -338,21 +341,20 @@ int sage_attn_fwd_masked(const int8_t* q, const int8_t* k, const void* v_panels,
 // ---- one-call pipeline --------------------------------------------------------------------
 namespace {
 // Up to this many keys per sequence and elements of K per call the pre-passes run as one launch whose workgroups read
-// their sequence's statistics themselves (sage_quant.hip: prepass_small_kernel).
+// their sequence's statistics themselves (sage_quant.hip: prepass_small_kernel) instead of two launches, statistics first.
 constexpr int kSmallPrepassRows = 1024;
-constexpr int64_t kSmallPrepassElements = (int64_t)4 << 20;
-// ... and the element reads it makes: every K tile and every V panel re-reads its whole sequence, elements of K times
-// (K tiles + V panels per sequence).  Measured end to end against the six launches: 8 M reads (1 x 8 heads of 1024 rows,
-// head_dim 64, K blocks of 128) 30.0 against 31.2 us; 38 M (the same with K blocks of 16) 33.9 / 33.2; 100 M (1 x 32 heads
-// of 1024 rows, head_dim 128, K blocks of 64) 70 / 81; 302 M (the same with K blocks of 16) 68.7 / 54.2, and 8 x 8 heads of
-// 1024 rows at head_dim 64 with K blocks of 16, also 302 M, 88.9 / 50.1.
-constexpr int64_t kSmallPrepassReads = (int64_t)128 << 20;
+constexpr int64_t kSmallPrepassElements = (int64_t)3 << 20;
+// ... and the element reads it makes: every K workgroup and every V panel re-reads its whole sequence.  Whole calls in bf16,
+// one launch / two, us: 32 heads of 512 rows, head_dim 128 (2.1 M elements), FP16 / FP8 P.V 29.7 / 30.9 and 27.5 / 30.9; 2 x 24 of 600
+// (3.7 M) 39.4 / 36.1 and 37.7 / 35.0; 2 x 16 of 1000 (4.1 M) 46.6 / 46.0 and 46.5 / 42.1; at head_dim 64 (2.1 M) 32.0 / 34.2
+// and 30.0 / 31.7; 8 heads of 1000, head_dim 128, K blocks of 16 (73 M reads) 37.6 / 37.7 and 33.1 / 35.3.
+constexpr int64_t kSmallPrepassReads = (int64_t)96 << 20;
 // A few query rows (sage_attn_few.hip) take four launches, 28-29 us end to end whatever the keys in this range; behind the
 // one-launch pre-pass the tiled kernel takes two, and longer with the keys of a head and with the re-reads.  bf16, K blocks of 64,
 // tiled / few rows: 1 x 8 heads of 768 keys, head_dim 128, 26.3 / 28.7 us, of 1024 keys 30.3 / 28.3; by re-reads, 4 x 8 heads
 // of 512 keys, head_dim 128 (25 M) 25.9 / 29.1; 16 x 8 of 512, head_dim 64 (50 M) 33.0 / 28.6; 4 x 8 of 768 (57 M) 34.7 / 28.4;
 // 8 x 8 of 1024, head_dim 64 (101 M) 47.7 / 28.3.
-constexpr int64_t kFewMinHeadElements = 896 * 128, kFewMinReads = (int64_t)32 << 20;
+constexpr int64_t kFewMinHeadElements = 896 * 128, kFewMinReads = (int64_t)32 << 20, kFewMinElements = (int64_t)4 << 20;
 // ... and with few keys, in great number: the FP32 results of a KV head's rows are written and read again, the tiled kernel with one
 // query head per KV head launches no more workgroups, and at head_dim 128 it wins where those bytes outweigh K and V.  16384 heads,
 // bf16, tiled / few rows: 24 rows, 16 keys 729 / 725 us; 28 rows, 16 keys 733 / 782, 48 keys 814 / 803; 32 rows, 16 keys 743 / 846,
@@ -502,9 +504,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   const int64_t ki_sb = varlen ? 0 : (int64_t)Hkv * Skv * D, ki_sh = varlen ? D : (int64_t)Skv * D, ki_sn = varlen ? (int64_t)Hkv * D : D;
   const int32_t *cu_qblk = nullptr, *cu_kblk = nullptr, *cu_panel = nullptr;
   if (varlen) {
-    int rc = sage_varlen_plan(cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, is_causal, plan,
-                              sage_varlen_plan_ints(B, total_q), stream);
-    if (rc) return rc;
+    if (B > 32767) return fail(SAGE_EINVAL, "number of sequences %d out of range (1..32767)", B);
     SagePlanLayout L = plan_layout(B, total_q);
     cu_qblk = plan + L.cu_qblk; cu_kblk = plan + L.cu_kblk; cu_panel = plan + L.cu_panel;
   }
@@ -514,12 +514,13 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   const bool no_keys = !varlen && Skv == 0;
   if (no_keys) smooth_k = 0;
   // Short sequences: all K and V pre-passes in one launch (every workgroup computes the statistic its tile needs over
-  // the whole sequence itself); otherwise six launches, the statistics in two stages.
+  // the whole sequence itself); otherwise two launches, the statistics in two stages.
   const int64_t k_elements = (int64_t)B * Hkv * Skv * D;
   const int64_t rereads = (Skv + blk_rows(blkk) - 1) / blk_rows(blkk) + (Skv + kPanelRows - 1) / kPanelRows;
   const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && k_elements <= kSmallPrepassElements &&
                              k_elements * rereads <= kSmallPrepassReads;
-  const bool short_keys = no_keys || (small_prepass && (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
+  const bool short_keys = no_keys || (!varlen && Skv <= kSmallPrepassRows && k_elements <= kFewMinElements &&
+                                      (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
   if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, B, Hkv, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
                     out, q_sn, k_sn, v_sn)) {
@@ -559,14 +560,6 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     va.v_sb = v_sb; va.v_sh = v_sh; va.v_sn = v_sn;
     hipError_t e = launch_prepass_small(qa, va, dtype, pv_mode == SAGE_PV_FP8, smooth_k != 0, km, v_scale, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sage_sageattn(pre-pass)");
-  } else {
-    if (smooth_k) {
-      rc = sage_k_mean(k, km, stat, stat_bytes, B, Hkv, Skv, D, k_sb, k_sh, k_sn, dtype, cu_seqlens_k, stream);
-      if (rc) return rc;
-    }
-    if (!no_keys) rc = sage_quant_int8(k, k_i8, k_scale, smooth_k ? km : nullptr, B, Hkv, Skv, D, k_sb, k_sh, k_sn, ki_sb, ki_sh, ki_sn,
-                         (int64_t)Hkv * D, D, blkk, 1.0f, dtype, cu_seqlens_k, cu_kblk, w.ks_sh, stream);
-    if (rc) return rc;
   }
   // Q is quantised by the attention kernel itself (each q-tile exactly where it is consumed) unless a feature needs the
   // standalone pass: an explicit mask or interleaved scales.
@@ -584,19 +577,12 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     lse_off = (float*)(ws + w.lse_off);
     dot.vec = km; dot.out = lse_off; dot.sb = (int64_t)Hkv * D; dot.sh = D; dot.group = Hq / Hkv; dot.total = total_q;
   }
-  if (!fuse_q) {
-    rc = quant_impl(q, q_i8, q_scale, nullptr, B, Hq, Sq, D, q_sb, q_sh, q_sn, qi_sb, qi_sh, qi_sn, 0, 0, blkq, q_mult, dtype,
-                    cu_seqlens_q, cu_qblk, w.qs_sh, dot, stream);
-    if (rc) return rc;
-  }
-  if (!no_keys && !small_prepass) {
-    rc = sage_prep_v(v, panels, v_scale, stat, stat_bytes, B, Hkv, Skv, D, v_sb, v_sh, v_sn, dtype, pv_mode, cu_seqlens_k,
-                     cu_panel, w.panel_sh, stream);
-    if (rc) return rc;
-  }
   QRawArg qr;
   if (fuse_q) { qr.ptr = q; qr.dtype = dtype; qr.mult = q_mult; qr.dot_km = want_dot ? km : nullptr; }
   MaskArg m;
+  MaskPackArgs pack;
+  memset(&pack, 0, sizeof(pack));
+  size_t used = w.total;   // of the workspace
   if (attn_mask) {
     // sageattn's additive mask is in natural-log units on top of sm_scale * q.k (test_sage_attention_mate.py:171-176)
     m.ptr = attn_mask; m.kind = mask_kind; m.sb = m_sb; m.sh = m_sh; m.sm = m_sm; m.sn = m_sn; m.mult = 1.44269504f;
@@ -604,11 +590,97 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     const bool pays = m_sn == 1 || p.ntk >= 5 || mask_tile_visits(p, B, Hq, Sq) >= 1024;
     if (!varlen && !is_causal && pays && mask_can_be_packed(p, B, Hq, Sq, Skv, mask_kind) && workspace_bytes - w.total >= (size_t)p.total_bytes) {
       uint8_t* bits = ws + w.total;
+      used += align_up((size_t)p.total_bytes);
       m.planes = p; m.bits = bits; m.seen = bits + p.bits_bytes;
-      hipError_t e = launch_mask_pack((const uint8_t*)attn_mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, bits + p.bits_bytes,
-                                      (hipStream_t)stream);
-      if (e != hipSuccess) return hip_fail(e, "sage_sageattn(mask)");
+      pack.mask = (const uint8_t*)attn_mask; pack.m_sb = m_sb; pack.m_sh = m_sh; pack.m_sm = m_sm; pack.m_sn = m_sn;
+      pack.p = p; pack.Sq = Sq; pack.Skv = Skv; pack.bits = bits; pack.seen = bits + p.bits_bytes;
     }
+  }
+  hipStream_t st = (hipStream_t)stream;
+  QuantArgs kq, qq;
+  memset(&kq, 0, sizeof(kq));
+  memset(&qq, 0, sizeof(qq));
+  if (!no_keys) {
+    if (int rc2 = quant_args(kq, k, k_i8, k_scale, smooth_k ? km : nullptr, B, Hkv, Skv, D, k_sb, k_sh, k_sn, ki_sb, ki_sh, ki_sn,
+                             (int64_t)Hkv * D, D, blkk, 1.0f, dtype, cu_seqlens_k, cu_kblk, w.ks_sh, RowDot())) return rc2;
+  }
+  if (!fuse_q) {
+    if (int rc2 = quant_args(qq, q, q_i8, q_scale, nullptr, B, Hq, Sq, D, q_sb, q_sh, q_sn, qi_sb, qi_sh, qi_sn, 0, 0, blkq, q_mult, dtype,
+                             cu_seqlens_q, cu_qblk, w.qs_sh, dot)) return rc2;
+  }
+  if (!no_keys && Skv > 0) {
+    if (!k || !v) return fail(SAGE_EINVAL, "null tensor pointer");
+    if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;
+    if (int rc2 = check_stride16("v", v_sb, v_sh, v_sn, 2, v)) return rc2;
+  }
+  const bool fp8 = pv_mode == SAGE_PV_FP8, keys = !no_keys && Skv > 0;
+  ColStatArgs ks, vs;
+  memset(&ks, 0, sizeof(ks));
+  ks.x = (const u16*)k; ks.partial = stat; ks.B = B; ks.H = Hkv; ks.L = Skv; ks.D = D;
+  ks.x_sb = k_sb; ks.x_sh = k_sh; ks.x_sn = k_sn; ks.nchunk = colstat_chunks(Skv); ks.cu_seqlens = cu_seqlens_k;
+  vs = ks;
+  vs.x = (const u16*)v; vs.x_sb = v_sb; vs.x_sh = v_sh; vs.x_sn = v_sn;
+  PrepVArgs pvn;
+  memset(&pvn, 0, sizeof(pvn));
+  pvn.v = (const u16*)v; pvn.panels = (uint8_t*)panels; pvn.vscale = v_scale; pvn.B = B; pvn.H = Hkv; pvn.L = Skv; pvn.D = D;
+  pvn.v_sb = v_sb; pvn.v_sh = v_sh; pvn.v_sn = v_sn; pvn.cu_seqlens = cu_seqlens_k; pvn.cu_panels = cu_panel; pvn.panel_sh = w.panel_sh;
+  PlanArgs pl;
+  memset(&pl, 0, sizeof(pl));
+  if (varlen) pl = {cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, attn_config(128, 1, true).nw * 32, 64, is_causal, plan};
+  // The pre-passes in two launches: what depends on nothing but the call's tensors, then what needs the statistics or the plan.  The two
+  // statistics then exist at the same time; where the workspace has no room for both (it is sized for one after the other), and for
+  // grids past one axis, every pass is a launch of its own.
+  FusedPrepass first, second;
+  memset(&first, 0, sizeof(first));
+  memset(&second, 0, sizeof(second));
+  const size_t v_stat_bytes = fp8 && smooth_k ? sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv_mode) : 0;
+  const bool k_long = smooth_k && ks.nchunk > kFusedChunks, v_long = fp8 && ks.nchunk > kFusedChunks;
+  bool fused = keys && !small_prepass && (int64_t)B <= 65535 && Hq <= 65535 && workspace_bytes - w.total >= v_stat_bytes + (used - w.total);
+  if (fused) {
+    first.plan = pl;
+    if (smooth_k) first.k_stat = ks;
+    if (fp8) { first.v_stat = vs; first.v_stat.partial = v_stat_bytes ? (void*)(ws + used) : stat; }
+    first.mask = pack;
+    (varlen || smooth_k ? second : first).k_quant = kq;
+    (varlen || fp8 ? second : first).v_panels = pvn;
+    if (smooth_k && !k_long) { second.k_quant.km_partial = (const double*)stat; second.k_quant.km_nchunk = ks.nchunk; second.k_quant.km_out = (u16*)km; }
+    if (fp8 && !v_long) { second.v_panels.vs_partial = (const float*)first.v_stat.partial; second.v_panels.vs_nchunk = vs.nchunk; second.v_panels.vscale_out = v_scale; }
+    if (!fuse_q && !qq.dot_out) {   // (with the row products it waits for the K mean in memory: a launch of its own)
+      FusedPrepass& f = varlen ? second : first;
+      if (!f.k_quant.out || fused_quant_together(D, f.k_quant.blk, qq.blk)) { f.q_quant = qq; qq.out = nullptr; }
+    }
+    fused = fused_prepass_workgroups(first) <= kFusedMaxWorkgroups && fused_prepass_workgroups(second) <= kFusedMaxWorkgroups;
+    if (!fused && !fuse_q) qq.out = q_i8;
+  }
+  hipError_t e = hipSuccess;
+  if (fused) {
+    e = launch_fused_prepass(first, dtype, D, fp8, st);
+    if (e == hipSuccess && k_long) e = launch_k_mean_finalize(ks, dtype, km, st);
+    if (e == hipSuccess && v_long) e = launch_v_scale_finalize(first.v_stat, v_scale, st);
+    if (e == hipSuccess) e = launch_fused_prepass(second, dtype, D, fp8, st);
+    if (e != hipSuccess) return hip_fail(e, "sage_sageattn(pre-pass)");
+  } else {
+    if (varlen) {
+      rc = sage_varlen_plan(cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, is_causal, plan, sage_varlen_plan_ints(B, total_q), stream);
+      if (rc) return rc;
+    }
+    if (!small_prepass && smooth_k) {
+      rc = sage_k_mean(k, km, stat, stat_bytes, B, Hkv, Skv, D, k_sb, k_sh, k_sn, dtype, cu_seqlens_k, stream);
+      if (rc) return rc;
+    }
+    if (!small_prepass && keys) e = launch_quant_int8(kq, dtype, Skv, st);
+    if (e != hipSuccess) return hip_fail(e, "sage_sageattn(K)");
+    if (!small_prepass && keys) {
+      rc = sage_prep_v(v, panels, v_scale, stat, stat_bytes, B, Hkv, Skv, D, v_sb, v_sh, v_sn, dtype, pv_mode, cu_seqlens_k,
+                       cu_panel, w.panel_sh, stream);
+      if (rc) return rc;
+    }
+    if (pack.bits) e = launch_mask_pack(pack, st);
+    if (e != hipSuccess) return hip_fail(e, "sage_sageattn(mask)");
+  }
+  if (qq.out) {
+    e = launch_quant_int8(qq, dtype, Sq, st);
+    if (e != hipSuccess) return hip_fail(e, "sage_sageattn(Q)");
   }
   // the attention kernel reads either the caller's floating-point q (its strides) or the int8 copy (dense strides)
   return attn_impl(q_i8, k_i8, panels, q_scale, k_scale, pv_mode == SAGE_PV_FP8 ? v_scale : nullptr, out, lse, B, Hq, Hkv, Sq,

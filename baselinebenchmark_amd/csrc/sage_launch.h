@@ -24,6 +24,11 @@ struct QuantArgs {
   int64_t dv_sb, dv_sh;
   int dv_group;
   int dot_total;
+  // K mean from its per-chunk sums (fused pre-pass): partial sums [B, H, nchunk, D], at most kFusedChunks chunks of a sequence; the
+  // workgroup of a sequence's first rows also writes the mean to km_out [B, H, D].  km is ignored then.
+  const double* km_partial;
+  int km_nchunk;
+  u16* km_out;
 };
 
 struct ColStatArgs {
@@ -44,6 +49,24 @@ struct PrepVArgs {
   const int32_t* cu_seqlens;
   const int32_t* cu_panels;
   int64_t panel_sh;
+  // V scales from their per-chunk maxima (fused pre-pass), like QuantArgs::km_partial; vscale is ignored then.
+  const float* vs_partial;
+  int vs_nchunk;
+  float* vscale_out;
+};
+
+struct MaskPackArgs {
+  const uint8_t* mask;
+  int64_t m_sb, m_sh, m_sm, m_sn;
+  MaskPlanes p;
+  int Sq, Skv;
+  uint8_t *bits, *seen;
+};
+
+struct PlanArgs {
+  const int32_t *cu_q, *cu_k;
+  int nseq, total_q, blkq, blkk, bm, bn, causal;
+  int32_t* plan;
 };
 
 // Division of a 32-bit unsigned number by a launch constant as a multiply-high and two shifts (exact for every 32-bit
@@ -151,8 +174,28 @@ hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dt
                                 float* vscale_out, hipStream_t st);
 
 // Packs a boolean mask [B, Hq, Sq, Skv] with element strides into the form of sage_common.h.
-hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,
-                            int Skv, uint8_t* bits, uint8_t* seen, hipStream_t st);
+hipError_t launch_mask_pack(const MaskPackArgs& a, hipStream_t st);
+
+// Several pre-passes in one launch: the jobs whose pointers are set, in the order of the members.  Jobs of one launch do not
+// see each other's results.
+constexpr int kFusedChunks = 8;   // chunks of a sequence whose statistics the quantiser and the panel job combine themselves
+struct FusedPrepass {
+  PlanArgs plan;          // if plan.plan
+  ColStatArgs k_stat;     // if k_stat.partial: sums
+  ColStatArgs v_stat;     // if v_stat.partial: abs-maxima
+  QuantArgs k_quant;      // if k_quant.out
+  QuantArgs q_quant;      // if q_quant.out
+  PrepVArgs v_panels;     // if v_panels.panels
+  MaskPackArgs mask;      // if mask.bits
+};
+// Whether one launch can run both quantisers (they share the rows per wavefront), and the workgroups it takes.
+bool fused_quant_together(int D, int blk_a, int blk_b);
+int64_t fused_prepass_workgroups(const FusedPrepass& f);
+constexpr int64_t kFusedMaxWorkgroups = (int64_t)1 << 23;   // one grid axis holds 2^31 threads
+hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv, hipStream_t st);
+// K mean / V scales from the per-chunk statistics a launch above has written (sequences of more than kFusedChunks chunks).
+hipError_t launch_k_mean_finalize(const ColStatArgs& a, int dtype, void* km, hipStream_t st);
+hipError_t launch_v_scale_finalize(const ColStatArgs& a, float* vscale, hipStream_t st);
 
 AttnConfig attn_config(int D, int pv, bool packed);
 // Fills in the launch constants of the tile decode from the dimensions already in `a` (B, Hq, Hkv, nqt, cu_q).

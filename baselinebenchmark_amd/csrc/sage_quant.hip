@@ -8,7 +8,9 @@
 // Arithmetic contract of the INT8 quantiser (bit-exact target): IEEE binary32 throughout,
 //   backends/_enflame/ops/sage_attention/quant_per_block.py:38-46  (+ :53-54 for k - km)
 //   backends/_hygon/ops/sageattention/sageattention_triton.py:35   (1e-12 floor)
+#include <cstring>
 #include "sage_launch.h"
+#include "sage_plan.h"
 
 #pragma clang fp contract(off)
 
@@ -25,14 +27,73 @@ __host__ __device__ constexpr int quant_wave_rows(int D) { return 64 / (D / 16);
 __host__ __device__ constexpr int quant_passes(int D, int blk) { return D == 128 ? (blk == 128 ? 4 : 2) : (blk >= 64 ? 2 : 1); }
 __host__ __device__ constexpr int quant_rows(int D, int blk) { return 4 * quant_passes(D, blk) * quant_wave_rows(D); }
 
+constexpr int kChunkRows = 512;   // rows of a chunk of the column statistics
+
+// Barrier that orders LDS traffic only: loads in flight stay in flight.
+__device__ inline void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Where a quantiser workgroup has the K mean from.  request() is called before the loads of the rows, read() after them (by every lane
+// of the workgroup): 16 channels from tc * 16 on, in the input type; false: nothing to subtract.
+template <int DT, int D>
+struct MeanInMemory {   // QuantArgs::km
+  const QuantArgs& a;
+  const int h, b;
+  __device__ void request(int) {}
+  __device__ bool read(uint4 (&km)[2], int tc, int, bool) {
+    if (a.km == nullptr) return false;
+    const uint4* p = reinterpret_cast<const uint4*>(a.km + (int64_t)b * a.km_sb + (int64_t)h * a.km_sh + tc * 16);
+    km[0] = p[0];
+    km[1] = p[1];
+    return true;
+  }
+};
+template <int DT, int D>
+struct MeanInLds {      // computed by the same workgroup; null: nothing to subtract
+  const u16* km_lds;
+  __device__ void request(int) {}
+  __device__ bool read(uint4 (&km)[2], int tc, int, bool) {
+    if (km_lds == nullptr) return false;
+    km[0] = *reinterpret_cast<const uint4*>(km_lds + tc * 16);
+    km[1] = *reinterpret_cast<const uint4*>(km_lds + tc * 16 + 8);
+    return true;
+  }
+};
+template <int DT, int D>
+struct MeanFromPartials {   // QuantArgs::km_partial, combined in chunk order like kmean_finalize_kernel
+  const QuantArgs& a;
+  const int h, b;
+  u16* km_lds;
+  double t[kFusedChunks];
+  __device__ int chunks(int L) const { return min((L + kChunkRows - 1) / kChunkRows, a.km_nchunk); }
+  __device__ void request(int L) {
+    const int nc = chunks(L);
+    const double* p = a.km_partial + ((int64_t)b * a.H + h) * a.km_nchunk * D + threadIdx.x;
+    if (threadIdx.x < D) {
+#pragma unroll
+      for (int c = 0; c < kFusedChunks; c++) t[c] = p[(int64_t)min(c, nc - 1) * D];
+    }
+  }
+  __device__ bool read(uint4 (&km)[2], int tc, int L, bool first) {
+    const int nc = chunks(L);
+    if (threadIdx.x < D) {
+      double s = 0;
+#pragma unroll
+      for (int c = 0; c < kFusedChunks; c++) s = c < nc ? s + t[c] : s;
+      const u16 m = from_f32<DT>((float)(s / (double)L));
+      km_lds[threadIdx.x] = m;
+      if (first) a.km_out[((int64_t)b * a.H + h) * D + threadIdx.x] = m;
+    }
+    lds_only_barrier();
+    return MeanInLds<DT, D>{km_lds}.read(km, tc, L, first);
+  }
+};
+
 // Quantises the rows chunk * quant_rows(D, blk) .. of (batch b, head h), which stay in registers, as floats, between the abs-max and
 // the rounding.  A lane owns 16 consecutive channels of a row (two 128-bit loads, one 128-bit store); all its loads are issued
 // before anything waits for one.
-// (km_lds: the K mean of this (batch, head) in LDS, D values in the input dtype, instead of a.km in global memory:
-// the fused pre-pass of short sequences computes it in the same workgroup.)
 // UNIT: the multiplier is 1 (every K call; x * 1.0f is x, so leaving the product out changes no bit).
-template <int DT, int D, int NP, bool UNIT>
-__device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int chunk, const int h, const int b, const u16* km_lds) {
+template <int DT, int D, int NP, bool UNIT, class Mean>
+__device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int chunk, const int h, const int b, Mean mean) {
   constexpr int TPR = D / 16;                  // lanes per row
   constexpr int RW = quant_wave_rows(D);       // rows per pass of a wavefront
   constexpr int WROWS = NP * RW;               // rows of a wavefront
@@ -58,6 +119,7 @@ __device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int ch
   if (n0 >= L) return;
   const int wrow = n0 + w * WROWS, row = wrow + tr;   // first row of the wavefront, of this lane
 
+  mean.request(L);
   // (rows past the end read the last one again: no branch between the loads)
   uint4 raw[NP][2];
 #pragma unroll
@@ -68,16 +130,8 @@ __device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int ch
   }
   // k - km is rounded to the input dtype (quant_per_block.py:53-54: the subtraction happens in torch, in
   // the tensor's dtype); both passes then see the rounded difference.
-  if (a.km != nullptr || km_lds != nullptr) {
-    uint4 kmr[2];
-    if (km_lds) {
-      kmr[0] = *reinterpret_cast<const uint4*>(km_lds + tc * 16);
-      kmr[1] = *reinterpret_cast<const uint4*>(km_lds + tc * 16 + 8);
-    } else {
-      const uint4* kp = reinterpret_cast<const uint4*>(a.km + (int64_t)b * a.km_sb + (int64_t)h * a.km_sh + tc * 16);
-      kmr[0] = kp[0];
-      kmr[1] = kp[1];
-    }
+  uint4 kmr[2];
+  if (mean.read(kmr, tc, L, chunk == 0)) {
     const uint32_t* km2 = reinterpret_cast<const uint32_t*>(kmr);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -181,10 +235,16 @@ __device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int ch
   }
 }
 
-template <int DT, int D, int NP>
+template <int DT, int D, int NP, bool PARTIAL = false>
 __global__ void __launch_bounds__(256) quant_int8_kernel(QuantArgs a) {
-  if (a.mult == 1.0f) quant_int8_rows<DT, D, NP, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
-  else quant_int8_rows<DT, D, NP, false>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
+  if constexpr (PARTIAL) {
+    __shared__ __align__(16) u16 km_lds[D];
+    quant_int8_rows<DT, D, NP, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, MeanFromPartials<DT, D>{a, (int)blockIdx.y, (int)blockIdx.z, km_lds});
+    return;
+  }
+  const MeanInMemory<DT, D> mean = {a, (int)blockIdx.y, (int)blockIdx.z};
+  if (a.mult == 1.0f) quant_int8_rows<DT, D, NP, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, mean);
+  else quant_int8_rows<DT, D, NP, false>(a, blockIdx.x, blockIdx.y, blockIdx.z, mean);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -192,14 +252,12 @@ __global__ void __launch_bounds__(256) quant_int8_kernel(QuantArgs a) {
 // Stage 1: one workgroup per (chunk of kChunkRows rows, head, batch) writes D partials.
 // Stage 2: one workgroup per (head, batch) combines the partials in chunk order.
 // ---------------------------------------------------------------------------------------------
-constexpr int kChunkRows = 512;
-
+constexpr int colstat_lds_bytes(int D) { return 256 / (D / 8) * D * 8; }
 
 template <int DT, int D, int MODE>
-__global__ void __launch_bounds__(256) colstat_partial_kernel(ColStatArgs a) {
+__device__ __forceinline__ void colstat_chunk(const ColStatArgs a, const int chunk, const int h, const int b, void* lds) {
   using acc_t = typename std::conditional<MODE == 0, double, float>::type;
   constexpr int TPR = D / 8, RPP = 256 / TPR;
-  const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, tr = tid / TPR, tc = tid % TPR;
   int L = a.L;
   int64_t xbase;
@@ -238,18 +296,32 @@ __global__ void __launch_bounds__(256) colstat_partial_kernel(ColStatArgs a) {
     for (int u = 0; u < UNR; u++) fold(raw[u]);
   }
   for (; n < n1; n += RPP) fold(load_stream16(base + (int64_t)n * a.x_sn));
-  __shared__ acc_t red[RPP][D];
+  acc_t(*red)[D] = reinterpret_cast<acc_t(*)[D]>(lds);
 #pragma unroll
   for (int i = 0; i < 8; i++) red[tr][tc * 8 + i] = acc[i];
   __syncthreads();
   if (tid < D) {
     acc_t t = red[0][tid];
-    for (int r = 1; r < RPP; r++) {
-      if constexpr (MODE == 0) t += red[r][tid];
-      else t = fmaxf(t, red[r][tid]);
+#pragma unroll 1
+    for (int r0 = 0; r0 < RPP; r0 += 8) {   // eight reads in flight; added in row order
+      acc_t u[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) u[i] = red[r0 + i][tid];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        if (r0 + i == 0) continue;
+        if constexpr (MODE == 0) t += u[i];
+        else t = fmaxf(t, u[i]);
+      }
     }
     reinterpret_cast<acc_t*>(a.partial)[(((int64_t)b * a.H + h) * a.nchunk + chunk) * D + tid] = t;
   }
+}
+
+template <int DT, int D, int MODE>
+__global__ void __launch_bounds__(256) colstat_partial_kernel(ColStatArgs a) {
+  __shared__ __align__(16) uint8_t lds[colstat_lds_bytes(D) / (MODE == 0 ? 1 : 2)];
+  colstat_chunk<DT, D, MODE>(a, blockIdx.x, blockIdx.y, blockIdx.z, lds);
 }
 
 // K mean: sum partials in chunk order (float64), /L, -> fp32 -> input dtype.
@@ -302,9 +374,45 @@ __global__ void vscale_finalize_kernel(const float* partial, float* vscale, int 
 // Elements are converted, scattered into LDS in panel byte order and streamed out linearly.
 // ---------------------------------------------------------------------------------------------
 
-// (vs_lds: the per-channel V scales of this (batch, head) in LDS instead of a.vscale in global memory.)
-template <int DT, int D, int PV>
-__device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, const int h, const int b, const float* vs_lds) {
+// Where a panel workgroup has the V scales from: like the K mean of the quantiser, D values in LDS or in memory.
+struct ScalesInMemory {
+  const float* p;
+  __device__ void request(int) {}
+  __device__ const float* ready(int, bool) { return p; }
+};
+template <int D>
+struct ScalesFromPartials {   // PrepVArgs::vs_partial, like vscale_finalize_kernel
+  const PrepVArgs& a;
+  const int h, b;
+  float* vs_lds;
+  float t[kFusedChunks];
+  __device__ void request(int L) {
+    const int nc = min((L + kChunkRows - 1) / kChunkRows, a.vs_nchunk);
+    const float* p = a.vs_partial + ((int64_t)b * a.H + h) * a.vs_nchunk * D + threadIdx.x;
+    if (threadIdx.x < D) {
+#pragma unroll
+      for (int c = 0; c < kFusedChunks; c++) t[c] = p[(int64_t)min(c, nc - 1) * D];
+    }
+  }
+  __device__ const float* ready(int, bool first) {
+    if (threadIdx.x < D) {
+      float m = 0.f;
+#pragma unroll
+      for (int c = 0; c < kFusedChunks; c++) m = fmaxf(m, t[c]);   // (chunks past the last repeat it)
+      const float s = fmaxf(m / 448.0f, kScaleFloor);
+      vs_lds[threadIdx.x] = s;
+      if (first) a.vscale_out[((int64_t)b * a.H + h) * D + threadIdx.x] = s;
+    }
+    lds_only_barrier();
+    return vs_lds;
+  }
+};
+
+// LDS of a panel job: T[channel][row quad], dword stride of a channel padded by one
+__host__ __device__ constexpr int prep_v_lds_bytes(int D, int PV) { return D * (kPanelRows / 4 * (PV == 1 ? 1 : 2) + 1) * 4; }
+
+template <int DT, int D, int PV, class Scales>
+__device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, const int h, const int b, Scales scales, uint32_t* T) {
   // A lane converts 4 consecutive rows x 8 consecutive channels at a time, so that the 4 row values of
   // a channel pack into one dword (fp8) or two (fp16): exactly the (b = 0..3) group of the panel
   // order.  They are staged in LDS as T[channel][row quad] and read back in panel order.
@@ -316,7 +424,7 @@ __device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, 
   constexpr int TS = NQ * QW + 1;               // dword stride of a channel in LDS (padded)
   constexpr int PANEL_BYTES = kPanelRows * D * ESZ;
   constexpr int DTN = D / 32;
-  __shared__ uint32_t T[D * TS];
+  static_assert(D * TS * 4 == prep_v_lds_bytes(D, PV), "LDS size");
   const int tid = threadIdx.x, tr = tid / TPR, tc = tid % TPR;
   int L = a.L;
   int64_t vbase, pbase;
@@ -331,48 +439,68 @@ __device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, 
   }
   const int n0 = pidx * kPanelRows;
   if (n0 >= L) return;
-  float sc[8], rc[8];
-  bool fast = true;
-  if constexpr (PV == 1) {
+  if constexpr (PV == 1) scales.request(L);
+  // (all rows are requested before anything waits; those past the end read the last one again and become zeros)
+  uint4 raw[QPT][4];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      sc[i] = vs_lds ? vs_lds[tc * 8 + i] : a.vscale[((int64_t)b * a.H + h) * D + tc * 8 + i];
-      rc[i] = 1.0f / sc[i];
-      fast = fast && ((__builtin_bit_cast(uint32_t, sc[i]) & 0x7fffffu) != 0x7fffffu) && sc[i] < 1.0e30f;
-    }
-    fast = __builtin_amdgcn_ballot_w64(!fast) == 0;   // the correction-step division for the whole wavefront, or not at all
-  }
-#pragma unroll
-  for (int qq = 0; qq < QPT; qq++) {
-    const int quad = qq * RPP + tr;
-    uint4 raw[4];
+  for (int qq = 0; qq < QPT; qq++)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      const int r = n0 + 4 * quad + j;
-      raw[j] = make_uint4(0, 0, 0, 0);
-      if (r < L) raw[j] = load_stream16(a.v + vbase + (int64_t)r * a.v_sn + tc * 8);
+      const int r = n0 + 4 * (qq * RPP + tr) + j;
+      raw[qq][j] = load_stream16(a.v + vbase + (int64_t)min(r, L - 1) * a.v_sn + tc * 8);
     }
+  auto row_there = [&](int qq, int j) { return n0 + 4 * (qq * RPP + tr) + j < L; };
+  if constexpr (PV == 1) {
+    const float* vs = scales.ready(L, pidx == 0);
+    float sc[8];
+    bool exact = true;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      float x[4];
+      sc[i] = vs[tc * 8 + i];
+      exact = exact && reciprocal_is_exact(sc[i]);
+    }
+    auto convert = [&](auto quotient) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) x[j] = to_f32<DT>(reinterpret_cast<const u16*>(&raw[j])[i]);
-      uint32_t* dst = &T[(tc * 8 + i) * TS + quad * QW];
-      if constexpr (PV == 1) {
-        float z[4];
+      for (int qq = 0; qq < QPT; qq++) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          float z[4];
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const float x = to_f32<DT>(reinterpret_cast<const u16*>(&raw[qq][j])[i]);
+            z[j] = fminf(fmaxf(quotient(row_there(qq, j) ? x : 0.f, i), -448.f), 448.f);
+          }
+          int pk = __builtin_amdgcn_cvt_pk_fp8_f32(z[0], z[1], 0, false);
+          pk = __builtin_amdgcn_cvt_pk_fp8_f32(z[2], z[3], pk, true);
+          T[(tc * 8 + i) * TS + qq * RPP + tr] = (uint32_t)pk;
+        }
+        __builtin_amdgcn_sched_barrier(0);   // (one pass after the other: both at once take twice the registers)
+      }
+    };
+    // (the correction-step division for the whole wavefront, or the general one)
+    if (__builtin_amdgcn_ballot_w64(!exact) == 0) {
+      float rc[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) rc[i] = 1.0f / sc[i];
+      convert([&](float x, int i) { return div_by_uniform(x, sc[i], rc[i]); });
+    } else {
+      convert([&](float x, int i) { return div_by_any(x, 1.0 / (double)sc[i]); });
+    }
+  } else {
+#pragma unroll
+    for (int qq = 0; qq < QPT; qq++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        float x[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          z[j] = fast ? div_by_uniform(x[j], sc[i], rc[i]) : x[j] / sc[i];
-          z[j] = fminf(fmaxf(z[j], -448.f), 448.f);
+          x[j] = to_f32<DT>(reinterpret_cast<const u16*>(&raw[qq][j])[i]);
+          if (!row_there(qq, j)) x[j] = 0.f;
         }
-        int pk = __builtin_amdgcn_cvt_pk_fp8_f32(z[0], z[1], 0, false);
-        pk = __builtin_amdgcn_cvt_pk_fp8_f32(z[2], z[3], pk, true);
-        dst[0] = (uint32_t)pk;
-      } else {
-        dst[0] = (uint32_t)f32_to_f16(x[0]) | ((uint32_t)f32_to_f16(x[1]) << 16);
-        dst[1] = (uint32_t)f32_to_f16(x[2]) | ((uint32_t)f32_to_f16(x[3]) << 16);
+        uint32_t* dst = &T[(tc * 8 + i) * TS + (qq * RPP + tr) * QW];
+        dst[0] = pack2<0>(x[0], x[1]);
+        dst[1] = pack2<0>(x[2], x[3]);
       }
-    }
   }
   __syncthreads();
   uint4* out = reinterpret_cast<uint4*>(a.panels + pbase);
@@ -396,9 +524,14 @@ __device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, 
   }
 }
 
-template <int DT, int D, int PV>
+template <int DT, int D, int PV, bool PARTIAL = false>
 __global__ void __launch_bounds__(256) prep_v_kernel(PrepVArgs a) {
-  prep_v_tile<DT, D, PV>(a, blockIdx.x, blockIdx.y, blockIdx.z, nullptr);
+  __shared__ __align__(16) uint32_t T[prep_v_lds_bytes(D, PV) / 4];
+  const int h = blockIdx.y, b = blockIdx.z;
+  if constexpr (PARTIAL) {
+    __shared__ float vs_lds[D];
+    prep_v_tile<DT, D, PV>(a, blockIdx.x, h, b, ScalesFromPartials<D>{a, h, b, vs_lds}, T);
+  } else prep_v_tile<DT, D, PV>(a, blockIdx.x, h, b, ScalesInMemory{a.vscale + ((int64_t)b * a.H + h) * D}, T);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -410,13 +543,37 @@ __global__ void __launch_bounds__(256) prep_v_kernel(PrepVArgs a) {
 // (batch, head): affordable while the sequence is short and the reads hit the L2; six dependent launches of a few
 // microseconds each become one.
 // ---------------------------------------------------------------------------------------------
+// Hands the rows n, n + RPP, ... below n1 of a lane's channels to `fold`, in that order, sixteen loads in flight: the statistic is
+// latency from end to end, and with the unrolling left to the compiler it took between four and thirty of them, 35 to 45 us for
+// the call on 8 heads of 1000 rows at head_dim 128.  (Rows past the end arrive as zeros, which no statistic notices.)
+template <int D, class Fold>
+__device__ __forceinline__ void stream_rows(const u16* base, int64_t stride, int n, int n0, int n1, Fold fold) {
+  constexpr int RPP = 256 / (D / 8);
+  auto batch = [&](auto unr) __attribute__((always_inline)) {
+    constexpr int UNR = decltype(unr)::value;
+    uint4 raw[UNR];
+#pragma unroll
+    for (int u = 0; u < UNR; u++) raw[u] = *reinterpret_cast<const uint4*>(base + (int64_t)min(n + u * RPP, n1 - 1) * stride);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < UNR; u++) fold(n + u * RPP < n1 ? raw[u] : make_uint4(0, 0, 0, 0));
+    n0 += UNR * RPP;
+    n += UNR * RPP;
+  };
+#pragma unroll 1
+  while (n1 - n0 > 8 * RPP) batch(std::integral_constant<int, 16>());
+  if (n1 - n0 > 4 * RPP) batch(std::integral_constant<int, 8>());
+  else if (n0 < n1) batch(std::integral_constant<int, 4>());
+}
+
 template <int DT, int D, int PV, int NP>
 __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVArgs va, int nk, int smooth, u16* km_out,
                                                             float* vscale_out) {
   constexpr int TPR = D / 8, RPP = 256 / TPR;
   const int h = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, tr = tid / TPR, tc = tid % TPR;
-  __shared__ double red[RPP][D];
+  __shared__ __align__(16) uint8_t lds[prep_v_lds_bytes(D, PV) > colstat_lds_bytes(D) ? prep_v_lds_bytes(D, PV) : colstat_lds_bytes(D)];
+  double(*red)[D] = reinterpret_cast<double(*)[D]>(lds);
   __shared__ __align__(16) u16 km_l[D];
   __shared__ float vs_l[D];
   if ((int)blockIdx.x < nk) {
@@ -429,13 +586,16 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
         double acc[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) acc[i] = 0;
-#pragma unroll 8
-        for (int n = n0 + tr; n < n1; n += RPP) {   // (unrolled for loads in flight; the additions keep their order)
-          uint4 raw = *reinterpret_cast<const uint4*>(qa.x + xbase + (int64_t)n * qa.x_sn + tc * 8);
-          const u16* e = reinterpret_cast<const u16*>(&raw);
+        stream_rows<D>(qa.x + xbase + tc * 8, qa.x_sn, n0 + tr, n0, n1, [&](const uint4& raw) {   // (the additions in row order)
+          const uint32_t* x2 = reinterpret_cast<const uint32_t*>(&raw);
 #pragma unroll
-          for (int i = 0; i < 8; i++) acc[i] += (double)to_f32<DT>(e[i]);
-        }
+          for (int i = 0; i < 4; i++) {
+            float lo, hi;
+            unpack2<DT>(x2[i], lo, hi);
+            acc[2 * i] += (double)lo;
+            acc[2 * i + 1] += (double)hi;
+          }
+        });
 #pragma unroll
         for (int i = 0; i < 8; i++) red[tr][tc * 8 + i] = acc[i];
         __syncthreads();
@@ -453,7 +613,7 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
       }
       __syncthreads();
     }
-    quant_int8_rows<DT, D, NP, true>(qa, blockIdx.x, h, b, smooth ? km_l : nullptr);   // (K: the multiplier is 1)
+    quant_int8_rows<DT, D, NP, true>(qa, blockIdx.x, h, b, MeanInLds<DT, D>{smooth ? km_l : nullptr});   // (K: the multiplier is 1)
   } else {
     const int pidx = blockIdx.x - nk;
     if constexpr (PV == 1) {
@@ -462,13 +622,16 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
       float acc[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) acc[i] = 0.f;
-#pragma unroll 8
-      for (int n = tr; n < L; n += RPP) {
-        uint4 raw = *reinterpret_cast<const uint4*>(va.v + vbase + (int64_t)n * va.v_sn + tc * 8);
-        const u16* e = reinterpret_cast<const u16*>(&raw);
+      stream_rows<D>(va.v + vbase + tc * 8, va.v_sn, tr, 0, L, [&](const uint4& raw) {
+        const uint32_t* x2 = reinterpret_cast<const uint32_t*>(&raw);
 #pragma unroll
-        for (int i = 0; i < 8; i++) acc[i] = fmaxf(acc[i], fabsf(to_f32<DT>(e[i])));
-      }
+        for (int i = 0; i < 4; i++) {
+          float lo, hi;
+          unpack2<DT>(x2[i], lo, hi);
+          acc[2 * i] = fmaxf(acc[2 * i], fabsf(lo));
+          acc[2 * i + 1] = fmaxf(acc[2 * i + 1], fabsf(hi));
+        }
+      });
       float* redf = reinterpret_cast<float*>(&red[0][0]);
 #pragma unroll
       for (int i = 0; i < 8; i++) redf[tr * D + tc * 8 + i] = acc[i];
@@ -482,7 +645,7 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
       }
       __syncthreads();
     }
-    prep_v_tile<DT, D, PV>(va, pidx, h, b, PV == 1 ? vs_l : nullptr);
+    prep_v_tile<DT, D, PV>(va, pidx, h, b, ScalesInMemory{vs_l}, reinterpret_cast<uint32_t*>(lds));
   }
 }
 
@@ -495,14 +658,15 @@ __device__ inline unsigned nonzero_bytes(unsigned x) {   // bit i: byte i of x i
   return (t * 0x10204080u) >> 28;
 }
 
-__global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn,
-                                                        MaskPlanes p, int Sq, int Skv, uint8_t* bits, uint8_t* seen) {
+__device__ __forceinline__ void mask_pack_tile(const MaskPackArgs& a, const int tile, const int qt, const int plane, uint8_t* packed) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4), aligned(1)));
-  __shared__ __align__(16) uint8_t packed[kMaskTileBytes];
   __shared__ unsigned wave_seen[4];
-  const int tile = blockIdx.x, qt = blockIdx.y, tid = threadIdx.x;
+  const uint8_t* mask = a.mask;
+  const int64_t m_sb = a.m_sb, m_sh = a.m_sh, m_sm = a.m_sm, m_sn = a.m_sn;
+  const MaskPlanes& p = a.p;
+  const int Sq = a.Sq, Skv = a.Skv, tid = threadIdx.x;
   const int heads = p.ph ? (p.pb ? p.pb : p.planes) : 1;   // planes of one batch entry
-  const int b = blockIdx.z / heads, hd = blockIdx.z - b * heads;
+  const int b = plane / heads, hd = plane - b * heads;
   const uint8_t* base = mask + (int64_t)b * m_sb + (int64_t)hd * m_sh;
   const int rows = m_sm ? min(kMaskRows, Sq - qt * kMaskRows) : kMaskRows;   // (rows that all read the same row are all valid)
   base += (int64_t)qt * kMaskRows * m_sm;
@@ -547,12 +711,65 @@ __global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int
   }
   __syncthreads();
   const uint4 row = reinterpret_cast<const uint4*>(packed)[tid];
-  const int64_t t = ((int64_t)blockIdx.z * p.nqt + qt) * p.ntk + tile;
-  reinterpret_cast<uint4*>(bits + t * kMaskTileBytes)[tid] = row;
+  const int64_t t = ((int64_t)plane * p.nqt + qt) * p.ntk + tile;
+  reinterpret_cast<uint4*>(a.bits + t * kMaskTileBytes)[tid] = row;
   const unsigned long long any = __builtin_amdgcn_ballot_w64((row.x | row.y | row.z | row.w) != 0);
   if ((tid & 63) == 0) wave_seen[tid >> 6] = ((unsigned)any != 0 ? 1 : 0) | ((any >> 32) != 0 ? 2 : 0);
   __syncthreads();
-  if (tid == 0) seen[t] = (uint8_t)(wave_seen[0] | wave_seen[1] << 2 | wave_seen[2] << 4 | wave_seen[3] << 6);
+  if (tid == 0) a.seen[t] = (uint8_t)(wave_seen[0] | wave_seen[1] << 2 | wave_seen[2] << 4 | wave_seen[3] << 6);
+}
+
+__global__ void __launch_bounds__(256) mask_pack_kernel(MaskPackArgs a) {
+  __shared__ __align__(16) uint8_t packed[kMaskTileBytes];
+  mask_pack_tile(a, blockIdx.x, blockIdx.y, blockIdx.z, packed);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Several pre-passes in one launch: a workgroup finds its job in the table of running workgroup counts and runs the code of that
+// job's own kernel.  The launches of a call on a few thousand rows take 3 to 8 us each, most of it the start, the memory
+// latency and the last workgroups of kernels too small to fill the chip, one after the other.
+// ---------------------------------------------------------------------------------------------
+enum FusedJob { kJobPlan, kJobKStat, kJobVStat, kJobKQuant, kJobQQuant, kJobVPanels, kJobMask, kJobs };
+struct FusedTable {
+  uint32_t end[kJobs];       // workgroups of the jobs up to this one
+  uint32_t nx[kJobs], nh[kJobs];
+  FastDiv div_x[kJobs], div_h[kJobs];   // workgroup of a job -> (x, head, batch)
+};
+constexpr int kFusedPlanSeqs = 1024;
+constexpr int fused_lds_bytes(int D, int PV) {
+  const int a = prep_v_lds_bytes(D, PV) > colstat_lds_bytes(D) ? prep_v_lds_bytes(D, PV) : colstat_lds_bytes(D);
+  return a > (int)sizeof(PlanLds<kFusedPlanSeqs>) ? a : (int)sizeof(PlanLds<kFusedPlanSeqs>);
+}
+
+// The jobs of the second launch alone (quantisers and panels, statistics combined on the way): fewer registers than with all of them.
+template <int DT, int D, int PV, int NP>
+__device__ __forceinline__ void fused_late_job(const FusedPrepass& f, const int job, const int x, const int h, const int b, uint32_t* lds, float* stat) {
+  if (job == kJobKQuant) {
+    if (f.k_quant.km_partial) quant_int8_rows<DT, D, NP, true>(f.k_quant, x, h, b, MeanFromPartials<DT, D>{f.k_quant, h, b, reinterpret_cast<u16*>(stat)});
+    else quant_int8_rows<DT, D, NP, true>(f.k_quant, x, h, b, MeanInMemory<DT, D>{f.k_quant, h, b});
+  } else if (job == kJobQQuant) {
+    quant_int8_rows<DT, D, NP, false>(f.q_quant, x, h, b, MeanInLds<DT, D>{nullptr});
+  } else {
+    if (PV == 1 && f.v_panels.vs_partial) prep_v_tile<DT, D, PV>(f.v_panels, x, h, b, ScalesFromPartials<D>{f.v_panels, h, b, stat}, lds);
+    else prep_v_tile<DT, D, PV>(f.v_panels, x, h, b, ScalesInMemory{f.v_panels.vscale + ((int64_t)b * f.v_panels.H + h) * D}, lds);
+  }
+}
+
+template <int DT, int D, int PV, int NP, bool ALL>
+__global__ void __launch_bounds__(256, ALL ? 3 : 4) fused_prepass_kernel(FusedPrepass f, FusedTable t) {
+  __shared__ __align__(16) uint8_t lds[ALL ? fused_lds_bytes(D, PV) : prep_v_lds_bytes(D, PV)];
+  __shared__ __align__(16) float stat[D];   // K mean or V scales of this workgroup's (batch, head)
+  int job = 0;
+  while (blockIdx.x >= t.end[job]) job++;
+  const uint32_t i = blockIdx.x - (job ? t.end[job - 1] : 0), y = fastdiv(i, t.div_x[job]);
+  const int x = i - y * t.nx[job], b = fastdiv(y, t.div_h[job]), h = y - b * t.nh[job];
+  if constexpr (ALL) {
+    if (job == kJobPlan) { varlen_plan<256, kFusedPlanSeqs>(f.plan, *reinterpret_cast<PlanLds<kFusedPlanSeqs>*>(lds)); return; }
+    if (job == kJobKStat) { colstat_chunk<DT, D, 0>(f.k_stat, x, h, b, lds); return; }
+    if (PV == 1 && job == kJobVStat) { colstat_chunk<DT, D, 1>(f.v_stat, x, h, b, lds); return; }
+    if (job == kJobMask) { mask_pack_tile(f.mask, x, h, b, lds); return; }
+  }
+  fused_late_job<DT, D, PV, NP>(f, job, x, h, b, reinterpret_cast<uint32_t*>(lds), stat);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -561,7 +778,7 @@ __global__ void __launch_bounds__(256) mask_pack_kernel(const uint8_t* mask, int
 hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_rows, hipStream_t st) {
   const int rows = quant_rows(a.D, a.blk);
   dim3 grid((max_rows + rows - 1) / rows, a.H, a.B), block(256);
-#define SAGE_QUANT(DT, DD, NP) quant_int8_kernel<DT, DD, NP><<<grid, block, 0, st>>>(a)
+#define SAGE_QUANT(DT, DD, NP) (a.km_partial ? quant_int8_kernel<DT, DD, NP, true><<<grid, block, 0, st>>>(a) : quant_int8_kernel<DT, DD, NP><<<grid, block, 0, st>>>(a))
 #define SAGE_QUANT_D(DT) \
   do { \
     if (a.D == 64) { if (quant_passes(64, a.blk) == 1) SAGE_QUANT(DT, 64, 1); else SAGE_QUANT(DT, 64, 2); } \
@@ -574,9 +791,105 @@ hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_rows, hipStr
   return hipGetLastError();
 }
 
-hipError_t launch_mask_pack(const uint8_t* mask, int64_t m_sb, int64_t m_sh, int64_t m_sm, int64_t m_sn, const MaskPlanes& p, int Sq,
-                            int Skv, uint8_t* bits, uint8_t* seen, hipStream_t st) {
-  mask_pack_kernel<<<dim3(p.ntk, p.nqt, p.planes), dim3(256), 0, st>>>(mask, m_sb, m_sh, m_sm, m_sn, p, Sq, Skv, bits, seen);
+hipError_t launch_mask_pack(const MaskPackArgs& a, hipStream_t st) {
+  mask_pack_kernel<<<dim3(a.p.ntk, a.p.nqt, a.p.planes), dim3(256), 0, st>>>(a);
+  return hipGetLastError();
+}
+
+bool fused_quant_together(int D, int blk_a, int blk_b) {
+  const int lo = blk_a < blk_b ? blk_a : blk_b, hi = blk_a < blk_b ? blk_b : blk_a;
+  return quant_passes(D, hi) * quant_wave_rows(D) <= lo;   // the wider one's wavefronts still own whole blocks of the other
+}
+
+// (x, head, batch) extents of the jobs; zero where a job is not asked for
+static void fused_extents(const FusedPrepass& f, int np_blk, int64_t (&e)[kJobs][3]) {
+  memset(e, 0, sizeof(e));
+  auto set = [&](int job, int64_t x, int64_t h, int64_t b) { e[job][0] = x; e[job][1] = h; e[job][2] = b; };
+  if (f.plan.plan) set(kJobPlan, 1, 1, 1);
+  if (f.k_stat.partial) set(kJobKStat, f.k_stat.nchunk, f.k_stat.H, f.k_stat.B);
+  if (f.v_stat.partial) set(kJobVStat, f.v_stat.nchunk, f.v_stat.H, f.v_stat.B);
+  auto quant = [&](int job, const QuantArgs& a) {
+    const int rows = quant_rows(a.D, np_blk);
+    if (a.out) set(job, (a.L + rows - 1) / rows, a.H, a.B);
+  };
+  quant(kJobKQuant, f.k_quant);
+  quant(kJobQQuant, f.q_quant);
+  if (f.v_panels.panels) set(kJobVPanels, (f.v_panels.L + kPanelRows - 1) / kPanelRows, f.v_panels.H, f.v_panels.B);
+  if (f.mask.bits) set(kJobMask, f.mask.p.ntk, f.mask.p.nqt, f.mask.p.planes);
+}
+static int fused_block(const FusedPrepass& f) {   // the scale block that sets the rows of a quantiser workgroup
+  const int k = f.k_quant.out ? f.k_quant.blk : 0, q = f.q_quant.out ? f.q_quant.blk : 0;
+  return k > q ? k : q;
+}
+
+int64_t fused_prepass_workgroups(const FusedPrepass& f) {
+  int64_t e[kJobs][3], n = 0;
+  fused_extents(f, fused_block(f), e);
+  for (auto& j : e) n += j[0] * j[1] * j[2];
+  return n;
+}
+
+template <int MODE>
+static hipError_t launch_colstat(const ColStatArgs& a, int dtype, hipStream_t st);
+
+// A job in a launch of its own.
+static hipError_t launch_job(const FusedPrepass& f, int job, int dtype, int pv, hipStream_t st) {
+  switch (job) {
+    case kJobPlan: return launch_varlen_plan(f.plan.cu_q, f.plan.cu_k, f.plan.nseq, f.plan.total_q, f.plan.blkq, f.plan.blkk, f.plan.bm, f.plan.bn, f.plan.causal, f.plan.plan, st);
+    case kJobKStat: return launch_colstat<0>(f.k_stat, dtype, st);
+    case kJobVStat: return launch_colstat<1>(f.v_stat, dtype, st);
+    case kJobKQuant: return launch_quant_int8(f.k_quant, dtype, f.k_quant.L, st);
+    case kJobQQuant: return launch_quant_int8(f.q_quant, dtype, f.q_quant.L, st);
+    case kJobVPanels: return launch_prep_v(f.v_panels, dtype, pv, (f.v_panels.L + kPanelRows - 1) / kPanelRows, st);
+    default: return launch_mask_pack(f.mask, st);
+  }
+}
+
+// Up to how many workgroups the jobs of a launch share it: past that each fills the chip by itself, and its own kernel, with fewer
+// registers and less LDS than the shared one, is the faster.  The plan, one workgroup of 8 us, always rides along.  Whole calls in
+// bf16, 40 query rows, us, before these launches / each job by itself / early, late or both jobs sharing: 8 heads of 4096 keys, FP8 P.V
+// (512 early and 768 late workgroups) 71.9 / 65.4 / 63.2, 63.7, 61.6; 32 heads of 4096, FP8 (1024 early, 3072 late) 87.9 / 82.0 / 81.8,
+// 83.0, 82.8; 4 x 32 of 4096, FP16 (5120 early) 181.8 / 174.3 / 177.1 early; packed, causal, 16 sequences of 100..600, 32/8 heads, FP16
+// (1920 late) 90.2 / 84.5 / 81.0, 82.9, 79.3; 96 of 16..1024 (18432 late) 571 / 547 / 544, 565, 563.
+constexpr int64_t kMergeEarly = 2048, kMergeLate = 8192;
+
+hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv, hipStream_t st) {
+  int64_t e[kJobs][3], n = 0;
+  const int blk = fused_block(f);
+  fused_extents(f, blk, e);
+  FusedTable t;
+  for (int j = 0; j < kJobs; j++) {
+    if (e[j][1] > 65535 || e[j][2] > 65535) return hipErrorInvalidConfiguration;   // (what the jobs' own grids take)
+    n += e[j][0] * e[j][1] * e[j][2];
+    if (n > kFusedMaxWorkgroups) return hipErrorInvalidConfiguration;
+    t.end[j] = (uint32_t)n;
+    t.nx[j] = e[j][0] ? (uint32_t)e[j][0] : 1;
+    t.nh[j] = e[j][1] ? (uint32_t)e[j][1] : 1;
+    t.div_x[j] = make_fastdiv(t.nx[j]);
+    t.div_h[j] = make_fastdiv(t.nh[j]);
+  }
+  if (n == 0) return hipSuccess;
+  int jobs = 0;
+  for (auto& j : e) jobs += j[0] * j[1] * j[2] > 0;
+  const bool all = e[kJobPlan][0] || e[kJobKStat][0] || e[kJobVStat][0] || e[kJobMask][0];
+  if (jobs == 1 || (!f.plan.plan && n > (all ? kMergeEarly : kMergeLate))) {
+    for (int j = 0; j < kJobs; j++)
+      if (e[j][0] * e[j][1] * e[j][2] > 0)
+        if (hipError_t err = launch_job(f, j, dtype, pv, st)) return err;
+    return hipSuccess;
+  }
+  const dim3 grid((uint32_t)n), block(256);
+  const int np = blk ? quant_passes(D, blk) : D == 128 ? 2 : 1;
+#define SAGE_FUSED(DT, DD, PVV, NP) (all ? fused_prepass_kernel<DT, DD, PVV, NP, true><<<grid, block, 0, st>>>(f, t) : fused_prepass_kernel<DT, DD, PVV, NP, false><<<grid, block, 0, st>>>(f, t))
+#define SAGE_FUSED_D(DT, PVV) \
+  do { \
+    if (D == 64) { if (np == 1) SAGE_FUSED(DT, 64, PVV, 1); else SAGE_FUSED(DT, 64, PVV, 2); } \
+    else { if (np == 2) SAGE_FUSED(DT, 128, PVV, 2); else SAGE_FUSED(DT, 128, PVV, 4); } \
+  } while (0)
+  if (dtype == 0) { if (pv) SAGE_FUSED_D(0, 1); else SAGE_FUSED_D(0, 0); }
+  else { if (pv) SAGE_FUSED_D(1, 1); else SAGE_FUSED_D(1, 0); }
+#undef SAGE_FUSED_D
+#undef SAGE_FUSED
   return hipGetLastError();
 }
 
@@ -595,7 +908,9 @@ static hipError_t launch_colstat(const ColStatArgs& a, int dtype, hipStream_t st
 hipError_t launch_k_mean(const ColStatArgs& a, int dtype, void* km, hipStream_t st) {
   if (a.nchunk == 0 || a.B == 0 || a.H == 0) return hipSuccess;
   hipError_t e = launch_colstat<0>(a, dtype, st);
-  if (e != hipSuccess) return e;
+  return e != hipSuccess ? e : launch_k_mean_finalize(a, dtype, km, st);
+}
+hipError_t launch_k_mean_finalize(const ColStatArgs& a, int dtype, void* km, hipStream_t st) {
   dim3 grid(a.H, a.B), block(a.D);
   if (dtype == 0) kmean_finalize_kernel<0><<<grid, block, 0, st>>>((const double*)a.partial, (u16*)km, a.H, a.L, a.D, a.nchunk, a.cu_seqlens);
   else kmean_finalize_kernel<1><<<grid, block, 0, st>>>((const double*)a.partial, (u16*)km, a.H, a.L, a.D, a.nchunk, a.cu_seqlens);
@@ -605,7 +920,9 @@ hipError_t launch_k_mean(const ColStatArgs& a, int dtype, void* km, hipStream_t 
 hipError_t launch_v_scale(const ColStatArgs& a, int dtype, float* vscale, hipStream_t st) {
   if (a.nchunk == 0 || a.B == 0 || a.H == 0) return hipSuccess;
   hipError_t e = launch_colstat<1>(a, dtype, st);
-  if (e != hipSuccess) return e;
+  return e != hipSuccess ? e : launch_v_scale_finalize(a, vscale, st);
+}
+hipError_t launch_v_scale_finalize(const ColStatArgs& a, float* vscale, hipStream_t st) {
   dim3 grid(a.H, a.B), block(a.D);
   vscale_finalize_kernel<<<grid, block, 0, st>>>((const float*)a.partial, vscale, a.H, a.L, a.D, a.nchunk, a.cu_seqlens);
   return hipGetLastError();
@@ -633,7 +950,7 @@ hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dt
 hipError_t launch_prep_v(const PrepVArgs& a, int dtype, int pv, int max_panels, hipStream_t st) {
   if (max_panels == 0 || a.B == 0 || a.H == 0) return hipSuccess;
   dim3 grid(max_panels, a.H, a.B), block(256);
-#define SAGE_PREPV(DT, DD, PVV) prep_v_kernel<DT, DD, PVV><<<grid, block, 0, st>>>(a)
+#define SAGE_PREPV(DT, DD, PVV) (PVV && a.vs_partial ? prep_v_kernel<DT, DD, PVV, PVV == 1><<<grid, block, 0, st>>>(a) : prep_v_kernel<DT, DD, PVV><<<grid, block, 0, st>>>(a))
   if (dtype == 0) {
     if (a.D == 64) { if (pv) SAGE_PREPV(0, 64, 1); else SAGE_PREPV(0, 64, 0); }
     else { if (pv) SAGE_PREPV(0, 128, 1); else SAGE_PREPV(0, 128, 0); }

@@ -429,6 +429,8 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
     lse = torch.empty((B, Hq, Sq), device=q.device, dtype=torch.float32) if return_lse else None
     ws_bytes = lib().sage_sageattn_workspace_bytes_for(B, Hq, Hkv, Sq, Skv, D, BLKQ | qflag, BLKK | kflag, pv, 0, 0, 0,
                                                        int(bool(smooth_k)), int(bool(return_lse)), int(attn_mask is not None))
+    if pv == PV_FP8:   # room for both statistics at a time: one launch for the two
+        ws_bytes += lib().sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv)
     if attn_mask is not None:
         if is_causal:
             raise NotImplementedError("attn_mask cannot be combined with is_causal")
@@ -501,6 +503,8 @@ def sageattn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqle
     lse = torch.empty((Hq, Tq), device=q.device, dtype=torch.float32) if return_lse else None
     ws_bytes = lib().sage_sageattn_workspace_bytes_for(nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D, BLKQ, BLKK, pv,
                                                        Tq, Tk, 1, int(bool(smooth_k)), int(bool(return_lse)), 0)
+    if pv == PV_FP8:   # (as in sageattn)
+        ws_bytes += lib().sage_prep_v_workspace_bytes(nseq, Hkv, int(max_seqlen_k), D, pv)
     ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
     check(lib().sage_sageattn(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(ws), ws_bytes,
                               nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D,

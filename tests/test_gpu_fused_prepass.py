@@ -1,0 +1,81 @@
+"""The pre-passes that share launches (statistics and plan first, quantiser and V panels second) against the same call made of
+the separate entry points: every intermediate is the same number, so outputs are equal bit for bit."""
+import pytest
+import torch
+
+import baselinebenchmark_amd as sa
+from baselinebenchmark_amd import _cabi
+from tests.helpers import randn
+
+pytestmark = [pytest.mark.gpu, pytest.mark.sage_attention]
+
+
+def _inputs(B, Hq, Hkv, Sq, Skv, D, dtype, layout, seed):
+    g = torch.Generator().manual_seed(seed)
+    q = randn(layout, B, Hq, Sq, D, dtype, g)
+    k = randn(layout, B, Hkv, Skv, D, dtype, g, offset_std=2.0)
+    return q.cuda(), k.cuda(), randn(layout, B, Hkv, Skv, D, dtype, g).cuda()
+
+
+def _steps(q, k, v, layout, pv, blkq, blkk, smooth, mask=None):
+    km = sa.k_mean(k, layout) if smooth else None
+    q8, qs, k8, ks = sa.per_block_int8(q, k, km=km, BLKQ=blkq, BLKK=blkk, tensor_layout=layout)
+    return sa.forward(q8, k8, v, qs, ks, tensor_layout=layout, output_dtype=q.dtype, pv_mode=pv, BLKQ=blkq, BLKK=blkk, attn_mask=mask)[0]
+
+
+# one chunk of 512 rows and a bit, whole chunks, the last length whose statistics the second launch combines itself (8 chunks)
+# and the first that has a launch for it; then grids whose jobs no longer share launches
+@pytest.mark.parametrize("B,H,Skv", [(1, 2, 1025), (1, 2, 1536), (2, 1, 1537), (1, 2, 4096), (1, 2, 4097), (2, 64, 4097)])
+@pytest.mark.parametrize("D,dtype,layout", [(64, torch.float16, "NHD"), (128, torch.bfloat16, "HND")])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("smooth", [True, False])
+def test_one_call_equals_the_separate_passes(B, H, Skv, D, dtype, layout, pv, smooth):
+    q, k, v = _inputs(B, H, H, 70, Skv, D, dtype, layout, Skv + D)
+    for blkq, blkk in ((128, 64), (64, 128), (32, 16)):
+        got = sa.sageattn(q, k, v, tensor_layout=layout, pv_mode=pv, smooth_k=smooth, BLKQ=blkq, BLKK=blkk)
+        assert torch.equal(got, _steps(q, k, v, layout, pv, blkq, blkk, smooth)), (blkq, blkk)
+
+
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("blkq,blkk", [(128, 64), (128, 16), (16, 128)])
+def test_masked_call_equals_the_separate_passes(pv, blkq, blkk):
+    """The Q quantiser and the packing of the mask share the first launch (or, where its rows per wavefront do not suit the K blocks,
+    have one of their own)."""
+    q, k, v = _inputs(2, 2, 2, 300, 1100, 64, torch.float16, "HND", 5)
+    mask = torch.rand((2, 1, 300, 1100), device="cuda") < 0.5
+    got = sa.sageattn(q, k, v, pv_mode=pv, BLKQ=blkq, BLKK=blkk, attn_mask=mask)
+    assert torch.equal(got, _steps(q, k, v, "HND", pv, blkq, blkk, True, mask))
+
+
+@pytest.mark.parametrize("Skv", [1500, 4500])
+def test_workspace_without_room_for_both_statistics(Skv):
+    """FP8 P.V through the C ABI with exactly sage_sageattn_workspace_bytes_for: the statistics run one after the other in the same
+    region; nothing is written past the end, and the output is the one of the call with room for both."""
+    B, H, S, D = 1, 3, 40, 128
+    q, k, v = _inputs(B, H, H, S, Skv, D, torch.bfloat16, "HND", 9)
+    lib = _cabi.lib()
+    need = lib.sage_sageattn_workspace_bytes_for(B, H, H, S, Skv, D, 128, 64, _cabi.PV_FP8, 0, 0, 0, 1, 0, 0)
+    out, ws = torch.empty_like(q), torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    hd = lambda n: (H * n * D, n * D, D)
+    rc = lib.sage_sageattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), None, ws.data_ptr(), need, B, H, H, S, Skv, D,
+                           *hd(S), *hd(Skv), *hd(Skv), *hd(S), 1, 128, 64, float(D ** -0.5), 0, 1, _cabi.PV_FP8, None, None, 0, 0,
+                           torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and bool((ws[need:] == 0xA5).all())
+    assert torch.equal(out, sa.sageattn(q, k, v, pv_mode="fp8"))
+
+
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("smooth", [True, False])
+def test_packed_call_equals_single_sequences(pv, smooth):
+    """The plan shares the first launch: lengths of nothing, one row, one chunk, and one sequence past eight chunks."""
+    lens = [0, 1, 130, 0, 512, 700, 4200]
+    g = torch.Generator().manual_seed(3)
+    T = sum(lens)
+    q, k, v = (torch.randn((T, h, 64), generator=g).to(torch.float16).cuda() for h in (4, 2, 2))
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device="cuda")
+    got = sa.sageattn_varlen(q, k, v, cu, cu, max(lens), max(lens), is_causal=True, pv_mode=pv, smooth_k=smooth)
+    for i, n in enumerate(lens):
+        if n:
+            s = slice(int(cu[i]), int(cu[i]) + n)
+            one = sa.sageattn(q[None, s], k[None, s], v[None, s], tensor_layout="NHD", is_causal=True, pv_mode=pv, smooth_k=smooth)
+            assert torch.equal(got[s], one[0]), n
