@@ -15,7 +15,10 @@ hipError_t launch_attn_qfused(const AttnArgs& a, int D, int pv, bool causal, int
     return pv ? SAGE_ATTN_Q(64, 1, 128, false, true) : SAGE_ATTN_Q(64, 0, 128, false, true);
   }
   if (D == 128) return pv ? (msum ? SAGE_ATTN_Q(128, 1, 128, true, false) : SAGE_ATTN_Q(128, 1, 128, false, false)) : SAGE_ATTN_Q(128, 0, 128, false, false);
-  return pv ? (msum ? SAGE_ATTN_Q(64, 1, 128, true, false) : SAGE_ATTN_Q(64, 1, 128, false, false)) : (msum ? SAGE_ATTN_Q(64, 0, 128, true, false) : SAGE_ATTN_Q(64, 0, 128, false, false));
+  if (pv || !msum) return pv ? (msum ? SAGE_ATTN_Q(64, 1, 128, true, false) : SAGE_ATTN_Q(64, 1, 128, false, false)) : SAGE_ATTN_Q(64, 0, 128, false, false);
+  // (as in launch_attn: 16 heads of 6000 rows 170.0 us instead of 175.3, 2 x 8 of 16384 951 instead of 971)
+  if (!causal) return a.blkk >= 64 ? launch_one<64, 8, 128, 0, false, true, 0, 1, true, 2>(a, grid, st) : launch_one<64, 8, 128, 0, false, true, 0, 1, true, 1>(a, grid, st);
+  return a.blkk >= 128 ? launch_one<64, 8, 128, 0, true, true, 0, 1, true, 4>(a, grid, st) : a.blkk == 64 ? launch_one<64, 8, 128, 0, true, true, 0, 1, true, 2>(a, grid, st) : launch_one<64, 8, 128, 0, true, true, 0, 1, true, 1>(a, grid, st);
 #undef SAGE_ATTN_QW
 #undef SAGE_ATTN_Q
 }
