@@ -16,6 +16,7 @@ Mirrored reference interfaces (same names, argument meaning and error classes):
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -35,12 +36,14 @@ def backend_name() -> str:
 # ------------------------------------------------------------------------------------------------
 # helpers
 # ------------------------------------------------------------------------------------------------
+# (Small calls are bound by the host: on 8 heads of 1024 rows the GPU needs 25 us, and the checks, allocations and the call through
+# ctypes took 22.  Plain integers as pointers, the raw stream handle and one look at shape and strides each keep them near half of that.)
 def _ptr(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _dt(dtype: torch.dtype) -> int:
@@ -62,10 +65,20 @@ def _check_float(name: str, x) -> None:
 def _layout(t: torch.Tensor, tensor_layout: str):
     """(B, H, L, D, stride_b, stride_h, stride_n), sageattention_triton.py:132-137."""
     if tensor_layout == "HND":
-        return t.shape[0], t.shape[1], t.shape[2], t.shape[3], t.stride(0), t.stride(1), t.stride(2)
+        (b, h, n, d), (sb, sh, sn, _) = t.shape, t.stride()
+        return b, h, n, d, sb, sh, sn
     if tensor_layout == "NHD":
-        return t.shape[0], t.shape[2], t.shape[1], t.shape[3], t.stride(0), t.stride(2), t.stride(1)
+        (b, n, h, d), (sb, sn, sh, _) = t.shape, t.stride()
+        return b, h, n, d, sb, sh, sn
     raise ValueError(f"tensor_layout {tensor_layout!r} is not supported")
+
+
+@functools.lru_cache(maxsize=1024)
+def _workspace_bytes(B, Hq, Hkv, Sq, Skv, D, blkq, blkk, pv, Tq, Tk, varlen, smooth, lse, mask) -> int:
+    """Workspace of a one-call pipeline, a function of these numbers alone; FP8 P.V with room for both statistics at a time, which
+    then share a launch."""
+    n = lib().sage_sageattn_workspace_bytes_for(B, Hq, Hkv, Sq, Skv, D, blkq, blkk, pv, Tq, Tk, varlen, smooth, lse, mask)
+    return n + (lib().sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv) if pv == PV_FP8 else 0)
 
 
 def _check_blocks_quant(BLKQ, BLKK):
@@ -194,6 +207,7 @@ def _pv(pv_mode) -> int:
     raise ValueError(f"pv_mode {pv_mode!r} is not 'fp16' or 'fp8'")
 
 
+@torch.no_grad()
 def _mask_args(attn_mask, B, Hq, Sq, Skv, device):
     """Validate an explicit mask and return (tensor kept alive, kind, element strides).
 
@@ -361,7 +375,6 @@ def _apply_recipe(quant_recipe, BLKQ, BLKK, pv_mode):
     return bq, bk, "fp8"
 
 
-@torch.no_grad()
 def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smooth_k=True, pv_mode=None,
              BLKQ=128, BLKK=64, return_lse=False, qk_quant_dtype="int8", quant_recipe=None, attn_mask=None,
              cu_seqlens_q=None, cu_seqlens_k=None, max_seqlen_q=None, max_seqlen_k=None, q_interleave=1,
@@ -424,19 +437,17 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
     if BLKQ not in (16, 32, 64, 128) or BLKK not in (16, 32, 64, 128):
         raise NotImplementedError("the attention kernel needs Q and K scale blocks of 16, 32, 64 or 128 rows")
     pv = _pv(pv_mode)
-    out = torch.empty(q.shape, device=q.device, dtype=q.dtype)
+    out = q.new_empty(q.shape)
     _, _, _, _, osb, osh, osn = _layout(out, tensor_layout)
     lse = torch.empty((B, Hq, Sq), device=q.device, dtype=torch.float32) if return_lse else None
-    ws_bytes = lib().sage_sageattn_workspace_bytes_for(B, Hq, Hkv, Sq, Skv, D, BLKQ | qflag, BLKK | kflag, pv, 0, 0, 0,
-                                                       int(bool(smooth_k)), int(bool(return_lse)), int(attn_mask is not None))
-    if pv == PV_FP8:   # room for both statistics at a time: one launch for the two
-        ws_bytes += lib().sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv)
+    ws_bytes = _workspace_bytes(B, Hq, Hkv, Sq, Skv, D, BLKQ | qflag, BLKK | kflag, pv, 0, 0, 0, int(bool(smooth_k)),
+                                int(bool(return_lse)), int(attn_mask is not None))
     if attn_mask is not None:
         if is_causal:
             raise NotImplementedError("attn_mask cannot be combined with is_causal")
         m, kind, ms = _mask_args(attn_mask, B, Hq, Sq, Skv, q.device)
         ws_bytes += lib().sage_sageattn_mask_bytes(B, Hq, Sq, Skv, kind, ms[0], ms[1], ms[2])
-    ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
+    ws = q.new_empty(max(ws_bytes, 256), dtype=torch.uint8)
     if attn_mask is not None:
         check(lib().sage_sageattn_masked(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(ws), ws_bytes,
                                          B, Hq, Hkv, Sq, Skv, D, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
@@ -470,7 +481,6 @@ def _check_cu(name, cu, device):
         raise ValueError(f"{name} must be on the same device as q")
 
 
-@torch.no_grad()
 def sageattn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, is_causal=False, sm_scale=None,
                     smooth_k=True, pv_mode="fp16", BLKQ=128, BLKK=64, return_lse=False):
     """Packed variable-length attention: q [Tq, Hq, D], k/v [Tk, Hkv, D], cu_seqlens int32 [nseq+1]
@@ -501,11 +511,9 @@ def sageattn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqle
     pv = _pv(pv_mode)
     out = torch.empty_like(q)
     lse = torch.empty((Hq, Tq), device=q.device, dtype=torch.float32) if return_lse else None
-    ws_bytes = lib().sage_sageattn_workspace_bytes_for(nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D, BLKQ, BLKK, pv,
-                                                       Tq, Tk, 1, int(bool(smooth_k)), int(bool(return_lse)), 0)
-    if pv == PV_FP8:   # (as in sageattn)
-        ws_bytes += lib().sage_prep_v_workspace_bytes(nseq, Hkv, int(max_seqlen_k), D, pv)
-    ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
+    ws_bytes = _workspace_bytes(nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D, BLKQ, BLKK, pv, Tq, Tk, 1,
+                                int(bool(smooth_k)), int(bool(return_lse)), 0)
+    ws = q.new_empty(max(ws_bytes, 256), dtype=torch.uint8)
     check(lib().sage_sageattn(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(ws), ws_bytes,
                               nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D,
                               0, q.stride(1), q.stride(0), 0, k.stride(1), k.stride(0), 0, v.stride(1), v.stride(0),
