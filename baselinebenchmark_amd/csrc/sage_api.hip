@@ -360,6 +360,11 @@ constexpr int64_t kFewMinHeadElements = 896 * 128, kFewMinReads = (int64_t)32 <<
 // bf16, tiled / few rows: 24 rows, 16 keys 729 / 725 us; 28 rows, 16 keys 733 / 782, 48 keys 814 / 803; 32 rows, 16 keys 743 / 846,
 // 64 keys 846 / 878, 80 keys 925 / 897.  (At head_dim 64, 32 rows, 32 keys 513 / 461; two query heads per KV head: few rows always.)
 bool few_rows_outweigh_keys(int64_t rows, int Sq, int Skv, int D) { return D == 128 && rows == Sq && Skv < 8 * (rows - 22); }
+// FP8 P.V: up to 16 rows the rules above hold (4 x 32/8 heads, 1 row, 8192 keys, head_dim 128, tiled / few rows 146 / 77 us; 2 heads of
+// 8192 keys 95 / 21).  With two score tiles the V quotients do not fit the registers of head_dim 128, and the pass that finds the first
+// tile's maximum costs more: 32 rows, 8 x 8 heads of 2500 / 4200 / 8192 keys 77 / 83, 115 / 114, 196 / 172; 8 x 32 of 8192 546 / 564; at
+// head_dim 64, 1500 / 1800 / 4200 keys 38.4 / 39.2, 41.7 / 37.2, 77.8 / 59.5.
+bool few_rows_pay_fp8(int64_t rows, int64_t pairs, int Skv, int D) { return rows <= 16 || (D == 64 ? Skv >= 1792 : Skv >= 4096 && pairs <= 64); }
 struct E2EWorkspace {
   size_t q_i8, k_i8, q_scale, k_scale, km, v_scale, panels, stat, plan, lse_off, total;
   int64_t qs_sh, ks_sh, panel_sh;
@@ -439,10 +444,10 @@ size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, i
 // Few query rows per KV head over a long history: sage_attn_few.hip.  Calls that the general
 // path refuses (its pre-passes have the batch and the heads on grid axes of 65535), slices of 2 GiB and more (32-bit row offsets),
 // rows that overlap and grids of 2^31 threads and more are left to that path.
-static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, int B, int Hkv, int64_t rows, int Sq, int Skv,
+static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, bool want_lse, int B, int Hkv, int64_t rows, int Sq, int Skv,
                           int D, int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
   const int64_t limit = 0x7fffffff;
-  return !varlen && !short_keys && !is_causal && !mask && pv_mode == SAGE_PV_FP16 && rows <= kFewRows && !few_rows_outweigh_keys(rows, Sq, Skv, D) && blk_groups(blkq) == 1 &&
+  return !varlen && !short_keys && !is_causal && !mask && (pv_mode == SAGE_PV_FP16 || (!want_lse && few_rows_pay_fp8(rows, (int64_t)B * Hkv, Skv, D))) && rows <= kFewRows && few_tiles_per_split(B, Hkv, (int)rows, Skv, D, (int64_t)sage_v_panel_bytes(B, Hkv, Skv, D, pv_mode)) > 0 && !few_rows_outweigh_keys(rows, Sq, Skv, D) && blk_groups(blkq) == 1 &&
          blk_groups(blkk) == 1 && B <= 65535 && Hkv <= 65535 && ((int64_t)B * Hkv + kFewWorkgroups) * 256 <= limit &&
          q && k && v && out && k_sn >= D && v_sn >= D && (int64_t)Sq * q_sn * 2 < limit &&
          ((int64_t)Skv + 128) * k_sn * 2 < limit && ((int64_t)Skv + 128) * v_sn * 2 < limit;
@@ -522,25 +527,36 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   const bool short_keys = no_keys || (!varlen && Skv <= kSmallPrepassRows && k_elements <= kFewMinElements &&
                                       (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
-  if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, B, Hkv, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
+  if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, lse != nullptr, B, Hkv, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
                     out, q_sn, k_sn, v_sn)) {
     if (int rc2 = check_stride16("q", q_sb, q_sh, q_sn, 2, q)) return rc2;
     if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;
     if (int rc2 = check_stride16("v", v_sb, v_sh, v_sn, 2, v)) return rc2;
     if (int rc2 = check_stride16("out", o_sb, o_sh, o_sn, 2, out)) return rc2;
-    if (smooth_k) {
-      rc = sage_k_mean(k, km, stat, stat_bytes, B, Hkv, Skv, D, k_sb, k_sh, k_sn, dtype, nullptr, stream);
-      if (rc) return rc;
-    }
+    // the statistics of K (smoothing) and V (FP8 P.V): per chunk; the kernel combines the chunks itself.  V's lie where the INT8 copy
+    // of K would (a float per channel and 512 rows, against a byte per channel and row), the partial results where the panels would.
+    FusedPrepass stats;
+    memset(&stats, 0, sizeof(stats));
+    ColStatArgs& ks = stats.k_stat;
+    ks.x = (const u16*)k; ks.B = B; ks.H = Hkv; ks.L = Skv; ks.D = D; ks.x_sb = k_sb; ks.x_sh = k_sh; ks.x_sn = k_sn;
+    ks.nchunk = colstat_chunks(Skv);
+    stats.v_stat = ks;
+    stats.v_stat.x = (const u16*)v; stats.v_stat.x_sb = v_sb; stats.v_stat.x_sh = v_sh; stats.v_stat.x_sn = v_sn;
+    if (smooth_k) ks.partial = stat;
+    if (pv_mode == SAGE_PV_FP8) stats.v_stat.partial = k_i8;
+    hipError_t e = launch_fused_prepass(stats, dtype, D, pv_mode == SAGE_PV_FP8, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "sage_sageattn(statistics)");
     FewArgs f;
     memset(&f, 0, sizeof(f));
-    f.q = (const u16*)q; f.k = (const u16*)k; f.v = (const u16*)v; f.km = smooth_k ? (const u16*)km : nullptr;
+    f.q = (const u16*)q; f.k = (const u16*)k; f.v = (const u16*)v;
+    f.km_partial = (const double*)ks.partial; f.vs_partial = (const float*)stats.v_stat.partial; f.nchunk = ks.nchunk;
     f.out = (u16*)out; f.lse = lse; f.part = (float*)panels;   // (no panels here: their region holds the partial results)
+    f.part_bytes = (int64_t)sage_v_panel_bytes(B, Hkv, Skv, D, pv_mode);
     f.B = B; f.Hq = Hq; f.Hkv = Hkv; f.Sq = Sq; f.Skv = Skv;
     f.q_sb = q_sb; f.q_sh = q_sh; f.q_sn = q_sn; f.k_sb = k_sb; f.k_sh = k_sh; f.k_sn = k_sn;
     f.v_sb = v_sb; f.v_sh = v_sh; f.v_sn = v_sn; f.o_sb = o_sb; f.o_sh = o_sh; f.o_sn = o_sn;
     f.blkq_shift = ilog2(blkq); f.blkk_shift = ilog2(blkk); f.q_mult = q_mult;
-    hipError_t e = launch_attn_few(f, dtype, D, (hipStream_t)stream);
+    e = launch_attn_few(f, dtype, D, pv_mode == SAGE_PV_FP8, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sage_sageattn(few rows)");
     return SAGE_OK;
   }
@@ -628,14 +644,14 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   memset(&pl, 0, sizeof(pl));
   if (varlen) pl = {cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, attn_config(128, 1, true).nw * 32, 64, is_causal, plan};
   // The pre-passes in two launches: what depends on nothing but the call's tensors, then what needs the statistics or the plan.  The two
-  // statistics then exist at the same time; where the workspace has no room for both (it is sized for one after the other), and for
-  // grids past one axis, every pass is a launch of its own.
+  // statistics then exist at the same time; where the workspace has no room for both (it is sized for one after the other) the
+  // passes follow each other.
   FusedPrepass first, second;
   memset(&first, 0, sizeof(first));
   memset(&second, 0, sizeof(second));
   const size_t v_stat_bytes = fp8 && smooth_k ? sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv_mode) : 0;
   const bool k_long = smooth_k && ks.nchunk > kFusedChunks, v_long = fp8 && ks.nchunk > kFusedChunks;
-  bool fused = keys && !small_prepass && (int64_t)B <= 65535 && Hq <= 65535 && workspace_bytes - w.total >= v_stat_bytes + (used - w.total);
+  const bool fused = keys && !small_prepass && (int64_t)B <= 65535 && Hq <= 65535 && workspace_bytes - w.total >= v_stat_bytes + (used - w.total);
   if (fused) {
     first.plan = pl;
     if (smooth_k) first.k_stat = ks;
@@ -649,8 +665,6 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
       FusedPrepass& f = varlen ? second : first;
       if (!f.k_quant.out || fused_quant_together(D, f.k_quant.blk, qq.blk)) { f.q_quant = qq; qq.out = nullptr; }
     }
-    fused = fused_prepass_workgroups(first) <= kFusedMaxWorkgroups && fused_prepass_workgroups(second) <= kFusedMaxWorkgroups;
-    if (!fused && !fuse_q) qq.out = q_i8;
   }
   hipError_t e = hipSuccess;
   if (fused) {

@@ -1,4 +1,4 @@
-// Attention of a few query rows over a long history (token generation): FP16 P.V, no mask, at most kFewRows rows per KV head
+// Attention of a few query rows over a long history (token generation): no mask, not causal, at most kFewRows rows per KV head
 // counting all query heads that share it.
 //
 // Bound by the bytes of K and V.  The tiled kernel gives a q-tile of 256 rows to every query head, so one row per head leaves
@@ -13,10 +13,13 @@
 // The order of the channels inside the Q.K^T contraction and of the keys inside the P.V one is free as long as both operands
 // agree: K fragments take the channels as whole 64-byte pieces of a row arrive, V fragments the keys as the 16x16 score tile
 // holds them, so neither the scores nor V go through LDS.
-// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 52.4 us
-// (this kernel 34 us = 3.9 TB/s of K and V, half of it vector arithmetic of the quantisation; K mean 15, merge 4); 8 rows: 170.8
-// -> 58.5; 8 x 32/8 heads, 4 rows, 16384 keys: 431.9 -> 158.9; 16 x 24 heads, 4096 keys: 452.4 -> 223.8; 1 x 2 heads, 32768
-// keys: 435.3 -> 53.2; 1 x 8/2 heads, 2048 keys: 47.1 -> 33.7.
+//   * the statistics (K mean, V scales) arrive per chunk of 512 rows and are combined by every workgroup: a launch less;
+//   * FP8 P.V: V is rounded to the e4m3 values of the panels in registers (a division per element: the vector ALU is what bounds it)
+//     and multiplied in fp16, which holds them; the probabilities are the tiled kernel's block-scaled codes, read back the same way.
+// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 46.3 us (this
+// kernel 33 us = 4.1 TB/s of K and V, half of it vector arithmetic of the quantisation; K sums 12, merge 4); 8 rows: 170.8
+// -> 55; 8 x 32/8 heads, 4 rows, 16384 keys: 431.9 -> 155; 16 x 32 heads, 4096 keys: 600 -> 286; 1 x 8/2 heads, 8 rows, 32768 keys:
+// 435 -> 62.  FP8 P.V: 146 -> 77, and 313 -> 67 for the last.
 #include "sage_launch.h"
 
 #pragma clang fp contract(off)
@@ -46,7 +49,7 @@ __device__ __forceinline__ v4i pack16(const float (&x)[16], Quotient quotient) {
   return v4i{(int)packed[0], (int)packed[1], (int)packed[2], (int)packed[3]};
 }
 
-template <int DT, int D, int MT>
+template <int DT, int D, int MT, int PV>
 __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   constexpr int LK = D / 32;   // 16-byte pieces of a K row per lane: piece i holds the channels 32 i + 8 (lane / 16) ..+7
   constexpr int KS = D / 64;   // contraction steps of Q.K^T
@@ -77,14 +80,50 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 #pragma unroll
       for (int i = 0; i < LK; i++) kraw[t][i] = __builtin_amdgcn_raw_buffer_load_b128(krsrc, off + t * 16 * (int)a.k_sn * 2 + 64 * i, 0, 0);
   };
-  if (t0 < t1) load_k(t0);
+  // ---- K mean and V scales from the per-chunk statistics, in chunk order (kmean_finalize_kernel, vscale_finalize_kernel) ----
+  __shared__ __align__(16) u16 km_lds[D];
+  [[maybe_unused]] __shared__ __align__(16) float2 vs_lds[PV ? D : 1];   // scale and its reciprocal
+  [[maybe_unused]] bool v_exact = true;
+  {
+    const int64_t at = (int64_t)bh * a.nchunk * D + tid % D;
+    // (head_dim 128: the lower half of the workgroup folds K, the upper one V; at 64 likewise with a quarter each)
+    if (a.km_partial && tid < D) {
+      double s = 0;
+      for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
+        double t[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) t[c] = a.km_partial[at + (int64_t)min(c0 + c, a.nchunk - 1) * D];
+#pragma unroll
+        for (int c = 0; c < 8; c++) s = c0 + c < a.nchunk ? s + t[c] : s;
+      }
+      km_lds[tid] = from_f32<DT>((float)(s / (double)L));
+    }
+    if constexpr (PV == 1) {
+      if (tid >= D && tid < 2 * D) {
+        float mx = 0.f;
+        for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
+#pragma unroll
+          for (int c = 0; c < 8; c++) mx = fmaxf(mx, a.vs_partial[at + (int64_t)min(c0 + c, a.nchunk - 1) * D]);
+        }
+        const float scale = fmaxf(mx / 448.0f, kScaleFloor);
+        vs_lds[tid - D] = make_float2(scale, 1.0f / scale);
+      }
+    }
+    __syncthreads();
+    if constexpr (PV == 1) v_exact = __builtin_amdgcn_ballot_w64(!reciprocal_is_exact(vs_lds[lane].x) || !reciprocal_is_exact(vs_lds[(lane + 64) % D].x)) == 0;
+  }
+  // FP8 P.V: the probability codes of a row are taken relative to the maximum of its first 128 keys (what the tiled kernel's running
+  // maximum is unless a later tile exceeds it by 2^20), so a range that starts later visits tile 0 first, for that maximum alone.
+  const bool reference_first = PV == 1 && t0 > 0 && t0 < t1;
+  const int first = reference_first ? 0 : t0;
+  auto next_tile = [&](int tile) { return reference_first && tile == 0 ? t0 : tile + 1; };
+  if (t0 < t1) load_k(first);
 
   float kmf[LK][8];
-  if (a.km) {
-    const u16* kp = a.km + ((int64_t)b * a.Hkv + kvh) * D + 8 * g;
+  if (a.km_partial) {
 #pragma unroll
     for (int i = 0; i < LK; i++) {
-      const v4u raw = *reinterpret_cast<const v4u*>(kp + 32 * i);
+      const v4u raw = *reinterpret_cast<const v4u*>(km_lds + 8 * g + 32 * i);
 #pragma unroll
       for (int e = 0; e < 8; e++) kmf[i][e] = to_f32<DT>((u16)(raw[e >> 1] >> (16 * (e & 1))));
     }
@@ -141,20 +180,25 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   }
 
   v4f o[MT][CV];
+  // m_used: the maximum that the probabilities are relative to; FP8 P.V: their binary exponent over m_ref instead
   float m_used[MT], lsum[MT];
+  [[maybe_unused]] float m_ref[MT];
+  [[maybe_unused]] __shared__ float tile_max[PV ? 2 : 1][4][PV ? 16 * MT : 1];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) {
-    m_used[mt] = kMInitFew;
+    m_used[mt] = PV == 1 ? kBlockMinExp : kMInitFew;
     lsum[mt] = 0.f;
 #pragma unroll
     for (int i = 0; i < CV; i++) o[mt][i] = v4f{0.f, 0.f, 0.f, 0.f};
   }
 
-  for (int tile = t0; tile < t1; tile++) {
+  int turn = 0;   // which of two sets in LDS: a wavefront writes the next tile's while a slower one still reads this tile's
+  for (int tile = first; tile < t1; tile = next_tile(tile), turn ^= 1) {
     const int n0 = tile * 128 + 32 * w;
+    const bool reference_only = reference_first && tile == 0;
     // V rows 16 t + 4 g + r of the 32 keys, CV channels each: the keys whose scores this lane will hold
     uint32_t vraw[2][4][CV / 2];
-    {
+    if (!reference_only) {
       const int off = ((n0 + 4 * g) * (int)a.v_sn + CV * m) * 2;
 #pragma unroll
       for (int t = 0; t < 2; t++)
@@ -193,10 +237,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     }
     if (a.blkk_shift >= 5) amax[0] = amax[1] = fmaxf(amax[0], amax[1]);
     if (a.blkk_shift >= 6) {
-      // (two sets in turn: a wavefront writes the next tile's while a slower one still reads this tile's)
-      if (lane == 0) block_amax[tile & 1][w] = amax[0];
+      if (lane == 0) block_amax[turn][w] = amax[0];
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (loads in flight stay in flight)
-      const float* p = block_amax[tile & 1];
+      const float* p = block_amax[turn];
       const float pair = fmaxf(p[w & ~1], p[w | 1]);
       amax[0] = amax[1] = a.blkk_shift == 6 ? pair : fmaxf(pair, fmaxf(p[(w & ~1) ^ 2], p[(w | 1) ^ 2]));
     }
@@ -216,13 +259,12 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
         else kreg[t][s] = pack16(x, [&, wide = 1.0 / (double)scale](float v) { return div_by_any(v, wide); });
       }
     }
-    if (tile + 1 < t1) load_k(tile + 1);
+    if (next_tile(tile) < t1) load_k(next_tile(tile));
 
     // ---- scores (lane: query row m, keys 16 t + 4 g + r), probabilities ----
     v8h p[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      float sv[8], mx = kNegInfFew;
+    auto scores = [&](int mt, float (&sv)[8]) __attribute__((always_inline)) -> float {   // returns the row maximum over the wavefront's keys
+      float mx = kNegInfFew;
 #pragma unroll
       for (int t = 0; t < 2; t++) {
         v4i acc = {0, 0, 0, 0};
@@ -236,33 +278,97 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
           mx = fmaxf(mx, sv[4 * t + r]);
         }
       }
-      mx = xor16_32_max(mx);
-      if (__builtin_amdgcn_ballot_w64(mx > m_used[mt] + kTauFew) != 0) {
-        const float m_new = fmaxf(m_used[mt], mx), alpha = __builtin_amdgcn_exp2f(m_used[mt] - m_new);
-        lsum[mt] *= alpha;
+      return xor16_32_max(mx);
+    };
+    auto rescale = [&](int mt, float m_new) __attribute__((always_inline)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_used[mt] - m_new);
+      lsum[mt] *= alpha;
 #pragma unroll
-        for (int i = 0; i < CV; i++) o[mt][i] *= alpha;
-        m_used[mt] = m_new;
+      for (int i = 0; i < CV; i++) o[mt][i] *= alpha;
+      m_used[mt] = m_new;
+    };
+    if constexpr (PV == 1) {
+      // The codes of the tiled kernel (block-scaled by the exponent e of the row's maximum in the tile), read back as the values they
+      // stand for: fp16 holds them, and 2^(e - m_used) keeps the sums of a range in fp32's reach however the tiles differ.
+      float sv[MT][8];
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        const float mx = scores(mt, sv[mt]);
+        if (g == 0) tile_max[turn][w][16 * mt + m] = mx;
       }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const float e = __builtin_amdgcn_exp2f(sv[j] - m_used[mt]);
-        lsum[mt] += e;
-        p[mt][j] = (_Float16)e;
+      for (int mt = 0; mt < MT; mt++) {
+        const int r = 16 * mt + m;
+        const float mall = fmaxf(fmaxf(tile_max[turn][0][r], tile_max[turn][1][r]), fmaxf(tile_max[turn][2][r], tile_max[turn][3][r]));
+        if (tile == 0) m_ref[mt] = mall;
+        const float e = fmaxf(__builtin_ceilf(mall - m_ref[mt]), kBlockMinExp);
+        if (__builtin_amdgcn_ballot_w64(e > m_used[mt]) != 0) rescale(mt, fmaxf(m_used[mt], e));
+        const float c = __builtin_fmaf(-kCodeStep, e, __builtin_fmaf(kCodeStep, kBlockTop - m_ref[mt], kCodeZero)), f = __builtin_amdgcn_exp2f(e - m_used[mt]);
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+          float x[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) x[i] = __builtin_fmaf(sv[mt][j + i], kCodeStep, c);
+          const int code = pack_probability_codes(x[0], x[1], x[2], x[3]);
+          const v2f lo = __builtin_amdgcn_cvt_pk_f32_fp8(code, false), hi = __builtin_amdgcn_cvt_pk_f32_fp8(code, true);
+          const float v[4] = {lo[0] * f, lo[1] * f, hi[0] * f, hi[1] * f};
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            lsum[mt] += v[i];
+            p[mt][j + i] = (_Float16)v[i];
+          }
+        }
+      }
+      if (reference_only) {   // (nothing but m_ref was wanted)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) { m_used[mt] = kBlockMinExp; lsum[mt] = 0.f; }
+        continue;
+      }
+    } else {
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        float sv[8];
+        const float mx = scores(mt, sv);
+        if (__builtin_amdgcn_ballot_w64(mx > m_used[mt] + kTauFew) != 0) rescale(mt, fmaxf(m_used[mt], mx));
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          const float e = __builtin_amdgcn_exp2f(sv[j] - m_used[mt]);
+          lsum[mt] += e;
+          p[mt][j] = (_Float16)e;
+        }
       }
     }
     // ---- O^T += V^T . P^T: matrix row c of product i is channel CV c + i ----
+    auto accumulate = [&](auto narrow) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < CV; i++) {
-      v8h vf;
+      for (int i = 0; i < CV; i++) {
+        v8h vf;
+        float2 vs = {1.f, 1.f};
+        if constexpr (PV == 1) vs = vs_lds[CV * m + i];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const u16 bits = (u16)(vraw[j >> 2][j & 3][i >> 1] >> (16 * (i & 1)));
-        vf[j] = DT == 0 ? __builtin_bit_cast(_Float16, bits) : (_Float16)bf16_to_f32(bits);
+        for (int j = 0; j < 8; j += 2) {
+          const u16 b0 = (u16)(vraw[j >> 2][j & 3][i >> 1] >> (16 * (i & 1))), b1 = (u16)(vraw[(j + 1) >> 2][(j + 1) & 3][i >> 1] >> (16 * (i & 1)));
+          if constexpr (PV == 1) {
+            // the e4m3 code of the panels (prep_v_tile), widened again: fp16 holds every e4m3 value, so only V is rounded to 8 bits
+            const float z0 = fminf(fmaxf(narrow(to_f32<DT>(b0), vs), -448.f), 448.f), z1 = fminf(fmaxf(narrow(to_f32<DT>(b1), vs), -448.f), 448.f);
+            const int code = __builtin_amdgcn_cvt_pk_fp8_f32(z0, z1, 0, false);
+            const v2f w2 = __builtin_amdgcn_cvt_pk_f32_fp8(code, false);
+            const v2h h2 = __builtin_convertvector(w2, v2h);
+            vf[j] = h2[0];
+            vf[j + 1] = h2[1];
+          } else {
+            vf[j] = DT == 0 ? __builtin_bit_cast(_Float16, b0) : (_Float16)bf16_to_f32(b0);
+            vf[j + 1] = DT == 0 ? __builtin_bit_cast(_Float16, b1) : (_Float16)bf16_to_f32(b1);
+          }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) o[mt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[mt], o[mt][i], 0, 0, 0);
+        if constexpr (PV == 1) __builtin_amdgcn_sched_barrier(0);   // (one channel's quotients at a time: several do not fit the registers)
       }
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) o[mt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[mt], o[mt][i], 0, 0, 0);
-    }
+    };
+    if (PV == 0 || v_exact) accumulate([](float x, float2 vs) { return div_by_uniform(x, vs.x, vs.y); });
+    else accumulate([](float x, float2 vs) { return div_by_any(x, 1.0 / (double)vs.x); });
   }
 
   // ---- the four wavefronts' parts into one, in their order ----
@@ -283,8 +389,8 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 #pragma unroll
     for (int i = 0; i < CV; i++) o[mt][i] *= f;
   }
-  for (int turn = 0; turn < 4; turn++) {
-    if (w == turn) {
+  for (int part_of = 0; part_of < 4; part_of++) {
+    if (w == part_of) {
 #pragma unroll
       for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -293,7 +399,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 #pragma unroll
           for (int i = 0; i < CV; i += 4) {
             float4 v = make_float4(o[mt][i][r], o[mt][i + 1][r], o[mt][i + 2][r], o[mt][i + 3][r]);
-            if (turn) {
+            if (part_of) {
               const float4 u = *reinterpret_cast<const float4*>(dst + i);
               v = make_float4(u.x + v.x, u.y + v.y, u.z + v.z, u.w + v.w);
             }
@@ -306,7 +412,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   float* part = a.part + ((int64_t)bh * a.nsplit + split) * few_part_floats(rows, D);
   for (int i = tid; i < rows * (D / 4); i += 256) {
     const int r = i / (D / 4), c = i - r * (D / 4);
-    reinterpret_cast<float4*>(part)[i] = *reinterpret_cast<const float4*>(merged + r * LDO + 4 * c);
+    float4 v = *reinterpret_cast<const float4*>(merged + r * LDO + 4 * c);
+    if constexpr (PV == 1) v = make_float4(v.x * vs_lds[4 * c].x, v.y * vs_lds[4 * c + 1].x, v.z * vs_lds[4 * c + 2].x, v.w * vs_lds[4 * c + 3].x);
+    reinterpret_cast<float4*>(part)[i] = v;
   }
   float* meta = part + rows * D;   // m, l and the smoothing term of every row
   if (tid < rows) {
@@ -343,25 +451,27 @@ __global__ void __launch_bounds__(128) attn_few_merge_kernel(FewArgs a, int D) {
     acc = __builtin_fmaf(part[i * stride + r * D + d], f, acc);
   }
   a.out[(int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + d] = from_f32<DT>(acc * (l > 0.f ? 1.0f / l : 0.f));
-  if (a.lse && d == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km ? meta[2 * rows] : 0.f) : kNegInfFew;
+  if (a.lse && d == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
 }
 
 }  // namespace
 
-hipError_t launch_attn_few(FewArgs a, int dtype, int D, hipStream_t st) {
+hipError_t launch_attn_few(FewArgs a, int dtype, int D, int pv, hipStream_t st) {
   const int rows = a.Hq / a.Hkv * a.Sq, ntiles = (a.Skv + 127) / 128, pairs = a.B * a.Hkv;
   // Two workgroups of four wavefronts per compute unit, no range shorter than one tile.
-  const int want = (kFewWorkgroups + pairs - 1) / pairs;
-  a.tiles_per_split = (ntiles + want - 1) / want;
+  a.tiles_per_split = few_tiles_per_split(a.B, a.Hkv, rows, a.Skv, D, a.part_bytes);
+  if (a.tiles_per_split < 1) return hipErrorInvalidValue;
   a.nsplit = (ntiles + a.tiles_per_split - 1) / a.tiles_per_split;
   a.div_nsplit = make_fastdiv(a.nsplit);
   // The pairs go on x, the one grid axis that is not limited to 65535.  In the main kernel the ranges of a pair stay neighbours:
   // with the pairs next to each other instead, 4 x 32/8 heads of 8192 keys took 50.9 us instead of 49.2.
   const dim3 grid(pairs * a.nsplit), block(256);
-#define SAGE_FEW(DT, DD) (rows > 16 ? attn_few_kernel<DT, DD, 2><<<grid, block, 0, st>>>(a) : attn_few_kernel<DT, DD, 1><<<grid, block, 0, st>>>(a))
+#define SAGE_FEW_P(DT, DD, PVV) (rows > 16 ? attn_few_kernel<DT, DD, 2, PVV><<<grid, block, 0, st>>>(a) : attn_few_kernel<DT, DD, 1, PVV><<<grid, block, 0, st>>>(a))
+#define SAGE_FEW(DT, DD) (pv ? SAGE_FEW_P(DT, DD, 1) : SAGE_FEW_P(DT, DD, 0))
   if (dtype == 0) { if (D == 64) SAGE_FEW(0, 64); else SAGE_FEW(0, 128); }
   else { if (D == 64) SAGE_FEW(1, 64); else SAGE_FEW(1, 128); }
 #undef SAGE_FEW
+#undef SAGE_FEW_P
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (dtype == 0) attn_few_merge_kernel<0><<<dim3(pairs, rows), dim3(D), 0, st>>>(a, D);

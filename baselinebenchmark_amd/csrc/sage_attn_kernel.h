@@ -55,7 +55,6 @@ constexpr float kBiasF = 12582912.0f;     // 1.5 * 2^23
 constexpr int kBiasBits = 0x4B400000;     // its bit pattern; int accumulators start here
 constexpr float kNegInf = -__builtin_inff();
 constexpr float kMInit = -1.0e30f;
-constexpr float kCodeBias = -0.3f;       // centres the linear-mantissa fp8 code of the probabilities (see softmax)
 
 template <int PV> struct PCfg;
 template <> struct PCfg<1> { static constexpr float tau = 3.0f, pshift = 5.0f; };   // fp8: p*32 <= 256 < 448
@@ -63,7 +62,7 @@ template <> struct PCfg<0> { static constexpr float tau = 8.0f, pshift = 0.0f; }
 // Block-scaled probability codes (FP8 P.V kernels without LSE or an explicit mask, see softmax): the largest probability of a
 // query row in a 128-key tile is coded within one binade below 2^kBlockTop (code <= 126 = 448), the block's power-of-two
 // scale goes to the MFMA as an E8M0 byte, kBlockScaleBias + exponent; the running maximum then only has to keep fp32 in range.
-constexpr float kBlockTop = 8.75f, kBlockTau = 20.0f, kBlockMinExp = -110.0f, kBlockScaleBias = 119.0f;   // 119 = 127 - 8
+constexpr float kBlockTau = 20.0f, kBlockScaleBias = 119.0f;   // 119 = 127 - 8 (the code itself: sage_common.h)
 
 // NOTE: __builtin_bit_cast applied directly to an element of an ext_vector_type value reads element
 // 0 whatever the index (clang miscompiles the element lvalue), so vector elements are always passed
@@ -925,8 +924,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       // below the largest key of ITS tile -- not below the row's running maximum, as a statically scaled code would do,
       // which loses a flat tail of many keys under a single large one.  The row sums of these very codes, with the
       // same scales, come from the matrix pipe too, so numerator and denominator of O see the same values.
-      constexpr float kN = 256.0f / 65535.0f, kN8 = 8.0f * kN;
-      constexpr float kC = kN * (56.0f + kCodeBias) + 127.5f / 65535.0f;
+      constexpr float kN8 = kCodeStep, kC = kCodeZero;
       // (a row with no visible key in the tile has maximum -inf: the clamp gives it a finite exponent, its codes are zero)
       const float e = fmaxf(__builtin_ceilf(mall - m_used), kBlockMinExp);
       const float k0 = __builtin_fmaf(-kN8, e, __builtin_fmaf(kN8, kBlockTop - m_used, kC));
@@ -944,9 +942,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
         for (int r = 0; r < 16; r++) t8[r] = __builtin_fmaf(as_f(acc[nt][r]), mul[subof(r)], c[subof(r)]);
 #pragma unroll
         for (int q4 = 0; q4 < 4; q4++) {
-          const unsigned w01 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pknorm_u16(t8[4 * q4], t8[4 * q4 + 1]));
-          const unsigned w23 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pknorm_u16(t8[4 * q4 + 2], t8[4 * q4 + 3]));
-          acc[0][4 * nt + q4] = (int)__builtin_amdgcn_perm(w23, w01, 0x07050301u);
+          acc[0][4 * nt + q4] = pack_probability_codes(t8[4 * q4], t8[4 * q4 + 1], t8[4 * q4 + 2], t8[4 * q4 + 3]);
         }
       }
     } else if constexpr (PV == 1) {

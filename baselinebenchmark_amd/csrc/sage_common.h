@@ -200,6 +200,17 @@ __device__ inline bool reciprocal_is_exact(float s) {
 // (Three instructions an element; inlined true divisions were a tenth of the attention kernels' code, nearly never run.)
 __device__ inline float div_by_any(float x, double r) { return (float)((double)x * r); }
 
+// FP8 probabilities as block-scaled linear-mantissa codes (explained at the softmax of sage_attn_kernel.h): the code of 2^t is
+// 8 t + 56 + kCodeBias, t = s - m - e + kBlockTop; pack_probability_codes takes (256 code + 127.5) / 65535 of four scores.
+constexpr float kCodeBias = -0.3f;       // centres the linear-mantissa code
+constexpr float kBlockTop = 8.75f, kBlockMinExp = -110.0f;
+constexpr float kCodeStep = 8.0f * 256.0f / 65535.0f, kCodeZero = 256.0f / 65535.0f * (56.0f + kCodeBias) + 127.5f / 65535.0f;
+__device__ inline int pack_probability_codes(float a, float b, float c, float d) {
+  const unsigned w01 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pknorm_u16(a, b));
+  const unsigned w23 = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pknorm_u16(c, d));
+  return (int)__builtin_amdgcn_perm(w23, w01, 0x07050301u);
+}
+
 // INT8 codes of N quotients (a multiple of four): q = trunc(z + 0.5 sgn(z)), four to a dword.  |z| <= 127.5, so the low byte of the
 // converted integer is the code, and three byte permutes gather four of them (masks and shifts took twice the instructions).
 template <int N, class Quotient>

@@ -97,9 +97,14 @@ __device__ inline uint32_t fastdiv(uint32_t n, const FastDiv& f) {
 constexpr int kFewRows = 32;          // query rows per KV head, over all query heads of its group
 constexpr int kFewWorkgroups = 512;   // two per compute unit, what the registers allow at once
 struct FewArgs {
-  const u16 *q, *k, *v, *km;   // km: [B, Hkv, D] or null
+  const u16 *q, *k, *v;
+  // per-chunk statistics (ColStatArgs), combined in the kernel: sums of K or null (no smoothing), abs-maxima of V (FP8 P.V) or null
+  const double* km_partial;
+  const float* vs_partial;
+  int nchunk;
   u16* out;
   float *lse, *part;
+  int64_t part_bytes;   // room for partial results
   int B, Hq, Hkv, Sq, Skv;
   int64_t q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, v_sb, v_sh, v_sn, o_sb, o_sh, o_sn;
   int blkq_shift, blkk_shift;
@@ -108,9 +113,18 @@ struct FewArgs {
   FastDiv div_nsplit;
 };
 __host__ __device__ inline int64_t few_part_floats(int rows, int D) { return (int64_t)rows * D + (3 * rows + 3) / 4 * 4; }
-// (at most one partial result per 128 keys: 32 rows of 524 bytes at head_dim 128, against the 32 KiB of an FP16 V panel)
+// (at most one partial result per 128 keys: 32 rows of 524 bytes at head_dim 128, against the 32 KiB of an FP16 V panel; an FP8 panel
+// has 16, and the launcher makes the ranges longer where they do not fit)
 static_assert((kFewRows * 128 + 3 * kFewRows) * 4 <= 128 * 128 * 2 && (kFewRows * 64 + 3 * kFewRows) * 4 <= 128 * 64 * 2, "partials fit the panel region");
-hipError_t launch_attn_few(FewArgs a, int dtype, int D, hipStream_t st);
+// Ranges of the keys, each of few_tiles_per_split() tiles; 0 where not even one range per pair fits.
+inline int few_tiles_per_split(int B, int Hkv, int rows, int Skv, int D, int64_t part_bytes) {
+  const int64_t ntiles = (Skv + 127) / 128, pairs = (int64_t)B * Hkv, want = (kFewWorkgroups + pairs - 1) / pairs;
+  const int64_t room = part_bytes / (pairs * few_part_floats(rows, D) * 4);   // ranges per pair
+  if (room < 1) return 0;
+  const int64_t n = want < room ? want : room;
+  return (int)((ntiles + n - 1) / n);
+}
+hipError_t launch_attn_few(FewArgs a, int dtype, int D, int pv, hipStream_t st);
 
 struct AttnArgs {
   const int8_t* q;
@@ -188,10 +202,8 @@ struct FusedPrepass {
   PrepVArgs v_panels;     // if v_panels.panels
   MaskPackArgs mask;      // if mask.bits
 };
-// Whether one launch can run both quantisers (they share the rows per wavefront), and the workgroups it takes.
+// Whether one launch can run both quantisers (they share the rows per wavefront).
 bool fused_quant_together(int D, int blk_a, int blk_b);
-int64_t fused_prepass_workgroups(const FusedPrepass& f);
-constexpr int64_t kFusedMaxWorkgroups = (int64_t)1 << 23;   // one grid axis holds 2^31 threads
 hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv, hipStream_t st);
 // K mean / V scales from the per-chunk statistics a launch above has written (sequences of more than kFusedChunks chunks).
 hipError_t launch_k_mean_finalize(const ColStatArgs& a, int dtype, void* km, hipStream_t st);

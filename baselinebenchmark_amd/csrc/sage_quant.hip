@@ -822,12 +822,7 @@ static int fused_block(const FusedPrepass& f) {   // the scale block that sets t
   return k > q ? k : q;
 }
 
-int64_t fused_prepass_workgroups(const FusedPrepass& f) {
-  int64_t e[kJobs][3], n = 0;
-  fused_extents(f, fused_block(f), e);
-  for (auto& j : e) n += j[0] * j[1] * j[2];
-  return n;
-}
+constexpr int64_t kFusedMaxWorkgroups = (int64_t)1 << 23;   // one grid axis holds 2^31 threads
 
 template <int MODE>
 static hipError_t launch_colstat(const ColStatArgs& a, int dtype, hipStream_t st);
@@ -861,8 +856,7 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
   for (int j = 0; j < kJobs; j++) {
     if (e[j][1] > 65535 || e[j][2] > 65535) return hipErrorInvalidConfiguration;   // (what the jobs' own grids take)
     n += e[j][0] * e[j][1] * e[j][2];
-    if (n > kFusedMaxWorkgroups) return hipErrorInvalidConfiguration;
-    t.end[j] = (uint32_t)n;
+    t.end[j] = (uint32_t)(n < kFusedMaxWorkgroups ? n : kFusedMaxWorkgroups);
     t.nx[j] = e[j][0] ? (uint32_t)e[j][0] : 1;
     t.nh[j] = e[j][1] ? (uint32_t)e[j][1] : 1;
     t.div_x[j] = make_fastdiv(t.nx[j]);
@@ -872,7 +866,7 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
   int jobs = 0;
   for (auto& j : e) jobs += j[0] * j[1] * j[2] > 0;
   const bool all = e[kJobPlan][0] || e[kJobKStat][0] || e[kJobVStat][0] || e[kJobMask][0];
-  if (jobs == 1 || (!f.plan.plan && n > (all ? kMergeEarly : kMergeLate))) {
+  if (jobs == 1 || n > kFusedMaxWorkgroups || (!f.plan.plan && n > (all ? kMergeEarly : kMergeLate))) {
     for (int j = 0; j < kJobs; j++)
       if (e[j][0] * e[j][1] * e[j][2] > 0)
         if (hipError_t err = launch_job(f, j, dtype, pv, st)) return err;
