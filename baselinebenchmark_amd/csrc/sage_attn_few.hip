@@ -107,6 +107,8 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
         }
         const float scale = fmaxf(mx / 448.0f, kScaleFloor);
         vs_lds[tid - D] = make_float2(scale, 1.0f / scale);
+        if (split == 0) a.vscale[(int64_t)bh * D + tid - D] = scale;   // (applied to the merged, normalised output: infinities and
+                                                                       // sums near fp32's end come out as in the tiled kernel)
       }
     }
     __syncthreads();
@@ -412,9 +414,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   float* part = a.part + ((int64_t)bh * a.nsplit + split) * few_part_floats(rows, D);
   for (int i = tid; i < rows * (D / 4); i += 256) {
     const int r = i / (D / 4), c = i - r * (D / 4);
-    float4 v = *reinterpret_cast<const float4*>(merged + r * LDO + 4 * c);
-    if constexpr (PV == 1) v = make_float4(v.x * vs_lds[4 * c].x, v.y * vs_lds[4 * c + 1].x, v.z * vs_lds[4 * c + 2].x, v.w * vs_lds[4 * c + 3].x);
-    reinterpret_cast<float4*>(part)[i] = v;
+    reinterpret_cast<float4*>(part)[i] = *reinterpret_cast<const float4*>(merged + r * LDO + 4 * c);
   }
   float* meta = part + rows * D;   // m, l and the smoothing term of every row
   if (tid < rows) {
@@ -431,27 +431,66 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   }
 }
 
-// One workgroup of D lanes per (row, batch x KV head): out = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s.
-// A few kilobytes per row out of the L2: bound by the latency of its two rounds of loads.
-template <int DT>
-__global__ void __launch_bounds__(128) attn_few_merge_kernel(FewArgs a, int D) {
-  const int bh = blockIdx.x, r = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv, d = threadIdx.x;
+// One workgroup per (row, batch x KV head): out = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s.
+// A few kilobytes per row out of the L2: bound by the latency of its rounds of loads.  D / 4 lanes take a partial result, as many
+// groups of them as there are partial results (four wavefronts at most) every group's first eight at once, ahead of the maxima.  (With
+// one lane per channel walking all of them, 256 ranges took 22 us: 2 heads of 32768 keys.)
+template <int DT, int D>
+__global__ void __launch_bounds__(256) attn_few_merge_kernel(FewArgs a) {
+  constexpr int LN = D / 4, MAXG = 256 / LN, AHEAD = 8;
+  const int bh = blockIdx.x, r = blockIdx.y, b = bh / a.Hkv, kvh = bh - b * a.Hkv, tid = threadIdx.x;
+  const int lane4 = tid % LN, group = tid / LN, groups = blockDim.x / LN, nwaves = blockDim.x / 64;
   const int G = a.Hq / a.Hkv, rows = G * a.Sq, hq = kvh * G + r / a.Sq, s = r % a.Sq;
   const int64_t stride = few_part_floats(rows, D);
   const float* part = a.part + (int64_t)bh * a.nsplit * stride;
   const float* meta = part + rows * D + r;
-  float top = kMInitFew;
-#pragma unroll 8
-  for (int i = 0; i < a.nsplit; i++) top = fmaxf(top, meta[i * stride]);
-  float l = 0.f, acc = 0.f;
-#pragma unroll 8
-  for (int i = 0; i < a.nsplit; i++) {
-    const float f = __builtin_amdgcn_exp2f(meta[i * stride] - top);
-    l = __builtin_fmaf(meta[i * stride + rows], f, l);
-    acc = __builtin_fmaf(part[i * stride + r * D + d], f, acc);
+  __shared__ float factor[kFewWorkgroups];
+  __shared__ float wave_top[4], wave_sum[4];
+  __shared__ float4 sums[MAXG][LN];
+  float4 o[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; i++) o[i] = reinterpret_cast<const float4*>(part + min(group + i * groups, a.nsplit - 1) * stride + r * D)[lane4];
+  float vs[4] = {1.f, 1.f, 1.f, 1.f};
+  if (a.vs_partial) {
+    const float4 t = reinterpret_cast<const float4*>(a.vscale + (int64_t)bh * D)[lane4];
+    vs[0] = t.x; vs[1] = t.y; vs[2] = t.z; vs[3] = t.w;
   }
-  a.out[(int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + d] = from_f32<DT>(acc * (l > 0.f ? 1.0f / l : 0.f));
-  if (a.lse && d == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+  float top = kMInitFew;
+  for (int i = tid; i < a.nsplit; i += blockDim.x) top = fmaxf(top, meta[i * stride]);
+  top = wave_max(top);
+  if ((tid & 63) == 0) wave_top[tid >> 6] = top;
+  __syncthreads();
+  for (int i = 0; i < nwaves; i++) top = fmaxf(top, wave_top[i]);
+  float l = 0.f;
+  for (int i = tid; i < a.nsplit; i += blockDim.x) {
+    const float f = __builtin_amdgcn_exp2f(meta[i * stride] - top);
+    factor[i] = f;
+    l = __builtin_fmaf(meta[i * stride + rows], f, l);
+  }
+#pragma unroll
+  for (int i = 1; i < 64; i <<= 1) l += __shfl_xor(l, i);
+  if ((tid & 63) == 0) wave_sum[tid >> 6] = l;
+  __syncthreads();
+  l = 0.f;
+  for (int i = 0; i < nwaves; i++) l += wave_sum[i];
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [&](const float4& v, float f) {
+    acc.x = __builtin_fmaf(v.x, f, acc.x); acc.y = __builtin_fmaf(v.y, f, acc.y); acc.z = __builtin_fmaf(v.z, f, acc.z); acc.w = __builtin_fmaf(v.w, f, acc.w);
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; i++)
+    if (group + i * groups < a.nsplit) add(o[i], factor[group + i * groups]);
+#pragma unroll 8
+  for (int i = group + AHEAD * groups; i < a.nsplit; i += groups) add(reinterpret_cast<const float4*>(part + i * stride + r * D)[lane4], factor[i]);
+  sums[group][lane4] = acc;
+  __syncthreads();
+  if (group == 0) {
+    for (int i = 1; i < groups; i++) add(sums[i][lane4], 1.0f);
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const uint2 out = make_uint2(pack2<DT>(acc.x * inv * vs[0], acc.y * inv * vs[1]), pack2<DT>(acc.z * inv * vs[2], acc.w * inv * vs[3]));
+    *reinterpret_cast<uint2*>(a.out + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + 4 * lane4) = out;
+    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+  }
 }
 
 }  // namespace
@@ -465,6 +504,7 @@ hipError_t launch_attn_few(FewArgs a, int dtype, int D, int pv, hipStream_t st) 
   a.div_nsplit = make_fastdiv(a.nsplit);
   // The pairs go on x, the one grid axis that is not limited to 65535.  In the main kernel the ranges of a pair stay neighbours:
   // with the pairs next to each other instead, 4 x 32/8 heads of 8192 keys took 50.9 us instead of 49.2.
+  if (a.nsplit > kFewWorkgroups) return hipErrorInvalidValue;   // (the merge holds a factor per range)
   const dim3 grid(pairs * a.nsplit), block(256);
 #define SAGE_FEW_P(DT, DD, PVV) (rows > 16 ? attn_few_kernel<DT, DD, 2, PVV><<<grid, block, 0, st>>>(a) : attn_few_kernel<DT, DD, 1, PVV><<<grid, block, 0, st>>>(a))
 #define SAGE_FEW(DT, DD) (pv ? SAGE_FEW_P(DT, DD, 1) : SAGE_FEW_P(DT, DD, 0))
@@ -474,8 +514,11 @@ hipError_t launch_attn_few(FewArgs a, int dtype, int D, int pv, hipStream_t st) 
 #undef SAGE_FEW_P
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (dtype == 0) attn_few_merge_kernel<0><<<dim3(pairs, rows), dim3(D), 0, st>>>(a, D);
-  else attn_few_merge_kernel<1><<<dim3(pairs, rows), dim3(D), 0, st>>>(a, D);
+  int threads = 64;   // of the merge: a group of D / 4 lanes per partial result
+  while (threads < 256 && threads < a.nsplit * (D / 4)) threads *= 2;
+  const dim3 mgrid(pairs, rows), mblock(threads);
+  if (dtype == 0) { if (D == 64) attn_few_merge_kernel<0, 64><<<mgrid, mblock, 0, st>>>(a); else attn_few_merge_kernel<0, 128><<<mgrid, mblock, 0, st>>>(a); }
+  else { if (D == 64) attn_few_merge_kernel<1, 64><<<mgrid, mblock, 0, st>>>(a); else attn_few_merge_kernel<1, 128><<<mgrid, mblock, 0, st>>>(a); }
   return hipGetLastError();
 }
 

@@ -101,6 +101,7 @@ struct FewArgs {
   // per-chunk statistics (ColStatArgs), combined in the kernel: sums of K or null (no smoothing), abs-maxima of V (FP8 P.V) or null
   const double* km_partial;
   const float* vs_partial;
+  float* vscale;   // [B, Hkv, D], written by the main kernel for the merge
   int nchunk;
   u16* out;
   float *lse, *part;

@@ -69,3 +69,20 @@ def test_workspace_by_need_is_not_exceeded(D, Sq, Skv):
                            None, 0, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and bool((ws[need:] == 0x5A).all())
     assert torch.equal(out, sa.sageattn(q, k, v, pv_mode="fp8"))
+
+
+@pytest.mark.parametrize("what", ["inf", "-inf", "nan", "huge"])
+def test_infinities_and_large_values_come_out_as_in_the_tiled_kernel(what):
+    """An infinity makes its channel infinite, values near the end of bfloat16's range stay finite: the V scale multiplies the
+    merged, normalised output."""
+    q, k, v = _inputs(1, 4, 2, 2, 2100, 64, torch.bfloat16, 5)
+    if what == "huge":
+        v *= 1e35
+    else:
+        v[0, 1, 1500, 3] = float(what)
+    got, want = sa.sageattn(q, k, v, pv_mode="fp8", BLKQ=16), _tiled(q, k, v, 16)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    if what in ("inf", "-inf"):
+        assert bool(torch.isinf(got).any())
+    elif what == "huge":
+        assert bool(torch.isfinite(got).all())
