@@ -29,6 +29,7 @@ struct QuantArgs {
   const double* km_partial;
   int km_nchunk;
   u16* km_out;
+  int heads_first;   // set by the launcher: grid is (head, rows) instead of (rows, head)
 };
 
 struct ColStatArgs {
@@ -38,6 +39,7 @@ struct ColStatArgs {
   int64_t x_sb, x_sh, x_sn;
   int nchunk;
   const int32_t* cu_seqlens;
+  int heads_first;   // as in QuantArgs
 };
 
 struct PrepVArgs {
@@ -53,6 +55,7 @@ struct PrepVArgs {
   const float* vs_partial;
   int vs_nchunk;
   float* vscale_out;
+  int heads_first;   // as in QuantArgs
 };
 
 struct MaskPackArgs {

@@ -237,14 +237,15 @@ __device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int ch
 
 template <int DT, int D, int NP, bool PARTIAL = false>
 __global__ void __launch_bounds__(256) quant_int8_kernel(QuantArgs a) {
+  const int chunk = a.heads_first ? blockIdx.y : blockIdx.x, h = a.heads_first ? blockIdx.x : blockIdx.y, b = blockIdx.z;
   if constexpr (PARTIAL) {
     __shared__ __align__(16) u16 km_lds[D];
-    quant_int8_rows<DT, D, NP, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, MeanFromPartials<DT, D>{a, (int)blockIdx.y, (int)blockIdx.z, km_lds});
+    quant_int8_rows<DT, D, NP, true>(a, chunk, h, b, MeanFromPartials<DT, D>{a, h, b, km_lds});
     return;
   }
-  const MeanInMemory<DT, D> mean = {a, (int)blockIdx.y, (int)blockIdx.z};
-  if (a.mult == 1.0f) quant_int8_rows<DT, D, NP, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, mean);
-  else quant_int8_rows<DT, D, NP, false>(a, blockIdx.x, blockIdx.y, blockIdx.z, mean);
+  const MeanInMemory<DT, D> mean = {a, h, b};
+  if (a.mult == 1.0f) quant_int8_rows<DT, D, NP, true>(a, chunk, h, b, mean);
+  else quant_int8_rows<DT, D, NP, false>(a, chunk, h, b, mean);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -321,7 +322,8 @@ __device__ __forceinline__ void colstat_chunk(const ColStatArgs a, const int chu
 template <int DT, int D, int MODE>
 __global__ void __launch_bounds__(256) colstat_partial_kernel(ColStatArgs a) {
   __shared__ __align__(16) uint8_t lds[colstat_lds_bytes(D) / (MODE == 0 ? 1 : 2)];
-  colstat_chunk<DT, D, MODE>(a, blockIdx.x, blockIdx.y, blockIdx.z, lds);
+  const bool hf = a.heads_first;
+  colstat_chunk<DT, D, MODE>(a, hf ? blockIdx.y : blockIdx.x, hf ? blockIdx.x : blockIdx.y, blockIdx.z, lds);
 }
 
 // K mean: sum partials in chunk order (float64), /L, -> fp32 -> input dtype.
@@ -527,11 +529,11 @@ __device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, 
 template <int DT, int D, int PV, bool PARTIAL = false>
 __global__ void __launch_bounds__(256) prep_v_kernel(PrepVArgs a) {
   __shared__ __align__(16) uint32_t T[prep_v_lds_bytes(D, PV) / 4];
-  const int h = blockIdx.y, b = blockIdx.z;
+  const int panel = a.heads_first ? blockIdx.y : blockIdx.x, h = a.heads_first ? blockIdx.x : blockIdx.y, b = blockIdx.z;
   if constexpr (PARTIAL) {
     __shared__ float vs_lds[D];
-    prep_v_tile<DT, D, PV>(a, blockIdx.x, h, b, ScalesFromPartials<D>{a, h, b, vs_lds}, T);
-  } else prep_v_tile<DT, D, PV>(a, blockIdx.x, h, b, ScalesInMemory{a.vscale + ((int64_t)b * a.H + h) * D}, T);
+    prep_v_tile<DT, D, PV>(a, panel, h, b, ScalesFromPartials<D>{a, h, b, vs_lds}, T);
+  } else prep_v_tile<DT, D, PV>(a, panel, h, b, ScalesInMemory{a.vscale + ((int64_t)b * a.H + h) * D}, T);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -734,6 +736,7 @@ struct FusedTable {
   uint32_t end[kJobs];       // workgroups of the jobs up to this one
   uint32_t nx[kJobs], nh[kJobs];
   FastDiv div_x[kJobs], div_h[kJobs];   // workgroup of a job -> (x, head, batch)
+  uint32_t heads_first;      // a bit per job: the heads are the inner index instead (nx and nh change places)
 };
 constexpr int kFusedPlanSeqs = 1024;
 constexpr int fused_lds_bytes(int D, int PV) {
@@ -762,7 +765,9 @@ __global__ void __launch_bounds__(256, ALL ? 3 : 4) fused_prepass_kernel(FusedPr
   int job = 0;
   while (blockIdx.x >= t.end[job]) job++;
   const uint32_t i = blockIdx.x - (job ? t.end[job - 1] : 0), y = fastdiv(i, t.div_x[job]);
-  const int x = i - y * t.nx[job], b = fastdiv(y, t.div_h[job]), h = y - b * t.nh[job];
+  const int b = fastdiv(y, t.div_h[job]), inner = i - y * t.nx[job], outer = y - b * t.nh[job];
+  const bool hf = t.heads_first >> job & 1;
+  const int x = hf ? outer : inner, h = hf ? inner : outer;
   if constexpr (ALL) {
     if (job == kJobPlan) { varlen_plan<256, kFusedPlanSeqs>(f.plan, *reinterpret_cast<PlanLds<kFusedPlanSeqs>*>(lds)); return; }
     if (job == kJobKStat) { colstat_chunk<DT, D, 0>(f.k_stat, x, h, b, lds); return; }
@@ -775,9 +780,19 @@ __global__ void __launch_bounds__(256, ALL ? 3 : 4) fused_prepass_kernel(FusedPr
 // ---------------------------------------------------------------------------------------------
 // Host-side launchers (called from the C ABI in sage_api.hip).
 // ---------------------------------------------------------------------------------------------
-hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_rows, hipStream_t st) {
+// Where the heads of a row lie next to each other (packed and [B, L, H, D] tensors), workgroups of the same rows are neighbours, so
+// that whole rows are on their way at a time; with the rows of one head first, a workgroup and its neighbours read 128 or 256 bytes out
+// of every few kilobytes.  96 packed prompts of 16..1024 rows, 8 KV heads of 128, bf16: K quantiser 51.2 -> 34.8 us (154 MB: 3.0 ->
+// 4.4 TB/s), FP16 V panels 49.3 -> 38.6 (205 MB: 4.2 -> 5.3 TB/s); 2 x 16 heads of 4096 rows, FP8: 27.3 -> 25.3 for both.  (The y axis of
+// a grid is limited to 65535.)
+static bool heads_first(int64_t head_stride, int64_t row_stride, int64_t chunks) { return head_stride < row_stride && chunks <= 65535; }
+
+hipError_t launch_quant_int8(const QuantArgs& args, int dtype, int max_rows, hipStream_t st) {
+  QuantArgs a = args;
   const int rows = quant_rows(a.D, a.blk);
-  dim3 grid((max_rows + rows - 1) / rows, a.H, a.B), block(256);
+  const uint32_t chunks = (max_rows + rows - 1) / rows;
+  a.heads_first = heads_first(a.x_sh, a.x_sn, chunks);
+  const dim3 grid = a.heads_first ? dim3(a.H, chunks, a.B) : dim3(chunks, a.H, a.B), block(256);
 #define SAGE_QUANT(DT, DD, NP) (a.km_partial ? quant_int8_kernel<DT, DD, NP, true><<<grid, block, 0, st>>>(a) : quant_int8_kernel<DT, DD, NP><<<grid, block, 0, st>>>(a))
 #define SAGE_QUANT_D(DT) \
   do { \
@@ -853,12 +868,18 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
   const int blk = fused_block(f);
   fused_extents(f, blk, e);
   FusedTable t;
+  const bool inner_heads[kJobs] = {false, heads_first(f.k_stat.x_sh, f.k_stat.x_sn, 0), heads_first(f.v_stat.x_sh, f.v_stat.x_sn, 0),
+                                   heads_first(f.k_quant.x_sh, f.k_quant.x_sn, 0), heads_first(f.q_quant.x_sh, f.q_quant.x_sn, 0),
+                                   heads_first(f.v_panels.v_sh, f.v_panels.v_sn, 0), false};
+  t.heads_first = 0;
   for (int j = 0; j < kJobs; j++) {
     if (e[j][1] > 65535 || e[j][2] > 65535) return hipErrorInvalidConfiguration;   // (what the jobs' own grids take)
     n += e[j][0] * e[j][1] * e[j][2];
     t.end[j] = (uint32_t)(n < kFusedMaxWorkgroups ? n : kFusedMaxWorkgroups);
-    t.nx[j] = e[j][0] ? (uint32_t)e[j][0] : 1;
-    t.nh[j] = e[j][1] ? (uint32_t)e[j][1] : 1;
+    const bool hf = inner_heads[j];
+    t.heads_first |= (uint32_t)hf << j;
+    t.nx[j] = e[j][hf] ? (uint32_t)e[j][hf] : 1;
+    t.nh[j] = e[j][!hf] ? (uint32_t)e[j][!hf] : 1;
     t.div_x[j] = make_fastdiv(t.nx[j]);
     t.div_h[j] = make_fastdiv(t.nh[j]);
   }
@@ -890,8 +911,10 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
 int colstat_chunks(int L) { return (L + kChunkRows - 1) / kChunkRows; }
 
 template <int MODE>
-static hipError_t launch_colstat(const ColStatArgs& a, int dtype, hipStream_t st) {
-  dim3 grid(a.nchunk, a.H, a.B), block(256);
+static hipError_t launch_colstat(const ColStatArgs& args, int dtype, hipStream_t st) {
+  ColStatArgs a = args;
+  a.heads_first = heads_first(a.x_sh, a.x_sn, a.nchunk);
+  const dim3 grid = a.heads_first ? dim3(a.H, a.nchunk, a.B) : dim3(a.nchunk, a.H, a.B), block(256);
   if (dtype == 0 && a.D == 64) colstat_partial_kernel<0, 64, MODE><<<grid, block, 0, st>>>(a);
   else if (dtype == 0 && a.D == 128) colstat_partial_kernel<0, 128, MODE><<<grid, block, 0, st>>>(a);
   else if (dtype == 1 && a.D == 64) colstat_partial_kernel<1, 64, MODE><<<grid, block, 0, st>>>(a);
@@ -941,9 +964,11 @@ hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dt
   return hipGetLastError();
 }
 
-hipError_t launch_prep_v(const PrepVArgs& a, int dtype, int pv, int max_panels, hipStream_t st) {
+hipError_t launch_prep_v(const PrepVArgs& args, int dtype, int pv, int max_panels, hipStream_t st) {
+  PrepVArgs a = args;
   if (max_panels == 0 || a.B == 0 || a.H == 0) return hipSuccess;
-  dim3 grid(max_panels, a.H, a.B), block(256);
+  a.heads_first = heads_first(a.v_sh, a.v_sn, max_panels);
+  const dim3 grid = a.heads_first ? dim3(a.H, max_panels, a.B) : dim3(max_panels, a.H, a.B), block(256);
 #define SAGE_PREPV(DT, DD, PVV) (PVV && a.vs_partial ? prep_v_kernel<DT, DD, PVV, PVV == 1><<<grid, block, 0, st>>>(a) : prep_v_kernel<DT, DD, PVV><<<grid, block, 0, st>>>(a))
   if (dtype == 0) {
     if (a.D == 64) { if (pv) SAGE_PREPV(0, 64, 1); else SAGE_PREPV(0, 64, 0); }

@@ -79,3 +79,32 @@ def test_packed_call_equals_single_sequences(pv, smooth):
             s = slice(int(cu[i]), int(cu[i]) + n)
             one = sa.sageattn(q[None, s], k[None, s], v[None, s], tensor_layout="NHD", is_causal=True, pv_mode=pv, smooth_k=smooth)
             assert torch.equal(got[s], one[0]), n
+
+
+@pytest.mark.parametrize("H", [1, 3, 8])
+@pytest.mark.parametrize("Skv", [1, 129, 1100, 4700])
+@pytest.mark.parametrize("D", [64, 128])
+def test_heads_in_a_row_equal_heads_apart(H, Skv, D):
+    """[B, L, H, D] and packed tensors are walked heads first, [B, H, L, D] rows first: the same numbers from every pre-pass."""
+    q, k, v = _inputs(2, H, H, 70, Skv, D, torch.bfloat16, "NHD", H + Skv)
+    t = [x.transpose(1, 2).contiguous() for x in (q, k, v)]
+    km, km_t = sa.k_mean(k, "NHD"), sa.k_mean(t[1], "HND")
+    assert torch.equal(km.flatten(1), km_t.flatten(1))   # ([B, 1, H, D] and [B, H, 1, D])
+    for blkq, blkk in ((128, 64), (32, 16)):
+        a = sa.per_block_int8(q, k, km=km, BLKQ=blkq, BLKK=blkk, tensor_layout="NHD")
+        b = sa.per_block_int8(t[0], t[1], km=km_t, BLKQ=blkq, BLKK=blkk, tensor_layout="HND")
+        assert torch.equal(a[0], b[0].transpose(1, 2)) and torch.equal(a[1], b[1])
+        assert torch.equal(a[2], b[2].transpose(1, 2)) and torch.equal(a[3], b[3])
+        for pv in ("fp16", "fp8"):
+            got = sa.sageattn(q, k, v, tensor_layout="NHD", pv_mode=pv, BLKQ=blkq, BLKK=blkk)
+            assert torch.equal(got, sa.sageattn(*t, pv_mode=pv, BLKQ=blkq, BLKK=blkk).transpose(1, 2)), pv
+
+
+@pytest.mark.parametrize("rows", [65535 * 64, 65535 * 64 + 1])
+def test_more_rows_than_the_second_grid_axis_holds(rows):
+    """16-row blocks at head_dim 64: 64 rows per workgroup, 65535 workgroups at most beside the heads."""
+    k = torch.randn((1, rows, 2, 64), device="cuda", dtype=torch.float16)
+    _, _, k8, ks = sa.per_block_int8(k[:, :16], k, BLKQ=16, BLKK=16, tensor_layout="NHD")
+    tail = rows - rows // 16 * 16 + 16 * 8
+    _, _, t8, ts = sa.per_block_int8(k[:, :16], k[:, -tail:], BLKQ=16, BLKK=16, tensor_layout="NHD")
+    assert torch.equal(k8[:, -tail:], t8) and torch.equal(ks[..., -ts.shape[-1]:], ts)
