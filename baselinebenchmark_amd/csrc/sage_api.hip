@@ -367,6 +367,7 @@ bool few_rows_outweigh_keys(int64_t rows, int Sq, int Skv, int D) { return D == 
 bool few_rows_pay_fp8(int64_t rows, int64_t pairs, int Skv, int D) { return rows <= 16 || (D == 64 ? Skv >= 1792 : Skv >= 4096 && pairs <= 64); }
 struct E2EWorkspace {
   size_t q_i8, k_i8, q_scale, k_scale, km, v_scale, panels, stat, plan, lse_off, total;
+  size_t k_i8_bytes;
   int64_t qs_sh, ks_sh, panel_sh;
 };
 // What a call's workspace holds beyond K, V and their statistics: the INT8 copy of Q with its scales (calls that may quantise Q by
@@ -384,7 +385,7 @@ E2EWorkspace e2e_layout(int B, int Hq, int Hkv, int Sq, int Skv, int D, int blkq
   size_t nq = varlen ? (size_t)total_q * Hq * D : (size_t)B * Hq * Sq * D;
   size_t nk = varlen ? (size_t)total_k * Hkv * D : (size_t)B * Hkv * Skv * D;
   w.q_i8 = off; off += q_pass ? align_up(nq) : 0;
-  w.k_i8 = off; off += align_up(nk);
+  w.k_i8 = off; w.k_i8_bytes = align_up(nk); off += w.k_i8_bytes;
   if (varlen) {
     w.qs_sh = total_q / blk_rows(blkq) + B; w.ks_sh = total_k / blk_rows(blkk) + B; w.panel_sh = total_k / SAGE_PANEL_ROWS + B;
     w.q_scale = off; off += q_pass ? align_up((size_t)Hq * w.qs_sh * 4) : 0;
@@ -444,13 +445,26 @@ size_t sage_sageattn_mask_bytes(int B, int Hq, int Sq, int Skv, int mask_kind, i
 // Few query rows per KV head over a long history: sage_attn_few.hip.  Calls that the general
 // path refuses (its pre-passes have the batch and the heads on grid axes of 65535), slices of 2 GiB and more (32-bit row offsets),
 // rows that overlap and grids of 2^31 threads and more are left to that path.
-static bool few_rows_path(int varlen, bool short_keys, int is_causal, const void* mask, int pv_mode, bool want_lse, int B, int Hkv, int64_t rows, int Sq, int Skv,
-                          int D, int blkq, int blkk, const void* q, const void* k, const void* v, const void* out, int64_t q_sn, int64_t k_sn, int64_t v_sn) {
-  const int64_t limit = 0x7fffffff;
-  return !varlen && !short_keys && !is_causal && !mask && (pv_mode == SAGE_PV_FP16 || (!want_lse && few_rows_pay_fp8(rows, (int64_t)B * Hkv, Skv, D))) && rows <= kFewRows && few_tiles_per_split(B, Hkv, (int)rows, Skv, D, (int64_t)sage_v_panel_bytes(B, Hkv, Skv, D, pv_mode)) > 0 && !few_rows_outweigh_keys(rows, Sq, Skv, D) && blk_groups(blkq) == 1 &&
-         blk_groups(blkk) == 1 && B <= 65535 && Hkv <= 65535 && ((int64_t)B * Hkv + kFewWorkgroups) * 256 <= limit &&
-         q && k && v && out && k_sn >= D && v_sn >= D && (int64_t)Sq * q_sn * 2 < limit &&
-         ((int64_t)Skv + 128) * k_sn * 2 < limit && ((int64_t)Skv + 128) * v_sn * 2 < limit;
+struct FewCall {
+  int varlen, is_causal, pv_mode, B, Hkv, Sq, Skv, D, blkq, blkk;
+  int64_t rows, q_sn, k_sn, v_sn;   // rows: of all query heads of a KV head
+  const void *q, *k, *v, *out, *mask;
+  bool short_keys, want_lse;
+  size_t k_i8_bytes;   // of the workspace: where the INT8 copy of K would be, the V statistics of FP8 P.V go
+};
+static bool few_rows_path(const FewCall& c) {
+  const int64_t limit = 0x7fffffff, pairs = (int64_t)c.B * c.Hkv;
+  if (c.varlen || c.short_keys || c.is_causal || c.mask || !c.q || !c.k || !c.v || !c.out) return false;
+  if (blk_groups(c.blkq) != 1 || blk_groups(c.blkk) != 1 || c.rows > kFewRows) return false;
+  if (c.B > 65535 || c.Hkv > 65535 || (pairs + kFewWorkgroups) * 256 > limit) return false;
+  if (c.k_sn < c.D || c.v_sn < c.D || (int64_t)c.Sq * c.q_sn * 2 >= limit) return false;
+  if (((int64_t)c.Skv + 128) * c.k_sn * 2 >= limit || ((int64_t)c.Skv + 128) * c.v_sn * 2 >= limit) return false;
+  if (few_tiles_per_split(c.B, c.Hkv, (int)c.rows, c.Skv, c.D, (int64_t)sage_v_panel_bytes(c.B, c.Hkv, c.Skv, c.D, c.pv_mode)) <= 0) return false;
+  if (few_rows_outweigh_keys(c.rows, c.Sq, c.Skv, c.D)) return false;
+  if (c.pv_mode == SAGE_PV_FP16) return true;
+  // (four bytes per channel and 512 rows against one per channel and row: one to three keys do not leave the room)
+  if (sage_prep_v_workspace_bytes(c.B, c.Hkv, c.Skv, c.D, c.pv_mode) > c.k_i8_bytes) return false;
+  return !c.want_lse && few_rows_pay_fp8(c.rows, pairs, c.Skv, c.D);
 }
 
 int sage_sageattn(const void* q, const void* k, const void* v, void* out, float* lse, void* workspace, size_t workspace_bytes,
@@ -527,14 +541,15 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   const bool short_keys = no_keys || (!varlen && Skv <= kSmallPrepassRows && k_elements <= kFewMinElements &&
                                       (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
-  if (few_rows_path(varlen, short_keys, is_causal, attn_mask, pv_mode, lse != nullptr, B, Hkv, Hq / Hkv * (int64_t)Sq, Sq, Skv, D, blkq, blkk, q, k, v,
-                    out, q_sn, k_sn, v_sn)) {
+  const FewCall few = {varlen, is_causal, pv_mode, B, Hkv, Sq, Skv, D, blkq, blkk, Hq / Hkv * (int64_t)Sq, q_sn, k_sn, v_sn,
+                       q, k, v, out, attn_mask, short_keys, lse != nullptr, w.k_i8_bytes};
+  if (few_rows_path(few)) {
     if (int rc2 = check_stride16("q", q_sb, q_sh, q_sn, 2, q)) return rc2;
     if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;
     if (int rc2 = check_stride16("v", v_sb, v_sh, v_sn, 2, v)) return rc2;
     if (int rc2 = check_stride16("out", o_sb, o_sh, o_sn, 2, out)) return rc2;
     // the statistics of K (smoothing) and V (FP8 P.V): per chunk; the kernel combines the chunks itself.  V's lie where the INT8 copy
-    // of K would (a float per channel and 512 rows, against a byte per channel and row), the partial results where the panels would.
+    // of K would (few_rows_path has made sure that they fit), the partial results where the panels would.
     FusedPrepass stats;
     memset(&stats, 0, sizeof(stats));
     ColStatArgs& ks = stats.k_stat;
