@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   v4f o[MT][CV];
   // m_used: the maximum that the probabilities are relative to; FP8 P.V: their binary exponent over m_ref instead
   float m_used[MT], lsum[MT];
-  [[maybe_unused]] float m_ref[MT];
+  [[maybe_unused]] float m_ref[MT], tile_scale[MT];   // tile_scale: of this tile's codes over m_used
   [[maybe_unused]] __shared__ float tile_max[PV ? 2 : 1][4][PV ? 16 * MT : 1];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) {
@@ -291,7 +291,8 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     };
     if constexpr (PV == 1) {
       // The codes of the tiled kernel (block-scaled by the exponent e of the row's maximum in the tile), read back as the values they
-      // stand for: fp16 holds them, and 2^(e - m_used) keeps the sums of a range in fp32's reach however the tiles differ.
+      // stand for, which fp16 holds.  Their common factor 2^(e - m_used) multiplies the tile's fp32 product, not the values: fp16 would
+      // lose those of a tile 16 binades below another one, which large values of V can still bring into the result.
       float sv[MT][8];
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
@@ -306,7 +307,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
         if (tile == 0) m_ref[mt] = mall;
         const float e = fmaxf(__builtin_ceilf(mall - m_ref[mt]), kBlockMinExp);
         if (__builtin_amdgcn_ballot_w64(e > m_used[mt]) != 0) rescale(mt, fmaxf(m_used[mt], e));
-        const float c = __builtin_fmaf(-kCodeStep, e, __builtin_fmaf(kCodeStep, kBlockTop - m_ref[mt], kCodeZero)), f = __builtin_amdgcn_exp2f(e - m_used[mt]);
+        const float c = __builtin_fmaf(-kCodeStep, e, __builtin_fmaf(kCodeStep, kBlockTop - m_ref[mt], kCodeZero));
+        tile_scale[mt] = __builtin_amdgcn_exp2f(e - m_used[mt]);
+        float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; j += 4) {
           float x[4];
@@ -314,13 +317,14 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
           for (int i = 0; i < 4; i++) x[i] = __builtin_fmaf(sv[mt][j + i], kCodeStep, c);
           const int code = pack_probability_codes(x[0], x[1], x[2], x[3]);
           const v2f lo = __builtin_amdgcn_cvt_pk_f32_fp8(code, false), hi = __builtin_amdgcn_cvt_pk_f32_fp8(code, true);
-          const float v[4] = {lo[0] * f, lo[1] * f, hi[0] * f, hi[1] * f};
+          const float v[4] = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
           for (int i = 0; i < 4; i++) {
-            lsum[mt] += v[i];
+            sum += v[i];
             p[mt][j + i] = (_Float16)v[i];
           }
         }
+        lsum[mt] = __builtin_fmaf(sum, tile_scale[mt], lsum[mt]);
       }
       if (reference_only) {   // (nothing but m_ref was wanted)
 #pragma unroll
@@ -365,7 +369,13 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
           }
         }
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) o[mt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[mt], o[mt][i], 0, 0, 0);
+        for (int mt = 0; mt < MT; mt++) {
+          if constexpr (PV == 1) {
+            const v4f part = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[mt], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[mt][i][r] = __builtin_fmaf(part[r], tile_scale[mt], o[mt][i][r]);
+          } else o[mt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, p[mt], o[mt][i], 0, 0, 0);
+        }
         if constexpr (PV == 1) __builtin_amdgcn_sched_barrier(0);   // (one channel's quotients at a time: several do not fit the registers)
       }
     };

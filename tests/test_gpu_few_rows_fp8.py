@@ -107,3 +107,25 @@ def test_a_handful_of_keys_in_very_many_heads(D, heads, Skv):
             assert float((got[part].double() - want.double()).norm() / want.double().norm()) < 5e-3, at
     if Skv == 1:   # the abs-maximum of a channel is the one value: code 448, scale |v| / 448
         assert float((got - v).abs().max()) <= float(v.abs().max()) * 2 ** -10
+
+
+@pytest.mark.parametrize("D,Sq", [(64, 1), (128, 4), (128, 16), (64, 32)])
+@pytest.mark.parametrize("binades", [10.3, 20.3, 36.3, 60.3, 100.3])
+def test_a_flat_tail_far_below_one_key(D, Sq, binades):
+    """One key lies `binades` above all others, and only keys of later tiles have values (those of its own tile lie below the tile's
+    codes): the output is their weight alone, n 2^-binades V.  512 heads are one range each, so the key and its tail meet in one accumulator.
+    A code is 2^t with a linear mantissa (up to 1.086), shifted by 0.3 of its 8 steps per binade (0.974) and rounded (2^(+-1/16)): 0.933
+    to 1.105 of the probability.  Both kernels have the same code; what is left between them is bfloat16 rounding."""
+    B, H, Skv = 64, 8, 128 * 15
+    a = binades * math.log(2.0) / math.sqrt(D)
+    q = torch.ones((B, H, Sq, D), device="cuda", dtype=torch.bfloat16)
+    k = torch.zeros((B, H, Skv, D), device="cuda", dtype=torch.bfloat16)
+    v = torch.full((B, H, Skv, D), 30000.0, device="cuda", dtype=torch.bfloat16)
+    k[:, :, 5], v[:, :, :128] = a, 0.0
+    got = sa.sageattn(q, k, v, pv_mode="fp8", BLKQ=16, smooth_k=False).double()
+    p = torch.softmax(k[0, 0].double().sum(-1) / math.sqrt(D), 0)
+    want = float(p @ v[0, 0, :, 0].double())
+    assert float((got / want - 1).abs().max()) < 0.105 + 2 ** -8
+    if Sq <= 16:
+        tiled = _tiled(q, k, v, 16, smooth_k=False).double()
+        assert float((got / tiled - 1).abs().max()) < 2 ** -7
