@@ -548,8 +548,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     if (int rc2 = check_stride16("k", k_sb, k_sh, k_sn, 2, k)) return rc2;
     if (int rc2 = check_stride16("v", v_sb, v_sh, v_sn, 2, v)) return rc2;
     if (int rc2 = check_stride16("out", o_sb, o_sh, o_sn, 2, out)) return rc2;
-    // the statistics of K (smoothing) and V (FP8 P.V): per chunk; the kernel combines the chunks itself.  V's lie where the INT8 copy
-    // of K would (few_rows_path has made sure that they fit), the partial results where the panels would.
+    // the statistics of K (smoothing) and V (FP8 P.V): per chunk; the kernel combines the chunks, but for very many of K.  V's lie where
+    // the INT8 copy of K would (few_rows_path has made sure that they fit), the partial results where the panels would.
     FusedPrepass stats;
     memset(&stats, 0, sizeof(stats));
     ColStatArgs& ks = stats.k_stat;
@@ -560,11 +560,15 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     if (smooth_k) ks.partial = stat;
     if (pv_mode == SAGE_PV_FP8) stats.v_stat.partial = k_i8;
     hipError_t e = launch_fused_prepass(stats, dtype, D, pv_mode == SAGE_PV_FP8, (hipStream_t)stream);
+    const bool mean_first = ks.partial && pv_mode == SAGE_PV_FP16 && ks.nchunk > kFewChunks;
+    if (e == hipSuccess && mean_first) e = launch_k_mean_finalize(ks, dtype, km, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sage_sageattn(statistics)");
     FewArgs f;
     memset(&f, 0, sizeof(f));
     f.q = (const u16*)q; f.k = (const u16*)k; f.v = (const u16*)v;
-    f.km_partial = (const double*)ks.partial; f.vs_partial = (const float*)stats.v_stat.partial; f.vscale = v_scale; f.nchunk = ks.nchunk;
+    if (mean_first) f.km = (const u16*)km;
+    else f.km_partial = (const double*)ks.partial;
+    f.vs_partial = (const float*)stats.v_stat.partial; f.vscale = v_scale; f.nchunk = ks.nchunk;
     f.out = (u16*)out; f.lse = lse; f.part = (float*)panels;   // (no panels here: their region holds the partial results)
     f.part_bytes = (int64_t)sage_v_panel_bytes(B, Hkv, Skv, D, pv_mode);
     f.B = B; f.Hq = Hq; f.Hkv = Hkv; f.Sq = Sq; f.Skv = Skv;

@@ -13,7 +13,8 @@
 // The order of the channels inside the Q.K^T contraction and of the keys inside the P.V one is free as long as both operands
 // agree: K fragments take the channels as whole 64-byte pieces of a row arrive, V fragments the keys as the 16x16 score tile
 // holds them, so neither the scores nor V go through LDS.
-//   * the statistics (K mean, V scales) arrive per chunk of 512 rows and are combined by every workgroup: a launch less;
+//   * the statistics (K mean, V scales) arrive per chunk of 512 rows and are combined by every workgroup: a launch less (not the K mean
+//     of very long histories, kFewChunks);
 //   * FP8 P.V: V is rounded to the e4m3 values of the panels in registers (a division per element: the vector ALU is what bounds it)
 //     and multiplied in fp16, which holds them; the probabilities are the tiled kernel's block-scaled codes, read back the same way.
 // Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 46.3 us (this
@@ -87,6 +88,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   {
     const int64_t at = (int64_t)bh * a.nchunk * D + tid % D;
     // (head_dim 128: the lower half of the workgroup folds K, the upper one V; at 64 likewise with a quarter each)
+    if (PV == 0 && a.km && tid < D) km_lds[tid] = a.km[(int64_t)bh * D + tid];
     if (a.km_partial && tid < D) {
       double s = 0;
       for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
@@ -122,7 +124,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   if (t0 < t1) load_k(first);
 
   float kmf[LK][8];
-  if (a.km_partial) {
+  if ((PV == 0 && a.km) || a.km_partial) {
 #pragma unroll
     for (int i = 0; i < LK; i++) {
       const v4u raw = *reinterpret_cast<const v4u*>(km_lds + 8 * g + 32 * i);
@@ -499,7 +501,7 @@ __global__ void __launch_bounds__(256) attn_few_merge_kernel(FewArgs a) {
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     const uint2 out = make_uint2(pack2<DT>(acc.x * inv * vs[0], acc.y * inv * vs[1]), pack2<DT>(acc.z * inv * vs[2], acc.w * inv * vs[3]));
     *reinterpret_cast<uint2*>(a.out + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + 4 * lane4) = out;
-    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km || a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
   }
 }
 

@@ -99,11 +99,18 @@ __device__ inline uint32_t fastdiv(uint32_t n, const FastDiv& f) {
 // (4 x 32 heads, 16 rows, 4096 keys) a call takes 86.4 us here and 173.0 with the tiled kernel.
 constexpr int kFewRows = 32;          // query rows per KV head, over all query heads of its group
 constexpr int kFewWorkgroups = 512;   // two per compute unit, what the registers allow at once
+// Chunks of a sequence up to which every workgroup combines the sums of K itself, FP16 P.V.  It walks them eight at a time, as the
+// finalise kernel does, but all 512 workgroups do and read them from the L2.  Whole calls, 1 row, bf16, in the kernel / by a launch: 1 KV
+// head of 64 chunks 25.2 / 25.6 us, 128 34.9 / 34.6, 512 79.2 / 74.5, 8192 1019 / 905; 8 heads of 64 48.2 / 49.3, 128 84.8 / 85.5, 1024
+// 599 / 588; 32 of 64 148 / 149, 128 283 / 283.  (FP8 P.V walks both statistics side by side, two launches one after the other: 1 head
+// of 8192 chunks 1364 / 1535, 8 of 256 253 / 263; always in the kernel.)
+constexpr int kFewChunks = 128;
 struct FewArgs {
   const u16 *q, *k, *v;
-  // per-chunk statistics (ColStatArgs), combined in the kernel: sums of K or null (no smoothing), abs-maxima of V (FP8 P.V) or null
+  // per-chunk statistics (ColStatArgs), combined in the kernel: sums of K or null, abs-maxima of V (FP8 P.V) or null
   const double* km_partial;
   const float* vs_partial;
+  const u16* km;   // [B, Hkv, D]: the mean itself, instead of km_partial, or null (both null: no smoothing)
   float* vscale;   // [B, Hkv, D], written by the main kernel for the merge
   int nchunk;
   u16* out;

@@ -171,3 +171,19 @@ def test_captured_call_replays_like_eager():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), seed
+
+
+@pytest.mark.parametrize("Skv", [128 * 512, 128 * 512 + 1])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+def test_mean_of_very_long_histories(Skv, D, dtype):
+    """The last number of chunks whose sums the kernel combines, and the first whose mean it finds ready: the same numbers as with keys that
+    were smoothed outside (difference rounded to the input type), bit for bit; LSE up to fp32 rounding of q . k_mean (some 2^-24 * 64)."""
+    g = torch.Generator(device="cuda").manual_seed(Skv + D)
+    q, k, v = (torch.randn((2, h, n, D), generator=g, device="cuda").to(dtype) for h, n in ((4, 3), (2, Skv), (2, Skv)))
+    k += 2.0
+    km = sa.k_mean(k)
+    out, lse = sa.sageattn(q, k, v, return_lse=True)
+    want, want_lse = sa.sageattn(q, k - km, v, smooth_k=False, return_lse=True)
+    assert torch.equal(out, want)
+    shift = (q.double() * km.double().repeat_interleave(2, 1)).sum(-1) * D ** -0.5
+    assert float((lse.double() - want_lse.double() - shift).abs().max()) < 1e-4
