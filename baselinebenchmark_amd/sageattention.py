@@ -437,7 +437,7 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
     if BLKQ not in (16, 32, 64, 128) or BLKK not in (16, 32, 64, 128):
         raise NotImplementedError("the attention kernel needs Q and K scale blocks of 16, 32, 64 or 128 rows")
     pv = _pv(pv_mode)
-    out = q.new_empty(q.shape)
+    out = torch.empty(q.shape, device=q.device, dtype=q.dtype)
     _, _, _, _, osb, osh, osn = _layout(out, tensor_layout)
     lse = torch.empty((B, Hq, Sq), device=q.device, dtype=torch.float32) if return_lse else None
     ws_bytes = _workspace_bytes(B, Hq, Hkv, Sq, Skv, D, BLKQ | qflag, BLKK | kflag, pv, 0, 0, 0, int(bool(smooth_k)),
@@ -447,7 +447,7 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
             raise NotImplementedError("attn_mask cannot be combined with is_causal")
         m, kind, ms = _mask_args(attn_mask, B, Hq, Sq, Skv, q.device)
         ws_bytes += lib().sage_sageattn_mask_bytes(B, Hq, Sq, Skv, kind, ms[0], ms[1], ms[2])
-    ws = q.new_empty(max(ws_bytes, 256), dtype=torch.uint8)
+    ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
     if attn_mask is not None:
         check(lib().sage_sageattn_masked(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(ws), ws_bytes,
                                          B, Hq, Hkv, Sq, Skv, D, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
@@ -513,7 +513,7 @@ def sageattn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqle
     lse = torch.empty((Hq, Tq), device=q.device, dtype=torch.float32) if return_lse else None
     ws_bytes = _workspace_bytes(nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D, BLKQ, BLKK, pv, Tq, Tk, 1,
                                 int(bool(smooth_k)), int(bool(return_lse)), 0)
-    ws = q.new_empty(max(ws_bytes, 256), dtype=torch.uint8)
+    ws = torch.empty(max(ws_bytes, 256), device=q.device, dtype=torch.uint8)
     check(lib().sage_sageattn(_ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(ws), ws_bytes,
                               nseq, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k), D,
                               0, q.stride(1), q.stride(0), 0, k.stride(1), k.stride(0), 0, v.stride(1), v.stride(0),

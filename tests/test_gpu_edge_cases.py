@@ -134,3 +134,23 @@ def test_strided_views_of_a_fused_qkv_buffer_through_the_c_abi(pv, causal, lse):
         ref, ref_lse = ref
         assert torch.allclose(lse_t * 0.6931471805599453, ref_lse, rtol=0, atol=1e-6)
     assert torch.equal(out.contiguous().view(torch.int16), ref.view(torch.int16))
+
+
+def test_a_tensor_subclass_gets_a_plain_tensor_back():
+    """The output and the scratch of a call are plain tensors whatever class q is of: nothing of the call runs through the class's
+    __torch_function__ but the look at the inputs, and a parameter that wants gradients leaves no graph behind."""
+    calls = []
+
+    class Logged(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            calls.append(getattr(func, "__name__", str(func)))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    q, k, v = (torch.randn((1, 2, 300, 64), device="cuda", dtype=torch.float16) for _ in range(3))
+    want = sa.sageattn(q, k, v)
+    got = sa.sageattn(q.as_subclass(Logged), k, v)
+    assert type(got) is torch.Tensor and torch.equal(got, want)
+    assert not [c for c in calls if "empty" in c]
+    grad = sa.sageattn(torch.nn.Parameter(q), k, v)
+    assert type(grad) is torch.Tensor and not grad.requires_grad and grad.grad_fn is None
