@@ -505,6 +505,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
                               lse != nullptr && smooth_k && !(!varlen && Skv == 0));
   if (workspace_bytes < w.total) return fail(SAGE_EWORKSPACE, "workspace too small: %zu < %zu", workspace_bytes, w.total);
   if (reinterpret_cast<uintptr_t>(workspace) % 256) return fail(SAGE_EINVAL, "workspace must be 256-byte aligned");
+  // (before anything is launched; a packed batch of no rows at all has no tensors)
+  if (((!varlen || total_q > 0) && (!q || !out)) || (!varlen && Skv > 0 && (!k || !v))) return fail(SAGE_EINVAL, "null tensor pointer");
   uint8_t* ws = (uint8_t*)workspace;
   int8_t* q_i8 = (int8_t*)(ws + w.q_i8);
   int8_t* k_i8 = (int8_t*)(ws + w.k_i8);

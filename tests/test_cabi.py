@@ -123,6 +123,20 @@ def test_attn_alignment_and_slice_limits(sage_lib):
     assert "2 GiB" in sage_lib.sage_last_error().decode()
 
 
+@pytest.mark.parametrize("missing", ["q", "k", "v", "out"])
+@pytest.mark.parametrize("Sq,Skv,packed", [(300, 300, False), (300, 2000, False), (1, 2000, False), (300, 300, True)])
+def test_a_missing_tensor_is_refused_before_any_launch(sage_lib, missing, Sq, Skv, packed):
+    """Short keys (all pre-passes in one launch), long ones, a few query rows, packed: without a GPU a launch would come back as
+    SAGE_ELAUNCH."""
+    t = {name: NULL if name == missing else FAKE for name in ("q", "k", "v", "out")}
+    st = lambda n: (8 * n * 64, n * 64, 64)
+    total = (Sq, Skv) if packed else (0, 0)
+    cu = FAKE if packed else NULL
+    rc = sage_lib.sage_sageattn(t["q"], t["k"], t["v"], t["out"], NULL, FAKE, 1 << 40, 1, 8, 8, Sq, Skv, 64, *st(Sq), *st(Skv), *st(Skv),
+                                *st(Sq), 0, 128, 64, 0.125, 0, 1, 0, cu, cu, *total, NULL)
+    assert rc == _cabi.SAGE_EINVAL and "null tensor pointer" in sage_lib.sage_last_error().decode()
+
+
 def test_empty_problem_is_a_no_op(sage_lib):
     rc = sage_lib.sage_quant_int8(NULL, NULL, NULL, NULL, 0, 4, 128, 128, 0, 0, 128, 0, 0, 128, 0, 0, 128, 1.0, 0,
                                   NULL, NULL, 0, NULL)
