@@ -780,18 +780,31 @@ __global__ void __launch_bounds__(256, ALL ? 3 : 4) fused_prepass_kernel(FusedPr
 // ---------------------------------------------------------------------------------------------
 // Host-side launchers (called from the C ABI in sage_api.hip).
 // ---------------------------------------------------------------------------------------------
-// Where the heads of a row lie next to each other (packed and [B, L, H, D] tensors), workgroups of the same rows are neighbours, so
-// that whole rows are on their way at a time; with the rows of one head first, a workgroup and its neighbours read 128 or 256 bytes out
-// of every few kilobytes.  96 packed prompts of 16..1024 rows, 8 KV heads of 128, bf16: K quantiser 51.2 -> 34.8 us (154 MB: 3.0 ->
-// 4.4 TB/s), FP16 V panels 49.3 -> 38.6 (205 MB: 4.2 -> 5.3 TB/s); 2 x 16 heads of 4096 rows, FP8: 27.3 -> 25.3 for both.  (The y axis of
-// a grid is limited to 65535.)
+// Where the heads of a row lie next to each other (packed and [B, L, H, D] tensors) the head can be the fastest grid index, so that whole
+// rows are on their way at a time; with the rows of one head first, a workgroup and its neighbours read 128 or 256 bytes out of every
+// few kilobytes.  (The y axis of a grid is limited to 65535.)
+// The quantiser always gains: bf16, 100 M elements, heads / rows first, 8 heads of 64 81.4 / 81.3 us, 24 80.9 / 89.8, 64 80.9 / 101.8, 8 of
+// 128 64.2 / 62.8, 24 65.1 / 69.7, 32 64.1 / 83.1.
 static bool heads_first(int64_t head_stride, int64_t row_stride, int64_t chunks) { return head_stride < row_stride && chunks <= 65535; }
+// Statistics and V panels, which read 128 rows and more per workgroup, gain where rows are a multiple of 4 KiB apart (a head's rows alone
+// then crowd into a few memory channels) and in packed batches of short sequences (most workgroups of a grid sized for the longest
+// one find nothing to do); elsewhere rows first is the faster one.  FP16 panels / FP8 panels with their statistic / K mean, 100 M elements in
+// us, heads first and rows first: 16 heads of 128 (4 KiB) 76 / 93 / 40 and 87 / 108 / 48; 32 of 64 (4 KiB) 80 / 99 / 41 and 87 / 113 / 50;
+// 24 of 128 (6 KiB) 77 / 93 / 39 and 71 / 91 / 39; 40 of 64 (5 KiB) 82 / 103 / 42 and 72 / 95 / 37.  Whole packed calls, a query row per
+// sequence, panels rows first, statistics rows first: 96 of 16..1024 rows, 24 heads of 128 447 -> 470, 453; 64 of 512..4096, 24 heads of
+// 64, FP8 649 -> 668, 660; 8 of 4096..8192 238 -> 236, 231; 16 of 512..32768 1248 -> 1225, 1192.
+static bool heads_first_streaming(int64_t head_stride, int64_t row_stride, int64_t chunks, bool packed, int max_rows) {
+  return heads_first(head_stride, row_stride, chunks) && (row_stride * 2 % 4096 == 0 || (packed && max_rows <= 4096));
+}
+static bool heads_first(const ColStatArgs& a, int64_t chunks) { return heads_first_streaming(a.x_sh, a.x_sn, chunks, a.cu_seqlens, a.L); }
+static bool heads_first(const PrepVArgs& a, int64_t chunks) { return heads_first_streaming(a.v_sh, a.v_sn, chunks, a.cu_seqlens, a.L); }
+static bool heads_first(const QuantArgs& a, int64_t chunks) { return heads_first(a.x_sh, a.x_sn, chunks); }
 
 hipError_t launch_quant_int8(const QuantArgs& args, int dtype, int max_rows, hipStream_t st) {
   QuantArgs a = args;
   const int rows = quant_rows(a.D, a.blk);
   const uint32_t chunks = (max_rows + rows - 1) / rows;
-  a.heads_first = heads_first(a.x_sh, a.x_sn, chunks);
+  a.heads_first = heads_first(a, chunks);
   const dim3 grid = a.heads_first ? dim3(a.H, chunks, a.B) : dim3(chunks, a.H, a.B), block(256);
 #define SAGE_QUANT(DT, DD, NP) (a.km_partial ? quant_int8_kernel<DT, DD, NP, true><<<grid, block, 0, st>>>(a) : quant_int8_kernel<DT, DD, NP><<<grid, block, 0, st>>>(a))
 #define SAGE_QUANT_D(DT) \
@@ -868,9 +881,8 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
   const int blk = fused_block(f);
   fused_extents(f, blk, e);
   FusedTable t;
-  const bool inner_heads[kJobs] = {false, heads_first(f.k_stat.x_sh, f.k_stat.x_sn, 0), heads_first(f.v_stat.x_sh, f.v_stat.x_sn, 0),
-                                   heads_first(f.k_quant.x_sh, f.k_quant.x_sn, 0), heads_first(f.q_quant.x_sh, f.q_quant.x_sn, 0),
-                                   heads_first(f.v_panels.v_sh, f.v_panels.v_sn, 0), false};
+  const bool inner_heads[kJobs] = {false, heads_first(f.k_stat, 0), heads_first(f.v_stat, 0), heads_first(f.k_quant, 0),
+                                   heads_first(f.q_quant, 0), heads_first(f.v_panels, 0), false};
   t.heads_first = 0;
   for (int j = 0; j < kJobs; j++) {
     if (e[j][1] > 65535 || e[j][2] > 65535) return hipErrorInvalidConfiguration;   // (what the jobs' own grids take)
@@ -913,7 +925,7 @@ int colstat_chunks(int L) { return (L + kChunkRows - 1) / kChunkRows; }
 template <int MODE>
 static hipError_t launch_colstat(const ColStatArgs& args, int dtype, hipStream_t st) {
   ColStatArgs a = args;
-  a.heads_first = heads_first(a.x_sh, a.x_sn, a.nchunk);
+  a.heads_first = heads_first(a, a.nchunk);
   const dim3 grid = a.heads_first ? dim3(a.H, a.nchunk, a.B) : dim3(a.nchunk, a.H, a.B), block(256);
   if (dtype == 0 && a.D == 64) colstat_partial_kernel<0, 64, MODE><<<grid, block, 0, st>>>(a);
   else if (dtype == 0 && a.D == 128) colstat_partial_kernel<0, 128, MODE><<<grid, block, 0, st>>>(a);
@@ -967,7 +979,7 @@ hipError_t launch_prepass_small(const QuantArgs& qa, const PrepVArgs& va, int dt
 hipError_t launch_prep_v(const PrepVArgs& args, int dtype, int pv, int max_panels, hipStream_t st) {
   PrepVArgs a = args;
   if (max_panels == 0 || a.B == 0 || a.H == 0) return hipSuccess;
-  a.heads_first = heads_first(a.v_sh, a.v_sn, max_panels);
+  a.heads_first = heads_first(a, max_panels);
   const dim3 grid = a.heads_first ? dim3(a.H, max_panels, a.B) : dim3(max_panels, a.H, a.B), block(256);
 #define SAGE_PREPV(DT, DD, PVV) (PVV && a.vs_partial ? prep_v_kernel<DT, DD, PVV, PVV == 1><<<grid, block, 0, st>>>(a) : prep_v_kernel<DT, DD, PVV><<<grid, block, 0, st>>>(a))
   if (dtype == 0) {

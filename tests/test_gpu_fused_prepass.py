@@ -100,6 +100,20 @@ def test_heads_in_a_row_equal_heads_apart(H, Skv, D):
             assert torch.equal(got, sa.sageattn(*t, pv_mode=pv, BLKQ=blkq, BLKK=blkk).transpose(1, 2)), pv
 
 
+@pytest.mark.parametrize("H,D", [(16, 128), (32, 64), (32, 128), (24, 64)])
+@pytest.mark.parametrize("Skv", [129, 1100, 4700])
+def test_rows_of_whole_pages_equal_heads_apart(H, D, Skv):
+    """Rows a multiple of 4 KiB apart, which the statistics and the V panels walk heads first, and 3 KiB, which they do not."""
+    q, k, v = _inputs(1, H, H, 40, Skv, D, torch.float16, "NHD", H + Skv)
+    t = [x.transpose(1, 2).contiguous() for x in (q, k, v)]
+    assert torch.equal(sa.k_mean(k, "NHD").flatten(1), sa.k_mean(t[1], "HND").flatten(1))
+    for pv in ("fp16", "fp8"):
+        for a, b in zip(sa.sageattention.prepare_v(v, "NHD", pv), sa.sageattention.prepare_v(t[2], "HND", pv)):
+            assert torch.equal(a, b) if a is not None else b is None
+        got = sa.sageattn(q, k, v, tensor_layout="NHD", pv_mode=pv)
+        assert torch.equal(got, sa.sageattn(*t, pv_mode=pv).transpose(1, 2)), pv
+
+
 @pytest.mark.parametrize("rows", [65535 * 64, 65535 * 64 + 1])
 def test_more_rows_than_the_second_grid_axis_holds(rows):
     """16-row blocks at head_dim 64: 64 rows per workgroup, 65535 workgroups at most beside the heads."""
