@@ -340,15 +340,18 @@ int sage_attn_fwd_masked(const int8_t* q, const int8_t* k, const void* v_panels,
 
 // ---- one-call pipeline --------------------------------------------------------------------
 namespace {
-// Up to this many keys per sequence and elements of K per call the pre-passes run as one launch whose workgroups read
-// their sequence's statistics themselves (sage_quant.hip: prepass_small_kernel) instead of two launches, statistics first.
+// Up to this many keys per sequence the pre-passes run as one launch whose workgroups read their sequence's statistics themselves
+// (sage_quant.hip: prepass_small_kernel) instead of two launches, statistics first ...
 constexpr int kSmallPrepassRows = 1024;
-constexpr int64_t kSmallPrepassElements = (int64_t)3 << 20;
-// ... and the element reads it makes: every K workgroup and every V panel re-reads its whole sequence.  Whole calls in bf16,
-// one launch / two, us: 32 heads of 512 rows, head_dim 128 (2.1 M elements), FP16 / FP8 P.V 29.7 / 30.9 and 27.5 / 30.9; 2 x 24 of 600
-// (3.7 M) 39.4 / 36.1 and 37.7 / 35.0; 2 x 16 of 1000 (4.1 M) 46.6 / 46.0 and 46.5 / 42.1; at head_dim 64 (2.1 M) 32.0 / 34.2
-// and 30.0 / 31.7; 8 heads of 1000, head_dim 128, K blocks of 16 (73 M reads) 37.6 / 37.7 and 33.1 / 35.3.
-constexpr int64_t kSmallPrepassReads = (int64_t)96 << 20;
+// ... and up to this many element reads, each workgroup of K and each V panel counted with its whole sequence.  Whole calls in bf16, one
+// launch / two, FP16 and FP8 P.V, us: 12 M reads (8 x 32 heads of 128 rows, head_dim 128) 20.5 / 25.3, 20.1 / 27.3; 16 M (32 x 32 of 64)
+// 52.4 / 62.4, 49.2 / 66.9; 24 M (16 x 32 of 128) 36.6 / 41.8, 34.1 / 46.1; (8 of 1024) 34.5 / 34.7, 30.2 / 32.3; (8 x 32 of 257, 64) 35.3 /
+// 38.2, 33.8 / 37.0; 28 M (4 x 24 of 300) 32.4 / 32.9, 28.9 / 32.8; 30 M (40 of 512) 30.7 / 31.8, 28.6 / 31.6; 32 M (4 x 32 of 512, 64)
+// 31.4 / 29.5, 27.9 / 29.5; 36 M (2 x 24 of 512) 32.5 / 33.1, 31.9 / 33.0; 40 M (24 of 768) 36.2 / 35.4, 32.4 / 33.8; 48 M (16 of 1024)
+// 41.4 / 38.2, 36.5 / 34.5; 64 M (8 x 32 of 257) 61.9 / 56.5, 56.2 / 56.2; 96 M (4 x 32 of 512) 52.4 / 43.6, 54.4 / 44.4.
+constexpr int64_t kSmallPrepassReads = (int64_t)30 << 20;
+// ... in this many heads: 12288 of a key, head_dim 64, 374 / 363; 16384 of 8 525 / 496; 8192 of 16 251 / 251, FP8 235 / 242.
+constexpr int64_t kSmallPrepassHeads = 8192;
 // A few query rows (sage_attn_few.hip) take four launches, 28-29 us end to end whatever the keys in this range; behind the
 // one-launch pre-pass the tiled kernel takes two, and longer with the keys of a head and with the re-reads.  bf16, K blocks of 64,
 // tiled / few rows: 1 x 8 heads of 768 keys, head_dim 128, 26.3 / 28.7 us, of 1024 keys 30.3 / 28.3; by re-reads, 4 x 8 heads
@@ -538,8 +541,9 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   // the whole sequence itself); otherwise two launches, the statistics in two stages.
   const int64_t k_elements = (int64_t)B * Hkv * Skv * D;
   const int64_t rereads = (Skv + blk_rows(blkk) - 1) / blk_rows(blkk) + (Skv + kPanelRows - 1) / kPanelRows;
-  const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && k_elements <= kSmallPrepassElements &&
-                             k_elements * rereads <= kSmallPrepassReads;
+  const int64_t prepass_workgroups = (Skv + quant_rows(D, blk_rows(blkk)) - 1) / quant_rows(D, blk_rows(blkk)) + (Skv + kPanelRows - 1) / kPanelRows;   // of a head
+  const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && k_elements * prepass_workgroups <= kSmallPrepassReads &&
+                             (int64_t)B * Hkv <= kSmallPrepassHeads;
   const bool short_keys = no_keys || (!varlen && Skv <= kSmallPrepassRows && k_elements <= kFewMinElements &&
                                       (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
