@@ -352,13 +352,29 @@ constexpr int kSmallPrepassRows = 1024;
 constexpr int64_t kSmallPrepassReads = (int64_t)30 << 20;
 // ... in this many heads: 12288 of a key, head_dim 64, 374 / 363; 16384 of 8 525 / 496; 8192 of 16 251 / 251, FP8 235 / 242.
 constexpr int64_t kSmallPrepassHeads = 8192;
-// A few query rows (sage_attn_few.hip) take four launches, 28-29 us end to end whatever the keys in this range; behind the
-// one-launch pre-pass the tiled kernel takes two, and longer with the keys of a head and with the re-reads.  bf16, K blocks of 64,
-// tiled / few rows: 1 x 8 heads of 768 keys, head_dim 128, 26.3 / 28.7 us, of 1024 keys 30.3 / 28.3; by re-reads, 4 x 8 heads
-// of 512 keys, head_dim 128 (25 M) 25.9 / 29.1; 16 x 8 of 512, head_dim 64 (50 M) 33.0 / 28.6; 4 x 8 of 768 (57 M) 34.7 / 28.4;
-// 8 x 8 of 1024, head_dim 64 (101 M) 47.7 / 28.3.
-constexpr int64_t kFewMinHeadElements = 896 * 128, kFewMinReads = (int64_t)32 << 20, kFewMinElements = (int64_t)4 << 20;
-// ... and with few keys, in great number: the FP32 results of a KV head's rows are written and read again, the tiled kernel with one
+// A few query rows (sage_attn_few.hip) take at most three launches, some 2.5 us of host time more than the two of the tiled kernel behind
+// the one-launch pre-pass, which is as fast as that as long as its workgroups (a 256-row tile per query head, two to a compute unit at
+// head_dim 64) are one round of the chip, the keys of a head are few and so are the re-reads of the pre-pass.  Past one round the rows
+// count: the few-rows kernel writes and reads FP32 results of every row.  Whole calls, K blocks of 64, bf16, tiled / few rows in us.
+// FP16 P.V, up to 16 rows: 8 heads of 768 keys, head_dim 64, 19.9 / 20.2, of 900 23.3 / 19.9; head_dim 128, of 257 18.6 / 19.5, of 512 21.0 /
+// 19.9; 64 of 256 (12 M reads) 18.7 / 19.5, 128 of 192 (15 M) 20.9 / 19.5; 320 of 64 26.8 / 19.1, head_dim 64 19.4 / 19.8, 640 of 64 27.5 /
+// 18.9; 512 heads on 128 KV heads of 128, head_dim 64, 17.4 / 19.7, 1024 on 256 28.6 / 19.4.  20, 24 and 32 rows, head_dim 64: 256 heads of 256
+// keys (16 M) 21.3 / 21.0, 21.1 / 22.2, 21.4 / 25.9; 1024 of 64 38.3 / 36.4, 38.0 / 39.3, 38.4 / 45.0.
+// FP8 P.V, 1 and 16 rows: head_dim 128, 8 heads of 768 keys 23.2 / 25.1 and 23.2 / 27.0, of 900 27.7 / 25.4 and 27.5 / 26.7; 32 of 512 (24 M)
+// 25.1 / 26.7 and 25.2 / 27.4; 16 of 768 (27 M) 28.8 / 26.7 and 28.8 / 27.9; 512 of 64 26.4 / 24.6 and 26.9 / 30.9; 1024 of 16 45.9 / 36.6 and
+// 46.7 / 48.0; 2048 of 16 86.2 / 55.7 and 86.7 / 80.5.
+bool tiled_beats_few_rows(int pv_mode, int D, int64_t rows, int Sq, int64_t query_heads, int Skv, int64_t prepass_reads) {
+  const bool apart = rows == Sq, many = apart && rows > 20;   // apart: every query head has a KV head of its own
+  const int64_t mega = 1 << 20;
+  if (Skv > kSmallPrepassRows) return false;
+  if (pv_mode == SAGE_PV_FP16) {
+    if ((int64_t)Skv * D > 48 * 1024 || prepass_reads > (many ? 20 : 12) * mega) return false;
+    return many || query_heads <= (D == 64 ? 512 : 256);
+  }
+  if ((int64_t)Skv * D > 896 * 128 || prepass_reads > 24 * mega) return false;
+  return query_heads <= (apart && rows > 8 ? 1024 : D == 64 ? 512 : 256);
+}
+// Few keys in great number: the FP32 results of a KV head's rows are written and read again, the tiled kernel with one
 // query head per KV head launches no more workgroups, and at head_dim 128 it wins where those bytes outweigh K and V.  16384 heads,
 // bf16, tiled / few rows: 24 rows, 16 keys 729 / 725 us; 28 rows, 16 keys 733 / 782, 48 keys 814 / 803; 32 rows, 16 keys 743 / 846,
 // 64 keys 846 / 878, 80 keys 925 / 897.  (At head_dim 64, 32 rows, 32 keys 513 / 461; two query heads per KV head: few rows always.)
@@ -540,12 +556,11 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   // Short sequences: all K and V pre-passes in one launch (every workgroup computes the statistic its tile needs over
   // the whole sequence itself); otherwise two launches, the statistics in two stages.
   const int64_t k_elements = (int64_t)B * Hkv * Skv * D;
-  const int64_t rereads = (Skv + blk_rows(blkk) - 1) / blk_rows(blkk) + (Skv + kPanelRows - 1) / kPanelRows;
-  const int64_t prepass_workgroups = (Skv + quant_rows(D, blk_rows(blkk)) - 1) / quant_rows(D, blk_rows(blkk)) + (Skv + kPanelRows - 1) / kPanelRows;   // of a head
-  const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && k_elements * prepass_workgroups <= kSmallPrepassReads &&
+  const int k_rows = quant_rows(D, blk_rows(blkk));
+  const int64_t prepass_reads = k_elements * ((Skv + k_rows - 1) / k_rows + (Skv + kPanelRows - 1) / kPanelRows);
+  const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && prepass_reads <= kSmallPrepassReads &&
                              (int64_t)B * Hkv <= kSmallPrepassHeads;
-  const bool short_keys = no_keys || (!varlen && Skv <= kSmallPrepassRows && k_elements <= kFewMinElements &&
-                                      (int64_t)Skv * D <= kFewMinHeadElements && k_elements * rereads <= kFewMinReads);
+  const bool short_keys = no_keys || tiled_beats_few_rows(pv_mode, D, Hq / Hkv * (int64_t)Sq, Sq, (int64_t)B * Hq, Skv, prepass_reads);
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
   const FewCall few = {varlen, is_causal, pv_mode, B, Hkv, Sq, Skv, D, blkq, blkk, Hq / Hkv * (int64_t)Sq, q_sn, k_sn, v_sn,
                        q, k, v, out, attn_mask, short_keys, lse != nullptr, w.k_i8_bytes};

@@ -187,3 +187,20 @@ def test_mean_of_very_long_histories(Skv, D, dtype):
     assert torch.equal(out, want)
     shift = (q.double() * km.double().repeat_interleave(2, 1)).sum(-1) * D ** -0.5
     assert float((lse.double() - want_lse.double() - shift).abs().max()) < 1e-4
+
+
+# one round of the tiled kernel's workgroups and the first head past it, more than 20 rows, the limits of keys and re-reads
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D", [(64, 8, 8, 2, 5, 64), (57, 9, 9, 2, 5, 64), (32, 8, 8, 3, 17, 128), (29, 9, 9, 3, 17, 128),
+                                               (33, 8, 8, 20, 17, 128), (33, 8, 8, 21, 17, 128), (65, 8, 4, 8, 33, 64), (130, 8, 8, 9, 7, 64),
+                                               (128, 8, 8, 9, 7, 128), (1, 2, 2, 1, 384, 128), (1, 2, 2, 1, 385, 128), (1, 2, 2, 1, 896, 128),
+                                               (1, 2, 2, 1, 897, 128), (4, 8, 8, 1, 512, 128), (4, 8, 8, 1, 513, 128)])
+def test_both_sides_of_the_rule_for_short_keys(B, Hq, Hkv, Sq, Skv, D, pv):
+    g = torch.Generator().manual_seed(Skv + D + Sq)
+    q, k, v = (torch.randn((B, h, n, D), generator=g) for h, n in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    q, k, v = q.half().cuda(), (k + 2.0 * torch.randn((D,), generator=g)).half().cuda(), v.half().cuda()
+    got = sa.sageattn(q, k, v, pv_mode=pv).cpu().double()
+    want, _ = _reference(q, k, v, "HND", 128, 64, True)
+    err = float((got - want).norm() / want.norm())
+    # P rounded to 11 bits; e4m3 V (3 mantissa bits: 2^-4 / sqrt(3) of a value) and codes of P (0.933 to 1.105, as much once normalised)
+    assert err < (2.0 ** -10 if pv == "fp16" else 0.055)
