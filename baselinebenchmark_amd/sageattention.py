@@ -37,7 +37,7 @@ def backend_name() -> str:
 # helpers
 # ------------------------------------------------------------------------------------------------
 # (Small calls are bound by the host: on 8 heads of 1024 rows the GPU needs 25 us, and the checks, allocations and the call through
-# ctypes took 22.  Plain integers as pointers, the raw stream handle and one look at shape and strides each keep them near half of that.)
+# ctypes took 22.  Plain integers as pointers, the raw stream handle and one look at shape and strides each bring that down to 16.)
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
@@ -437,7 +437,8 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
     if BLKQ not in (16, 32, 64, 128) or BLKK not in (16, 32, 64, 128):
         raise NotImplementedError("the attention kernel needs Q and K scale blocks of 16, 32, 64 or 128 rows")
     pv = _pv(pv_mode)
-    out = torch.empty(q.shape, device=q.device, dtype=q.dtype)
+    # (a plain tensor whatever class q is of; new_empty, which keeps the class, saves a microsecond)
+    out = q.new_empty(q.shape) if type(q) is torch.Tensor else torch.empty(q.shape, device=q.device, dtype=q.dtype)
     _, _, _, _, osb, osh, osn = _layout(out, tensor_layout)
     lse = torch.empty((B, Hq, Sq), device=q.device, dtype=torch.float32) if return_lse else None
     ws_bytes = _workspace_bytes(B, Hq, Hkv, Sq, Skv, D, BLKQ | qflag, BLKK | kflag, pv, 0, 0, 0, int(bool(smooth_k)),
