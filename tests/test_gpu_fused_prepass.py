@@ -135,3 +135,78 @@ def test_limits_of_the_one_launch_prepass(B, H, Skv, D, blkk, pv):
     for smooth in (True, False):
         got = sa.sageattn(q, k, v, pv_mode=pv, smooth_k=smooth, BLKK=blkk)
         assert torch.equal(got, _steps(q, k, v, "HND", pv, 128, blkk, smooth))
+
+
+def _cu(lens):
+    return torch.tensor([0, *lens], dtype=torch.int64).cumsum(0).to(torch.int32).cuda()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("nseq,longest", [(1, 20000), (63, 900), (65, 5000), (1023, 70), (1024, 70), (1025, 70), (5000, 40)])
+def test_plan_of_a_one_call_batch_equals_the_plan_on_its_own(nseq, longest, causal):
+    """The plan that rides along with the statistics has 256 lanes and keeps 1024 lengths in LDS, the one of varlen_plan 1024 and 4096: the
+    same block offsets and tile list, read back from the end of the call's workspace (empty sequences, other key than query lengths)."""
+    g = torch.Generator().manual_seed(nseq)
+    lq, lk = (torch.randint(0, longest + 1, (nseq,), generator=g).tolist() for _ in range(2))
+    lq[0], lk[-1] = longest, longest
+    cuq, cuk, Tq, Tk = _cu(lq), _cu(lk), sum(lq), sum(lk)
+    q, k, v = (torch.randn((n, 2, 64), device="cuda", dtype=torch.float16) for n in (Tq, Tk, Tk))
+    lib = _cabi.lib()
+    need = lib.sage_sageattn_workspace_bytes_for(nseq, 2, 2, max(lq), max(lk), 64, 64, 16, _cabi.PV_FP16, Tq, Tk, 1, 1, 0, 0)
+    out, ws = torch.empty_like(q), torch.empty(need, dtype=torch.uint8, device="cuda")
+    row = (0, 64, 128)
+    rc = lib.sage_sageattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), None, ws.data_ptr(), need, nseq, 2, 2, max(lq), max(lk),
+                           64, *row, *row, *row, *row, 0, 64, 16, 0.125, int(causal), 1, _cabi.PV_FP16, cuq.data_ptr(), cuk.data_ptr(), Tq, Tk,
+                           torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    want, offs = sa.varlen_plan(cuq, cuk, Tq, 64, 16, is_causal=causal)
+    ints = lib.sage_varlen_plan_ints(nseq, Tq)
+    at = need - (4 * ints + 255) // 256 * 256   # the last region of a call without LSE
+    got = ws[at:at + 4 * ints].view(torch.int32)
+    used = offs[4] + int(want[offs[3]])
+    assert torch.equal(got[:used], want[:used])
+
+
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("smooth", [True, False])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+def test_packed_call_of_up_to_eight_chunks(D, dtype, pv, smooth):
+    """No sequence past 4096 keys: the second launch combines the statistics itself, of nothing, a part of a chunk, one chunk and a row,
+    and eight of them side by side; other key than query lengths."""
+    lq, lk = [40, 0, 300, 33, 257, 64, 90], [0, 130, 1, 513, 4096, 512, 3500]
+    cuq, cuk = _cu(lq), _cu(lk)
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn((n, h, D), generator=g).to(dtype).cuda() for n, h in ((sum(lq), 4), (sum(lk), 2), (sum(lk), 2)))
+    k += 1.5
+    got = sa.sageattn_varlen(q, k, v, cuq, cuk, max(lq), max(lk), pv_mode=pv, smooth_k=smooth)
+    for i, (n, m) in enumerate(zip(lq, lk)):
+        rows = slice(int(cuq[i]), int(cuq[i]) + n)
+        keys = slice(int(cuk[i]), int(cuk[i]) + m)
+        if n and m:
+            one = sa.sageattn(q[None, rows], k[None, keys], v[None, keys], tensor_layout="NHD", pv_mode=pv, smooth_k=smooth)
+            assert torch.equal(got[rows], one[0]), (n, m)
+        else:
+            assert not bool(got[rows].any())
+
+
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+def test_packed_call_of_more_sequences_than_the_plan_keeps(pv):
+    """1300 sequences, some of them empty, keys of other lengths: each kind of sequence equals the batch of its own, bit for bit."""
+    g = torch.Generator().manual_seed(11)
+    kinds = [(0, 5), (33, 0), (40, 7), (65, 130), (130, 33), (34, 600)]
+    pick = torch.randint(0, len(kinds), (1300,), generator=g).tolist()
+    lq, lk = [kinds[i][0] for i in pick], [kinds[i][1] for i in pick]
+    cuq, cuk = _cu(lq), _cu(lk)
+    q, k, v = (torch.randn((n, 2, 64), generator=g).half().cuda() for n in (sum(lq), sum(lk), sum(lk)))
+    got = sa.sageattn_varlen(q, k, v, cuq, cuk, max(lq), max(lk), pv_mode=pv)
+    for kind, (n, m) in enumerate(kinds):
+        members = [i for i, p in enumerate(pick) if p == kind]
+        if not n:
+            continue
+        rows = torch.stack([got[int(cuq[i]):int(cuq[i]) + n] for i in members])
+        if not m:
+            assert not bool(rows.any())
+            continue
+        part = lambda x, cu, length: torch.stack([x[int(cu[i]):int(cu[i]) + length] for i in members])  # noqa: E731
+        one = sa.sageattn(part(q, cuq, n), part(k, cuk, m), part(v, cuk, m), tensor_layout="NHD", pv_mode=pv)
+        assert torch.equal(rows, one), (n, m)
