@@ -54,8 +54,10 @@ hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, 
 #define SAGE_ATTN(DD, PVV, BNN, MS) (a.blkk >= 128 ? SAGE_ATTN_W(DD, PVV, BNN, MS, 4) : a.blkk == 64 ? SAGE_ATTN_W(DD, PVV, BNN, MS, 2) : SAGE_ATTN_W(DD, PVV, BNN, MS, 1))
   if (D == 128) return pv ? (msum ? SAGE_ATTN(128, 1, 128, true) : SAGE_ATTN(128, 1, 128, false)) : SAGE_ATTN(128, 0, 128, false);
   if (pv || !msum) return pv ? (msum ? SAGE_ATTN(64, 1, 128, true) : SAGE_ATTN(64, 1, 128, false)) : SAGE_ATTN(64, 0, 128, false);
-  // (FP16 P.V without LSE, not causal: the variant for 64-key scales also where they cover 128 keys, the same numbers: 16 heads of 6000
-  // rows 165.1 us instead of 169.2; causal it is the slower one)
+  // (FP16 P.V without LSE, not causal: the variant for 64-key scales also where they cover 128 keys, the same numbers.  The one for 128-key
+  // scales comes out of the compiler with a phase of the loop in two copies, 3133 instructions against 2889: 16 heads of 6000 rows 161.4 us
+  // instead of 166.1, 48 of 2222 74.1 / 75.8, 48 of 4096 182.5 / 185.1, 32 of 8192 460 / 468, 2 of 20000 236 / 246.  Causal, where neither
+  // has that, the 128-key one is the smaller and faster.)
   if (!causal) return a.blkk >= 64 ? launch_one<64, 8, 128, 0, false, true, 0, 1, false, 2>(a, grid, st) : launch_one<64, 8, 128, 0, false, true, 0, 1, false, 1>(a, grid, st);
   return a.blkk >= 128 ? launch_one<64, 8, 128, 0, true, true, 0, 1, false, 4>(a, grid, st) : a.blkk == 64 ? launch_one<64, 8, 128, 0, true, true, 0, 1, false, 2>(a, grid, st) : launch_one<64, 8, 128, 0, true, true, 0, 1, false, 1>(a, grid, st);
 #undef SAGE_ATTN_W

@@ -1085,7 +1085,8 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // their tile count at every use: as a flag that is computed first and carried through the period, the condition cost the
     // FP16 P.V ones of head_dim 64 1 % (8 heads of 1024 rows: 28.8 instead of 28.4 us; 2 of 20000, 128-key scales: 268 / 260).  Causal
     // ones with 128-key scales are the exception (2 heads of 20000 rows on ready INT8 operands: 228 us carried, 232 at every use;
-    // head_dim 64, Q quantised in the prologue, no LSE, 2 x 8 heads of 16384: 503.4 / 507.5).
+    // head_dim 64, Q quantised in the prologue, no LSE: 8 heads of 1024 rows 25.5 / 25.8, 48 of 2222 59.7 / 59.9, 48 of 4096 134.0 / 135.4, 32
+    // of 8192 283 / 289, 2 of 20000 253 / 259).  The two forms differ by a handful of instructions: it is their order that differs.
     constexpr bool CARRIED = LISTED || (PV == 0 && CAUSAL && KW == 4 && (!QF || (D == 64 && MSUM)));
     [[maybe_unused]] bool on = false, on_prev = false;
     auto enter = [&](int j) { if constexpr (CARRIED) { on_prev = on; on = LISTED ? j < ntiles && sees(j) : j < wave_ntiles; } };

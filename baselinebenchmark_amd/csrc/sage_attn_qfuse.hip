@@ -16,7 +16,8 @@ hipError_t launch_attn_qfused(const AttnArgs& a, int D, int pv, bool causal, int
   }
   if (D == 128) return pv ? (msum ? SAGE_ATTN_Q(128, 1, 128, true, false) : SAGE_ATTN_Q(128, 1, 128, false, false)) : SAGE_ATTN_Q(128, 0, 128, false, false);
   if (pv || !msum) return pv ? (msum ? SAGE_ATTN_Q(64, 1, 128, true, false) : SAGE_ATTN_Q(64, 1, 128, false, false)) : SAGE_ATTN_Q(64, 0, 128, false, false);
-  // (as in launch_attn: 16 heads of 6000 rows 170.0 us instead of 175.3, 2 x 8 of 16384 951 instead of 971)
+  // (as in launch_attn: 8 heads of 1024 rows 25.3 us instead of 25.7, 48 of 2222 88.9 / 91.6, 48 of 4096 208 / 211, 32 of 8192 490 / 499, 16 of
+  // 16384 924 / 955)
   if (!causal) return a.blkk >= 64 ? launch_one<64, 8, 128, 0, false, true, 0, 1, true, 2>(a, grid, st) : launch_one<64, 8, 128, 0, false, true, 0, 1, true, 1>(a, grid, st);
   return a.blkk >= 128 ? launch_one<64, 8, 128, 0, true, true, 0, 1, true, 4>(a, grid, st) : a.blkk == 64 ? launch_one<64, 8, 128, 0, true, true, 0, 1, true, 2>(a, grid, st) : launch_one<64, 8, 128, 0, true, true, 0, 1, true, 1>(a, grid, st);
 #undef SAGE_ATTN_QW

@@ -858,8 +858,12 @@ static hipError_t launch_job(const FusedPrepass& f, int job, int dtype, int pv, 
 }
 
 // Up to how many workgroups the jobs of a launch share it: past that each fills the chip by itself, and its own kernel, with fewer
-// registers and less LDS than the shared one, is the faster.  The plan, one workgroup of 8 us, always rides along.  Whole calls in
-// bf16, 40 query rows, us, before these launches / each job by itself / early, late or both jobs sharing: 8 heads of 4096 keys, FP8 P.V
+// registers and less LDS than the shared one, is the faster.  With a plan the statistics share its launch whatever their size: its one
+// workgroup starts first and works beside theirs, and a launch of its own costs more than they gain.  Packed, head_dim 128, 8 KV heads, a
+// query row per sequence, shared / apart in us: 16 sequences of 512..32768 keys (15873 workgroups) FP8 841 / 852, FP16 943 / 950; 64 of
+// 512..4096 FP8 380 / 385; 200 of 100..1500 442 / 452; whole causal calls, 32/8 heads, of 256 sequences 1497 / 1493 and FP8 1308 / 1316, of
+// 4096 4551 / 4571 and FP8 4406 / 4364 (the plan has 256 lanes here and 1024 apart), of 32000 34.1 / 34.3 ms.
+// Without one, whole calls in bf16, 40 query rows, us, before these launches / each job by itself / early, late or both jobs sharing: 8 heads of 4096 keys, FP8 P.V
 // (512 early and 768 late workgroups) 71.9 / 65.4 / 63.2, 63.7, 61.6; 32 heads of 4096, FP8 (1024 early, 3072 late) 87.9 / 82.0 / 81.8,
 // 83.0, 82.8; 4 x 32 of 4096, FP16 (5120 early) 181.8 / 174.3 / 177.1 early; packed, causal, 16 sequences of 100..600, 32/8 heads, FP16
 // (1920 late) 90.2 / 84.5 / 81.0, 82.9, 79.3; 96 of 16..1024 (18432 late) 571 / 547 / 544, 565, 563.
