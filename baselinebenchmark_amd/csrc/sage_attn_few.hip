@@ -508,22 +508,25 @@ __global__ void __launch_bounds__(256) attn_few_merge_kernel(FewArgs a) {
 // One range per (batch, KV head): nothing to merge, D / 4 lanes normalise a row, 1024 / D rows per workgroup.  (A workgroup of the merge
 // kernel per row, with three barriers and eight loads of the one partial result: whole calls of 16384 heads, head_dim 64, 32 rows and 32 keys
 // 535 -> 311 us, 1 row and 64 keys 164 -> 156; head_dim 128, 16 rows and 32 keys 467 -> 365.)
+// At most kFewNormaliseGroups workgroups, which then walk the rows: 4 M pairs of 32 rows would be more threads than a grid axis holds.
+constexpr int kFewNormaliseGroups = 1 << 16;
 template <int DT, int D>
 __global__ void __launch_bounds__(256) attn_few_normalise_kernel(FewArgs a) {
-  constexpr int LN = D / 4;
-  const int G = a.Hq / a.Hkv, rows = G * a.Sq, row = blockIdx.x * (256 / LN) + threadIdx.x / LN, lane4 = threadIdx.x % LN;
-  if (row >= a.B * a.Hkv * rows) return;
-  const int bh = row / rows, r = row - bh * rows, b = bh / a.Hkv, kvh = bh - b * a.Hkv, head = r / a.Sq, hq = kvh * G + head, s = r - head * a.Sq;
-  const float* part = a.part + (int64_t)bh * few_part_floats(rows, D);
-  const float* meta = part + rows * D + r;
-  const float4 o = reinterpret_cast<const float4*>(part + r * D)[lane4];
-  const float m = meta[0], top = fmaxf(kMInitFew, m), f = __builtin_amdgcn_exp2f(m - top), l = meta[rows] * f;   // (f: 1, or NaN with m)
-  float4 vs = make_float4(1.f, 1.f, 1.f, 1.f);
-  if (a.vs_partial) vs = reinterpret_cast<const float4*>(a.vscale + (int64_t)bh * D)[lane4];
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
-  const uint2 out = make_uint2(pack2<DT>(o.x * f * inv * vs.x, o.y * f * inv * vs.y), pack2<DT>(o.z * f * inv * vs.z, o.w * f * inv * vs.w));
-  *reinterpret_cast<uint2*>(a.out + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + 4 * lane4) = out;
-  if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km || a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+  constexpr int LN = D / 4, RPW = 256 / LN;
+  const int G = a.Hq / a.Hkv, rows = G * a.Sq, total = a.B * a.Hkv * rows, lane4 = threadIdx.x % LN;
+  for (int row = blockIdx.x * RPW + threadIdx.x / LN; row < total; row += gridDim.x * RPW) {
+    const int bh = row / rows, r = row - bh * rows, b = bh / a.Hkv, kvh = bh - b * a.Hkv, head = r / a.Sq, hq = kvh * G + head, s = r - head * a.Sq;
+    const float* part = a.part + (int64_t)bh * few_part_floats(rows, D);
+    const float* meta = part + rows * D + r;
+    const float4 o = reinterpret_cast<const float4*>(part + r * D)[lane4];
+    const float m = meta[0], top = fmaxf(kMInitFew, m), f = __builtin_amdgcn_exp2f(m - top), l = meta[rows] * f;   // (f: 1, or NaN with m)
+    float4 vs = make_float4(1.f, 1.f, 1.f, 1.f);
+    if (a.vs_partial) vs = reinterpret_cast<const float4*>(a.vscale + (int64_t)bh * D)[lane4];
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const uint2 out = make_uint2(pack2<DT>(o.x * f * inv * vs.x, o.y * f * inv * vs.y), pack2<DT>(o.z * f * inv * vs.z, o.w * f * inv * vs.w));
+    *reinterpret_cast<uint2*>(a.out + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + 4 * lane4) = out;
+    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km || a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+  }
 }
 
 }  // namespace
@@ -548,7 +551,8 @@ hipError_t launch_attn_few(FewArgs a, int dtype, int D, int pv, hipStream_t st) 
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (a.nsplit == 1) {
-    const dim3 ngrid((uint32_t)(((int64_t)pairs * rows * (D / 4) + 255) / 256));
+    const int64_t groups = ((int64_t)pairs * rows * (D / 4) + 255) / 256;
+    const dim3 ngrid((uint32_t)(groups < kFewNormaliseGroups ? groups : kFewNormaliseGroups));
     if (dtype == 0) { if (D == 64) attn_few_normalise_kernel<0, 64><<<ngrid, block, 0, st>>>(a); else attn_few_normalise_kernel<0, 128><<<ngrid, block, 0, st>>>(a); }
     else { if (D == 64) attn_few_normalise_kernel<1, 64><<<ngrid, block, 0, st>>>(a); else attn_few_normalise_kernel<1, 128><<<ngrid, block, 0, st>>>(a); }
     return hipGetLastError();

@@ -204,3 +204,26 @@ def test_both_sides_of_the_rule_for_short_keys(B, Hq, Hkv, Sq, Skv, D, pv):
     err = float((got - want).norm() / want.norm())
     # P rounded to 11 bits; e4m3 V (3 mantissa bits: 2^-4 / sqrt(3) of a value) and codes of P (0.933 to 1.105, as much once normalised)
     assert err < (2.0 ** -10 if pv == "fp16" else 0.055)
+
+
+@pytest.mark.parametrize("D,heads,G,Sq", [(64, 2050, 1, 32), (128, 1030, 2, 16)])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+def test_one_range_per_head_and_more_rows_than_one_walk(D, heads, G, Sq, pv):
+    """One range per head is normalised 256 / (D / 4) rows to a workgroup by at most 65536 workgroups, which then walk on: the last heads equal
+    a call of their own, which one walk covers (the same kernel, so the same numbers)."""
+    B, Skv, rows = 16, 100, G * Sq
+    assert B * heads * rows * D // 4 > 256 << 16
+    if pv == "fp8" and rows > 16:   # (FP8 takes one score tile here: twice the heads of half the rows)
+        heads, Sq = 2 * heads, Sq // 2
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v = (torch.randn((B, h, n, D), generator=g, device="cuda").half() for h, n in ((heads * G, Sq), (heads, Skv), (heads, Skv)))
+    out, lse = sa.sageattn(q, k, v, pv_mode=pv), None
+    if pv == "fp16":
+        out, lse = sa.sageattn(q, k, v, return_lse=True)
+    for at in (0, B - 1):
+        part = slice(at, at + 1)
+        want, want_lse = sa.sageattn(q[part], k[part], v[part], pv_mode=pv), None
+        assert torch.equal(out[part], want)
+        if lse is not None:
+            want, want_lse = sa.sageattn(q[part], k[part], v[part], return_lse=True)
+            assert torch.equal(lse[part], want_lse) and torch.equal(out[part], want)
