@@ -242,7 +242,11 @@ size_t sage_sageattn_workspace_bytes(int B, int Hq, int Hkv, int Sq, int Skv, in
 /* The same for ONE kind of call: without an explicit mask, and unless LSE is returned from smoothed keys or the Q scales
  * are interleaved, Q is quantised inside the attention kernel and its INT8 copy (a third of the upper bound) is not
  * part of the workspace.  sage_sageattn / sage_sageattn_masked accept any workspace of at least this size for the call
- * they are given; sage_sageattn_static checks it against its capacity. */
+ * they are given; sage_sageattn_static checks it against its capacity.
+ * With FP8 P.V and smooth_k, sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv_mode) bytes more than this size (behind those of
+ * sage_sageattn_mask_bytes, if a mask is packed) let the statistics of K and V exist at the same time
+ * and the pre-passes share two launches; in a workspace without them the same pre-passes run one after the other, with the same
+ * results.  (The upper bound above has them to spare where it counts an INT8 copy of Q that the call does not make.) */
 size_t sage_sageattn_workspace_bytes_for(int B, int Hq, int Hkv, int Sq, int Skv, int D,
                                          int blkq, int blkk, int pv_mode,
                                          int total_q, int total_k, int varlen,
@@ -266,7 +270,8 @@ int sage_sageattn(const void* q, const void* k, const void* v, void* out, float*
  * softmax(sm_scale * q.k^T + mask) at :171-178: here the additive mask is in NATURAL-log units on top
  * of sm_scale * q.k^T (it is multiplied by log2(e) internally); boolean masks as in
  * sage_attn_fwd_masked.  attn_mask == NULL makes it identical to sage_sageattn.
- * A workspace that is larger than sage_sageattn_workspace_bytes_for by sage_sageattn_mask_bytes lets the call pack a boolean
+ * A workspace that is larger than sage_sageattn_workspace_bytes_for by sage_sageattn_mask_bytes (FP8 P.V of smoothed keys: and by
+ * sage_prep_v_workspace_bytes, see there) lets the call pack a boolean
  * mask into bits first (one per row and key, for each distinct slice of the mask): the attention then skips the key tiles
  * that no row of a q-tile sees.  With finite V the results are the same, bit for bit; an infinity or NaN in V at a key that a row
  * may not see reaches that row's output as 0 * V = NaN where its tile is visited, and not where it is skipped (as above the
