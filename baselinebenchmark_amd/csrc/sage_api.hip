@@ -587,9 +587,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     FewArgs f;
     memset(&f, 0, sizeof(f));
     f.q = (const u16*)q; f.k = (const u16*)k; f.v = (const u16*)v;
-    if (mean_first) f.km = (const u16*)km;
-    else f.km_partial = (const double*)ks.partial;
-    f.vs_partial = (const float*)stats.v_stat.partial; f.vscale = v_scale; f.nchunk = ks.nchunk;
+    f.km_partial = mean_first ? (const double*)km : (const double*)ks.partial; f.nchunk = mean_first ? 0 : ks.nchunk;
+    f.vs_partial = (const float*)stats.v_stat.partial; f.vscale = v_scale;
     f.out = (u16*)out; f.lse = lse; f.part = (float*)panels;   // (no panels here: their region holds the partial results)
     f.part_bytes = (int64_t)sage_v_panel_bytes(B, Hkv, Skv, D, pv_mode);
     f.B = B; f.Hq = Hq; f.Hkv = Hkv; f.Sq = Sq; f.Skv = Skv;

@@ -88,8 +88,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   {
     const int64_t at = (int64_t)bh * a.nchunk * D + tid % D;
     // (head_dim 128: the lower half of the workgroup folds K, the upper one V; at 64 likewise with a quarter each)
-    if (PV == 0 && a.km && tid < D) km_lds[tid] = a.km[(int64_t)bh * D + tid];
-    if (a.km_partial && tid < D) {
+    if (PV == 0 && a.km_partial && a.nchunk == 0) {
+      if (tid < D) km_lds[tid] = reinterpret_cast<const u16*>(a.km_partial)[(int64_t)bh * D + tid];
+    } else if (a.km_partial && tid < D) {
       double s = 0;
       for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
         double t[8];
@@ -124,7 +125,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   if (t0 < t1) load_k(first);
 
   float kmf[LK][8];
-  if ((PV == 0 && a.km) || a.km_partial) {
+  if (a.km_partial) {
 #pragma unroll
     for (int i = 0; i < LK; i++) {
       const v4u raw = *reinterpret_cast<const v4u*>(km_lds + 8 * g + 32 * i);
@@ -501,7 +502,7 @@ __global__ void __launch_bounds__(256) attn_few_merge_kernel(FewArgs a) {
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     const uint2 out = make_uint2(pack2<DT>(acc.x * inv * vs[0], acc.y * inv * vs[1]), pack2<DT>(acc.z * inv * vs[2], acc.w * inv * vs[3]));
     *reinterpret_cast<uint2*>(a.out + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + 4 * lane4) = out;
-    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km || a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
   }
 }
 
@@ -525,7 +526,7 @@ __global__ void __launch_bounds__(256) attn_few_normalise_kernel(FewArgs a) {
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     const uint2 out = make_uint2(pack2<DT>(o.x * f * inv * vs.x, o.y * f * inv * vs.y), pack2<DT>(o.z * f * inv * vs.z, o.w * f * inv * vs.w));
     *reinterpret_cast<uint2*>(a.out + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)s * a.o_sn + 4 * lane4) = out;
-    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km || a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
+    if (a.lse && lane4 == 0) a.lse[((int64_t)b * a.Hq + hq) * a.Sq + s] = l > 0.f ? top + __builtin_amdgcn_logf(l) + (a.km_partial ? meta[2 * rows] : 0.f) : kNegInfFew;
   }
 }
 

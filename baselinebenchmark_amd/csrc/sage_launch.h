@@ -118,10 +118,10 @@ constexpr int kFewWorkgroups = 512;   // two per compute unit, what the register
 constexpr int kFewChunks = 128;
 struct FewArgs {
   const u16 *q, *k, *v;
-  // per-chunk statistics (ColStatArgs), combined in the kernel: sums of K or null, abs-maxima of V (FP8 P.V) or null
+  // per-chunk statistics (ColStatArgs), combined in the kernel: sums of K or null (no smoothing), abs-maxima of V (FP8 P.V) or null.
+  // nchunk 0, FP16 P.V: km_partial is the mean itself, [B, Hkv, D] in K's type
   const double* km_partial;
   const float* vs_partial;
-  const u16* km;   // [B, Hkv, D]: the mean itself, instead of km_partial, or null (both null: no smoothing)
   float* vscale;   // [B, Hkv, D], written by the main kernel for the merge
   int nchunk;
   u16* out;
