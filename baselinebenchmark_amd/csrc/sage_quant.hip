@@ -775,18 +775,27 @@ __global__ void __launch_bounds__(256, ALL ? 3 : 4) fused_prepass_kernel(FusedPr
 // The quantiser always gains: bf16, 100 M elements, heads / rows first, 8 heads of 64 81.4 / 81.3 us, 24 80.9 / 89.8, 64 80.9 / 101.8, 8 of
 // 128 64.2 / 62.8, 24 65.1 / 69.7, 32 64.1 / 83.1.
 static bool heads_first(int64_t head_stride, int64_t row_stride, int64_t chunks) { return head_stride < row_stride && chunks <= 65535; }
-// Statistics and V panels, which read 128 rows and more per workgroup, gain where rows are a multiple of 4 KiB apart (a head's rows alone
-// then crowd into a few memory channels) and in packed batches of short sequences (most workgroups of a grid sized for the longest
-// one find nothing to do); elsewhere rows first is the faster one.  FP16 panels / FP8 panels with their statistic / K mean, 100 M elements in
-// us, heads first and rows first: 16 heads of 128 (4 KiB) 76 / 93 / 40 and 87 / 108 / 48; 32 of 64 (4 KiB) 80 / 99 / 41 and 87 / 113 / 50;
-// 24 of 128 (6 KiB) 77 / 93 / 39 and 71 / 91 / 39; 40 of 64 (5 KiB) 82 / 103 / 42 and 72 / 95 / 37.  Whole packed calls, a query row per
-// sequence, panels rows first, statistics rows first: 96 of 16..1024 rows, 24 heads of 128 447 -> 470, 453; 64 of 512..4096, 24 heads of
-// 64, FP8 649 -> 668, 660; 8 of 4096..8192 238 -> 236, 231; 16 of 512..32768 1248 -> 1225, 1192.
-static bool heads_first_streaming(int64_t head_stride, int64_t row_stride, int64_t chunks, bool packed, int max_rows) {
-  return heads_first(head_stride, row_stride, chunks) && (row_stride * 2 % 4096 == 0 || (packed && max_rows <= 4096));
+// Statistics (512 rows per workgroup) and V panels (128), in packed batches: up to 4096 rows a sequence, heads first (most workgroups of a grid
+// sized for the longest sequence find nothing to do), longer ones rows first.  Whole causal calls, heads first / rows first: 64 of 256..4096, 24
+// heads of 128, FP8 2268 / 2379 us, of 64 1421 / 1472; 96 of 16..1024, 8 heads of 128 235 / 244; 16 of 512..32768, 24 heads of 64 17224 / 17117.
+// Otherwise heads first where rows are a multiple of 4 KiB apart (a head's rows alone then crowd into a few memory channels), and
+//   statistics at head_dim 128, and at 64 as long as a head is four chunks.  Whole calls, 40 query rows: 4 x 32 heads of 8000 rows, 128, FP8 313 / 322,
+//   24 of 1559 42.6 / 43.2; head_dim 64: 4 x 24 of 1559 48.0 / 48.9, 24 of 9000, FP8 110.2 / 109.3, 4 x 40 of 8000 231 / 224;
+//   the panels of a shared launch, up to 1024 in FP16 and 512 in FP8 (the K quantiser beside them walks heads first too; what exactly gains has
+//   not been isolated).  Whole calls, FP16: 2 x 8 heads of 4000 rows, 128 (512 panels) 81.8 / 85.6, 2 x 12, 64 (768) 65.2 / 68.5, 2 x 20, 128 (1280)
+//   106.4 / 106.2, 4 x 40 of 1559, 64 (2080) 64.1 / 62.7; FP8: 4 of 9000, 128 (284) 109.5 / 110.5, 12 of 9000 (852) 126.5 / 125.8.
+// Panels alone, 100 M elements: 16 heads of 128 (4 KiB) 71.6 / 77.7, 32 (8 KiB) 71.1 / 73.7, 24 (6 KiB) 73.2 / 67.7; 32 of 64 (4 KiB) 75.8 / 78.6,
+// 40 (5 KiB) 78.9 / 68.0.
+static bool heads_first_streaming(int64_t head_stride, int64_t row_stride, int64_t chunks, bool packed, int max_rows, bool otherwise) {
+  return heads_first(head_stride, row_stride, chunks) && (packed ? max_rows <= 4096 : otherwise || row_stride * 2 % 4096 == 0);
 }
-static bool heads_first(const ColStatArgs& a, int64_t chunks) { return heads_first_streaming(a.x_sh, a.x_sn, chunks, a.cu_seqlens, a.L); }
-static bool heads_first(const PrepVArgs& a, int64_t chunks) { return heads_first_streaming(a.v_sh, a.v_sn, chunks, a.cu_seqlens, a.L); }
+static bool heads_first(const ColStatArgs& a, int64_t chunks) {
+  return heads_first_streaming(a.x_sh, a.x_sn, chunks, a.cu_seqlens, a.L, a.D == 128 || a.L <= 4 * kChunkRows);
+}
+constexpr int64_t kFewPanels[2] = {1024, 512};   // FP16, FP8
+static bool heads_first(const PrepVArgs& a, int64_t chunks, bool few = false) {
+  return heads_first_streaming(a.v_sh, a.v_sn, chunks, a.cu_seqlens, a.L, few);
+}
 static bool heads_first(const QuantArgs& a, int64_t chunks) { return heads_first(a.x_sh, a.x_sn, chunks); }
 
 hipError_t launch_quant_int8(const QuantArgs& args, int dtype, int max_rows, hipStream_t st) {
@@ -874,8 +883,9 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
   const int blk = fused_block(f);
   fused_extents(f, blk, e);
   FusedTable t;
+  const bool few_panels = e[kJobVPanels][0] * e[kJobVPanels][1] * e[kJobVPanels][2] <= kFewPanels[pv != 0];
   const bool inner_heads[kJobs] = {false, heads_first(f.k_stat, 0), heads_first(f.v_stat, 0), heads_first(f.k_quant, 0),
-                                   heads_first(f.q_quant, 0), heads_first(f.v_panels, 0), false};
+                                   heads_first(f.q_quant, 0), heads_first(f.v_panels, 0, few_panels), false};
   t.heads_first = 0;
   for (int j = 0; j < kJobs; j++) {
     if (e[j][1] > 65535 || e[j][2] > 65535) return hipErrorInvalidConfiguration;   // (what the jobs' own grids take)
