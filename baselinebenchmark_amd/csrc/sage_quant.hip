@@ -772,31 +772,45 @@ __global__ void __launch_bounds__(256, ALL ? 3 : 4) fused_prepass_kernel(FusedPr
 // Where the heads of a row lie next to each other (packed and [B, L, H, D] tensors) the head can be the fastest grid index, so that whole
 // rows are on their way at a time; with the rows of one head first, a workgroup and its neighbours read 128 or 256 bytes out of every
 // few kilobytes.  (The y axis of a grid is limited to 65535.)
-// The quantiser always gains: bf16, 100 M elements, heads / rows first, 8 heads of 64 81.4 / 81.3 us, 24 80.9 / 89.8, 64 80.9 / 101.8, 8 of
-// 128 64.2 / 62.8, 24 65.1 / 69.7, 32 64.1 / 83.1.
 static bool heads_first(int64_t head_stride, int64_t row_stride, int64_t chunks) { return head_stride < row_stride && chunks <= 65535; }
 // Statistics (512 rows per workgroup) and V panels (128), in packed batches: up to 4096 rows a sequence, heads first (most workgroups of a grid
 // sized for the longest sequence find nothing to do), longer ones rows first.  Whole causal calls, heads first / rows first: 64 of 256..4096, 24
 // heads of 128, FP8 2268 / 2379 us, of 64 1421 / 1472; 96 of 16..1024, 8 heads of 128 235 / 244; 16 of 512..32768, 24 heads of 64 17224 / 17117.
 // Otherwise heads first where rows are a multiple of 4 KiB apart (a head's rows alone then crowd into a few memory channels), and
-//   statistics at head_dim 128, and at 64 as long as a head is four chunks.  Whole calls, 40 query rows: 4 x 32 heads of 8000 rows, 128, FP8 313 / 322,
-//   24 of 1559 42.6 / 43.2; head_dim 64: 4 x 24 of 1559 48.0 / 48.9, 24 of 9000, FP8 110.2 / 109.3, 4 x 40 of 8000 231 / 224;
-//   the panels of a shared launch, up to 1024 in FP16 and 512 in FP8 (the K quantiser beside them walks heads first too; what exactly gains has
-//   not been isolated).  Whole calls, FP16: 2 x 8 heads of 4000 rows, 128 (512 panels) 81.8 / 85.6, 2 x 12, 64 (768) 65.2 / 68.5, 2 x 20, 128 (1280)
-//   106.4 / 106.2, 4 x 40 of 1559, 64 (2080) 64.1 / 62.7; FP8: 4 of 9000, 128 (284) 109.5 / 110.5, 12 of 9000 (852) 126.5 / 125.8.
+//   statistics at head_dim 128, and at 64 as long as a head is four chunks or all of them are 256.  Whole calls, 40 query rows: 4 x 32 heads of 8000
+//   rows, 128, FP8 313 / 322, 24 of 1559 42.6 / 43.2; head_dim 64: 4 x 24 of 1559 48.0 / 48.9, 2 x 4 of 5696, FP8 69.1 / 70.1, 24 of 9000 110.2 /
+//   109.3, 4 x 40 of 8000 231 / 224;
+//   up to 1024 panels (which reader of them gains has not been isolated).  Whole calls, FP16: 2 x 8 heads of 4000 rows,
+//   128 (512 panels) 81.8 / 85.6, 2 x 12, 64 (768) 65.2 / 68.5, 2 x 20, 128 (1280) 106.4 / 106.2, 4 x 40 of 1559, 64 (2080) 64.1 / 62.7; FP8: 4 of
+//   9000, 128 (284) 109.5 / 110.5, 8 x 12 of 886 (672) 65.1 / 66.0, 12 of 9000 (852) 126.5 / 125.8, 4 x 12 of 2471, 64 (960) 45.2 / 46.1.
 // Panels alone, 100 M elements: 16 heads of 128 (4 KiB) 71.6 / 77.7, 32 (8 KiB) 71.1 / 73.7, 24 (6 KiB) 73.2 / 67.7; 32 of 64 (4 KiB) 75.8 / 78.6,
 // 40 (5 KiB) 78.9 / 68.0.
+constexpr int64_t kFewStats = 256, kFewPanels = 1024;
 static bool heads_first_streaming(int64_t head_stride, int64_t row_stride, int64_t chunks, bool packed, int max_rows, bool otherwise) {
   return heads_first(head_stride, row_stride, chunks) && (packed ? max_rows <= 4096 : otherwise || row_stride * 2 % 4096 == 0);
 }
 static bool heads_first(const ColStatArgs& a, int64_t chunks) {
-  return heads_first_streaming(a.x_sh, a.x_sn, chunks, a.cu_seqlens, a.L, a.D == 128 || a.L <= 4 * kChunkRows);
+  return heads_first_streaming(a.x_sh, a.x_sn, chunks, a.cu_seqlens, a.L, a.D == 128 || a.L <= 4 * kChunkRows || (int64_t)a.B * a.H * a.nchunk <= kFewStats);
 }
-constexpr int64_t kFewPanels[2] = {1024, 512};   // FP16, FP8
-static bool heads_first(const PrepVArgs& a, int64_t chunks, bool few = false) {
-  return heads_first_streaming(a.v_sh, a.v_sn, chunks, a.cu_seqlens, a.L, few);
+static bool heads_first(const PrepVArgs& a, int64_t chunks) {
+  const int64_t panels = (int64_t)a.B * a.H * ((a.L + kPanelRows - 1) / kPanelRows);
+  return heads_first_streaming(a.v_sh, a.v_sn, chunks, a.cu_seqlens, a.L, panels <= kFewPanels);
 }
-static bool heads_first(const QuantArgs& a, int64_t chunks) { return heads_first(a.x_sh, a.x_sn, chunks); }
+// The quantiser.  Packed batches: heads first where the grid's row chunks are even in number: rows first, the same chunks of all heads and
+// sequences then go to the same XCDs, and those with the last ones of a grid sized for the longest sequence run dry.  Whole causal calls, heads
+// first / rows first: 96 of 16..1024, 24 heads of 64 441 / 467 us, of 128 624 / 660; 60 of 64..2000 554 / 584 and 835 / 879; 64 of 256..4096 1430 / 1485;
+// an odd number: 23 of 52..2880 391 / 385 and 581 / 581.
+// Otherwise in small tensors, in the largest, and from 48 M elements where rows of heads of 128 are a multiple of 4 KiB apart.  Whole calls, 40
+// query rows: 8 heads of 1500 rows, 64, 34.5 / 36.6, 12 of 1500 33.4 / 34.1, 32 of 1500, 128 (6 M elements) 40.8 / 41.0; 4 x 24 of 2471, 128 (30 M)
+// 101.9 / 100.9, 4 x 32 of 8000, 64 (66 M) 195 / 189, 2 x 40 of 16000, 64 (82 M) 276 / 263, 24 of 32760, 128 (101 M) 472 / 468; 2 x 16 of 16000, 128
+// (4 KiB, 66 M) 267.7 / 269.6, 2 x 32 of 16384 383 / 388.  Alone, 160 M elements: 24 heads of 64 117 / 126, 12 of 128 91 / 96, 32 of 128 90 / 113;
+// 8 of 128 (2 KiB) 90.5 / 88.6.
+static bool heads_first(const QuantArgs& a, int64_t chunks) {
+  if (!heads_first(a.x_sh, a.x_sn, chunks)) return false;
+  const int64_t mega = 1 << 20, elements = (int64_t)a.B * a.H * a.L * a.D, row_bytes = a.x_sn * 2;
+  if (a.cu_seqlens) return chunks % 2 == 0;
+  return elements <= 8 * mega || (elements >= 48 * mega && a.D == 128 && row_bytes % 4096 == 0) || (elements >= 128 * mega && row_bytes > 2048);
+}
 
 hipError_t launch_quant_int8(const QuantArgs& args, int dtype, int max_rows, hipStream_t st) {
   QuantArgs a = args;
@@ -883,9 +897,8 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
   const int blk = fused_block(f);
   fused_extents(f, blk, e);
   FusedTable t;
-  const bool few_panels = e[kJobVPanels][0] * e[kJobVPanels][1] * e[kJobVPanels][2] <= kFewPanels[pv != 0];
-  const bool inner_heads[kJobs] = {false, heads_first(f.k_stat, 0), heads_first(f.v_stat, 0), heads_first(f.k_quant, 0),
-                                   heads_first(f.q_quant, 0), heads_first(f.v_panels, 0, few_panels), false};
+  const bool inner_heads[kJobs] = {false, heads_first(f.k_stat, 0), heads_first(f.v_stat, 0), heads_first(f.k_quant, e[kJobKQuant][0]),
+                                   heads_first(f.q_quant, e[kJobQQuant][0]), heads_first(f.v_panels, 0), false};
   t.heads_first = 0;
   for (int j = 0; j < kJobs; j++) {
     if (e[j][1] > 65535 || e[j][2] > 65535) return hipErrorInvalidConfiguration;   // (what the jobs' own grids take)

@@ -137,6 +137,18 @@ def test_limits_of_the_one_launch_prepass(B, H, Skv, D, blkk, pv):
         assert torch.equal(got, _steps(q, k, v, "HND", pv, 128, blkk, smooth))
 
 
+@pytest.mark.parametrize("H,D,L", [(24, 64, 5461), (24, 64, 5462), (16, 128, 24575), (16, 128, 24577), (24, 64, 87381), (24, 64, 87382),
+                                   (16, 64, 131073)])
+def test_quantiser_walks_of_small_and_large_tensors(H, D, L):
+    """Around 8, 48 and 128 M elements, where the walk over the heads of a row changes: the same codes as from heads that lie apart."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    k = torch.randn((1, L, H, D), generator=g, device="cuda", dtype=torch.float16)
+    t = k.transpose(1, 2).contiguous()
+    _, _, got, scale = sa.per_block_int8(k[:, :16], k, BLKK=64, tensor_layout="NHD")
+    _, _, want, want_scale = sa.per_block_int8(t[:, :, :16].contiguous(), t, BLKK=64)
+    assert torch.equal(got.transpose(1, 2), want) and torch.equal(scale, want_scale)
+
+
 def _cu(lens):
     return torch.tensor([0, *lens], dtype=torch.int64).cumsum(0).to(torch.int32).cuda()
 
