@@ -343,13 +343,15 @@ namespace {
 // Up to this many keys per sequence the pre-passes run as one launch whose workgroups read their sequence's statistics themselves
 // (sage_quant.hip: prepass_small_kernel) instead of two launches, statistics first ...
 constexpr int kSmallPrepassRows = 1024;
-// ... and up to this many element reads, each workgroup of K and each V panel counted with its whole sequence.  Whole calls in bf16, one
-// launch / two, FP16 and FP8 P.V, us: 12 M reads (8 x 32 heads of 128 rows, head_dim 128) 20.5 / 25.3, 20.1 / 27.3; 16 M (32 x 32 of 64)
-// 52.4 / 62.4, 49.2 / 66.9; 24 M (16 x 32 of 128) 36.6 / 41.8, 34.1 / 46.1; (8 of 1024) 34.5 / 34.7, 30.2 / 32.3; (8 x 32 of 257, 64) 35.3 /
-// 38.2, 33.8 / 37.0; 28 M (4 x 24 of 300) 32.4 / 32.9, 28.9 / 32.8; 30 M (40 of 512) 30.7 / 31.8, 28.6 / 31.6; 32 M (4 x 32 of 512, 64)
-// 31.4 / 29.5, 27.9 / 29.5; 36 M (2 x 24 of 512) 32.5 / 33.1, 31.9 / 33.0; 40 M (24 of 768) 36.2 / 35.4, 32.4 / 33.8; 48 M (16 of 1024)
-// 41.4 / 38.2, 36.5 / 34.5; 64 M (8 x 32 of 257) 61.9 / 56.5, 56.2 / 56.2; 96 M (4 x 32 of 512) 52.4 / 43.6, 54.4 / 44.4.
-constexpr int64_t kSmallPrepassReads = (int64_t)30 << 20;
+// ... and up to this many element reads, where a K workgroup reads its sequence for the mean and a V panel for the scales, and a tensor without
+// a statistic is read once.  More reads pay where two statistics would be two passes.  Whole calls in bf16, one launch / two, us:
+//   mean alone (FP16 P.V): 20 M reads (72 heads of 452 rows, head_dim 128) 39.0 / 39.1; 21 M (96 of 590, 64) 39.9 / 40.1; 24 M (256 of 384, 64) 38.4 /
+//   42.7; 23 M (24 of 648) 57.2 / 55.5; 27 M (32 of 852) 73.0 / 70.6; 29 M (96 of 704, 64) 49.6 / 48.1; 40 M (256 of 512, 64) 58.5 / 51.7;
+//   scales alone (FP8, keys as they are): 25 M (32 of 795) 32.6 / 35.1; 27 M (96 of 647, 64) 38.8 / 40.5; 35 M (256 of 443, 64) 45.1 / 44.4;
+//   both: 36 M (48 of 505) 29.9 / 33.9, (32 of 622) 33.0 / 33.3; 40 M (96 of 380) 34.0 / 36.6; 44 M (64 of 809, 64) 73.1 / 70.8; 47 M (96 of 671, 64)
+//   32.3 / 31.4; 61 M (64 of 983, 64) 41.6 / 33.3;
+//   neither: 10 M (48 of 832) 35.5 / 36.8: no reads twice, one launch either way, the smaller kernel is the faster.
+constexpr int64_t small_prepass_reads(bool mean, bool scales) { return (int64_t)(mean && scales ? 42 : scales ? 32 : 24) << 20; }
 // ... in this many heads: 12288 of a key, head_dim 64, 374 / 363; 16384 of 8 525 / 496; 8192 of 16 251 / 251, FP8 235 / 242.
 constexpr int64_t kSmallPrepassHeads = 8192;
 // A few query rows (sage_attn_few.hip) take at most three launches, some 2.5 us of host time more than the two of the tiled kernel behind
@@ -363,15 +365,15 @@ constexpr int64_t kSmallPrepassHeads = 8192;
 // FP8 P.V, 1 and 16 rows: head_dim 128, 8 heads of 768 keys 23.2 / 25.1 and 23.2 / 27.0, of 900 27.7 / 25.4 and 27.5 / 26.7; 32 of 512 (24 M)
 // 25.1 / 26.7 and 25.2 / 27.4; 16 of 768 (27 M) 28.8 / 26.7 and 28.8 / 27.9; 512 of 64 26.4 / 24.6 and 26.9 / 30.9; 1024 of 16 45.9 / 36.6 and
 // 46.7 / 48.0; 2048 of 16 86.2 / 55.7 and 86.7 / 80.5.
-bool tiled_beats_few_rows(int pv_mode, int D, int64_t rows, int Sq, int64_t query_heads, int Skv, int64_t prepass_reads) {
+bool tiled_beats_few_rows(int pv_mode, int D, int64_t rows, int Sq, int64_t query_heads, int Skv, int64_t group_reads) {
   const bool apart = rows == Sq, many = apart && rows > 20;   // apart: every query head has a KV head of its own
   const int64_t mega = 1 << 20;
   if (Skv > kSmallPrepassRows) return false;
   if (pv_mode == SAGE_PV_FP16) {
-    if ((int64_t)Skv * D > 48 * 1024 || prepass_reads > (many ? 20 : 12) * mega) return false;
+    if ((int64_t)Skv * D > 48 * 1024 || group_reads > (many ? 20 : 12) * mega) return false;
     return many || query_heads <= (D == 64 ? 512 : 256);
   }
-  if ((int64_t)Skv * D > 896 * 128 || prepass_reads > 24 * mega) return false;
+  if ((int64_t)Skv * D > 896 * 128 || group_reads > 24 * mega) return false;
   return query_heads <= (apart && rows > 8 ? 1024 : D == 64 ? 512 : 256);
 }
 // Few keys in great number: the FP32 results of a KV head's rows are written and read again, the tiled kernel with one
@@ -557,10 +559,11 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   // the whole sequence itself); otherwise two launches, the statistics in two stages.
   const int64_t k_elements = (int64_t)B * Hkv * Skv * D;
   const int k_rows = quant_rows(D, blk_rows(blkk));
-  const int64_t prepass_reads = k_elements * ((Skv + k_rows - 1) / k_rows + (Skv + kPanelRows - 1) / kPanelRows);
-  const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && prepass_reads <= kSmallPrepassReads &&
+  const int k_groups = (Skv + k_rows - 1) / k_rows, v_groups = (Skv + kPanelRows - 1) / kPanelRows;
+  const int64_t prepass_reads = k_elements * ((smooth_k ? k_groups : 1) + (pv_mode == SAGE_PV_FP8 ? v_groups : 1));
+  const bool small_prepass = !varlen && !no_keys && Skv <= kSmallPrepassRows && prepass_reads <= small_prepass_reads(smooth_k, pv_mode == SAGE_PV_FP8) &&
                              (int64_t)B * Hkv <= kSmallPrepassHeads;
-  const bool short_keys = no_keys || tiled_beats_few_rows(pv_mode, D, Hq / Hkv * (int64_t)Sq, Sq, (int64_t)B * Hq, Skv, prepass_reads);
+  const bool short_keys = no_keys || tiled_beats_few_rows(pv_mode, D, Hq / Hkv * (int64_t)Sq, Sq, (int64_t)B * Hq, Skv, k_elements * (k_groups + v_groups));
   const float q_mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
   const FewCall few = {varlen, is_causal, pv_mode, B, Hkv, Sq, Skv, D, blkq, blkk, Hq / Hkv * (int64_t)Sq, q_sn, k_sn, v_sn,
                        q, k, v, out, attn_mask, short_keys, lse != nullptr, w.k_i8_bytes};

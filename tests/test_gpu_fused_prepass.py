@@ -124,11 +124,12 @@ def test_more_rows_than_the_second_grid_axis_holds(rows):
     assert torch.equal(k8[:, -tail:], t8) and torch.equal(ks[..., -ts.shape[-1]:], ts)
 
 
-# element reads (whole sequences, once per K workgroup and V panel) around the limit of the one-launch pre-pass, 30 Mi, and heads around
-# its 8192: either way the same numbers as from the separate entry points
+# element reads (whole sequences, once per K workgroup with a mean and V panel with scales) around the limits of the one-launch pre-pass, 24 Mi
+# with a mean, 32 Mi with scales and 42 Mi with both, and heads around its 8192: either way the same numbers as from the separate entry points
 @pytest.mark.parametrize("B,H,Skv,D,blkk", [(1, 40, 512, 128, 64), (1, 40, 513, 128, 64), (1, 30, 1024, 64, 64), (1, 31, 1024, 64, 64),
                                             (1, 20, 1024, 64, 16), (1, 21, 1024, 64, 16), (64, 128, 3, 64, 64), (64, 129, 3, 64, 64),
-                                            (16, 32, 128, 128, 16), (1, 8, 1024, 128, 64), (1, 8, 1025, 128, 64)])
+                                            (16, 32, 128, 128, 16), (1, 8, 1024, 128, 64), (1, 8, 1025, 128, 64), (1, 56, 512, 128, 64),
+                                            (1, 57, 512, 128, 64), (1, 102, 512, 128, 64), (1, 103, 512, 128, 64)])
 @pytest.mark.parametrize("pv", ["fp16", "fp8"])
 def test_limits_of_the_one_launch_prepass(B, H, Skv, D, blkk, pv):
     q, k, v = _inputs(B, H, H, 40, Skv, D, torch.float16, "HND", Skv + H)
