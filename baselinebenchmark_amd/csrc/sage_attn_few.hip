@@ -17,10 +17,10 @@
 //     of very long histories, kFewChunks);
 //   * FP8 P.V: V is rounded to the e4m3 values of the panels in registers (a division per element: the vector ALU is what bounds it)
 //     and multiplied in fp16, which holds them; the probabilities are the tiled kernel's block-scaled codes, read back the same way.
-// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 46.3 us (this
-// kernel 33 us = 4.1 TB/s of K and V, half of it vector arithmetic of the quantisation; K sums 12, merge 4); 8 rows: 170.8
-// -> 55; 8 x 32/8 heads, 4 rows, 16384 keys: 431.9 -> 155; 16 x 32 heads, 4096 keys: 600 -> 286; 1 x 8/2 heads, 8 rows, 32768 keys:
-// 435 -> 62.  FP8 P.V: 146 -> 77, and 313 -> 67 for the last.
+// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 48.7 us (this
+// kernel 33 us = 4.1 TB/s of K and V, half of it vector arithmetic of the quantisation; K sums 10, merge 5); 8 rows: 170.8
+// -> 54; 8 x 32/8 heads, 4 rows, 16384 keys: 431.9 -> 150; 16 x 32 heads, 4096 keys: 600 -> 279; 1 x 8/2 heads, 8 rows, 32768 keys:
+// 435 -> 34.  FP8 P.V: 146 -> 82 for the first, 311 -> 51 for the last.
 #include "sage_launch.h"
 
 #pragma clang fp contract(off)

@@ -35,8 +35,8 @@ struct QuantArgs {
 // Geometry of the quantiser: a workgroup of 256 lanes takes quant_rows(D, blk) consecutive rows of one (batch, head), whole scale
 // blocks of them, and a wavefront quant_passes(D, blk) times quant_wave_rows(D) neighbouring ones, never more than a scale block: the
 // maximum of a block crosses wavefronts only where the block does, and no lane is idle at any block size.
-// Bound by HBM (3 bytes per element) with the vector ALU close behind it: some 12 instructions per element, 19 when the differences
-// were narrowed one by one, widened twice and packed by masks and shifts.  bf16, K mean subtracted, head_dim 128, one kernel: 4 x 32
+// Bound by HBM (3 bytes per element) with the vector ALU close behind it: 14.6 vector instructions per element (SQ_INSTS_VALU), 17.6 when the
+// differences were narrowed one by one, widened twice and packed by masks and shifts.  bf16, K mean subtracted, head_dim 128, one kernel: 4 x 32
 // heads of 4096 rows, blocks of 64: 52.0 -> 40.8 us (201 MB, 4.9 TB/s); blocks of 16, 2 x 16 heads of 4096 rows, where a block a
 // workgroup left half the lanes idle: 24.5 -> 13.1.
 __host__ __device__ constexpr int quant_wave_rows(int D) { return 64 / (D / 16); }   // rows of a pass of a wavefront
