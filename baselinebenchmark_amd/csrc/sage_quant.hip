@@ -536,8 +536,11 @@ __global__ void __launch_bounds__(256) prep_v_kernel(PrepVArgs a) {
 // ---------------------------------------------------------------------------------------------
 // Hands the rows n, n + RPP, ... below n1 of a lane's channels to `fold`, in that order, sixteen loads in flight: the statistic is
 // latency from end to end, and with the unrolling left to the compiler it took between four and thirty of them, 35 to 45 us for
-// the call on 8 heads of 1000 rows at head_dim 128.  (Rows past the end arrive as zeros, which no statistic notices.)
-template <int D, class Fold>
+// the call on 8 heads of 1000 rows at head_dim 128.  (Rows past the end arrive as zeros, which no statistic notices.  Their loads are of
+// one line, but their binary64 additions take as long as others: SUMS leaves them out, workgroup by workgroup.  3 x 32/8 heads of 648 rows, head_dim
+// 128, FP16 P.V 57.3 -> 56.2 us, 2 x 24 of 4095 queries and 257 keys, 64, 42.3 -> 41.6.  Maxima are cheaper than the branches: FP8, no
+// smoothing, 2 x 16 heads of 795 32.6 us without, 34.0 with them.)
+template <int D, bool SUMS, class Fold>
 __device__ __forceinline__ void stream_rows(const u16* base, int64_t stride, int n, int n0, int n1, Fold fold) {
   constexpr int RPP = 256 / (D / 8);
   auto batch = [&](auto unr) __attribute__((always_inline)) {
@@ -547,7 +550,10 @@ __device__ __forceinline__ void stream_rows(const u16* base, int64_t stride, int
     for (int u = 0; u < UNR; u++) raw[u] = *reinterpret_cast<const uint4*>(base + (int64_t)min(n + u * RPP, n1 - 1) * stride);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < UNR; u++) fold(n + u * RPP < n1 ? raw[u] : make_uint4(0, 0, 0, 0));
+    for (int u = 0; u < UNR; u++) {
+      if (SUMS && n0 + u * RPP >= n1) break;
+      fold(n + u * RPP < n1 ? raw[u] : make_uint4(0, 0, 0, 0));
+    }
     n0 += UNR * RPP;
     n += UNR * RPP;
   };
@@ -577,7 +583,7 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
         double acc[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) acc[i] = 0;
-        stream_rows<D>(qa.x + xbase + tc * 8, qa.x_sn, n0 + tr, n0, n1, [&](const uint4& raw) {   // (the additions in row order)
+        stream_rows<D, true>(qa.x + xbase + tc * 8, qa.x_sn, n0 + tr, n0, n1, [&](const uint4& raw) {   // (the additions in row order)
           const uint32_t* x2 = reinterpret_cast<const uint32_t*>(&raw);
 #pragma unroll
           for (int i = 0; i < 4; i++) {
@@ -613,7 +619,7 @@ __global__ void __launch_bounds__(256) prepass_small_kernel(QuantArgs qa, PrepVA
       float acc[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) acc[i] = 0.f;
-      stream_rows<D>(va.v + vbase + tc * 8, va.v_sn, tr, 0, L, [&](const uint4& raw) {
+      stream_rows<D, false>(va.v + vbase + tc * 8, va.v_sn, tr, 0, L, [&](const uint4& raw) {
         const uint32_t* x2 = reinterpret_cast<const uint32_t*>(&raw);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
