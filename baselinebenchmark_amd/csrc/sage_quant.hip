@@ -806,16 +806,16 @@ static bool heads_first(const PrepVArgs& a, int64_t chunks) {
 // sequences then go to the same XCDs, and those with the last ones of a grid sized for the longest sequence run dry.  Whole causal calls, heads
 // first / rows first: 96 of 16..1024, 24 heads of 64 441 / 467 us, of 128 624 / 660; 60 of 64..2000 554 / 584 and 835 / 879; 64 of 256..4096 1430 / 1485;
 // an odd number: 23 of 52..2880 391 / 385 and 581 / 581.
-// Otherwise in small tensors, in the largest, and from 48 M elements where rows of heads of 128 are a multiple of 4 KiB apart.  Whole calls, 40
+// Otherwise in small tensors, in the largest, and where rows of heads of 128 are a multiple of 4 KiB apart.  Whole calls, 40
 // query rows: 8 heads of 1500 rows, 64, 34.5 / 36.6, 12 of 1500 33.4 / 34.1, 32 of 1500, 128 (6 M elements) 40.8 / 41.0; 4 x 24 of 2471, 128 (30 M)
 // 101.9 / 100.9, 4 x 32 of 8000, 64 (66 M) 195 / 189, 2 x 40 of 16000, 64 (82 M) 276 / 263, 24 of 32760, 128 (101 M) 472 / 468; 2 x 16 of 16000, 128
-// (4 KiB, 66 M) 267.7 / 269.6, 2 x 32 of 16384 383 / 388.  Alone, 160 M elements: 24 heads of 64 117 / 126, 12 of 128 91 / 96, 32 of 128 90 / 113;
+// (4 KiB, 66 M) 267.7 / 269.6, 2 x 32 of 16384 383 / 388; causal, as many query rows, 16 of 4096, 128, 98.2 / 101.8, 2 x 32 of 2048 100.5 / 101.3.  Alone, 160 M elements: 24 heads of 64 117 / 126, 12 of 128 91 / 96, 32 of 128 90 / 113;
 // 8 of 128 (2 KiB) 90.5 / 88.6.
 static bool heads_first(const QuantArgs& a, int64_t chunks) {
   if (!heads_first(a.x_sh, a.x_sn, chunks)) return false;
   const int64_t mega = 1 << 20, elements = (int64_t)a.B * a.H * a.L * a.D, row_bytes = a.x_sn * 2;
   if (a.cu_seqlens) return chunks % 2 == 0;
-  return elements <= 8 * mega || (elements >= 48 * mega && a.D == 128 && row_bytes % 4096 == 0) || (elements >= 128 * mega && row_bytes > 2048);
+  return elements <= 8 * mega || (a.D == 128 && row_bytes % 4096 == 0) || (elements >= 128 * mega && row_bytes > 2048);
 }
 
 hipError_t launch_quant_int8(const QuantArgs& args, int dtype, int max_rows, hipStream_t st) {

@@ -141,7 +141,8 @@ def test_limits_of_the_one_launch_prepass(B, H, Skv, D, blkk, pv):
 @pytest.mark.parametrize("H,D,L", [(24, 64, 5461), (24, 64, 5462), (16, 128, 24575), (16, 128, 24577), (24, 64, 87381), (24, 64, 87382),
                                    (16, 64, 131073)])
 def test_quantiser_walks_of_small_and_large_tensors(H, D, L):
-    """Around 8, 48 and 128 M elements, where the walk over the heads of a row changes: the same codes as from heads that lie apart."""
+    """Around 8 and 128 M elements, where the walk over the heads of a row changes, and rows 4 KiB apart: the same codes as from heads that lie
+    apart."""
     g = torch.Generator(device="cuda").manual_seed(L)
     k = torch.randn((1, L, H, D), generator=g, device="cuda", dtype=torch.float16)
     t = k.transpose(1, 2).contiguous()
