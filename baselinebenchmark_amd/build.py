@@ -15,7 +15,7 @@ from pathlib import Path
 CSRC = Path(__file__).resolve().parent / "csrc"
 LIB = CSRC / "libsage_mi355x.so"
 SOURCES = ["sage_quant.hip", "sage_attn.hip", "sage_attn_mask.hip", "sage_attn_maskwide.hip", "sage_attn_maskbits.hip", "sage_attn_qfuse.hip",
-           "sage_attn_kinterleave.hip", "sage_attn_few.hip", "sage_api.hip", "sage_static.hip"]
+           "sage_attn_kinterleave.hip", "sage_attn_small.hip", "sage_attn_few.hip", "sage_api.hip", "sage_static.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # correctly rounded fp32 divide (the INT8 quantiser's contract) and no packed-fp32 selection
@@ -32,7 +32,7 @@ FLAGS = [
 # loaded or exchanged value is preceded by an instruction that only quiets signalling NaNs (four per tile: 0.6 % on
 # config 2, bit-identical outputs).
 EXTRA_FLAGS = {src: ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-fno-honor-nans"]
-               for src in ("sage_attn.hip", "sage_attn_qfuse.hip", "sage_attn_kinterleave.hip")}
+               for src in ("sage_attn.hip", "sage_attn_qfuse.hip", "sage_attn_kinterleave.hip", "sage_attn_small.hip")}
 
 
 def _hipcc() -> str:

@@ -196,8 +196,7 @@ int sage_varlen_plan(const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, i
   if (!cu_seqlens_q || !cu_seqlens_k || !plan) return fail(SAGE_EINVAL, "null pointer");
   if (!valid_blk_quant(blkq) || !valid_blk_quant(blkk)) return fail(SAGE_ENOTIMPL, "block sizes %d/%d not supported", blkq, blkk);
   if (plan_ints < sage_varlen_plan_ints(nseq, total_q)) return fail(SAGE_EWORKSPACE, "plan buffer too small");
-  AttnConfig cfg = attn_config(128, 1, true);
-  hipError_t e = launch_varlen_plan(cu_seqlens_q, cu_seqlens_k, nseq, total_q, blkq, blkk, cfg.nw * 32, 64, is_causal, plan,
+  hipError_t e = launch_varlen_plan(cu_seqlens_q, cu_seqlens_k, nseq, total_q, blkq, blkk, kLargeTileRows, 64, is_causal, plan,
                                     (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "sage_varlen_plan");
   return SAGE_OK;
@@ -223,12 +222,51 @@ struct MaskArg {
   float mult = 1.0f;   // additive masks are multiplied by this (1 for base-2 units, log2(e) for natural units)
 };
 
+// Query rows per workgroup: 256 (eight wavefronts, two groups in step on one tile stream, sage_attn.hip) or 128 (four wavefronts,
+// two or three workgroups to a compute unit, sage_attn_small.hip).  The results are the same bits; the line between them is cost.
+// The small ones let a workgroup's prologue and epilogue run under another's tiles, leave fewer padded rows and fill the chip with half
+// the rows, but fetch every K and V tile twice as often.  Whole calls, bf16, 256 rows / 128 rows, us:
+//   chip not filled (128 q-tiles of 256 rows and fewer): 8 heads of 2000 rows, head_dim 128, FP16 full 54.0 / 50.1, causal 54.0 / 50.1, FP8 47.1 /
+//     43.1; of 4000 89.4 / 85.6, 89.3 / 84.5, 70.0 / 64.7; head_dim 64 FP16 of 4000 65.0 / 58.4;
+//   one round of the chip, all of the same cost: two small workgroups share some compute units and not others: 12 heads of 4000 rows, full,
+//     head_dim 128 FP16 102 / 115, FP8 78 / 84; 100 of 500 45.0 / 45.0, 44.9 / 44.0; 64 of 700 43.0 / 43.7, 43.2 / 42.8; head_dim 64 FP16 64 of 700
+//     30.2 / 29.4, 48 of 1000 36.1 / 36.6, FP8 24 of 2000 41.9 / 41.9, 16 of 2800 45.3 / 45.9.  Causal tiles differ by themselves: 12 of 4000 91 / 86;
+//   several rounds, head_dim 128: FP16 full, 160 of 1400 rows 194 / 190, 128 of 2000 263 / 275; causal, 64 of 2800 157 / 155, 64 of 4000 259 / 268; FP8
+//     full 1400 173 / 159, 2000 216 / 213, 2800 187 / 191; causal 2800 135 / 132, 4000 209 / 210, 32 of 8000 315 / 329;
+//   head_dim 64, three to a compute unit: FP16 full 64 of 4000 270 / 264, 32 of 8000 480 / 482, causal 8000 275 / 264, 32 of 16000 959 / 924; FP8 full 4000
+//     204 / 194, 8000 341 / 337, causal 8000 205 / 203, 16000 665 / 657;
+//   FP8 with LSE: 2000 rows full 255 / 245, causal 187 / 173, 32 of 16000 2663 / 2503 and 1371 / 1286: at every length;
+//   packed, 32/8 heads, the length between mean and maximum: head_dim 64, causal FP16, 200 prompts of 8..300 259 / 162, 96 of 16..512 208 / 146, 16 of
+//     512..8000 1544 / 1434, 8 of 4000..16000 4345 / 4006, full FP8 5158 / 4910: always; head_dim 128, causal FP16 64 of 16..1024 424 / 370, 40 of
+//     200..2000 680 / 635, 30 of 1000..4000 1822 / 1840, FP8 1366 / 1302, 16 of 512..8000 1666 / 1661, full FP16 40 of 200..2000 988 / 972, FP8 30 of
+//     1000..4000 2124 / 2119.
+struct TileRows { int B, Hq, Sq, Skv, D, pv, causal, blkk, kgroups; bool lse, mask, packed; int total_q, total_k; };
+bool small_tiles_pay(const TileRows& c) {
+  if (c.mask || c.kgroups != 1 || c.blkk == 16) return false;   // (no such variants)
+  if (c.packed && c.total_q >= kSmallTileRows << 16) return false;   // (a plan has 16 bits for the q-tile of a sequence)
+  if (c.pv == SAGE_PV_FP8 && c.lse) return true;
+  int64_t keys = c.packed ? ((int64_t)c.total_k / c.B + c.Skv) / 2 : c.Skv;
+  const int64_t large = (int64_t)c.B * c.Hq * ((c.Sq + 255) / 256);
+  if (c.packed && c.D == 64) return true;
+  if (!c.packed && large <= 128) return true;
+  if (!c.packed && !c.causal && large <= 256) return keys <= (c.D == 64 ? (c.pv == SAGE_PV_FP8 ? 2048 : 768) : c.pv == SAGE_PV_FP8 ? 768 : 512);
+  if (c.causal) keys /= 2;
+  if (c.D == 64) return keys <= (c.causal && c.pv == SAGE_PV_FP16 ? 8192 : 4096);
+  return keys <= (c.pv == SAGE_PV_FP8 ? 1800 : 1500);
+}
+int tile_rows(const TileRows& c) { return small_tiles_pay(c) ? kSmallTileRows : kLargeTileRows; }
+// ... of the entry points that take a plan of the caller's, whose q-tiles have 256 rows.
+int public_tile_rows(int B, int Hq, int Sq, int Skv, int D, int pv_mode, int is_causal, int blkk, const float* lse, const int32_t* cu_seqlens_q) {
+  if (cu_seqlens_q) return kLargeTileRows;
+  return tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, false, false, 0, 0});
+}
+
 int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const float* q_scale, const float* k_scale,
               const float* v_scale, void* out, float* lse, int B, int Hq, int Hkv, int Sq, int Skv, int D, int64_t q_sb,
               int64_t q_sh, int64_t q_sn, int64_t k_sb, int64_t k_sh, int64_t k_sn, int64_t o_sb, int64_t o_sh,
               int64_t o_sn, int blkq, int blkk, int is_causal, int pv_mode, int out_dtype, const int32_t* cu_seqlens_q,
               const int32_t* cu_seqlens_k, const int32_t* plan, int total_q, int64_t q_scale_sh, int64_t k_scale_sh,
-              int64_t panel_sh, const MaskArg& mask, const float* lse_offset, const QRawArg& qraw, sage_stream_t stream) {
+              int64_t panel_sh, const MaskArg& mask, const float* lse_offset, const QRawArg& qraw, int tile_rows, sage_stream_t stream) {
   if (int rc = check_common(B, Hq, Sq, D, out_dtype)) return rc;
   if (Hkv <= 0 || Hq % Hkv) return fail(SAGE_EINVAL, "query heads (%d) must be divisible by KV heads (%d)", Hq, Hkv);
   if (Skv < 0) return fail(SAGE_EINVAL, "negative kv length");
@@ -263,10 +301,10 @@ int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const floa
   }
   if (packed && (!cu_seqlens_k || !plan)) return fail(SAGE_EINVAL, "packed mode needs cu_seqlens_k and plan");
   if (packed && B > 32767) return fail(SAGE_EINVAL, "too many sequences");
-  AttnConfig cfg = attn_config(D, pv_mode, packed);
-  const int BM = cfg.nw * 32;
+  const int BM = tile_rows;
   AttnArgs a;
   memset(&a, 0, sizeof(a));
+  a.tile_rows = BM;
   a.q = q; a.k = k; a.vp = (const uint8_t*)v_panels; a.qs = q_scale; a.ks = k_scale; a.vs = v_scale;
   a.out = out; a.lse = lse;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Skv = Skv;
@@ -307,7 +345,8 @@ int sage_attn_fwd(const int8_t* q, const int8_t* k, const void* v_panels, const 
                   int64_t o_sn, int blkq, int blkk, int is_causal, int pv_mode, int out_dtype, const int32_t* cu_seqlens_q,
                   const int32_t* cu_seqlens_k, const int32_t* plan, int total_q, int64_t q_scale_sh, int64_t k_scale_sh,
                   int64_t panel_sh, sage_stream_t stream) {
-  return attn_impl(q, k, v_panels, q_scale, k_scale, v_scale, out, lse, B, Hq, Hkv, Sq, Skv, D, q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, o_sb, o_sh, o_sn, blkq, blkk, is_causal, pv_mode, out_dtype, cu_seqlens_q, cu_seqlens_k, plan, total_q, q_scale_sh, k_scale_sh, panel_sh, MaskArg(), nullptr, QRawArg(), stream);
+  const int rows = public_tile_rows(B, Hq, Sq, Skv, D, pv_mode, is_causal, blkk, lse, cu_seqlens_q);
+  return attn_impl(q, k, v_panels, q_scale, k_scale, v_scale, out, lse, B, Hq, Hkv, Sq, Skv, D, q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, o_sb, o_sh, o_sn, blkq, blkk, is_causal, pv_mode, out_dtype, cu_seqlens_q, cu_seqlens_k, plan, total_q, q_scale_sh, k_scale_sh, panel_sh, MaskArg(), nullptr, QRawArg(), rows, stream);
 }
 
 int sage_attn_fwd_qfused(const void* q, int q_dtype, double sm_scale, const int8_t* k, const void* v_panels,
@@ -320,9 +359,10 @@ int sage_attn_fwd_qfused(const void* q, int q_dtype, double sm_scale, const int8
   if (!q) return fail(SAGE_EINVAL, "null tensor pointer");
   QRawArg qr;
   qr.ptr = q; qr.dtype = q_dtype; qr.mult = (float)((sm_scale > 0 ? sm_scale : 1.0 / sqrt((double)D)) * 1.44269504);
+  const int rows = public_tile_rows(B, Hq, Sq, Skv, D, pv_mode, is_causal, blkk, lse, cu_seqlens_q);
   return attn_impl(nullptr, k, v_panels, nullptr, k_scale, v_scale, out, lse, B, Hq, Hkv, Sq, Skv, D, q_sb, q_sh, q_sn, k_sb,
                    k_sh, k_sn, o_sb, o_sh, o_sn, blkq, blkk, is_causal, pv_mode, out_dtype, cu_seqlens_q, cu_seqlens_k, plan,
-                   total_q, 0, k_scale_sh, panel_sh, MaskArg(), nullptr, qr, stream);
+                   total_q, 0, k_scale_sh, panel_sh, MaskArg(), nullptr, qr, rows, stream);
 }
 
 int sage_attn_fwd_masked(const int8_t* q, const int8_t* k, const void* v_panels, const float* q_scale, const float* k_scale,
@@ -335,7 +375,7 @@ int sage_attn_fwd_masked(const int8_t* q, const int8_t* k, const void* v_panels,
   m.ptr = attn_mask; m.kind = mask_kind; m.sb = m_sb; m.sh = m_sh; m.sm = m_sm; m.sn = m_sn;
   return attn_impl(q, k, v_panels, q_scale, k_scale, v_scale, out, lse, B, Hq, Hkv, Sq, Skv, D, q_sb, q_sh, q_sn, k_sb, k_sh,
                    k_sn, o_sb, o_sh, o_sn, blkq, blkk, 0, pv_mode, out_dtype, nullptr, nullptr, nullptr, 0, 0, 0, 0, m, nullptr,
-                   QRawArg(), stream);
+                   QRawArg(), kLargeTileRows, stream);
 }
 
 // ---- one-call pipeline --------------------------------------------------------------------
@@ -684,7 +724,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   pvn.v_sb = v_sb; pvn.v_sh = v_sh; pvn.v_sn = v_sn; pvn.cu_seqlens = cu_seqlens_k; pvn.cu_panels = cu_panel; pvn.panel_sh = w.panel_sh;
   PlanArgs pl;
   memset(&pl, 0, sizeof(pl));
-  if (varlen) pl = {cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, attn_config(128, 1, true).nw * 32, 64, is_causal, plan};
+  const int bm = tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, attn_mask != nullptr, varlen != 0, total_q, total_k});
+  if (varlen) pl = {cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, bm, 64, is_causal, plan};
   // The pre-passes in two launches: what depends on nothing but the call's tensors, then what needs the statistics or the plan.  The two
   // statistics then exist at the same time; where the workspace has no room for both (it is sized for one after the other) the
   // passes follow each other.
@@ -717,8 +758,8 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     if (e != hipSuccess) return hip_fail(e, "sage_sageattn(pre-pass)");
   } else {
     if (varlen) {
-      rc = sage_varlen_plan(cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, is_causal, plan, sage_varlen_plan_ints(B, total_q), stream);
-      if (rc) return rc;
+      e = launch_varlen_plan(cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, bm, 64, is_causal, plan, st);
+      if (e != hipSuccess) return hip_fail(e, "sage_sageattn(plan)");
     }
     if (!small_prepass && smooth_k) {
       rc = sage_k_mean(k, km, stat, stat_bytes, B, Hkv, Skv, D, k_sb, k_sh, k_sn, dtype, cu_seqlens_k, stream);
@@ -742,7 +783,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   return attn_impl(q_i8, k_i8, panels, q_scale, k_scale, pv_mode == SAGE_PV_FP8 ? v_scale : nullptr, out, lse, B, Hq, Hkv, Sq,
                    Skv, D, fuse_q ? q_sb : qi_sb, fuse_q ? q_sh : qi_sh, fuse_q ? q_sn : qi_sn, ki_sb, ki_sh, ki_sn, o_sb, o_sh,
                    o_sn, blkq, blkk, is_causal, pv_mode, dtype, cu_seqlens_q, cu_seqlens_k, plan, total_q, w.qs_sh, w.ks_sh,
-                   w.panel_sh, m, lse_off, qr, stream);
+                   w.panel_sh, m, lse_off, qr, bm, stream);
 }
 
 }  // extern "C"

@@ -7,14 +7,6 @@ namespace sage {
 // ---------------------------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------------------------
-AttnConfig attn_config(int D, int pv, bool packed) {
-  (void)D; (void)packed;
-  AttnConfig c;
-  c.nw = 8;
-  c.bn = 128;
-  return c;
-}
-
 void finish_attn_args(AttnArgs& a, bool causal) {
   const bool packed = a.cu_q != nullptr;
   a.G = a.Hq / a.Hkv;
@@ -41,6 +33,7 @@ void finish_attn_args(AttnArgs& a, bool causal) {
 
 hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st) {
   if (grid == 0) return hipSuccess;
+  if (a.tile_rows == kSmallTileRows) return launch_attn_small(a, D, pv, causal, grid, st);
   if (a.mask_bits) return launch_attn_packed_mask(a, D, pv, grid, st);
   if (a.mask) return launch_attn_masked(a, D, pv, grid, st);
   if (a.k_interleave) return launch_attn_kinterleaved(a, D, pv, causal, grid, st);

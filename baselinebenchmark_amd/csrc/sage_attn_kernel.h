@@ -122,28 +122,33 @@ __device__ inline int kswz(int n) {
 // non-causal kernels from 1k to 16k keys, neutral for causal ones; three slots measured 1-2 % slower
 // than four, the slot index being a modulo in the loop).  FP16 P.V tiles are twice as large: two
 // slots, one period (three slots measured 1-3 % slower there).
-template <int PV, bool CAUSAL>
-constexpr int attn_tile_slots() { return PV == 1 ? 4 : 2; }
-template <int PV, bool CAUSAL>
-constexpr int attn_tile_lead() { return attn_tile_slots<PV, CAUSAL>() > 2 ? 2 : 1; }
+// Workgroups of four wavefronts (attn_is_small) take what still lets as many of them as the registers allow fit a compute unit: FP16 P.V
+// two K slots and one V slot, FP8 P.V two or three slots of a K and a V tile side by side (attn_is_paired).
+constexpr bool attn_is_small(int NW) { return NW == 4; }
+constexpr bool attn_is_paired(int PV, int NW) { return attn_is_small(NW) && PV == 1; }
+template <int D, int PV, int NW>
+constexpr int attn_k_slots() { return attn_is_paired(PV, NW) ? (D == 64 ? 3 : 2) : PV == 1 ? 4 : 2; }
+template <int D, int PV, int NW>
+constexpr int attn_v_slots() { return attn_is_small(NW) && PV == 0 ? 1 : attn_k_slots<D, PV, NW>(); }
+template <int D, int PV, int NW>
+constexpr int attn_tile_lead() { return attn_k_slots<D, PV, NW>() > 2 ? 2 : 1; }
 
 // Dynamic LDS of a kernel variant: the K slots and as many V slots; a kernel that quantises its own Q also
 // stages the raw q-tile behind the K slots that are requested in the prologue (over slots that are idle
 // until the main loop); FP8 kernels keep the D per-channel V scales behind all of that.
-template <int D, int NW, int BN, int PV, bool CAUSAL, bool QF>
+template <int D, int NW, int BN, int PV, bool QF>
 constexpr int attn_tile_lds_bytes() {
-  constexpr int slots = attn_tile_slots<PV, CAUSAL>();
-  constexpr int tiles = slots * (BN * D + BN * D * (PV ? 1 : 2));
-  constexpr int qstage = attn_tile_lead<PV, CAUSAL>() * BN * D + NW * 32 * D * 2;
+  constexpr int tiles = attn_k_slots<D, PV, NW>() * BN * D + attn_v_slots<D, PV, NW>() * BN * D * (PV ? 1 : 2);
+  constexpr int qstage = attn_tile_lead<D, PV, NW>() * BN * D * (attn_is_paired(PV, NW) ? 2 : 1) + NW * 32 * D * 2;
   return (QF && qstage > tiles) ? qstage : tiles;
 }
 // Kernels that follow a packed mask (MASK == 3) keep their list of visible tiles and the mask bits of the tiles in flight
 // behind that: four slots, because group 1 still reads the bits of tile j - 1 in period j while those of tile j + 1 (FP16
 // P.V) or j + 2 (FP8 P.V) arrive.
 constexpr int kMaskSlots = 4;
-template <int D, int NW, int BN, int PV, bool CAUSAL, bool QF, int MASK>
+template <int D, int NW, int BN, int PV, bool QF, int MASK>
 constexpr int attn_lds_bytes() {
-  return attn_tile_lds_bytes<D, NW, BN, PV, CAUSAL, QF>() + (PV ? D * 4 : 0) + (MASK == 3 ? kMaskSlots * kMaskTileBytes + kMaskMaxTiles * 4 : 0);
+  return attn_tile_lds_bytes<D, NW, BN, PV, QF>() + (PV ? D * 4 : 0) + (MASK == 3 ? kMaskSlots * kMaskTileBytes + kMaskMaxTiles * 4 : 0);
 }
 
 // Timing build (-DSAGE_TIMING=1, not the shipped library): every wavefront stamps eight points of its
@@ -185,9 +190,11 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 // looks its scale up), 2 for blocks of 64 keys and more, 4 for blocks of 128: the row maximum then runs one integer chain
 // per scale and the per-scale constants of the softmax are computed once (a tenth of the vector instructions of a tile).
 template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
-__global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2) : 1) attn_kernel(AttnArgs a) {
   constexpr int GSH = SAGE_GSH;   // which bit of the wavefront index picks the group
-  static_assert(NW == (2 << GSH), "the two groups pair wavefront w with w + NW/2");
+  constexpr bool SMALL = attn_is_small(NW);
+  static_assert(SMALL || NW == (2 << GSH), "the two groups pair wavefront w with w + NW/2");
+  static_assert(!SMALL || MASK == 0, "explicit masks: eight wavefronts");
   constexpr int BM = NW * 32;
   constexpr int NTHR = NW * 64;
   constexpr int KS = D / 32;   // contraction steps of S^T
@@ -199,7 +206,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   constexpr int PANEL_BYTES = kPanelRows * D * VESZ;
   constexpr int CPR = D / 16;
   constexpr float TAU = PCfg<PV>::tau, PSHIFT = PCfg<PV>::pshift;
-  constexpr int NSLOT = attn_tile_slots<PV, CAUSAL>(), LEAD = attn_tile_lead<PV, CAUSAL>();   // tiles are requested LEAD periods ahead
+  constexpr int KSLOTS = attn_k_slots<D, PV, NW>(), VSLOTS = attn_v_slots<D, PV, NW>(), LEAD = attn_tile_lead<D, PV, NW>();   // tiles are requested LEAD periods ahead
   // FP8 P.V: the softmax denominator of O always comes from the matrix pipe (the sum of the very fp8 values that
   // multiply V); MSUM additionally means that no fp32 sum is kept (no LSE wanted), and then the probabilities are
   // coded without v_exp_f32 (FASTP, see softmax).  FP16 P.V kernels instantiated with MSUM (no LSE wanted) take the sum
@@ -345,7 +352,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   const int my_row = row0 + m;
   const int kv_end = CAUSAL ? min(Lk, qt * BM + BM) : Lk;
   constexpr bool LISTED = MASK == 3;
-  uint8_t* mask_lds = smem + attn_tile_lds_bytes<D, NW, BN, PV, CAUSAL, QF>() + (PV ? D * 4 : 0);
+  uint8_t* mask_lds = smem + attn_tile_lds_bytes<D, NW, BN, PV, QF>() + (PV ? D * 4 : 0);
   int* tile_list = reinterpret_cast<int*>(mask_lds + kMaskSlots * kMaskTileBytes);
   int ntiles = (kv_end + BN - 1) / BN;
   const uint8_t* mask_bits = nullptr;
@@ -376,7 +383,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   // ---- tile loads: global memory -> LDS directly (no registers), 1 KB per wavefront instruction ----
   // Lane l of a wavefront writes LDS bytes [16*l, 16*l+16) of the 1 KB piece, so the K swizzle is
   // applied on the global side: the lane fetches the 16-byte chunk that belongs in its slot.
-  // K tiles and V tiles each rotate through NSLOT LDS slots.
+  // K tiles and V tiles each rotate through their LDS slots.
   constexpr int KPIECES = KBYTES / 1024 / NW, VPIECES = VBYTES / 1024 / NW;
   static_assert(KPIECES * 1024 * NW == KBYTES && VPIECES * 1024 * NW == VBYTES, "tile must split into 1 KB pieces per wavefront");
   // The buffer form of the LDS load is used on purpose: the compiler treats the global form as a flat
@@ -386,14 +393,15 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   auto dma16 = [&](__amdgpu_buffer_rsrc_t rsrc, int lane_offset, int uniform_offset, uint8_t* dst_uniform) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst_uniform, 16, lane_offset, uniform_offset, 0, 0);
   };
-  auto kslot = [&](int j) { return smem + (j % NSLOT) * KBYTES; };
-  auto vslot = [&](int j) { return smem + NSLOT * KBYTES + (j % NSLOT) * VBYTES; };
+  constexpr bool PAIRED = attn_is_paired(PV, NW);
+  auto kslot = [&](int j) { return smem + (j % KSLOTS) * (PAIRED ? STAGE : KBYTES); };
+  auto vslot = [&](int j) { return PAIRED ? smem + KBYTES + (j % VSLOTS) * STAGE : smem + KSLOTS * KBYTES + (j % VSLOTS) * VBYTES; };
   // Per-lane byte offsets of this wavefront's pieces inside a tile are loop invariant; the tile index
   // only adds a uniform term.  Rows past the end of the sequence (last tile only) are clamped.
   // Piece offsets are those of the lower wavefront of the SIMD pair (wl); dw selects which wavefront's pieces a
   // request covers: dw_self for this wavefront's own (prologue), 0 and PARTNER_DW for both of the pair (main
   // loop, where one wavefront issues for two).  Offsets added per request are therefore never negative.
-  constexpr int PARTNER_DW = 1 << GSH;
+  constexpr int PARTNER_DW = SMALL ? 0 : 1 << GSH;
   const int wl = w & ~PARTNER_DW, dw_self = w - wl;
   int koffv[KPIECES], voffv[VPIECES];
 #pragma unroll
@@ -434,11 +442,13 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   // The K tiles of the lead are requested before anything waits on memory, and the per-channel V scales of the epilogue
   // come along (4 bytes per lane, D / 64 wavefronts).  Kernels that quantise their own Q put the raw q-tile's requests in
   // front of these (the quantisation is what the prologue waits for; the K tiles then arrive under it).
-  float* vs_lds = reinterpret_cast<float*>(smem + attn_tile_lds_bytes<D, NW, BN, PV, CAUSAL, QF>());
+  float* vs_lds = reinterpret_cast<float*>(smem + attn_tile_lds_bytes<D, NW, BN, PV, QF>());
   // returns the number of requests this wavefront issued
   auto request_lead_tiles = [&]() -> int {
     int n = 0;
     if (ntiles > 0) { load_k(0, dw_self); n += KPIECES; }
+    if constexpr (PAIRED)
+      if (ntiles > 0) { load_v(0, dw_self); n += VPIECES; }
     if constexpr (PV == 1) {
       if (w < D / 64) {
         if (Lk > 0) {
@@ -453,7 +463,11 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     }
 #pragma unroll
     for (int t = 1; t < LEAD; t++)
-      if (t < ntiles) { load_k(t, dw_self); n += KPIECES; }
+      if (t < ntiles) {
+        load_k(t, dw_self);
+        n += KPIECES;
+        if constexpr (PAIRED) { load_v(t, dw_self); n += VPIECES; }
+      }
     return n;
   };
   // Tile loads complete in the order they were requested, so waiting until only the n newest are in
@@ -467,6 +481,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
       case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
       case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+      case 9: asm volatile("s_waitcnt vmcnt(9)" ::: "memory"); break;
       case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
       case 10: asm volatile("s_waitcnt vmcnt(10)" ::: "memory"); break;
       case 12: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
@@ -499,7 +514,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // per instruction.  16-byte units of a row are XOR-swizzled with the row index, on the global side as
     // for K.  Only this wavefront reads its region, so its own vmcnt wait is all the ordering needed.
     constexpr int QUPR = D * 2 / 16, QRPP = 64 / QUPR, QPIECES = 32 * D * 2 / 1024;
-    uint8_t* qstage = smem + LEAD * KBYTES + w * (32 * D * 2);
+    uint8_t* qstage = smem + LEAD * (PAIRED ? STAGE : KBYTES) + w * (32 * D * 2);
     // LSE of smoothed keys: the K mean of this head, whose product with the scaled row every logit of the row has lost.
     // Requested ahead of the rows themselves, which complete after it.
     [[maybe_unused]] v4u kmr[KS][2];
@@ -577,7 +592,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     SAGE_T(2, amax);   // the raw Q rows have arrived
     const int wpb = a.blkq >> 5;   // wavefronts per scale block
     if (wpb > 1) {
-      static_assert(NW == 8, "a scale block of 128 rows is one half of the wavefronts");
+      static_assert(NW == 8 || NW == 4, "a scale block of 128 rows is four wavefronts");
       if (lane == 0) q_block_amax[w] = amax;
       lds_barrier();
       const v4f half = lds_read1(lds_address(q_block_amax) + 16 * (w >> 2));
@@ -665,14 +680,15 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   [[maybe_unused]] int pscale = 0;
 
   // ---- S^T = K . Q^T (int8 -> int32 on the biased accumulators), then mask and row maximum ----
-  auto qk = [&](int j) {
+  auto qk = [&](int j, auto live) {
+    constexpr int NL = decltype(live)::value;
     const uint8_t* kbuf = kslot(j);
     // K fragments run KPF MFMAs ahead of their use so that no MFMA waits for the LDS read issued
     // just before it; the k-step is the outer index so that consecutive MFMAs hit different accumulators.
     {
-      constexpr int NF = NT * KS, KPF = SAGE_KPF;
+      constexpr int NF = NL * KS, KPF = SAGE_KPF < NF ? SAGE_KPF : NF;
       auto kfrag = [&](int i) {
-        const int nt = i % NT, ks = i / NT, n = 32 * nt + m;
+        const int nt = i % NL, ks = i / NL, n = 32 * nt + m;
         return *reinterpret_cast<const v4i*>(kbuf + n * D + 16 * ((2 * ks + h) ^ kswz<D>(n)));
       };
       v4i kf[NF];
@@ -681,7 +697,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
 #pragma unroll
       for (int i = 0; i < NF; i++) {
         if (i + KPF < NF) kf[i + KPF] = kfrag(i + KPF);
-        const int nt = i % NT, ks = i / NT;
+        const int nt = i % NL, ks = i / NL;
         acc[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[i], qreg[ks], ks == 0 ? bias : acc[nt], 0, 0, 0);
       }
       __builtin_amdgcn_sched_group_barrier(0x100, KPF, 0);
@@ -700,7 +716,9 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     for (int i = 0; i < NSC; i++) sc[i] = qscale * kscale_at(j, i);
   };
 
-  auto rowmax = [&](int j) {
+  auto rowmax = [&](int j, auto live, auto masked) {
+    constexpr int NL = decltype(live)::value;
+    static_assert(NL == NT || MASK == 0);
     const int n0 = j * BN;
     if constexpr (LISTED) {
       // Scores as in the explicit-mask variants below, the keep-mask one bit per score: bit 16 * (nt % 2) + r of word
@@ -807,8 +825,9 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       return;
     }
     // ---- masking: only tiles that cross the diagonal or the end of the sequence ----
+    // (tiles that neither can reach come without the question)
     const bool need_mask = (CAUSAL && (n0 + BN - 1 > row0)) || (n0 + BN > Lk);
-    if (need_mask) {
+    if (decltype(masked)::value && need_mask) {
       // Register r of 32-key group nt holds key n0 + 32*nt + 8*(r/4) + r%4 + 4*h: it is masked when that index
       // exceeds lim.  In causal kernels (two diagonal tiles per q-tile) the bounds of lim over the wavefront (its 32
       // rows, both lane halves) sort the groups first: most are visible or masked as a whole, and only the one the
@@ -816,7 +835,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       const int lim = (CAUSAL ? min(my_row, Lk - 1) : Lk - 1) - n0 - 4 * h;
       const int lim_hi = min(row0 + 31, Lk - 1) - n0, lim_lo = min(row0, Lk - 1) - n0 - 4;
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
+      for (int nt = 0; nt < NL; nt++) {
         if constexpr (CAUSAL) {
           if (32 * nt + 27 <= lim_lo) continue;
           if (32 * nt > lim_hi) {
@@ -841,24 +860,25 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     if constexpr (GPS > 1) {
       // groups that share a scale share one integer chain
 #pragma unroll
-      for (int g = 0; g < NSC; g++) {
+      for (int g = 0; g < (NL + GPS - 1) / GPS; g++) {
         // (one chain per 32-key group, combined at the end: independent chains issue back to back)
-        int mxg[GPS];
+        constexpr int GL = GPS < NL ? GPS : NL;
+        int mxg[GL];
 #pragma unroll
-        for (int t = 0; t < GPS; t++) {
+        for (int t = 0; t < GL; t++) {
           mxg[t] = acc[g * GPS + t][0];
 #pragma unroll
           for (int r = 1; r < 16; r++) mxg[t] = max(mxg[t], acc[g * GPS + t][r]);
         }
         int mx = mxg[0];
 #pragma unroll
-        for (int t = 1; t < GPS; t++) mx = max(mx, mxg[t]);
+        for (int t = 1; t < GL; t++) mx = max(mx, mxg[t]);
         mloc = fmaxf(mloc, __builtin_fmaf(as_f(mx), sc[g], -kBiasF * sc[g]));
       }
       return;
     }
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
+    for (int nt = 0; nt < NL; nt++) {
 #pragma unroll
       for (int sub = 0; sub < SUBS; sub++) {
         float smx;
@@ -881,7 +901,8 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   };
 
   // ---- online softmax of the tile whose scores are in acc: pure VALU work ----
-  auto softmax = [&](int j) {
+  auto softmax = [&](int j, auto live) {
+    constexpr int NL = decltype(live)::value;
     // next tile's K scales: requested first, consumed last
     float kraw[NSC];
 #pragma unroll
@@ -930,7 +951,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       const float k0 = __builtin_fmaf(-kN8, e, __builtin_fmaf(kN8, kBlockTop - m_used, kC));
       pscale = (int)(unsigned)(e + kBlockScaleBias);
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
+      for (int nt = 0; nt < NL; nt++) {
         float c[SUBS], mul[SUBS];
 #pragma unroll
         for (int sub = 0; sub < SUBS; sub++) {
@@ -947,7 +968,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       }
     } else if constexpr (PV == 1) {
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
+      for (int nt = 0; nt < NL; nt++) {
         float c[SUBS], mul[SUBS];
 #pragma unroll
         for (int sub = 0; sub < SUBS; sub++) {
@@ -971,7 +992,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       }
     } else {
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
+      for (int nt = 0; nt < NL; nt++) {
         float c[SUBS], mul[SUBS];
 #pragma unroll
         for (int sub = 0; sub < SUBS; sub++) {
@@ -998,10 +1019,12 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   };
 
   // ---- O^T += V^T . P^T ----
-  auto pv = [&](int j) {
+  auto pv = [&](int j, auto live) {
+    constexpr int NL = decltype(live)::value;
+    static_assert(PV == 0 || NL % 2 == 0, "FP8 products contract over 64 keys");
     const uint8_t* vbuf = vslot(j);
     if constexpr (PV == 1) {
-      constexpr int NV = (BN / 64) * DTN, VPF = SAGE_VPF;
+      constexpr int NV = NL / 2 * DTN, VPF = SAGE_VPF < NV ? SAGE_VPF : NV;
       auto vfrag = [&](int i) {
         const uint8_t* vp0 = vbuf + ((i * 2) * 64 + lane) * 16;
         v4i lo = *reinterpret_cast<const v4i*>(vp0);
@@ -1042,7 +1065,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
         if (i + VPF < NV) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
       }
     } else {
-      constexpr int NV = (BN / 16) * DTN, VPF = 4;
+      constexpr int NV = NL * 2 * DTN, VPF = 4;
       auto vfrag = [&](int i) { return *reinterpret_cast<const v8h*>(vbuf + (i * 64 + lane) * 16); };
       v8h vf[NV];
 #pragma unroll
@@ -1080,6 +1103,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
   // K tile j is read in phases 2j and 2j+1, V tile j in phases 2j+2 and 2j+3.
   SAGE_T(3, qreg[0]);   // Q operand ready
   if (ntiles > 0) {
+    constexpr std::integral_constant<int, NT> all{};   // 32-key groups of a tile
     const int grp = (w >> GSH) & 1;
     // Work of this wavefront on the tile of period j, and on that of period j - 1, if it sees them.  Unlisted kernels branch on
     // their tile count at every use: as a flag that is computed first and carried through the period, the condition cost the
@@ -1127,12 +1151,12 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // FP16 kernels of head_dim 128 (twelve requests per period, the V tiles being twice as large) leave the V pieces of
     // group 1's wavefronts to group 1, which requests them at the start of its matrix phase: both matrix phases then
     // carry part of the requests instead of one carrying all of them (+2 % from 4k to 16k keys).
-    constexpr bool SPLIT_REQ = PV == 0 && VECMAX;
+    constexpr bool SPLIT_REQ = !SMALL && PV == 0 && VECMAX;
     // FP8 kernels: group 0 requests the K tile of the period (after its matrix half), group 1 the V tile, as the first
     // thing it does in the period: group 0's period (matrix half, requests, vector half) is the longer one, and V
     // requests at any other place of group 1's period, or the K requests there, measured slower (+1.4 % for this one on
     // config 2, +1.7 % on config 3, +3 % at head_dim 64).
-    constexpr bool V_BY_GROUP1 = PV == 1 && LEAD == 2;
+    constexpr bool V_BY_GROUP1 = !SMALL && PV == 1 && LEAD == 2;
     static_assert(!SPLIT_REQ || LEAD == 1, "group 1 requests V(j) in period j");
     auto first_value_tile = [&]() { load_v(0, 0); load_v(0, PARTNER); };
     auto request_tiles = [&](int j, bool with_first_value = true) {
@@ -1156,7 +1180,58 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
     // it: a group that finishes its half early starts the other half at once (+1.5 % at head_dim 128, +6 % at
     // head_dim 64, where the vector half is much the longer one); FP16 P.V kernels measured equal or slower without.
     auto odd_barrier = [&]() { if constexpr (PV == 0) lds_barrier(); };
-    if constexpr (VECMAX) {
+    if constexpr (SMALL) {
+      // One tile after the other; the matrix and the vector work of a compute unit overlap because several workgroups share it.
+      auto tile_landed = [&](int j) __attribute__((always_inline)) {   // K(j), and V(j) of PAIRED; everyone is done with tile j - 1
+        wait_all_but(LEAD == 2 && j + 1 < ntiles ? KPIECES + VPIECES : 0);
+        lds_barrier();
+        if constexpr (PAIRED) {
+          if (j + LEAD < ntiles) { [[clang::always_inline]] load_k(j + LEAD, 0); [[clang::always_inline]] load_v(j + LEAD, 0); }
+        } else {
+          [[clang::always_inline]] load_v(j, 0);
+          if (j + 1 < ntiles) [[clang::always_inline]] load_k(j + 1, 0);
+        }
+      };
+      auto values_landed = [&](int j) __attribute__((always_inline)) {
+        if constexpr (!PAIRED) {
+          wait_all_but(j + 1 < ntiles ? KPIECES : 0);
+          lds_barrier();
+        }
+      };
+      auto step = [&](int j, auto live, auto masked) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_setprio(1);
+        [[clang::always_inline]] qk(j, live);
+        __builtin_amdgcn_s_setprio(0);
+        [[clang::always_inline]] rowmax(j, live, masked);
+        [[clang::always_inline]] softmax(j, live);
+        values_landed(j);
+        __builtin_amdgcn_s_setprio(1);
+        [[clang::always_inline]] pv(j, live);
+        __builtin_amdgcn_s_setprio(0);
+        // The three ways through the last tile meet in register copies of O.  The compiler counts sched_group_barrier as an instruction
+        // when it spaces such a copy from the product it reads, and came out one wait state short (two registers of a product
+        // copied before they were written): the products are waited for here, with states to spare.
+        if constexpr (decltype(masked)::value) {
+          asm volatile("s_nop 7" : "+v"(o[0]));
+#pragma unroll
+          for (int dt = 1; dt < DTN; dt++) asm volatile("" : "+v"(o[dt]));
+        }
+      };
+      const int last = ntiles - 1;
+      for (int j = 0; j < last; j++) {
+        tile_landed(j);
+        if (j < wave_ntiles) step(j, all, std::false_type());
+        else values_landed(j);
+      }
+      // The last tile is the only one that the diagonal or the end of the sequence cuts: as many of its 32-key groups as the
+      // wavefront sees (FP8 products contract over 64 keys).
+      tile_landed(last);
+      const int groups = (wave_end - last * BN + 31) >> 5;
+      if (groups > 2) step(last, all, std::true_type());
+      else if (PV == 1 ? groups > 0 : groups == 2) step(last, std::integral_constant<int, 2>(), std::true_type());
+      else if (PV == 0 && groups == 1) step(last, std::integral_constant<int, PV == 1 ? 2 : 1>(), std::true_type());
+      else values_landed(last);
+    } else if constexpr (VECMAX) {
       // FP8 P.V, and FP16 P.V of head_dim 128: the matrix half is nothing but MFMAs and their LDS reads (P.V of the
       // previous tile, Q.K^T of the next); the row maximum and the probabilities belong to the vector half.  Group 0
       // issues its tile requests, for both wavefronts of each SIMD pair, after its last Q.K^T MFMA (a request holds up
@@ -1168,13 +1243,13 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
           SAGE_PH(0);
           if (LEAD == 2 && j == 0) first_value_tile();   // V(0) has one period only: ahead of the first Q.K^T, not after it
           enter(j);
-          if_was_on(j, [&, j] { pv(j - 1); }, nothing);
-          if_on(j, [&, j] { qk(j); }, forget_scores);
+          if_was_on(j, [&, j] { pv(j - 1, all); }, nothing);
+          if_on(j, [&, j] { qk(j, all); }, forget_scores);
           request_tiles(j, false);
           SAGE_PH(1);
           odd_barrier();
           SAGE_PH(2);
-          if_on(j, [&, j] { rowmax(j); softmax(j); }, [&, j] { load_scales(j + 1); });   // (a skipped tile's softmax would have fetched them)
+          if_on(j, [&, j] { rowmax(j, all, std::true_type()); softmax(j, all); }, [&, j] { load_scales(j + 1); });   // (a skipped tile's softmax would have fetched them)
         }
       } else {
         for (int j = 0; j <= ntiles; j++) {
@@ -1184,13 +1259,13 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
           SAGE_PH(0);
           if (V_BY_GROUP1 && j + 1 < ntiles) { load_v(j + 1, 0); load_v(j + 1, PARTNER); }
           enter(j);
-          if_was_on(j, [&, j] { rowmax(j - 1); softmax(j - 1); }, [&, j] { load_scales(j); });
+          if_was_on(j, [&, j] { rowmax(j - 1, all, std::true_type()); softmax(j - 1, all); }, [&, j] { load_scales(j); });
           SAGE_PH(1);
           odd_barrier();
           SAGE_PH(2);
           if (SPLIT_REQ && j < ntiles) load_v(j, PARTNER);   // V(j) of the pair's second wavefront: LEAD is 1 here
-          if_was_on(j, [&, j] { pv(j - 1); }, nothing);
-          if_on(j, [&, j] { qk(j); }, forget_scores);
+          if_was_on(j, [&, j] { pv(j - 1, all); }, nothing);
+          if_on(j, [&, j] { qk(j, all); }, forget_scores);
         }
       }
     } else if (grp == 0) {
@@ -1199,20 +1274,20 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
       for (int j = 0; j <= ntiles; j++) {
         even_barrier(j, issuer_in_flight(j));
         enter(j);
-        if_was_on(j, [&, j] { pv(j - 1); }, nothing);
+        if_was_on(j, [&, j] { pv(j - 1, all); }, nothing);
         request_tiles(j);
-        if_on(j, [&, j] { qk(j); rowmax(j); }, forget_scores);
+        if_on(j, [&, j] { qk(j, all); rowmax(j, all, std::true_type()); }, forget_scores);
         lds_barrier();
-        if_on(j, [&, j] { softmax(j); }, [&, j] { load_scales(j + 1); });
+        if_on(j, [&, j] { softmax(j, all); }, [&, j] { load_scales(j + 1); });
       }
     } else {
       for (int j = 0; j <= ntiles; j++) {
         even_barrier(j, j == 0 ? first_in_flight : 0);
         enter(j);
-        if_was_on(j, [&, j] { softmax(j - 1); }, [&, j] { load_scales(j); });
+        if_was_on(j, [&, j] { softmax(j - 1, all); }, [&, j] { load_scales(j); });
         lds_barrier();
-        if_was_on(j, [&, j] { pv(j - 1); }, nothing);
-        if_on(j, [&, j] { qk(j); rowmax(j); }, forget_scores);
+        if_was_on(j, [&, j] { pv(j - 1, all); }, nothing);
+        if_on(j, [&, j] { qk(j, all); rowmax(j, all, std::true_type()); }, forget_scores);
       }
     }
   }
@@ -1324,7 +1399,7 @@ __global__ void __launch_bounds__(NW * 64) attn_kernel(AttnArgs a) {
 
 template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
 static hipError_t launch_one(const AttnArgs& a, int grid, hipStream_t st) {
-  constexpr int smem = attn_lds_bytes<D, NW, BN, PV, CAUSAL, QF, MASK>();
+  constexpr int smem = attn_lds_bytes<D, NW, BN, PV, QF, MASK>();
   auto kern = attn_kernel<D, NW, BN, PV, CAUSAL, MSUM, MASK, KSUB, QF, KW, DOT>;
   // More than 64 KB of dynamic LDS has to be allowed once per kernel and device.
   constexpr int kMaxDevices = 64;

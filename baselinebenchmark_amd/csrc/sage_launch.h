@@ -195,9 +195,10 @@ struct AttnArgs {
   const uint8_t* mask_bits; // packed boolean mask (sage_common.h) or null: taken instead of `mask`
   const uint8_t* mask_seen;
   int mask_pb, mask_ph, mask_nqt, mask_ntk;
+  int tile_rows;            // query rows per workgroup; host-side dispatch only
 };
 
-struct AttnConfig { int nw, bn; };
+constexpr int kLargeTileRows = 256, kSmallTileRows = 128;   // query rows per workgroup: eight or four wavefronts of 32
 
 hipError_t launch_quant_int8(const QuantArgs& a, int dtype, int max_rows, hipStream_t st);
 int colstat_chunks(int L);
@@ -231,10 +232,10 @@ hipError_t launch_fused_prepass(const FusedPrepass& f, int dtype, int D, int pv,
 hipError_t launch_k_mean_finalize(const ColStatArgs& a, int dtype, void* km, hipStream_t st);
 hipError_t launch_v_scale_finalize(const ColStatArgs& a, float* vscale, hipStream_t st);
 
-AttnConfig attn_config(int D, int pv, bool packed);
 // Fills in the launch constants of the tile decode from the dimensions already in `a` (B, Hq, Hkv, nqt, cu_q).
 void finish_attn_args(AttnArgs& a, bool causal);
 hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
+hipError_t launch_attn_small(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_masked(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_masked_wide(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_packed_mask(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);

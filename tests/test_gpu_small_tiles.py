@@ -1,0 +1,47 @@
+"""Attention in workgroups of 128 query rows (four wavefronts): sequence ends and diagonals at every edge of a 32-key group."""
+import pytest
+import torch
+
+import baselinebenchmark_amd as sa
+from oracle import attention as oa
+from tests.helpers import randn
+
+pytestmark = [pytest.mark.gpu, pytest.mark.sage_attention]
+DEV = "cuda"
+EDGES = [1, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 160, 161, 255, 256, 257, 384, 385]
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_every_end_of_a_tile_matches_the_formula(D, pv, causal):
+    # tolerances of test_gpu_attention.py: FP16 P.V relative RMSE 2e-3, FP8 5e-2 (e4m3), LSE2 1e-3
+    for Skv in EDGES:
+        Sq = Skv if causal else 130
+        g = torch.Generator().manual_seed(11 * Skv + D)
+        q, k, v = (randn("HND", 1, 2, n, D, torch.float16, g) for n in (Sq, Skv, Skv))
+        qi, qs, ki, ks = sa.per_block_int8(q.to(DEV), k.to(DEV), BLKQ=64, BLKK=32)
+        ref, ref_lse = oa.sage_reference(qi.cpu(), ki.cpu(), v, qs.cpu(), ks.cpu(), "HND", 64, 32, is_causal=causal)
+        kw = dict(output_dtype=torch.float16, BLKQ=64, BLKK=32, is_causal=causal, pv_mode=pv)
+        for lse in (False, True):
+            out, l2 = sa.forward(qi, ki, v.to(DEV), qs, ks, return_lse=lse, **kw)
+            m = oa.metrics(out.cpu().float(), ref)
+            assert m["finite"] and m["rel_rmse"] < (2e-3 if pv == "fp16" else 5e-2), (Skv, lse, m)
+            if lse:
+                assert (l2.cpu().double() - ref_lse).abs().max().item() < 1e-3, Skv
+        assert torch.equal(sa.forward_fused_q(q.to(DEV), ki, v.to(DEV), ks, **kw)[0], sa.forward(qi, ki, v.to(DEV), qs, ks, **kw)[0]), Skv
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("blkk", [32, 64, 128])
+def test_packed_batches_get_the_same_bits_from_128_and_256_rows(blkk, pv, causal):
+    # head_dim 128: a bound on the lengths far above them makes the call take the workgroups of 256 rows
+    T, H, D = sum(EDGES), 4, 128
+    cu = torch.tensor([sum(EDGES[:i]) for i in range(len(EDGES) + 1)], dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn((T, h, D), generator=g).to(torch.bfloat16).to(DEV) for h in (H, 2, 2))
+    kw = dict(is_causal=causal, pv_mode=pv, BLKQ=128, BLKK=blkk)
+    small = sa.sageattn_varlen(q, k, v, cu, cu, max(EDGES), max(EDGES), **kw)
+    large = sa.sageattn_varlen(q, k, v, cu, cu, 8192, 8192, **kw)
+    assert torch.isfinite(small.float()).all() and torch.equal(small, large)
