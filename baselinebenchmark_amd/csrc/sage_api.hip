@@ -239,17 +239,23 @@ struct MaskArg {
 //   packed, 32/8 heads, the length between mean and maximum: head_dim 64, causal FP16, 200 prompts of 8..300 259 / 162, 96 of 16..512 208 / 146, 16 of
 //     512..8000 1544 / 1434, 8 of 4000..16000 4345 / 4006, full FP8 5158 / 4910: always; head_dim 128, causal FP16 64 of 16..1024 424 / 370, 40 of
 //     200..2000 680 / 635, 30 of 1000..4000 1822 / 1840, FP8 1366 / 1302, 16 of 512..8000 1666 / 1661, full FP16 40 of 200..2000 988 / 972, FP8 30 of
-//     1000..4000 2124 / 2119.
-struct TileRows { int B, Hq, Sq, Skv, D, pv, causal, blkk, kgroups; bool lse, mask, packed; int total_q, total_k; };
+//     1000..4000 2124 / 2119;
+//   masks: one bias per head, 2 x 16 heads of 1000 rows, head_dim 64 69 / 49, 128 82 / 60, 1 x 4 of 6000 325 / 211, 363 / 232; documents, head_dim 64, 2
+//     x 16 of 1500 53 / 50, 4 x 32 123 / 110, FP8 128 1 x 32 of 2200 133 / 101; padding, head_dim 64, 1 x 32 of 2200 109 / 85, but, head_dim 128, FP16,
+//     in one round of the chip, 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), of 1000 52 / 48, and in three whole ones, 4 x 32 of 1500, 195 / 200.
+enum MaskClass { kNoMask, kKeepMask, kBiasMask, kOtherMask };   // boolean (in bits, or contiguous keys), additive with contiguous keys, other strides
+struct TileRows { int B, Hq, Sq, Skv, D, pv, causal, blkk, kgroups; bool lse; MaskClass mask; bool packed; int total_q, total_k; };
 bool small_tiles_pay(const TileRows& c) {
-  if (c.mask || c.kgroups != 1 || c.blkk == 16) return false;   // (no such variants)
+  if (c.mask == kOtherMask || c.kgroups != 1 || c.blkk == 16) return false;   // (no such variants)
   if (c.packed && c.total_q >= kSmallTileRows << 16) return false;   // (a plan has 16 bits for the q-tile of a sequence)
   if (c.pv == SAGE_PV_FP8 && c.lse) return true;
+  if (c.mask != kNoMask && !(c.mask == kKeepMask && c.D == 128 && c.pv == SAGE_PV_FP16)) return true;
   int64_t keys = c.packed ? ((int64_t)c.total_k / c.B + c.Skv) / 2 : c.Skv;
   const int64_t large = (int64_t)c.B * c.Hq * ((c.Sq + 255) / 256);
   if (c.packed && c.D == 64) return true;
   if (!c.packed && large <= 128) return true;
   if (!c.packed && !c.causal && large <= 256) return keys <= (c.D == 64 ? (c.pv == SAGE_PV_FP8 ? 2048 : 768) : c.pv == SAGE_PV_FP8 ? 768 : 512);
+  if (c.mask != kNoMask) return keys <= 1024 || large <= 512;
   if (c.causal) keys /= 2;
   if (c.D == 64) return keys <= (c.causal && c.pv == SAGE_PV_FP16 ? 8192 : 4096);
   return keys <= (c.pv == SAGE_PV_FP8 ? 1800 : 1500);
@@ -258,7 +264,13 @@ int tile_rows(const TileRows& c) { return small_tiles_pay(c) ? kSmallTileRows : 
 // ... of the entry points that take a plan of the caller's, whose q-tiles have 256 rows.
 int public_tile_rows(int B, int Hq, int Sq, int Skv, int D, int pv_mode, int is_causal, int blkk, const float* lse, const int32_t* cu_seqlens_q) {
   if (cu_seqlens_q) return kLargeTileRows;
-  return tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, false, false, 0, 0});
+  return tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, kNoMask, false, 0, 0});
+}
+
+MaskClass mask_class(const MaskArg& m, int Skv) {
+  if (!m.ptr) return kNoMask;
+  if (!m.bits && !mask_is_wide(m.sn, m.kind, Skv)) return kOtherMask;
+  return m.kind == SAGE_MASK_BOOL ? kKeepMask : kBiasMask;
 }
 
 int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const float* q_scale, const float* k_scale,
@@ -373,9 +385,10 @@ int sage_attn_fwd_masked(const int8_t* q, const int8_t* k, const void* v_panels,
   if (!attn_mask) return fail(SAGE_EINVAL, "null mask");
   MaskArg m;
   m.ptr = attn_mask; m.kind = mask_kind; m.sb = m_sb; m.sh = m_sh; m.sm = m_sm; m.sn = m_sn;
+  const int rows = tile_rows({B, Hq, Sq, Skv, D, pv_mode, 0, blk_rows(blkk), blk_groups(blkk), lse != nullptr, mask_class(m, Skv), false, 0, 0});
   return attn_impl(q, k, v_panels, q_scale, k_scale, v_scale, out, lse, B, Hq, Hkv, Sq, Skv, D, q_sb, q_sh, q_sn, k_sb, k_sh,
                    k_sn, o_sb, o_sh, o_sn, blkq, blkk, 0, pv_mode, out_dtype, nullptr, nullptr, nullptr, 0, 0, 0, 0, m, nullptr,
-                   QRawArg(), kLargeTileRows, stream);
+                   QRawArg(), rows, stream);
 }
 
 // ---- one-call pipeline --------------------------------------------------------------------
@@ -724,7 +737,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   pvn.v_sb = v_sb; pvn.v_sh = v_sh; pvn.v_sn = v_sn; pvn.cu_seqlens = cu_seqlens_k; pvn.cu_panels = cu_panel; pvn.panel_sh = w.panel_sh;
   PlanArgs pl;
   memset(&pl, 0, sizeof(pl));
-  const int bm = tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, attn_mask != nullptr, varlen != 0, total_q, total_k});
+  const int bm = tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, mask_class(m, Skv), varlen != 0, total_q, total_k});
   if (varlen) pl = {cu_seqlens_q, cu_seqlens_k, B, total_q, blkq, blkk, bm, 64, is_causal, plan};
   // The pre-passes in two launches: what depends on nothing but the call's tensors, then what needs the statistics or the plan.  The two
   // statistics then exist at the same time; where the workspace has no room for both (it is sized for one after the other) the

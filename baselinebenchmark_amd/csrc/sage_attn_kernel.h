@@ -144,11 +144,13 @@ constexpr int attn_tile_lds_bytes() {
 }
 // Kernels that follow a packed mask (MASK == 3) keep their list of visible tiles and the mask bits of the tiles in flight
 // behind that: four slots, because group 1 still reads the bits of tile j - 1 in period j while those of tile j + 1 (FP16
-// P.V) or j + 2 (FP8 P.V) arrive.
-constexpr int kMaskSlots = 4;
+// P.V) or j + 2 (FP8 P.V) arrive; workgroups of four wavefronts as many as K slots, of half a mask tile each.
+template <int D, int PV, int NW>
+constexpr int attn_mask_slots() { return attn_is_small(NW) ? attn_k_slots<D, PV, NW>() : 4; }
+constexpr int attn_mask_tile_bytes(int NW) { return kMaskTileBytes / kMaskRows * 32 * NW; }
 template <int D, int NW, int BN, int PV, bool QF, int MASK>
 constexpr int attn_lds_bytes() {
-  return attn_tile_lds_bytes<D, NW, BN, PV, QF>() + (PV ? D * 4 : 0) + (MASK == 3 ? kMaskSlots * kMaskTileBytes + kMaskMaxTiles * 4 : 0);
+  return attn_tile_lds_bytes<D, NW, BN, PV, QF>() + (PV ? D * 4 : 0) + (MASK == 3 ? attn_mask_slots<D, PV, NW>() * attn_mask_tile_bytes(NW) + kMaskMaxTiles * 4 : 0);
 }
 
 // Timing build (-DSAGE_TIMING=1, not the shipped library): every wavefront stamps eight points of its
@@ -190,11 +192,10 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 // looks its scale up), 2 for blocks of 64 keys and more, 4 for blocks of 128: the row maximum then runs one integer chain
 // per scale and the per-scale constants of the softmax are computed once (a tenth of the vector instructions of a tile).
 template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
-__global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2) : 1) attn_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 && (MASK == 0 || MASK == 3) ? 3 : 2) : 1) attn_kernel(AttnArgs a) {
   constexpr int GSH = SAGE_GSH;   // which bit of the wavefront index picks the group
   constexpr bool SMALL = attn_is_small(NW);
   static_assert(SMALL || NW == (2 << GSH), "the two groups pair wavefront w with w + NW/2");
-  static_assert(!SMALL || MASK == 0, "explicit masks: eight wavefronts");
   constexpr int BM = NW * 32;
   constexpr int NTHR = NW * 64;
   constexpr int KS = D / 32;   // contraction steps of S^T
@@ -353,19 +354,22 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2)
   const int kv_end = CAUSAL ? min(Lk, qt * BM + BM) : Lk;
   constexpr bool LISTED = MASK == 3;
   uint8_t* mask_lds = smem + attn_tile_lds_bytes<D, NW, BN, PV, QF>() + (PV ? D * 4 : 0);
-  int* tile_list = reinterpret_cast<int*>(mask_lds + kMaskSlots * kMaskTileBytes);
+  constexpr int MSLOTS = attn_mask_slots<D, PV, NW>(), MBYTES = attn_mask_tile_bytes(NW);
+  int* tile_list = reinterpret_cast<int*>(mask_lds + MSLOTS * MBYTES);
   int ntiles = (kv_end + BN - 1) / BN;
   const uint8_t* mask_bits = nullptr;
   if constexpr (LISTED) {
     // The tiles this workgroup has to visit, in order: tile index | which of its eight 32-row groups see it << 16.
     // Every wavefront writes the same list (and reads back only what it wrote itself), so no barrier is needed.
-    const int64_t qtile = (int64_t)(b * a.mask_pb + hq_idx * a.mask_ph) * a.mask_nqt + (a.mask_nqt > 1 ? qt : 0);
+    constexpr int PART = kMaskRows / BM;   // workgroups to a q-tile of the mask
+    const int part = qt % PART;
+    const int64_t qtile = (int64_t)(b * a.mask_pb + hq_idx * a.mask_ph) * a.mask_nqt + (a.mask_nqt > 1 ? qt / PART : 0);
     const uint8_t* seen = a.mask_seen + qtile * a.mask_ntk;
-    mask_bits = a.mask_bits + qtile * a.mask_ntk * kMaskTileBytes;
+    mask_bits = a.mask_bits + qtile * a.mask_ntk * kMaskTileBytes + part * MBYTES;
     int n = 0;
     for (int t0 = 0; t0 < a.mask_ntk; t0 += 64) {
       const int t = t0 + lane;
-      const int c = t < a.mask_ntk ? seen[t] : 0;
+      const int c = t < a.mask_ntk ? (PART == 1 ? seen[t] : seen[t] >> NW * part & ((1 << NW) - 1)) : 0;
       const unsigned long long on = __builtin_amdgcn_ballot_w64(c != 0);
       if (c != 0) tile_list[n + __popcll(on & ((1ull << lane) - 1))] = t | (c << 16);
       n += __popcll(on);
@@ -414,13 +418,13 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2)
   const int ktile_bytes = BN * (int)a.k_sn;
   // dw is a multiple of 4, so the rows move by a multiple of 16 and keep their swizzle: only the uniform offset changes.
   [[maybe_unused]] const __amdgpu_buffer_rsrc_t mrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)mask_bits, 0, 0x7fffffff, 0x00020000);
-  auto mslot = [&](int j) { return mask_lds + (j % kMaskSlots) * kMaskTileBytes; };
+  auto mslot = [&](int j) { return mask_lds + (j % MSLOTS) * MBYTES; };
   auto load_k = [&](int period, int dw) {
     uint8_t* dst = kslot(period) + dw * 1024;
     const int j = tile_at(period);
-    // (the mask bits of the tile: four 1 KB pieces, one each for the wavefronts of group 0)
+    // (the mask bits of the tile: 1 KB pieces, one each for the wavefronts of the lower half)
     if constexpr (LISTED)
-      if (dw == 0) dma16(mrsrc, wl * 1024 + lane * 16, j * kMaskTileBytes, mslot(period) + wl * 1024);
+      if (SMALL ? w < NW / 2 : dw == 0) dma16(mrsrc, wl * 1024 + lane * 16, j * kMaskTileBytes, mslot(period) + wl * 1024);
     if (j * BN + BN <= Lk) {
       const int uo = j * ktile_bytes + dw * (64 / CPR) * (int)a.k_sn;
 #pragma unroll
@@ -1182,8 +1186,9 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2)
     auto odd_barrier = [&]() { if constexpr (PV == 0) lds_barrier(); };
     if constexpr (SMALL) {
       // One tile after the other; the matrix and the vector work of a compute unit overlap because several workgroups share it.
+      const int k_requests = KPIECES + (LISTED && w < NW / 2);   // of this wavefront for a K tile (and its mask bits)
       auto tile_landed = [&](int j) __attribute__((always_inline)) {   // K(j), and V(j) of PAIRED; everyone is done with tile j - 1
-        wait_all_but(LEAD == 2 && j + 1 < ntiles ? KPIECES + VPIECES : 0);
+        wait_all_but(LEAD == 2 && j + 1 < ntiles ? k_requests + VPIECES : 0);
         lds_barrier();
         if constexpr (PAIRED) {
           if (j + LEAD < ntiles) { [[clang::always_inline]] load_k(j + LEAD, 0); [[clang::always_inline]] load_v(j + LEAD, 0); }
@@ -1194,7 +1199,7 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2)
       };
       auto values_landed = [&](int j) __attribute__((always_inline)) {
         if constexpr (!PAIRED) {
-          wait_all_but(j + 1 < ntiles ? KPIECES : 0);
+          wait_all_but(j + 1 < ntiles ? k_requests : 0);
           lds_barrier();
         }
       };
@@ -1217,6 +1222,17 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2)
           for (int dt = 1; dt < DTN; dt++) asm volatile("" : "+v"(o[dt]));
         }
       };
+      if constexpr (MASK != 0) {
+        for (int j = 0; j < ntiles; j++) {
+          const bool on = LISTED ? sees(j) : j < wave_ntiles;
+          tile_landed(j);
+          if (on) step(j, all, std::true_type());
+          else {
+            values_landed(j);
+            if constexpr (LISTED) load_scales(j + 1);   // (a skipped tile's softmax would have fetched them)
+          }
+        }
+      } else {
       const int last = ntiles - 1;
       for (int j = 0; j < last; j++) {
         tile_landed(j);
@@ -1231,6 +1247,7 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 ? 3 : 2)
       else if (PV == 1 ? groups > 0 : groups == 2) step(last, std::integral_constant<int, 2>(), std::true_type());
       else if (PV == 0 && groups == 1) step(last, std::integral_constant<int, PV == 1 ? 2 : 1>(), std::true_type());
       else values_landed(last);
+      }
     } else if constexpr (VECMAX) {
       // FP8 P.V, and FP16 P.V of head_dim 128: the matrix half is nothing but MFMAs and their LDS reads (P.V of the
       // previous tile, Q.K^T of the next); the row maximum and the probabilities belong to the vector half.  Group 0

@@ -12,7 +12,7 @@ namespace sage {
 // less than one whole key tile stay here too (500 rows, 77 keys, head_dim 64, FP8 P.V: 21.4 us here, 24 there); boolean ones of
 // that size measure the same or better there (21.2 / 22.0, FP16 P.V 15.3 / 16.4).
 hipError_t launch_attn_masked(const AttnArgs& a, int D, int pv, int grid, hipStream_t st) {
-  if (a.m_sn == 1 && (a.mask_kind == 1 || a.Skv >= 128)) return launch_attn_masked_wide(a, D, pv, grid, st);
+  if (mask_is_wide(a.m_sn, a.mask_kind, a.Skv)) return launch_attn_masked_wide(a, D, pv, grid, st);
   // K scale granularity: one scale per 32-key group or coarser, two per group (K blocks of 16 keys), or four interleaved
   // scales per block -- the masked kernels turn the accumulators into scores element by element and look the scale of
   // every element up, so the finer granularities only change that lookup.

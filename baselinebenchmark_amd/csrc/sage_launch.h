@@ -236,6 +236,8 @@ hipError_t launch_v_scale_finalize(const ColStatArgs& a, float* vscale, hipStrea
 void finish_attn_args(AttnArgs& a, bool causal);
 hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
 hipError_t launch_attn_small(const AttnArgs& a, int D, int pv, bool causal, int grid, hipStream_t st);
+// Masks that the kernels of sage_attn_maskwide.hip take, rather than those of sage_attn_mask.hip (which gives the reasons).
+inline bool mask_is_wide(int64_t m_sn, int kind, int Skv) { return m_sn == 1 && (kind == 1 || Skv >= 128); }
 hipError_t launch_attn_masked(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_masked_wide(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);
 hipError_t launch_attn_packed_mask(const AttnArgs& a, int D, int pv, int grid, hipStream_t st);

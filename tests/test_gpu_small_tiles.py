@@ -45,3 +45,24 @@ def test_packed_batches_get_the_same_bits_from_128_and_256_rows(blkk, pv, causal
     small = sa.sageattn_varlen(q, k, v, cu, cu, max(EDGES), max(EDGES), **kw)
     large = sa.sageattn_varlen(q, k, v, cu, cu, 8192, 8192, **kw)
     assert torch.isfinite(small.float()).all() and torch.equal(small, large)
+
+
+@pytest.mark.parametrize("kind", ["keep", "keep_rows_alike", "bias"])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_masks_get_the_same_bits_from_128_and_256_rows(D, pv, kind):
+    # a mask whose keys are not contiguous makes the call take the workgroups of 256 rows; sageattn packs a boolean one into bits
+    for Sq, Skv in [(1, 128), (33, 300), (128, 127), (129, 385), (200, 129), (256, 500), (257, 640), (400, 1100)]:
+        g = torch.Generator().manual_seed(Sq + Skv)
+        q, k, v = (randn("HND", 2, 2, n, D, torch.bfloat16, g).to(DEV) for n in (Sq, Skv, Skv))
+        shape = (2, 1, 1 if kind == "keep_rows_alike" else Sq, Skv)
+        mask = torch.randn(shape, generator=g).to(DEV) if kind == "bias" else (torch.rand(shape, generator=g) < 0.6).to(DEV)
+        spread = torch.zeros((*shape, 2), dtype=mask.dtype, device=DEV)
+        spread[..., 0] = mask
+        qi, qs, ki, ks = sa.per_block_int8(q, k, BLKQ=64, BLKK=64)
+        kw = dict(output_dtype=torch.bfloat16, BLKQ=64, BLKK=64, pv_mode=pv, return_lse=True)
+        small, large = (sa.forward(qi, ki, v, qs, ks, attn_mask=m, **kw) for m in (mask, spread[..., 0]))
+        assert torch.equal(small[0], large[0]) and torch.equal(small[1], large[1]), (Sq, Skv)
+        if kind != "bias":
+            packed = sa.sageattn(q, k, v, attn_mask=mask, smooth_k=False, pv_mode=pv, BLKQ=64, BLKK=64)
+            assert torch.equal(packed, large[0]), (Sq, Skv)
