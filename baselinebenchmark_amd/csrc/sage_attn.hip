@@ -35,9 +35,9 @@ hipError_t launch_attn(const AttnArgs& a, int D, int pv, bool causal, int grid, 
   if (grid == 0) return hipSuccess;
   if (a.mask_bits) return launch_attn_packed_mask(a, D, pv, grid, st);
   if (a.mask) return launch_attn_masked(a, D, pv, grid, st);
-  if (a.tile_rows == kSmallTileRows) return launch_attn_small(a, D, pv, causal, grid, st);
   if (a.k_interleave) return launch_attn_kinterleaved(a, D, pv, causal, grid, st);
   if (a.blkk == 16) return launch_attn_k16(a, D, pv, causal, grid, st);
+  if (a.tile_rows == kSmallTileRows) return launch_attn_small(a, D, pv, causal, grid, st);
   if (a.q_raw) return launch_attn_qfused(a, D, pv, causal, grid, st);
   // Row sums on the matrix pipe unless LSE is wanted (FP16 P.V: only head_dim 64 gains by it; head_dim 128 is
   // bound by its matrix phases and keeps the sums on the vector ALU).

@@ -1,5 +1,6 @@
 // Fused attention kernel variants of four wavefronts (128 query rows to a workgroup), for short sequences and calls that do not fill the
-// chip (the rule: small_tiles_pay in sage_api.hip; those with an explicit mask: sage_attn_maskbits.hip, sage_attn_maskwide.hip).  Own translation unit so that the sets of instantiations compile in parallel.
+// chip (the rule: small_tiles_pay in sage_api.hip; those with an explicit mask, K blocks of 16 keys or interleaved K scales stand beside their
+// larger brothers).  Own translation unit so that the sets of instantiations compile in parallel.
 //
 // With eight wavefronts a workgroup takes a compute unit for itself, and the 9 us that a q-tile spends on its addresses, raw rows,
 // quantisation and output run beside nothing; at 1000 keys that is half of its time.  Four wavefronts use half the registers and

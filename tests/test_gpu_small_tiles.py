@@ -14,15 +14,16 @@ EDGES = [1, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 160, 161, 255, 256, 257, 
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("pv", ["fp16", "fp8"])
 @pytest.mark.parametrize("D", [64, 128])
-def test_every_end_of_a_tile_matches_the_formula(D, pv, causal):
+@pytest.mark.parametrize("blkk", [16, 32])
+def test_every_end_of_a_tile_matches_the_formula(blkk, D, pv, causal):
     # tolerances of test_gpu_attention.py: FP16 P.V relative RMSE 2e-3, FP8 5e-2 (e4m3), LSE2 1e-3
     for Skv in EDGES:
         Sq = Skv if causal else 130
         g = torch.Generator().manual_seed(11 * Skv + D)
         q, k, v = (randn("HND", 1, 2, n, D, torch.float16, g) for n in (Sq, Skv, Skv))
-        qi, qs, ki, ks = sa.per_block_int8(q.to(DEV), k.to(DEV), BLKQ=64, BLKK=32)
-        ref, ref_lse = oa.sage_reference(qi.cpu(), ki.cpu(), v, qs.cpu(), ks.cpu(), "HND", 64, 32, is_causal=causal)
-        kw = dict(output_dtype=torch.float16, BLKQ=64, BLKK=32, is_causal=causal, pv_mode=pv)
+        qi, qs, ki, ks = sa.per_block_int8(q.to(DEV), k.to(DEV), BLKQ=64, BLKK=blkk)
+        ref, ref_lse = oa.sage_reference(qi.cpu(), ki.cpu(), v, qs.cpu(), ks.cpu(), "HND", 64, blkk, is_causal=causal)
+        kw = dict(output_dtype=torch.float16, BLKQ=64, BLKK=blkk, is_causal=causal, pv_mode=pv)
         for lse in (False, True):
             out, l2 = sa.forward(qi, ki, v.to(DEV), qs, ks, return_lse=lse, **kw)
             m = oa.metrics(out.cpu().float(), ref)
@@ -45,6 +46,22 @@ def test_packed_batches_get_the_same_bits_from_128_and_256_rows(blkk, pv, causal
     small = sa.sageattn_varlen(q, k, v, cu, cu, max(EDGES), max(EDGES), **kw)
     large = sa.sageattn_varlen(q, k, v, cu, cu, 8192, 8192, **kw)
     assert torch.isfinite(small.float()).all() and torch.equal(small, large)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("pv", ["fp16", "fp8"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_interleaved_k_scales_match_the_formula_at_every_end_of_a_tile(D, pv, causal):
+    for Skv in EDGES:
+        Sq = Skv if causal else 130
+        g = torch.Generator().manual_seed(7 * Skv + D)
+        q, k, v = (randn("HND", 1, 2, n, D, torch.float16, g) for n in (Sq, Skv, Skv))
+        qi, qs, ki, ks = sa.per_block_int8(q.to(DEV), k.to(DEV), BLKQ=32, BLKK=64, k_interleave=4)
+        out, _ = sa.forward(qi, ki, v.to(DEV), qs, ks, output_dtype=torch.float16, BLKQ=32, BLKK=64, is_causal=causal, pv_mode=pv, k_interleave=4)
+        n = torch.arange(Skv)
+        ref, _ = oa.sage_reference(qi.cpu(), ki.cpu(), v, qs.cpu(), ks.cpu()[..., (n // 64) * 4 + (n % 8) // 2], "HND", 32, 1, is_causal=causal)
+        m = oa.metrics(out.cpu().float(), ref)
+        assert m["finite"] and m["rel_rmse"] < (2e-3 if pv == "fp16" else 5e-2), (Skv, m)
 
 
 @pytest.mark.parametrize("kind", ["keep", "keep_rows_alike", "bias"])
