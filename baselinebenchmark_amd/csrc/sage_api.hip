@@ -72,6 +72,20 @@ const char* sage_last_error(void) { return g_err; }
 }  // extern "C"
 
 namespace {
+constexpr int64_t kStatElements = (int64_t)56 << 20, kInputElements = (int64_t)20 << 20;
+// What is read past the caches is faster by itself (sage_common.h) but found in none of them again.  Up to kStatElements elements, the
+// tensors that a call takes statistics of are read through the caches: the quantiser, the panels or the few-rows kernel then find part of them in
+// the last-level cache (256 MB).  Whole calls, bf16, past / through, us: 1 row, 32/8 heads, 8192 keys, K of 34 MB 30.9 / 29.7, 67 MB 48.6 / 47.8, 100 MB 82.2 /
+// 79.4, 268 MB 149 / 153; 32 heads of 4096 rows (34 MB), FP16 P.V 142 / 140, FP8 (K and V) 113 / 112; 64 heads 272 / 274, FP8 212 / 215 (134 MB: not taken);
+// 128 of them FP8 409 / 421; 220 of 1200 168.7 / 163.8.
+// Up to kInputElements elements of K and V together the second reads go through the caches too, where the L2s still hold the first
+// ones (past them, a line that others want is given up): with both, 31 heads of 2000 rows, head_dim 128, FP16 64.5 / 61.6, FP8 59.3 / 55.2, of 64 62.3 /
+// 60.2; 7 of 4000, 64, 56.9 / 55.6.  So do those of the one-launch pre-pass, whose workgroups read each other's rows for their statistics: 52 of
+// 600, FP8, 128, 39.4 / 36.7.  FP16 panels of head_dim 64 are then written through them as well: 15 of 4000 60.7 / 58.7, 31 of 2000 42.7 /
+// 41.5; at 128 (28 of 1100 41.6 / 42.8), FP8 (15 of 2000 43.7 / 44.9) and INT8 K it is the slower.
+bool statistics_stay(int64_t elements) { return elements <= kStatElements; }
+bool inputs_stay(int64_t elements) { return elements <= kInputElements; }
+
 struct RowDot {   // optional side output of the quantiser (see QuantArgs)
   const void* vec = nullptr;
   float* out = nullptr;
@@ -137,6 +151,7 @@ int sage_k_mean(const void* k, void* km, void* workspace, size_t workspace_bytes
   ColStatArgs a;
   a.x = (const u16*)k; a.partial = workspace; a.B = B; a.H = H; a.L = L; a.D = D;
   a.x_sb = k_sb; a.x_sh = k_sh; a.x_sn = k_sn; a.nchunk = colstat_chunks(L); a.cu_seqlens = cu_seqlens;
+  a.cached = !cu_seqlens && statistics_stay((int64_t)B * H * L * D);   // (its quantiser comes next)
   if (a.nchunk == 0) a.nchunk = 1;  // L == 0: the finalize kernel still writes zeros
   hipError_t e = launch_k_mean(a, dtype, km, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "sage_k_mean");
@@ -171,6 +186,7 @@ int sage_prep_v(const void* v, void* panels, float* v_scale, void* workspace, si
     ColStatArgs c;
     c.x = (const u16*)v; c.partial = workspace; c.B = B; c.H = H; c.L = L; c.D = D;
     c.x_sb = v_sb; c.x_sh = v_sh; c.x_sn = v_sn; c.nchunk = colstat_chunks(L); c.cu_seqlens = cu_seqlens;
+    c.cached = !cu_seqlens && statistics_stay((int64_t)B * H * L * D);
     hipError_t e = launch_v_scale(c, dtype, v_scale, st);
     if (e != hipSuccess) return hip_fail(e, "sage_prep_v(scale)");
   }
@@ -636,6 +652,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     ColStatArgs& ks = stats.k_stat;
     ks.x = (const u16*)k; ks.B = B; ks.H = Hkv; ks.L = Skv; ks.D = D; ks.x_sb = k_sb; ks.x_sh = k_sh; ks.x_sn = k_sn;
     ks.nchunk = colstat_chunks(Skv);
+    ks.cached = statistics_stay(k_elements * ((smooth_k != 0) + (pv_mode == SAGE_PV_FP8)));
     stats.v_stat = ks;
     stats.v_stat.x = (const u16*)v; stats.v_stat.x_sb = v_sb; stats.v_stat.x_sh = v_sh; stats.v_stat.x_sn = v_sn;
     if (smooth_k) ks.partial = stat;
@@ -668,11 +685,12 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     qa.x = (const u16*)k; qa.out = k_i8; qa.scale = k_scale; qa.km = nullptr;
     qa.B = B; qa.H = Hkv; qa.L = Skv; qa.D = D;
     qa.x_sb = k_sb; qa.x_sh = k_sh; qa.x_sn = k_sn; qa.o_sb = ki_sb; qa.o_sh = ki_sh; qa.o_sn = ki_sn;
+    qa.cached = true;   // (other workgroups read the rows for their statistics)
     qa.blk = kb; qa.blk_shift = ilog2(kb); qa.groups = blk_groups(blkk); qa.mult = 1.0f; qa.dv_group = 1;
     PrepVArgs va;
     memset(&va, 0, sizeof(va));
     va.v = (const u16*)v; va.panels = (uint8_t*)panels; va.vscale = v_scale; va.B = B; va.H = Hkv; va.L = Skv; va.D = D;
-    va.v_sb = v_sb; va.v_sh = v_sh; va.v_sn = v_sn;
+    va.v_sb = v_sb; va.v_sh = v_sh; va.v_sn = v_sn; va.cached = true;
     hipError_t e = launch_prepass_small(qa, va, dtype, pv_mode == SAGE_PV_FP8, smooth_k != 0, km, v_scale, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sage_sageattn(pre-pass)");
   }
@@ -733,12 +751,15 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
   memset(&ks, 0, sizeof(ks));
   ks.x = (const u16*)k; ks.partial = stat; ks.B = B; ks.H = Hkv; ks.L = Skv; ks.D = D;
   ks.x_sb = k_sb; ks.x_sh = k_sh; ks.x_sn = k_sn; ks.nchunk = colstat_chunks(Skv); ks.cu_seqlens = cu_seqlens_k;
+  const int64_t kv_elements = varlen ? (int64_t)total_k * Hkv * D : k_elements;   // of either
+  ks.cached = statistics_stay(kv_elements * ((smooth_k != 0) + fp8));
   vs = ks;
   vs.x = (const u16*)v; vs.x_sb = v_sb; vs.x_sh = v_sh; vs.x_sn = v_sn;
   PrepVArgs pvn;
   memset(&pvn, 0, sizeof(pvn));
   pvn.v = (const u16*)v; pvn.panels = (uint8_t*)panels; pvn.vscale = v_scale; pvn.B = B; pvn.H = Hkv; pvn.L = Skv; pvn.D = D;
   pvn.v_sb = v_sb; pvn.v_sh = v_sh; pvn.v_sn = v_sn; pvn.cu_seqlens = cu_seqlens_k; pvn.cu_panels = cu_panel; pvn.panel_sh = w.panel_sh;
+  kq.cached = pvn.cached = !varlen && inputs_stay(2 * kv_elements);
   PlanArgs pl;
   memset(&pl, 0, sizeof(pl));
   const int bm = tile_rows({B, Hq, Sq, Skv, D, pv_mode, is_causal, blk_rows(blkk), blk_groups(blkk), lse != nullptr, mask_class(m, Skv), varlen != 0, total_q, total_k});

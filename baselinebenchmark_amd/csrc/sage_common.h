@@ -144,9 +144,20 @@ __device__ inline uint4 load_stream16(const void* p) {
   const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
+// ... unless a later pass of the same call finds them in the last-level cache (256 MB), or in an L2, which is for the caller to know:
+// `load` is handed to the work as a function, so that the choice is one uniform branch around it.
+template <class Work>
+__device__ __forceinline__ void with_loads(bool cached, Work work) {
+  if (cached) work([](const void* p) __attribute__((always_inline)) { return *reinterpret_cast<const uint4*>(p); });
+  else work([](const void* p) __attribute__((always_inline)) { return load_stream16(p); });
+}
 __device__ inline void store_stream16(void* p, uint4 v) {
   const v4u t = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(t, reinterpret_cast<v4u*>(p));
+}
+__device__ inline void store16(bool cached, void* p, uint4 v) {
+  if (cached) *reinterpret_cast<uint4*>(p) = v;
+  else store_stream16(p, v);
 }
 
 // ---------------------------------------------------------------------------------------------

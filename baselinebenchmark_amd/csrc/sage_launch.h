@@ -30,6 +30,7 @@ struct QuantArgs {
   int km_nchunk;
   u16* km_out;
   int heads_first;   // set by the launcher: grid is (head, rows) instead of (rows, head)
+  int cached;        // read through the caches (with_loads) instead of past them
 };
 
 // Geometry of the quantiser: a workgroup of 256 lanes takes quant_rows(D, blk) consecutive rows of one (batch, head), whole scale
@@ -50,7 +51,7 @@ struct ColStatArgs {
   int64_t x_sb, x_sh, x_sn;
   int nchunk;
   const int32_t* cu_seqlens;
-  int heads_first;   // as in QuantArgs
+  int heads_first, cached;   // as in QuantArgs
 };
 
 struct PrepVArgs {
@@ -66,7 +67,7 @@ struct PrepVArgs {
   const float* vs_partial;
   int vs_nchunk;
   float* vscale_out;
-  int heads_first;   // as in QuantArgs
+  int heads_first, cached;   // as in QuantArgs
 };
 
 struct MaskPackArgs {

@@ -111,12 +111,14 @@ __device__ __forceinline__ void quant_int8_rows(const QuantArgs& a, const int ch
   mean.request(L);
   // (rows past the end read the last one again: no branch between the loads)
   uint4 raw[NP][2];
+  with_loads(a.cached, [&](auto load) __attribute__((always_inline)) {
 #pragma unroll
-  for (int p = 0; p < NP; p++) {
-    const u16* src = a.x + xbase + (int64_t)min(row + p * RW, L - 1) * a.x_sn + tc * 16;
-    raw[p][0] = load_stream16(src);
-    raw[p][1] = load_stream16(src + 8);
-  }
+    for (int p = 0; p < NP; p++) {
+      const u16* src = a.x + xbase + (int64_t)min(row + p * RW, L - 1) * a.x_sn + tc * 16;
+      raw[p][0] = load(src);
+      raw[p][1] = load(src + 8);
+    }
+  });
   // k - km is rounded to the input dtype (quant_per_block.py:53-54: the subtraction happens in torch, in
   // the tensor's dtype); both passes then see the rounded difference.
   uint4 kmr[2];
@@ -278,14 +280,16 @@ __device__ __forceinline__ void colstat_chunk(const ColStatArgs a, const int chu
   constexpr int UNR = 8;
   const u16* base = a.x + xbase + tc * 8;
   int n = n0 + tr;
-  for (; n + (UNR - 1) * RPP < n1; n += UNR * RPP) {
-    uint4 raw[UNR];
+  with_loads(a.cached, [&](auto load) __attribute__((always_inline)) {
+    for (; n + (UNR - 1) * RPP < n1; n += UNR * RPP) {
+      uint4 raw[UNR];
 #pragma unroll
-    for (int u = 0; u < UNR; u++) raw[u] = load_stream16(base + (int64_t)(n + u * RPP) * a.x_sn);
+      for (int u = 0; u < UNR; u++) raw[u] = load(base + (int64_t)(n + u * RPP) * a.x_sn);
 #pragma unroll
-    for (int u = 0; u < UNR; u++) fold(raw[u]);
-  }
-  for (; n < n1; n += RPP) fold(load_stream16(base + (int64_t)n * a.x_sn));
+      for (int u = 0; u < UNR; u++) fold(raw[u]);
+    }
+    for (; n < n1; n += RPP) fold(load(base + (int64_t)n * a.x_sn));
+  });
   acc_t(*red)[D] = reinterpret_cast<acc_t(*)[D]>(lds);
 #pragma unroll
   for (int i = 0; i < 8; i++) red[tr][tc * 8 + i] = acc[i];
@@ -433,13 +437,15 @@ __device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, 
   if constexpr (PV == 1) scales.request(L);
   // (all rows are requested before anything waits; those past the end read the last one again and become zeros)
   uint4 raw[QPT][4];
+  with_loads(a.cached, [&](auto load) __attribute__((always_inline)) {
 #pragma unroll
-  for (int qq = 0; qq < QPT; qq++)
+    for (int qq = 0; qq < QPT; qq++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int r = n0 + 4 * (qq * RPP + tr) + j;
-      raw[qq][j] = load_stream16(a.v + vbase + (int64_t)min(r, L - 1) * a.v_sn + tc * 8);
-    }
+      for (int j = 0; j < 4; j++) {
+        const int r = n0 + 4 * (qq * RPP + tr) + j;
+        raw[qq][j] = load(a.v + vbase + (int64_t)min(r, L - 1) * a.v_sn + tc * 8);
+      }
+  });
   auto row_there = [&](int qq, int j) { return n0 + 4 * (qq * RPP + tr) + j < L; };
   if constexpr (PV == 1) {
     const float* vs = scales.ready(L, pidx == 0);
@@ -511,7 +517,7 @@ __device__ __forceinline__ void prep_v_tile(const PrepVArgs& a, const int pidx, 
       const uint32_t* src = &T[(32 * dt + d_lo) * TS + (4 * ks16 + hh) * 2];
       v = make_uint4(src[0], src[1], src[4], src[5]);
     }
-    store_stream16(out + c, v);
+    store16(D == 64 && PV == 0 && a.cached, out + c, v);   // (see inputs_stay)
   }
 }
 
