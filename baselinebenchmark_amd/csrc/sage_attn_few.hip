@@ -17,8 +17,9 @@
 //     of very long histories, kFewChunks);
 //   * FP8 P.V: V is rounded to the e4m3 values of the panels in registers (a division per element: the vector ALU is what bounds it)
 //     and multiplied in fp16, which holds them; the probabilities are the tiled kernel's block-scaled codes, read back the same way.
-// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 48.7 us (this
-// kernel 33 us = 4.1 TB/s of K and V, half of it vector arithmetic of the quantisation; K sums 10, merge 5); 8 rows: 170.8
+// Measured, whole calls in bf16, tiled kernel -> this one: 4 x 32/8 heads, 1 row, 8192 keys, head_dim 128: 170.7 -> 46.0 us (this
+// kernel 30 us = 4.5 TB/s of K and V, half of it vector arithmetic of the quantisation; K sums 10, merge 5; requesting everything that the
+// prologue needs before it waits for any of it took 1.0 of 47.8, keeping the differences as floats 0.8); 8 rows: 170.8
 // -> 54; 8 x 32/8 heads, 4 rows, 16384 keys: 431.9 -> 150; 16 x 32 heads, 4096 keys: 600 -> 279; 1 x 8/2 heads, 8 rows, 32768 keys:
 // 435 -> 34.  FP8 P.V: 146 -> 82 for the first, 311 -> 51 for the last.
 #include "sage_launch.h"
@@ -42,6 +43,9 @@ __device__ inline float xor16_32_sum(float x) {
   x += __shfl_xor(x, 16);
   return x + __shfl_xor(x, 32);
 }
+
+// Waits for this wavefront's LDS operations only: loads in flight stay in flight.
+__device__ inline void lds_only_barrier_few() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 template <class Quotient>
 __device__ __forceinline__ v4i pack16(const float (&x)[16], Quotient quotient) {
@@ -81,18 +85,50 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
 #pragma unroll
       for (int i = 0; i < LK; i++) kraw[t][i] = __builtin_amdgcn_raw_buffer_load_b128(krsrc, off + t * 16 * (int)a.k_sn * 2 + 64 * i, 0, 0);
   };
+  // FP8 P.V: the probability codes of a row are taken relative to the maximum of its first 128 keys (what the tiled kernel's running
+  // maximum is unless a later tile exceeds it by 2^20), so a range that starts later visits tile 0 first, for that maximum alone.
+  const bool reference_first = PV == 1 && t0 > 0 && t0 < t1;
+  const int first = reference_first ? 0 : t0;
+  auto next_tile = [&](int tile) { return reference_first && tile == 0 ? t0 : tile + 1; };
+  // The first statistics of K are requested, then Q and the first K tile, and only then does anything wait: one memory latency instead of
+  // three.  (Loads complete in order: behind the K tile, the statistics would wait for it.)
+  constexpr int AHEAD = 16;
+  const int64_t stat_at = (int64_t)bh * a.nchunk * D + tid % D;
+  double sums[AHEAD];
+  if (a.km_partial && a.nchunk > 0 && tid < D) {
+#pragma unroll
+    for (int c = 0; c < AHEAD; c++) sums[c] = a.km_partial[stat_at + (int64_t)min(c, a.nchunk - 1) * D];
+  }
+  [[maybe_unused]] float maxima[PV ? AHEAD : 1];
+  if constexpr (PV == 1) {
+    if (tid >= D && tid < 2 * D) {
+#pragma unroll
+      for (int c = 0; c < AHEAD; c++) maxima[c] = a.vs_partial[stat_at + (int64_t)min(c, a.nchunk - 1) * D];
+    }
+  }
+  v4u qraw[MT][LK];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
+    const u16* qp = a.q + (int64_t)b * a.q_sb + (int64_t)(kvh * G + head) * a.q_sh + (int64_t)s * a.q_sn + 8 * g;
+#pragma unroll
+    for (int i = 0; i < LK; i++) qraw[mt][i] = *reinterpret_cast<const v4u*>(qp + 32 * i);
+  }
+  if (t0 < t1) load_k(first);
   // ---- K mean and V scales from the per-chunk statistics, in chunk order (kmean_finalize_kernel, vscale_finalize_kernel) ----
   __shared__ __align__(16) u16 km_lds[D];
   [[maybe_unused]] __shared__ __align__(16) float2 vs_lds[PV ? D : 1];   // scale and its reciprocal
   [[maybe_unused]] bool v_exact = true;
   {
-    const int64_t at = (int64_t)bh * a.nchunk * D + tid % D;
+    const int64_t at = stat_at;
     // (head_dim 128: the lower half of the workgroup folds K, the upper one V; at 64 likewise with a quarter each)
     if (PV == 0 && a.km_partial && a.nchunk == 0) {
       if (tid < D) km_lds[tid] = reinterpret_cast<const u16*>(a.km_partial)[(int64_t)bh * D + tid];
     } else if (a.km_partial && tid < D) {
       double s = 0;
-      for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
+#pragma unroll
+      for (int c = 0; c < AHEAD; c++) s = c < a.nchunk ? s + sums[c] : s;
+      for (int c0 = AHEAD; c0 < a.nchunk; c0 += 8) {
         double t[8];
 #pragma unroll
         for (int c = 0; c < 8; c++) t[c] = a.km_partial[at + (int64_t)min(c0 + c, a.nchunk - 1) * D];
@@ -104,7 +140,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     if constexpr (PV == 1) {
       if (tid >= D && tid < 2 * D) {
         float mx = 0.f;
-        for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
+#pragma unroll
+        for (int c = 0; c < AHEAD; c++) mx = fmaxf(mx, maxima[c]);
+        for (int c0 = AHEAD; c0 < a.nchunk; c0 += 8) {
 #pragma unroll
           for (int c = 0; c < 8; c++) mx = fmaxf(mx, a.vs_partial[at + (int64_t)min(c0 + c, a.nchunk - 1) * D]);
         }
@@ -114,16 +152,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
                                                                        // sums near fp32's end come out as in the tiled kernel)
       }
     }
-    __syncthreads();
+    lds_only_barrier_few();
     if constexpr (PV == 1) v_exact = __builtin_amdgcn_ballot_w64(!reciprocal_is_exact(vs_lds[lane].x) || !reciprocal_is_exact(vs_lds[(lane + 64) % D].x)) == 0;
   }
-  // FP8 P.V: the probability codes of a row are taken relative to the maximum of its first 128 keys (what the tiled kernel's running
-  // maximum is unless a later tile exceeds it by 2^20), so a range that starts later visits tile 0 first, for that maximum alone.
-  const bool reference_first = PV == 1 && t0 > 0 && t0 < t1;
-  const int first = reference_first ? 0 : t0;
-  auto next_tile = [&](int tile) { return reference_first && tile == 0 ? t0 : tile + 1; };
-  if (t0 < t1) load_k(first);
-
   float kmf[LK][8];
   if (a.km_partial) {
 #pragma unroll
@@ -146,12 +177,10 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     float x[MT][KS][16];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
-      const u16* qp = a.q + (int64_t)b * a.q_sb + (int64_t)(kvh * G + head) * a.q_sh + (int64_t)s * a.q_sn + 8 * g;
       float amax = 0.f, sum = 0.f;
 #pragma unroll
       for (int i = 0; i < LK; i++) {
-        const v4u raw = *reinterpret_cast<const v4u*>(qp + 32 * i);
+        const v4u raw = qraw[mt][i];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           const float v = to_f32<DT>((u16)(raw[e >> 1] >> (16 * (e & 1)))) * a.q_mult;
@@ -164,7 +193,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
       dot[mt] = xor16_32_sum(sum);   // what K smoothing takes from every logit of the row
       if (w == 0 && g == 0) row_amax[16 * mt + m] = amax;
     }
-    __syncthreads();
+    lds_only_barrier_few();
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
       const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
@@ -222,10 +251,12 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
         }
     }
     // ---- K: subtract the mean in the input type, block maxima, quantise ----
+    // (one score tile and no V quotients: the differences stay as floats, a widening less each; the others have no registers for it)
+    constexpr bool WIDE = MT == 1 && PV == 0;
+    float xk[2][WIDE ? D / 4 : 1];
     float amax[2];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-      const bool gone = n0 + 16 * t + m >= L;
       float mx = 0.f;
 #pragma unroll
       for (int i = 0; i < LK; i++)
@@ -234,11 +265,24 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
           float lo, hi;
           unpack2<DT>(kraw[t][i][e], lo, hi);
           const uint32_t x = pack2<DT>(lo - kmf[i][2 * e], hi - kmf[i][2 * e + 1]);
-          kraw[t][i][e] = gone ? 0u : x;
           unpack2<DT>(x, lo, hi);
+          if constexpr (WIDE) {
+            xk[t][8 * i + 2 * e] = lo;
+            xk[t][8 * i + 2 * e + 1] = hi;
+          } else kraw[t][i][e] = x;
           mx = fmaxf(mx, fmaxf(fabsf(lo), fabsf(hi)));
         }
-      amax[t] = wave_max(gone ? 0.f : mx);
+      if (tile * 128 + 128 > L && n0 + 16 * t + m >= L) {   // (a tile that the sequence ends in: rows past it are zeros)
+        mx = 0.f;
+        if constexpr (WIDE) {
+#pragma unroll
+          for (int e = 0; e < D / 4; e++) xk[t][e] = 0.f;
+        } else {
+#pragma unroll
+          for (int i = 0; i < LK; i++) kraw[t][i] = v4u{0, 0, 0, 0};
+        }
+      }
+      amax[t] = wave_max(mx);
     }
     if (a.blkk_shift >= 5) amax[0] = amax[1] = fmaxf(amax[0], amax[1]);
     if (a.blkk_shift >= 6) {
@@ -259,7 +303,10 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
       for (int s = 0; s < KS; s++) {
         float x[16];
 #pragma unroll
-        for (int e = 0; e < 16; e++) x[e] = to_f32<DT>((u16)(kraw[t][2 * s + (e >> 3)][(e & 7) >> 1] >> (16 * (e & 1))));
+        for (int e = 0; e < 16; e++) {
+          if constexpr (WIDE) x[e] = xk[t][16 * s + e];
+          else x[e] = to_f32<DT>((u16)(kraw[t][2 * s + (e >> 3)][(e & 7) >> 1] >> (16 * (e & 1))));
+        }
         if (fast) kreg[t][s] = pack16(x, [&](float v) { return div_by_uniform(v, scale, rcp); });
         else kreg[t][s] = pack16(x, [&, wide = 1.0 / (double)scale](float v) { return div_by_any(v, wide); });
       }
@@ -367,8 +414,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
             vf[j] = h2[0];
             vf[j + 1] = h2[1];
           } else {
-            vf[j] = DT == 0 ? __builtin_bit_cast(_Float16, b0) : (_Float16)bf16_to_f32(b0);
-            vf[j + 1] = DT == 0 ? __builtin_bit_cast(_Float16, b1) : (_Float16)bf16_to_f32(b1);
+            const v2h h2 = __builtin_bit_cast(v2h, DT == 0 ? (uint32_t)b0 | (uint32_t)b1 << 16 : pack2<0>(bf16_to_f32(b0), bf16_to_f32(b1)));
+            vf[j] = h2[0];
+            vf[j + 1] = h2[1];
           }
         }
 #pragma unroll
