@@ -274,7 +274,7 @@ bool small_tiles_pay(const TileRows& c) {
   const int64_t large = (int64_t)c.B * c.Hq * ((c.Sq + 255) / 256);
   if (c.packed && c.D == 64) return true;
   if (!c.packed && large <= 128) return !(c.kgroups != 1 && c.D == 64 && c.pv == SAGE_PV_FP8);
-  if (!c.packed && !c.causal && large <= 256) return keys <= (c.D == 64 ? (c.pv == SAGE_PV_FP8 ? 2048 : 768) : c.pv == SAGE_PV_FP8 ? 768 : 512);
+  if (!c.packed && !c.causal && large <= 256) return keys <= (c.D == 64 ? (c.pv == SAGE_PV_FP8 && c.kgroups == 1 ? 2048 : 768) : c.pv == SAGE_PV_FP8 ? 768 : 512);
   if (c.mask != kNoMask) return keys <= 1024 || large <= 512;
   if (c.causal) keys /= 2;
   if (c.D == 64) return keys <= (c.causal && c.pv == SAGE_PV_FP16 ? 8192 : 4096);

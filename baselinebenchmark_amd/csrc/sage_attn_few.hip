@@ -90,31 +90,31 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
   const bool reference_first = PV == 1 && t0 > 0 && t0 < t1;
   const int first = reference_first ? 0 : t0;
   auto next_tile = [&](int tile) { return reference_first && tile == 0 ? t0 : tile + 1; };
-  // The first statistics of K are requested, then Q and the first K tile, and only then does anything wait: one memory latency instead of
-  // three.  (Loads complete in order: behind the K tile, the statistics would wait for it.)
-  constexpr int AHEAD = 16;
+  // FP16 P.V: the first statistics of K are requested, then Q and the first K tile, and only then does anything wait: one memory latency
+  // instead of three.  (Loads complete in order: behind the K tile, the statistics would wait for it.  FP8 P.V, whose statistics of V come
+  // along, has no registers left for it at head_dim 128 and gained nothing: 8 heads of 8192 keys 82.5 us, 82.9 like this.)
+  constexpr bool EARLY = PV == 0;
+  constexpr int AHEAD = EARLY ? 16 : 0;   // chunks
   const int64_t stat_at = (int64_t)bh * a.nchunk * D + tid % D;
-  double sums[AHEAD];
-  if (a.km_partial && a.nchunk > 0 && tid < D) {
-#pragma unroll
-    for (int c = 0; c < AHEAD; c++) sums[c] = a.km_partial[stat_at + (int64_t)min(c, a.nchunk - 1) * D];
-  }
-  [[maybe_unused]] float maxima[PV ? AHEAD : 1];
-  if constexpr (PV == 1) {
-    if (tid >= D && tid < 2 * D) {
-#pragma unroll
-      for (int c = 0; c < AHEAD; c++) maxima[c] = a.vs_partial[stat_at + (int64_t)min(c, a.nchunk - 1) * D];
-    }
-  }
-  v4u qraw[MT][LK];
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++) {
+  [[maybe_unused]] double sums[EARLY ? AHEAD : 1];
+  [[maybe_unused]] v4u qraw[MT][LK];
+  auto q_row = [&](int mt) {
     const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
-    const u16* qp = a.q + (int64_t)b * a.q_sb + (int64_t)(kvh * G + head) * a.q_sh + (int64_t)s * a.q_sn + 8 * g;
+    return a.q + (int64_t)b * a.q_sb + (int64_t)(kvh * G + head) * a.q_sh + (int64_t)s * a.q_sn + 8 * g;
+  };
+  if constexpr (EARLY) {
+    if (a.km_partial && a.nchunk > 0 && tid < D) {
 #pragma unroll
-    for (int i = 0; i < LK; i++) qraw[mt][i] = *reinterpret_cast<const v4u*>(qp + 32 * i);
+      for (int c = 0; c < AHEAD; c++) sums[c] = a.km_partial[stat_at + (int64_t)min(c, a.nchunk - 1) * D];
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const u16* qp = q_row(mt);
+#pragma unroll
+      for (int i = 0; i < LK; i++) qraw[mt][i] = *reinterpret_cast<const v4u*>(qp + 32 * i);
+    }
+    if (t0 < t1) load_k(first);
   }
-  if (t0 < t1) load_k(first);
   // ---- K mean and V scales from the per-chunk statistics, in chunk order (kmean_finalize_kernel, vscale_finalize_kernel) ----
   __shared__ __align__(16) u16 km_lds[D];
   [[maybe_unused]] __shared__ __align__(16) float2 vs_lds[PV ? D : 1];   // scale and its reciprocal
@@ -140,9 +140,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     if constexpr (PV == 1) {
       if (tid >= D && tid < 2 * D) {
         float mx = 0.f;
-#pragma unroll
-        for (int c = 0; c < AHEAD; c++) mx = fmaxf(mx, maxima[c]);
-        for (int c0 = AHEAD; c0 < a.nchunk; c0 += 8) {
+        for (int c0 = 0; c0 < a.nchunk; c0 += 8) {
 #pragma unroll
           for (int c = 0; c < 8; c++) mx = fmaxf(mx, a.vs_partial[at + (int64_t)min(c0 + c, a.nchunk - 1) * D]);
         }
@@ -155,6 +153,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     lds_only_barrier_few();
     if constexpr (PV == 1) v_exact = __builtin_amdgcn_ballot_w64(!reciprocal_is_exact(vs_lds[lane].x) || !reciprocal_is_exact(vs_lds[(lane + 64) % D].x)) == 0;
   }
+  if constexpr (!EARLY)
+    if (t0 < t1) load_k(first);
+
   float kmf[LK][8];
   if (a.km_partial) {
 #pragma unroll
@@ -180,7 +181,9 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
       float amax = 0.f, sum = 0.f;
 #pragma unroll
       for (int i = 0; i < LK; i++) {
-        const v4u raw = qraw[mt][i];
+        v4u raw;
+        if constexpr (EARLY) raw = qraw[mt][i];
+        else raw = *reinterpret_cast<const v4u*>(q_row(mt) + 32 * i);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           const float v = to_f32<DT>((u16)(raw[e >> 1] >> (16 * (e & 1)))) * a.q_mult;
@@ -257,6 +260,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
     float amax[2];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
+      const bool gone = n0 + 16 * t + m >= L;   // rows past the end are zeros
       float mx = 0.f;
 #pragma unroll
       for (int i = 0; i < LK; i++)
@@ -269,19 +273,16 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
           if constexpr (WIDE) {
             xk[t][8 * i + 2 * e] = lo;
             xk[t][8 * i + 2 * e + 1] = hi;
-          } else kraw[t][i][e] = x;
+          } else kraw[t][i][e] = gone ? 0u : x;
           mx = fmaxf(mx, fmaxf(fabsf(lo), fabsf(hi)));
         }
-      if (tile * 128 + 128 > L && n0 + 16 * t + m >= L) {   // (a tile that the sequence ends in: rows past it are zeros)
-        mx = 0.f;
-        if constexpr (WIDE) {
+      if constexpr (WIDE) {
+        if (tile * 128 + 128 > L && gone) {   // (in the one tile that has any)
 #pragma unroll
           for (int e = 0; e < D / 4; e++) xk[t][e] = 0.f;
-        } else {
-#pragma unroll
-          for (int i = 0; i < LK; i++) kraw[t][i] = v4u{0, 0, 0, 0};
         }
       }
+      if (gone) mx = 0.f;
       amax[t] = wave_max(mx);
     }
     if (a.blkk_shift >= 5) amax[0] = amax[1] = fmaxf(amax[0], amax[1]);
