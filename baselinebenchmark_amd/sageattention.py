@@ -81,6 +81,19 @@ def _workspace_bytes(B, Hq, Hkv, Sq, Skv, D, blkq, blkk, pv, Tq, Tk, varlen, smo
     return n + (lib().sage_prep_v_workspace_bytes(B, Hkv, Skv, D, pv) if pv == PV_FP8 else 0)
 
 
+# (Sizes asked for once per shape, and no torch.no_grad around functions that run no differentiable operation: the two-step calls of 4
+# heads of 576 rows, bound by the host, 64.7 -> 57 us, FP8 76 -> 67.)
+@functools.lru_cache(maxsize=1024)
+def _k_mean_bytes(B, H, L, D) -> int:
+    return lib().sage_k_mean_workspace_bytes(B, H, L, D)
+
+
+@functools.lru_cache(maxsize=1024)
+def _prep_v_bytes(B, H, L, D, pv):
+    """(panels, workspace), in bytes."""
+    return lib().sage_v_panel_bytes(B, H, L, D, pv), lib().sage_prep_v_workspace_bytes(B, H, L, D, pv) if pv == PV_FP8 else 0
+
+
 def _check_blocks_quant(BLKQ, BLKK):
     for b in (BLKQ, BLKK):
         if b not in (16, 32, 64, 128):
@@ -96,7 +109,6 @@ def _q_mult(head_dim: int, sm_scale) -> float:
 # ------------------------------------------------------------------------------------------------
 # quantisers
 # ------------------------------------------------------------------------------------------------
-@torch.no_grad()
 def k_mean(k: torch.Tensor, tensor_layout: str = "HND") -> torch.Tensor:
     """Per-(batch, kv-head, channel) mean of K over the sequence in k's dtype, shaped to broadcast
     against k ([B,H,1,D] for HND, [B,1,H,D] for NHD): the `km` argument of per_block_int8."""
@@ -105,7 +117,7 @@ def k_mean(k: torch.Tensor, tensor_layout: str = "HND") -> torch.Tensor:
     if D not in (64, 128):
         raise NotImplementedError("head_dim must be 64 or 128")
     km = torch.empty((B, H, D), device=k.device, dtype=k.dtype)
-    ws_bytes = lib().sage_k_mean_workspace_bytes(B, H, L, D)
+    ws_bytes = _k_mean_bytes(B, H, L, D)
     ws = torch.empty(max(ws_bytes, 8), device=k.device, dtype=torch.uint8)
     check(lib().sage_k_mean(_ptr(k), _ptr(km), _ptr(ws), ws_bytes, B, H, L, D, sb, sh, sn, _dt(k.dtype), None, _stream(k)))
     return km.view(B, H, 1, D) if tensor_layout == "HND" else km.view(B, 1, H, D)
@@ -148,7 +160,6 @@ def _quant_one(x, km, blk, mult, tensor_layout, groups=1):
     return out, scale
 
 
-@torch.no_grad()
 def per_block_int8(q, k, km=None, BLKQ=128, BLKK=64, sm_scale=None, tensor_layout="HND", q_interleave=1, k_interleave=1):
     """Per-block INT8 quantisation of Q and K; returns (q_int8, q_scale, k_int8, k_scale).
 
@@ -179,7 +190,6 @@ def per_block_int8(q, k, km=None, BLKQ=128, BLKK=64, sm_scale=None, tensor_layou
     return q_int8, q_scale, k_int8, k_scale
 
 
-@torch.no_grad()
 def prepare_v(v: torch.Tensor, tensor_layout: str = "HND", pv_mode: str = "fp16"):
     """V -> MFMA-ready panels.  Returns (panels uint8 tensor, v_scale [B,H,D] float32 or None)."""
     _check_float("v", v)
@@ -187,12 +197,11 @@ def prepare_v(v: torch.Tensor, tensor_layout: str = "HND", pv_mode: str = "fp16"
     B, H, L, D, sb, sh, sn = _layout(v, tensor_layout)
     if D not in (64, 128):
         raise NotImplementedError("head_dim must be 64 or 128")
-    panels = torch.empty(max(lib().sage_v_panel_bytes(B, H, L, D, pv), 16), device=v.device, dtype=torch.uint8)
+    panel_bytes, ws_bytes = _prep_v_bytes(B, H, L, D, pv)
+    panels = torch.empty(max(panel_bytes, 16), device=v.device, dtype=torch.uint8)
     v_scale = ws = None
-    ws_bytes = 0
     if pv == PV_FP8:
         v_scale = torch.empty((B, H, D), device=v.device, dtype=torch.float32)
-        ws_bytes = lib().sage_prep_v_workspace_bytes(B, H, L, D, pv)
         ws = torch.empty(max(ws_bytes, 8), device=v.device, dtype=torch.uint8)
     check(lib().sage_prep_v(_ptr(v), _ptr(panels), _ptr(v_scale), _ptr(ws), ws_bytes, B, H, L, D, sb, sh, sn,
                             _dt(v.dtype), pv, None, None, 0, _stream(v)))
