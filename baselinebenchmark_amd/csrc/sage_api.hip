@@ -280,7 +280,12 @@ bool small_tiles_pay(const TileRows& c) {
   if (c.D == 64) return keys <= (c.causal && c.pv == SAGE_PV_FP16 ? 8192 : 4096);
   return keys <= (c.pv == SAGE_PV_FP8 ? 1800 : 1500);
 }
-int tile_rows(const TileRows& c) { return small_tiles_pay(c) ? kSmallTileRows : kLargeTileRows; }
+int tile_rows(const TileRows& c) {
+#ifdef SAGE_TIMING   // (the timers that are read are those of the workgroups of 256 rows)
+  return kLargeTileRows;
+#endif
+  return small_tiles_pay(c) ? kSmallTileRows : kLargeTileRows;
+}
 // ... of the entry points that take a plan of the caller's, whose q-tiles have 256 rows.
 int public_tile_rows(int B, int Hq, int Sq, int Skv, int D, int pv_mode, int is_causal, int blkk, const float* lse, const int32_t* cu_seqlens_q) {
   if (cu_seqlens_q) return kLargeTileRows;
@@ -428,8 +433,8 @@ constexpr int64_t small_prepass_reads(bool mean, bool scales) { return (int64_t)
 // ... in this many heads: 12288 of a key, head_dim 64, 374 / 363; 16384 of 8 525 / 496; 8192 of 16 251 / 251, FP8 235 / 242.
 constexpr int64_t kSmallPrepassHeads = 8192;
 // A few query rows (sage_attn_few.hip) take at most three launches, some 2.5 us of host time more than the two of the tiled kernel behind
-// the one-launch pre-pass, which is as fast as that as long as its workgroups (a 256-row tile per query head, two to a compute unit at
-// head_dim 64) are one round of the chip, the keys of a head are few and so are the re-reads of the pre-pass.  Past one round the rows
+// the one-launch pre-pass, which is as fast as that as long as its workgroups (one per query head; measured with tiles of 256 rows, one
+// to a compute unit) are one round of the chip, the keys of a head are few and so are the re-reads of the pre-pass.  Past one round the rows
 // count: the few-rows kernel writes and reads FP32 results of every row.  Whole calls, K blocks of 64, bf16, tiled / few rows in us.
 // FP16 P.V, up to 16 rows: 8 heads of 768 keys, head_dim 64, 19.9 / 20.2, of 900 23.3 / 19.9; head_dim 128, of 257 18.6 / 19.5, of 512 21.0 /
 // 19.9; 64 of 256 (12 M reads) 18.7 / 19.5, 128 of 192 (15 M) 20.9 / 19.5; 320 of 64 26.8 / 19.1, head_dim 64 19.4 / 19.8, 640 of 64 27.5 /

@@ -37,6 +37,8 @@
 //     SIMD always has matrix work and vector work to overlap.  One barrier per tile period hands the tile
 //     slots over; the FP16 P.V kernels keep a second one in the middle of the period (their two slots are
 //     what it protects the pace of), the FP8 P.V kernels, with four slots, run their two halves unsynchronised.
+//   * Workgroups of four wavefronts (NW = 4: sage_attn_small.hip says what for) have no groups: each wavefront takes a tile through
+//     Q.K^T, softmax and P.V in turn, and what overlaps is the work of the two or three workgroups of a compute unit.
 #pragma once
 #include "sage_launch.h"
 #include <atomic>

@@ -82,7 +82,7 @@ def _workspace_bytes(B, Hq, Hkv, Sq, Skv, D, blkq, blkk, pv, Tq, Tk, varlen, smo
 
 
 # (Sizes asked for once per shape, and no torch.no_grad around functions that run no differentiable operation: the two-step calls of 4
-# heads of 576 rows, bound by the host, 64.7 -> 57 us, FP8 76 -> 67.)
+# heads of 576 rows, bound by the host, 64.7 -> 56 us, FP8 76 -> 65.)
 @functools.lru_cache(maxsize=1024)
 def _k_mean_bytes(B, H, L, D) -> int:
     return lib().sage_k_mean_workspace_bytes(B, H, L, D)
