@@ -1235,20 +1235,20 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 && (MASK
           }
         }
       } else {
-      const int last = ntiles - 1;
-      for (int j = 0; j < last; j++) {
-        tile_landed(j);
-        if (j < wave_ntiles) step(j, all, std::false_type());
-        else values_landed(j);
-      }
-      // The last tile is the only one that the diagonal or the end of the sequence cuts: as many of its 32-key groups as the
-      // wavefront sees (FP8 products contract over 64 keys).
-      tile_landed(last);
-      const int groups = (wave_end - last * BN + 31) >> 5;
-      if (groups > 2) step(last, all, std::true_type());
-      else if (PV == 1 ? groups > 0 : groups == 2) step(last, std::integral_constant<int, 2>(), std::true_type());
-      else if (PV == 0 && groups == 1) step(last, std::integral_constant<int, PV == 1 ? 2 : 1>(), std::true_type());
-      else values_landed(last);
+        const int last = ntiles - 1;
+        for (int j = 0; j < last; j++) {
+          tile_landed(j);
+          if (j < wave_ntiles) step(j, all, std::false_type());
+          else values_landed(j);
+        }
+        // The last tile is the only one that the diagonal or the end of the sequence cuts: as many of its 32-key groups as the
+        // wavefront sees (FP8 products contract over 64 keys).
+        tile_landed(last);
+        const int groups = (wave_end - last * BN + 31) >> 5;
+        if (groups > 2) step(last, all, std::true_type());
+        else if (PV == 1 ? groups > 0 : groups == 2) step(last, std::integral_constant<int, 2>(), std::true_type());
+        else if (PV == 0 && groups == 1) step(last, std::integral_constant<int, PV == 1 ? 2 : 1>(), std::true_type());
+        else values_landed(last);
       }
     } else if constexpr (VECMAX) {
       // FP8 P.V, and FP16 P.V of head_dim 128: the matrix half is nothing but MFMAs and their LDS reads (P.V of the
