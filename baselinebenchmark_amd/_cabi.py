@@ -27,6 +27,7 @@ _I, _L, _P = c_int, c_int64, c_void_p
 SIGNATURES = {
     "sage_backend_name": (c_char_p, []),
     "sage_last_error": (c_char_p, []),
+    "sage_last_tile_rows": (c_int, []),
     "sage_quant_int8": (c_int, [_P, _P, _P, _P, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _L, _L, _I, c_float, _I,
                                 _P, _P, _L, _P]),
     "sage_k_mean_workspace_bytes": (c_size_t, [_I, _I, _I, _I]),

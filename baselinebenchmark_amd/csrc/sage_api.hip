@@ -15,6 +15,7 @@ using namespace sage;
 namespace {
 
 thread_local char g_err[512] = "";
+thread_local int g_tile_rows = 0;   // sage_last_tile_rows
 
 int fail(int code, const char* fmt, ...) {
   va_list ap;
@@ -68,6 +69,8 @@ extern "C" {
 const char* sage_backend_name(void) { return "mi355x_hip_int8_qk_fp8_fp16_pv"; }
 
 const char* sage_last_error(void) { return g_err; }
+
+int sage_last_tile_rows(void) { return g_tile_rows; }
 
 }  // extern "C"
 
@@ -304,6 +307,7 @@ int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const floa
               int64_t o_sn, int blkq, int blkk, int is_causal, int pv_mode, int out_dtype, const int32_t* cu_seqlens_q,
               const int32_t* cu_seqlens_k, const int32_t* plan, int total_q, int64_t q_scale_sh, int64_t k_scale_sh,
               int64_t panel_sh, const MaskArg& mask, const float* lse_offset, const QRawArg& qraw, int tile_rows, sage_stream_t stream) {
+  g_tile_rows = 0;
   if (int rc = check_common(B, Hq, Sq, D, out_dtype)) return rc;
   if (Hkv <= 0 || Hq % Hkv) return fail(SAGE_EINVAL, "query heads (%d) must be divisible by KV heads (%d)", Hq, Hkv);
   if (Skv < 0) return fail(SAGE_EINVAL, "negative kv length");
@@ -370,6 +374,7 @@ int attn_impl(const int8_t* q, const int8_t* k, const void* v_panels, const floa
   finish_attn_args(a, is_causal != 0);
   hipError_t e = launch_attn(a, D, pv_mode, is_causal != 0, (int)grid, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "sage_attn_fwd");
+  g_tile_rows = BM;
   return SAGE_OK;
 }
 }  // namespace
@@ -583,6 +588,7 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
                          int is_causal, int smooth_k, int pv_mode, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                          int total_q, int total_k, const void* attn_mask, int mask_kind, int64_t m_sb, int64_t m_sh,
                          int64_t m_sm, int64_t m_sn, sage_stream_t stream) {
+  g_tile_rows = 0;
   if (int rc = check_common(B, Hq, Sq, D, dtype)) return rc;
   if (Hkv <= 0 || Hq % Hkv) return fail(SAGE_EINVAL, "query heads (%d) must be divisible by KV heads (%d)", Hq, Hkv);
   if (!valid_blk_attn(blk_rows(blkq)) || !valid_blkk_attn(blk_rows(blkk)))

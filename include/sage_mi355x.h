@@ -72,6 +72,10 @@ const char* sage_backend_name(void);
 /* Message for the last non-zero return on this thread ("" if none). */
 const char* sage_last_error(void);
 
+/* Query rows per workgroup (256 or 128) of the tiled attention kernel that the calling thread's last attention call launched; 0 if it
+ * launched none (an error, nothing to do, or the kernel for a few query rows).  The results do not depend on it: for tests and tuning. */
+int sage_last_tile_rows(void);
+
 /*
  * Per-block INT8 quantiser for one operand.  Replaces one launch of
  * quant_per_block_int8_kernel (backends/_enflame/ops/sage_attention/quant_per_block.py:20-46,
