@@ -260,7 +260,8 @@ struct MaskArg {
 //     200..2000 680 / 635, 30 of 1000..4000 1822 / 1840, FP8 1366 / 1302, 16 of 512..8000 1666 / 1661, full FP16 40 of 200..2000 988 / 972, FP8 30 of
 //     1000..4000 2124 / 2119;
 //   K blocks of 16 and interleaved scales the same: FP8, head_dim 128, blocks of 16, full 160 of 1400 rows 176 / 164, 2000 220 / 219, 2800 192 / 197, causal 2800 138 /
-//     132, 4000 215 / 214, 8 heads of 4000 74 / 70; head_dim 64, in one round, 2 x 32/8 of 704 24.4 / 25.3; head_dim 64, interleaved, FP16 8 heads of 2000 44 / 39, but FP8, causal, which spills, 36 / 37;
+//     132, 4000 215 / 214, 8 heads of 4000 74 / 70; head_dim 64, in one round, 2 x 32/8 of 704 24.4 / 25.3; head_dim 64, interleaved, FP16 8 heads of 2000 44 / 39, FP8 causal 12 of 2000 38 / 37, but full, which
+//     keeps 36 bytes a lane in scratch memory, 33 of 700 27.0 / 27.8;
 //   masks: one bias per head, 2 x 16 heads of 1000 rows, head_dim 64 69 / 49, 128 82 / 60, 1 x 4 of 6000 325 / 211, 363 / 232; documents, head_dim 64, 2
 //     x 16 of 1500 53 / 50, 4 x 32 123 / 110, FP8 128 1 x 32 of 2200 133 / 101; padding, head_dim 64, 1 x 32 of 2200 109 / 85, but, head_dim 128, FP16,
 //     in one round of the chip, 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), of 1000 52 / 48, and in three whole ones, 4 x 32 of 1500, 195 / 200.
@@ -276,7 +277,7 @@ bool small_tiles_pay(const TileRows& c) {
   int64_t keys = c.packed ? ((int64_t)c.total_k / c.B + c.Skv) / 2 : c.Skv;
   const int64_t large = (int64_t)c.B * c.Hq * ((c.Sq + 255) / 256);
   if (c.packed && c.D == 64) return true;
-  if (!c.packed && large <= 128) return !(c.kgroups != 1 && c.D == 64 && c.pv == SAGE_PV_FP8);
+  if (!c.packed && large <= 128) return c.causal || !(c.kgroups != 1 && c.D == 64 && c.pv == SAGE_PV_FP8);
   if (!c.packed && !c.causal && large <= 256) return keys <= (c.D == 64 ? (c.pv == SAGE_PV_FP16 ? 768 : fine ? 512 : 2048) : c.pv == SAGE_PV_FP8 ? 768 : 512);
   if (c.mask != kNoMask) return keys <= 1024 || large <= 512;
   if (c.causal) keys /= 2;

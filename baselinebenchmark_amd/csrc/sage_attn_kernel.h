@@ -184,6 +184,17 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 #define SAGE_PH(k) do { } while (0)
 #define SAGE_T(k, x) do { } while (0)
 #endif
+// Workgroups of four wavefronts to a compute unit that the registers are held to.  Three (head_dim 64) leave 168: the FP8 P.V kernels then
+// keep 12 to 48 bytes a lane in scratch memory and still gain by the third workgroup.  With interleaved K scales and LSE it is 80 to 116,
+// a dozen accesses a tile, each waiting for the tiles requested ahead of it (loads complete in order): two workgroups, nothing in scratch.  16 heads of 8000
+// rows, 256 rows / three / two, us: full 299 / 395 / 287, causal 181 / 244 / 174; 25 of 3000, full, 134 / 118 / 107.  The
+// interleaved causal ones without LSE likewise: 26 heads of 4200 rows 81 / 84 / 79, 21 of 3000 54 / 56 / 52; full ones not: 25 of 3000 91 / 75 / 84.
+template <int D, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB>
+constexpr int attn_small_per_cu() {
+  if (D != 64 || (MASK != 0 && MASK != 3)) return 2;
+  return PV == 1 && KSUB == 3 && (CAUSAL || !MSUM) ? 2 : 3;
+}
+
 // MASK: 0 none, 1 boolean keep-mask (bytes), 2 additive fp32 bias in base-2 score units
 // (sageattention_triton.py:92-105), both [B, Hq, Sq, Skv] with element strides; 3 = a boolean mask in the packed form of
 // mask_pack_kernel (sage_common.h): the workgroup walks only the tiles in which one of its rows sees a key, a wavefront
@@ -198,7 +209,7 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 // looks its scale up), 2 for blocks of 64 keys and more, 4 for blocks of 128: the row maximum then runs one integer chain
 // per scale and the per-scale constants of the softmax are computed once (a tenth of the vector instructions of a tile).
 template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
-__global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (D == 64 && (MASK == 0 || MASK == 3) ? 3 : 2) : 1) attn_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (attn_small_per_cu<D, PV, CAUSAL, MSUM, MASK, KSUB>()) : 1) attn_kernel(AttnArgs a) {
   constexpr int GSH = SAGE_GSH;   // which bit of the wavefront index picks the group
   constexpr bool SMALL = attn_is_small(NW);
   static_assert(SMALL || NW == (2 << GSH), "the two groups pair wavefront w with w + NW/2");
