@@ -188,11 +188,13 @@ static __device__ unsigned long long g_wg_timeline[kTimelineMax][4];
 // keep 12 to 48 bytes a lane in scratch memory and still gain by the third workgroup.  With interleaved K scales and LSE it is 80 to 116,
 // a dozen accesses a tile, each waiting for the tiles requested ahead of it (loads complete in order): two workgroups, nothing in scratch.  16 heads of 8000
 // rows, 256 rows / three / two, us: full 299 / 395 / 287, causal 181 / 244 / 174; 25 of 3000, full, 134 / 118 / 107.  The
-// interleaved causal ones without LSE likewise: 26 heads of 4200 rows 81 / 84 / 79, 21 of 3000 54 / 56 / 52; full ones not: 25 of 3000 91 / 75 / 84.
+// interleaved causal ones without LSE likewise: 26 heads of 4200 rows 81 / 84 / 79, 21 of 3000 54 / 56 / 52; full ones not: 25 of 3000 91 / 75 / 84.  With a packed
+// mask the LDS of FP8 P.V (64 KB) has room for two: 2 x 16 heads of 1000 rows, documents 49 / 45 / 44, 1 x 8 of 3000 54 / 50 / 48; two tile slots instead of
+// three make room for a third, 4 x 32 of 1500 133 / 129 / 125 and 119 like that, but the first two 48 and 52.
 template <int D, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB>
 constexpr int attn_small_per_cu() {
   if (D != 64 || (MASK != 0 && MASK != 3)) return 2;
-  return PV == 1 && KSUB == 3 && (CAUSAL || !MSUM) ? 2 : 3;
+  return PV == 1 && (MASK == 3 || KSUB == 3 && (CAUSAL || !MSUM)) ? 2 : 3;
 }
 
 // MASK: 0 none, 1 boolean keep-mask (bytes), 2 additive fp32 bias in base-2 score units
@@ -1436,6 +1438,8 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (attn_small_per_c
 template <int D, int NW, int BN, int PV, bool CAUSAL, bool MSUM, int MASK, int KSUB = 1, bool QF = false, int KW = 1, bool DOT = false>
 static hipError_t launch_one(const AttnArgs& a, int grid, hipStream_t st) {
   constexpr int smem = attn_lds_bytes<D, NW, BN, PV, QF, MASK>();
+  static_assert(!attn_is_small(NW) || smem * attn_small_per_cu<D, PV, CAUSAL, MSUM, MASK, KSUB>() <= 160 * 1024,
+                "the registers are held to more workgroups than the LDS of a compute unit has room for");
   auto kern = attn_kernel<D, NW, BN, PV, CAUSAL, MSUM, MASK, KSUB, QF, KW, DOT>;
   // More than 64 KB of dynamic LDS has to be allowed once per kernel and device.
   constexpr int kMaxDevices = 64;

@@ -143,8 +143,9 @@ def attention_kernel(D, NW, pv, causal, msum, mask, ksub):
 def test_kernels_that_lose_by_scratch_memory_have_none(code_objects):
     # 128 rows, FP8 P.V, head_dim 64, interleaved K scales: with LSE up to 1.46 times as long as with 256 rows when they spilled
     wanted = [attention_kernel(64, 4, 1, causal, msum, 0, 3) for causal, msum in ((False, False), (True, False), (True, True))]
-    seen = {name: int(n) for path in code_objects for name, n in scratch_bytes(path).items() if name.startswith(tuple(wanted))}
-    assert len(seen) == 2 * len(wanted)   # (with INT8 and with floating-point Q)
+    masked = attention_kernel(64, 4, 1, False, False, 3, 1)   # ... and with a packed mask, whose LDS leaves room for two workgroups only
+    seen = {name: int(n) for path in code_objects for name, n in scratch_bytes(path).items() if name.startswith((*wanted, masked))}
+    assert len(seen) == 2 * len(wanted) + 1   # (with INT8 and with floating-point Q)
     assert not any(seen.values()), seen
 
 
