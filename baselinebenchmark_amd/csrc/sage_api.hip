@@ -244,45 +244,76 @@ struct MaskArg {
 // Query rows per workgroup: 256 (eight wavefronts, two groups in step on one tile stream, sage_attn.hip) or 128 (four wavefronts,
 // two or three workgroups to a compute unit, sage_attn_small.hip).  The results are the same bits; the line between them is cost.
 // The small ones let a workgroup's prologue and epilogue run under another's tiles, leave fewer padded rows and fill the chip with half
-// the rows, but fetch every K and V tile twice as often.  Whole calls, bf16, 256 rows / 128 rows, us:
-//   chip not filled (128 q-tiles of 256 rows and fewer): 8 heads of 2000 rows, head_dim 128, FP16 full 54.0 / 50.1, causal 54.0 / 50.1, FP8 47.1 /
-//     43.1; of 4000 89.4 / 85.6, 89.3 / 84.5, 70.0 / 64.7; head_dim 64 FP16 of 4000 65.0 / 58.4;
-//   one round of the chip, all of the same cost: two small workgroups share some compute units and not others: 12 heads of 4000 rows, full,
-//     head_dim 128 FP16 102 / 115, FP8 78 / 84; 100 of 500 45.0 / 45.0, 44.9 / 44.0; 64 of 700 43.0 / 43.7, 43.2 / 42.8; head_dim 64 FP16 64 of 700
-//     30.2 / 29.4, 48 of 1000 36.1 / 36.6, FP8 24 of 2000 41.9 / 41.9, 16 of 2800 45.3 / 45.9.  Causal tiles differ by themselves: 12 of 4000 91 / 86;
-//   several rounds, head_dim 128: FP16 full, 160 of 1400 rows 194 / 190, 128 of 2000 263 / 275; causal, 64 of 2800 157 / 155, 64 of 4000 259 / 268; FP8
-//     full 1400 173 / 159, 2000 216 / 213, 2800 187 / 191; causal 2800 135 / 132, 4000 209 / 210, 32 of 8000 315 / 329;
-//   head_dim 64, three to a compute unit: FP16 full 64 of 4000 270 / 264, 32 of 8000 480 / 482, causal 8000 275 / 264, 32 of 16000 959 / 924; FP8 full 4000
-//     204 / 194, 8000 341 / 337, causal 8000 205 / 203, 16000 665 / 657;
-//   FP8 with LSE: 2000 rows full 255 / 245, causal 187 / 173, 32 of 16000 2663 / 2503 and 1371 / 1286: at every length;
+// the rows, but fetch every K and V tile twice as often.  Which is the faster depends on how many rounds of the chip either makes: 7872 whole calls
+// without a mask (2 head_dims, both P.V, full and causal, with and without LSE, the three kinds of K scales, 300 to 8000 rows, 150 to 1540 q-tiles of
+// 256 rows; bf16) are 0.1 % longer than the better size by the rules below, 48 of them more than 2 % longer than with 256 rows (7.4 % always with 256); of 5808
+// others of the same ranges 56 are, at most 6 %.
+// Some of them, and what the rules do not compare, whole calls, 256 rows / 128 rows, us:
+//   not filled (128 q-tiles of 256 rows and fewer): 8 heads of 2000 rows, head_dim 128, FP16 full 54.0 / 50.1, causal 54.0 / 50.1, FP8 47.1 / 43.1; of 4000
+//     89.4 / 85.6, 89.3 / 84.5, 70.0 / 64.7; head_dim 64 FP16 of 4000 65.0 / 58.4; interleaved, FP8, causal 12 of 2000 38 / 37, but full, where the
+//     small kernel keeps 36 bytes a lane in scratch memory, 33 of 700 27.0 / 27.8;
 //   packed, 32/8 heads, the length between mean and maximum: head_dim 64, causal FP16, 200 prompts of 8..300 259 / 162, 96 of 16..512 208 / 146, 16 of
 //     512..8000 1544 / 1434, 8 of 4000..16000 4345 / 4006, full FP8 5158 / 4910: always; head_dim 128, causal FP16 64 of 16..1024 424 / 370, 40 of
 //     200..2000 680 / 635, 30 of 1000..4000 1822 / 1840, FP8 1366 / 1302, 16 of 512..8000 1666 / 1661, full FP16 40 of 200..2000 988 / 972, FP8 30 of
 //     1000..4000 2124 / 2119;
-//   K blocks of 16 and interleaved scales the same: FP8, head_dim 128, blocks of 16, full 160 of 1400 rows 176 / 164, 2000 220 / 219, 2800 192 / 197, causal 2800 138 /
-//     132, 4000 215 / 214, 8 heads of 4000 74 / 70; head_dim 64, in one round, 2 x 32/8 of 704 24.4 / 25.3; head_dim 64, interleaved, FP16 8 heads of 2000 44 / 39, FP8 causal 12 of 2000 38 / 37, but full, which
-//     keeps 36 bytes a lane in scratch memory, 33 of 700 27.0 / 27.8;
 //   masks: one bias per head, 2 x 16 heads of 1000 rows, head_dim 64 69 / 49, 128 82 / 60, 1 x 4 of 6000 325 / 211, 363 / 232; documents, head_dim 64, 2
 //     x 16 of 1500 53 / 50, 4 x 32 123 / 110, FP8 128 1 x 32 of 2200 133 / 101; padding, head_dim 64, 1 x 32 of 2200 109 / 85, but, head_dim 128, FP16,
 //     in one round of the chip, 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), of 1000 52 / 48, and in three whole ones, 4 x 32 of 1500, 195 / 200.
 enum MaskClass { kNoMask, kKeepMask, kBiasMask, kOtherMask };   // boolean (in bits, or contiguous keys), additive with contiguous keys, other strides
 struct TileRows { int B, Hq, Sq, Skv, D, pv, causal, blkk, kgroups; bool lse; MaskClass mask; bool packed; int total_q, total_k; };
+
+// Calls that are not causal: all workgroups of a size cost the same.  A round of the chip of 256-row workgroups takes as long as their tiles
+// and `hidden` tiles more than small ones (what of a prologue and an epilogue does not run beside another workgroup; less of it in the
+// first round, where compute units with one small workgroup wait for those with two); one, two or three small ones together on a compute unit take
+// `together` times their tiles.  Fitted to the calls above.  Examples, 256 / 128 rows, us: head_dim 128, FP16, 75 heads of 1500 rows 116 / 126, 37 of 1700 102 / 96, 47 of
+// 2600 203 / 186, FP8 73 of 1700 112 / 118, 47 of 2600 158 / 143; head_dim 64, FP16, 18 of 4200 136 / 110, 32 of 3500 125 / 129, FP8 9 of 8000 160 / 125, 14 of 8000
+// 168 / 180, 200 of 700 66 / 55.
+struct RoundCost { float together[3], hidden; };
+constexpr RoundCost kRoundCost128[2] = {{{0.68f, 1.25f, 0}, 1.6f}, {{0.80f, 1.22f, 0}, 1.8f}};   // FP16, FP8 P.V
+constexpr RoundCost kRoundCost64[2] = {{{0.62f, 1.10f, 1.48f}, 0.9f}, {{0.65f, 1.08f, 1.46f}, 0.6f}};
+constexpr RoundCost kRoundCost64Fp8Lse = {{0.50f, 1.04f, 1.33f}, 0.2f}, kRoundCost64Fp8Fine = {{0.78f, 1.15f, 1.46f}, 0.4f};   // (fine: see below)
+bool fewer_rounds_pay(const RoundCost& cost, int per_cu, int64_t large, int64_t small, int Skv) {
+  constexpr int kComputeUnits = 256;
+  const int64_t rounds = (large + kComputeUnits - 1) / kComputeUnits, deepest = (small + kComputeUnits - 1) / kComputeUnits;
+  const int rest = (int)(deepest % per_cu);
+  const float tiles = Skv / 128.0f, small_tiles = (float)(deepest / per_cu) * cost.together[per_cu - 1] + (rest ? cost.together[rest - 1] : 0);
+  return small_tiles * tiles <= rounds * tiles + (rounds == 1 ? 0.6f : (float)rounds) * cost.hidden;
+}
+
 bool small_tiles_pay(const TileRows& c) {
-  const bool fine = c.kgroups != 1 || c.blkk == 16;   // two or four K scales per 32 keys
+  const bool fine = c.kgroups != 1 || c.blkk == 16, fp8 = c.pv == SAGE_PV_FP8;   // fine: two or four K scales per 32 keys
   if (c.mask == kOtherMask || (c.mask != kNoMask && fine)) return false;   // (no such variants)
   if (c.packed && c.blkk == 16) return false;   // (their plan stays the one of sage_varlen_plan)
   if (c.packed && c.total_q >= kSmallTileRows << 16) return false;   // (a plan has 16 bits for the q-tile of a sequence)
-  if (c.pv == SAGE_PV_FP8 && c.lse) return true;
-  if (c.mask != kNoMask && !(c.mask == kKeepMask && c.D == 128 && c.pv == SAGE_PV_FP16)) return true;
-  int64_t keys = c.packed ? ((int64_t)c.total_k / c.B + c.Skv) / 2 : c.Skv;
-  const int64_t large = (int64_t)c.B * c.Hq * ((c.Sq + 255) / 256);
-  if (c.packed && c.D == 64) return true;
-  if (!c.packed && large <= 128) return c.causal || !(c.kgroups != 1 && c.D == 64 && c.pv == SAGE_PV_FP8);
-  if (!c.packed && !c.causal && large <= 256) return keys <= (c.D == 64 ? (c.pv == SAGE_PV_FP16 ? 768 : fine ? 512 : 2048) : c.pv == SAGE_PV_FP8 ? 768 : 512);
-  if (c.mask != kNoMask) return keys <= 1024 || large <= 512;
-  if (c.causal) keys /= 2;
-  if (c.D == 64) return keys <= (c.causal && c.pv == SAGE_PV_FP16 ? 8192 : 4096);
-  return keys <= (c.pv == SAGE_PV_FP8 ? 1800 : 1500);
+  if (c.packed) {
+    if (c.D == 64 || (fp8 && c.lse)) return true;
+    const int64_t keys = ((int64_t)c.total_k / c.B + c.Skv) / 2;
+    return keys <= (fp8 ? 1800 : 1500) * (c.causal ? 2 : 1);
+  }
+  const int64_t heads = (int64_t)c.B * c.Hq, large = heads * ((c.Sq + kLargeTileRows - 1) / kLargeTileRows);
+  if (c.mask != kNoMask) {
+    if (c.mask != kKeepMask || c.D == 64 || fp8 || large <= 128) return true;
+    return large <= 256 ? c.Skv <= 512 : c.Skv <= 1024 || large <= 512;
+  }
+  // FP8 P.V with LSE: the exact exponentials are the longer half, and nothing is lost by fetching a tile twice; full calls of head_dim 64 in
+  // one round of the chip are the exception.
+  if (fp8 && c.lse && (c.D == 128 || c.kgroups != 1 || c.causal)) return true;
+  if (fp8 && c.D == 64 && !c.lse) {
+    if (c.kgroups != 1 && !c.causal && large <= 128) return false;                  // (scratch memory, see above)
+    if (c.blkk == 16 && c.causal && large > 128 && large <= 256) return false;      // 32 heads of 2000 rows 44.3 / 45.5, 27 of 1400 36.5 / 37.6
+  }
+  if (large <= 128) return true;
+  if (!c.causal) {
+    const RoundCost& cost = c.D == 128 ? kRoundCost128[fp8] : !fp8 ? kRoundCost64[0] : c.lse ? kRoundCost64Fp8Lse : fine ? kRoundCost64Fp8Fine : kRoundCost64[1];
+    return fewer_rounds_pay(cost, c.D == 64 ? 3 : 2, large, heads * ((c.Sq + kSmallTileRows - 1) / kSmallTileRows), c.Skv);
+  }
+  // Causal ones differ by themselves.  Up to five quarters of a round the small ones spread the longest tiles over compute units that have
+  // nothing else; in the second round 256 rows pair a long tile with a short one and come out even; beyond, the tiles' cost decides, at half
+  // the keys.  256 / 128 rows, us: head_dim 128, FP16, 12 heads of 5600 rows 127 / 122, 32 of 3500 114 / 124, 75 of 1500 86 / 88, 100 of 1500
+  // 109 / 104, 85 of 2300 159 / 162, 73 of 3500 258 / 274, FP8 12 of 5600 101 / 98, 73 of 3500 205 / 227, with K blocks of 16 100 of 2300 167 / 158; head_dim 64, FP16, 20 of 5600
+  // 104 / 107, 47 of 5600 237 / 218, FP8 32 of 3000 53 / 55, 64 of 3000 95 / 92.
+  if (c.D == 128) return c.Skv <= (large <= 320 ? 8192 : large <= 512 ? 1400 : c.blkk == 16 ? 2700 : 2048);
+  return large <= 320 || (!fp8 && fine) || c.Skv <= (large <= 512 ? (fp8 ? 2700 : 3000) : fp8 ? 8192 : 16384);
 }
 int tile_rows(const TileRows& c) {
 #ifdef SAGE_TIMING   // (the timers that are read are those of the workgroups of 256 rows)

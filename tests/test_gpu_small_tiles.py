@@ -180,3 +180,20 @@ def test_masks_get_the_same_bits_from_128_and_256_rows(D, pv, kind):
             packed, rows = rows_of(lambda: sa.sageattn(q, k, v, attn_mask=mask, smooth_k=False, pv_mode=pv, BLKQ=64, BLKK=64))
             assert rows == 128, (Sq, Skv)
             assert torch.equal(packed, large[0]), (Sq, Skv)
+
+
+PLAIN, FINE, INTERLEAVED = dict(BLKQ=128, BLKK=64), dict(BLKQ=128, BLKK=16), dict(BLKQ=32, BLKK=64, q_interleave=8, k_interleave=4)
+
+
+@pytest.mark.parametrize("D,pv,causal,lse,scales,H,L,rows", [
+    (128, "fp16", False, False, PLAIN, 75, 1500, 256), (128, "fp16", False, True, PLAIN, 75, 1500, 256), (128, "fp16", False, False, PLAIN, 37, 1700, 128),
+    (128, "fp8", False, False, PLAIN, 73, 1700, 256), (128, "fp8", False, False, PLAIN, 47, 2600, 128), (128, "fp8", False, True, PLAIN, 73, 1700, 128),
+    (128, "fp16", False, False, INTERLEAVED, 85, 1500, 256), (128, "fp16", True, False, PLAIN, 32, 3500, 256), (128, "fp8", True, False, PLAIN, 73, 3500, 256),
+    (128, "fp8", True, False, FINE, 100, 2300, 128), (128, "fp8", True, False, PLAIN, 8, 16000, 256), (64, "fp16", False, False, PLAIN, 32, 3500, 256),
+    (64, "fp16", False, False, PLAIN, 18, 4200, 128), (64, "fp16", True, False, PLAIN, 20, 5600, 256), (64, "fp16", True, False, INTERLEAVED, 20, 5600, 128),
+    (64, "fp8", False, False, FINE, 14, 8000, 256), (64, "fp8", False, True, FINE, 8, 8000, 256), (64, "fp8", False, False, INTERLEAVED, 85, 1500, 256),
+    (64, "fp8", False, False, INTERLEAVED, 10, 2000, 256), (64, "fp8", False, True, INTERLEAVED, 16, 4200, 128), (64, "fp8", True, False, INTERLEAVED, 16, 4200, 128),
+])
+def test_calls_take_the_size_that_measured_faster(D, pv, causal, lse, scales, H, L, rows):
+    q, k, v = (torch.zeros((1, H, L, D), device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    assert rows_of(lambda: sa.sageattn(q, k, v, is_causal=causal, pv_mode=pv, return_lse=lse, **scales))[1] == rows
