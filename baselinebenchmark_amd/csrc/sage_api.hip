@@ -695,7 +695,10 @@ int sage_sageattn_masked(const void* q, const void* k, const void* v, void* out,
     ColStatArgs& ks = stats.k_stat;
     ks.x = (const u16*)k; ks.B = B; ks.H = Hkv; ks.L = Skv; ks.D = D; ks.x_sb = k_sb; ks.x_sh = k_sh; ks.x_sn = k_sn;
     ks.nchunk = colstat_chunks(Skv);
-    ks.cached = statistics_stay(k_elements * ((smooth_k != 0) + (pv_mode == SAGE_PV_FP8)));
+    // (FP8 P.V of head_dim 128, float16: its kernel is as long whether it finds the tensors or not.  1 row, through / past, us: 32 heads of 523 keys
+    // 29.7 / 27.8, 24 of 900 28.5 / 27.2, 16 of 1600 28.9 / 27.6, but 64 of 1245 42.6 / 44.0, 128 of 900 46.1 / 47.5; bfloat16 32 of 523 27.4 / 28.5, 16 of 1600 27.8 / 28.8)
+    const bool kept = pv_mode != SAGE_PV_FP8 || D != 128 || dtype != SAGE_DT_F16 || k_elements > (int64_t)5 << 20;
+    ks.cached = kept && statistics_stay(k_elements * ((smooth_k != 0) + (pv_mode == SAGE_PV_FP8)));
     stats.v_stat = ks;
     stats.v_stat.x = (const u16*)v; stats.v_stat.x_sb = v_sb; stats.v_stat.x_sh = v_sh; stats.v_stat.x_sn = v_sn;
     if (smooth_k) ks.partial = stat;
