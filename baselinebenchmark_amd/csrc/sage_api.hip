@@ -316,8 +316,8 @@ bool small_tiles_pay(const TileRows& c) {
   return large <= 320 || (!fp8 && fine) || c.Skv <= (large <= 512 ? (fp8 ? 2700 : 3000) : fp8 ? 8192 : 16384);
 }
 int tile_rows(const TileRows& c) {
-#ifdef SAGE_TIMING   // (the timers that are read are those of the workgroups of 256 rows)
-  return kLargeTileRows;
+#ifdef SAGE_TIMING   // (the timers that are read are those of the workgroups of 256 rows, of calls without a mask and interleaved scales)
+  if (c.mask == kNoMask && c.kgroups == 1) return kLargeTileRows;
 #endif
   return small_tiles_pay(c) ? kSmallTileRows : kLargeTileRows;
 }

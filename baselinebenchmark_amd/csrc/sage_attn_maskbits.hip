@@ -5,15 +5,20 @@
 
 namespace sage {
 
+namespace {
+template <int D, int PV>
+hipError_t launch_kind(const AttnArgs& a, int grid, hipStream_t st) {
+  if (a.k_interleave) return launch_one<D, 8, 128, PV, false, false, 3, 3>(a, grid, st);
+  if (a.blkk == 16) return launch_one<D, 8, 128, PV, false, false, 3, 2>(a, grid, st);
+  if (a.tile_rows == kSmallTileRows) return launch_one<D, 4, 128, PV, false, false, 3, 1>(a, grid, st);
+  if constexpr (D == 128 && PV == 0) return launch_one<D, 8, 128, PV, false, false, 3, 1>(a, grid, st);
+  else return hipErrorInvalidValue;   // (they take 128 rows at every size: small_tiles_pay)
+}
+}  // namespace
+
 hipError_t launch_attn_packed_mask(const AttnArgs& a, int D, int pv, int grid, hipStream_t st) {
-  if (a.tile_rows == kSmallTileRows) {
-    if (D == 128) return pv ? launch_one<128, 4, 128, 1, false, false, 3, 1>(a, grid, st) : launch_one<128, 4, 128, 0, false, false, 3, 1>(a, grid, st);
-    return pv ? launch_one<64, 4, 128, 1, false, false, 3, 1>(a, grid, st) : launch_one<64, 4, 128, 0, false, false, 3, 1>(a, grid, st);
-  }
-#define SAGE_ATTN_B(DD, PVV) (a.k_interleave ? launch_one<DD, 8, 128, PVV, false, false, 3, 3>(a, grid, st) : a.blkk == 16 ? launch_one<DD, 8, 128, PVV, false, false, 3, 2>(a, grid, st) : launch_one<DD, 8, 128, PVV, false, false, 3, 1>(a, grid, st))
-  if (D == 128) return pv ? SAGE_ATTN_B(128, 1) : SAGE_ATTN_B(128, 0);
-  return pv ? SAGE_ATTN_B(64, 1) : SAGE_ATTN_B(64, 0);
-#undef SAGE_ATTN_B
+  if (D == 128) return pv ? launch_kind<128, 1>(a, grid, st) : launch_kind<128, 0>(a, grid, st);
+  return pv ? launch_kind<64, 1>(a, grid, st) : launch_kind<64, 0>(a, grid, st);
 }
 
 }  // namespace sage

@@ -4,16 +4,24 @@
 
 namespace sage {
 
+namespace {
+template <int D, int PV, int MASK>
+hipError_t launch_mask(const AttnArgs& a, int grid, hipStream_t st) {
+  if (a.k_interleave) return launch_one<D, 8, 128, PV, false, false, MASK, 3>(a, grid, st);
+  if (a.blkk == 16) return launch_one<D, 8, 128, PV, false, false, MASK, 2>(a, grid, st);
+  if (a.tile_rows == kSmallTileRows) return launch_one<D, 4, 128, PV, false, false, MASK, 1>(a, grid, st);
+  if constexpr (D == 128 && PV == 0 && MASK == 4) return launch_one<D, 8, 128, PV, false, false, MASK, 1>(a, grid, st);
+  else return hipErrorInvalidValue;   // (they take 128 rows at every size: small_tiles_pay)
+}
+template <int D, int PV>
+hipError_t launch_kind(const AttnArgs& a, int grid, hipStream_t st) {
+  return a.mask_kind == 1 ? launch_mask<D, PV, 4>(a, grid, st) : launch_mask<D, PV, 5>(a, grid, st);
+}
+}  // namespace
+
 hipError_t launch_attn_masked_wide(const AttnArgs& a, int D, int pv, int grid, hipStream_t st) {
-#define SAGE_ATTN_WS(DD, PVV) (a.mask_kind == 1 ? launch_one<DD, 4, 128, PVV, false, false, 4, 1>(a, grid, st) : launch_one<DD, 4, 128, PVV, false, false, 5, 1>(a, grid, st))
-  if (a.tile_rows == kSmallTileRows) return D == 128 ? (pv ? SAGE_ATTN_WS(128, 1) : SAGE_ATTN_WS(128, 0)) : pv ? SAGE_ATTN_WS(64, 1) : SAGE_ATTN_WS(64, 0);
-#undef SAGE_ATTN_WS
-#define SAGE_ATTN_WK(DD, PVV, KS) (a.mask_kind == 1 ? launch_one<DD, 8, 128, PVV, false, false, 4, KS>(a, grid, st) : launch_one<DD, 8, 128, PVV, false, false, 5, KS>(a, grid, st))
-#define SAGE_ATTN_W(DD, PVV) (a.k_interleave ? SAGE_ATTN_WK(DD, PVV, 3) : a.blkk == 16 ? SAGE_ATTN_WK(DD, PVV, 2) : SAGE_ATTN_WK(DD, PVV, 1))
-  if (D == 128) return pv ? SAGE_ATTN_W(128, 1) : SAGE_ATTN_W(128, 0);
-  return pv ? SAGE_ATTN_W(64, 1) : SAGE_ATTN_W(64, 0);
-#undef SAGE_ATTN_W
-#undef SAGE_ATTN_WK
+  if (D == 128) return pv ? launch_kind<128, 1>(a, grid, st) : launch_kind<128, 0>(a, grid, st);
+  return pv ? launch_kind<64, 1>(a, grid, st) : launch_kind<64, 0>(a, grid, st);
 }
 
 }  // namespace sage
