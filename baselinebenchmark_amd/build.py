@@ -26,11 +26,14 @@ FLAGS = [
 
 
 # The instantiation units of the shipped attention kernels are scheduled for instruction-level parallelism rather than
-# for occupancy (which is fixed at two wavefronts per SIMD anyway): +0.9 % on config 2 and on FP16 P.V at 16k keys, equal
-# elsewhere, no scratch.  The explicit-mask variants (sage_attn_mask.hip), which spill under either strategy, keep the default.
+# for occupancy, which the launch bounds fix at two wavefronts per SIMD, three in the 128-row kernels of head_dim 64: +0.9 % on
+# 2 x 32 causal heads of 16384 rows (FP8 P.V) and on FP16 P.V at 16k keys, equal elsewhere.  Kernels of 256 rows and of head_dim 128 come out
+# without scratch memory; the 128-row ones of head_dim 64 keep up to 28 bytes a lane there (FP8 P.V; 36 to 48 with interleaved K scales),
+# 8 or 12 in five FP16 ones, within their 168 registers, and are the faster for it (attn_small_per_cu).  The explicit-mask variants
+# (sage_attn_mask.hip), which spill under either strategy, keep the default.
 # -fno-honor-nans: these kernels produce -inf (masked scores) but never a NaN, and without the flag every fmaxf on a
 # loaded or exchanged value is preceded by an instruction that only quiets signalling NaNs (four per tile: 0.6 % on
-# config 2, bit-identical outputs).
+# 2 x 32 causal heads of 16384 rows, bit-identical outputs).
 EXTRA_FLAGS = {src: ["-mllvm", "-amdgpu-sched-strategy=max-ilp", "-fno-honor-nans"]
                for src in ("sage_attn.hip", "sage_attn_qfuse.hip", "sage_attn_kinterleave.hip", "sage_attn_small.hip")}
 

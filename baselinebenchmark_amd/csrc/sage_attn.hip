@@ -17,7 +17,8 @@ void finish_attn_args(AttnArgs& a, bool causal) {
   a.tier_shift = -1;
   a.div_range = a.div_last = make_fastdiv(1);
   // Per-XCD tile order (fixed-length batches whose heads and KV groups spread evenly over the eight XCDs): ranges of
-  // R = 2^tier_shift consecutive q-tiles, R at most 32 and at most half of a head's q-tiles.  Causal problems with fewer than
+  // R = 2^tier_shift consecutive q-tiles, R at most 32 and at most half of a head's q-tiles.  (The lines below were measured with q-tiles of
+  // 256 rows and are the same numbers of q-tiles for those of 128.)  Causal problems with fewer than
   // 16 q-tiles per compute unit keep the plain heaviest-first order -- with so few rounds the balance of the last one
   // matters more than locality (1 x 32 heads of 4096 rows: 7 % slower with ranges) -- unless an XCD holds 16 heads or
   // more and 8 q-tiles per compute unit (4 x 32 heads of 4096 rows: 2 % faster with ranges, 8 x 32 of 2048 rows 5 %).

@@ -44,9 +44,6 @@ __device__ inline float xor16_32_sum(float x) {
   return x + __shfl_xor(x, 32);
 }
 
-// Waits for this wavefront's LDS operations only: loads in flight stay in flight.
-__device__ inline void lds_only_barrier_few() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <class Quotient>
 __device__ __forceinline__ v4i pack16(const float (&x)[16], Quotient quotient) {
   uint32_t packed[4];
@@ -150,7 +147,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
                                                                        // sums near fp32's end come out as in the tiled kernel)
       }
     }
-    lds_only_barrier_few();
+    lds_barrier();
     if constexpr (PV == 1) v_exact = __builtin_amdgcn_ballot_w64(!reciprocal_is_exact(vs_lds[lane].x) || !reciprocal_is_exact(vs_lds[(lane + 64) % D].x)) == 0;
   }
   if constexpr (!EARLY)
@@ -196,7 +193,7 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
       dot[mt] = xor16_32_sum(sum);   // what K smoothing takes from every logit of the row
       if (w == 0 && g == 0) row_amax[16 * mt + m] = amax;
     }
-    lds_only_barrier_few();
+    lds_barrier();
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
       const int r = min(16 * mt + m, rows - 1), head = r / a.Sq, s = r - head * a.Sq;
@@ -254,7 +251,8 @@ __global__ void __launch_bounds__(256, 2) attn_few_kernel(FewArgs a) {
         }
     }
     // ---- K: subtract the mean in the input type, block maxima, quantise ----
-    // (one score tile and no V quotients: the differences stay as floats, a widening less each; the others have no registers for it)
+    // (one score tile and no V quotients: the differences stay as floats, a widening less each; at head_dim 128 this takes all 256 registers
+    // and, with the sixteen sums ahead, 12 bytes a lane of scratch memory outside the loop; the others have no registers for it)
     constexpr bool WIDE = MT == 1 && PV == 0;
     float xk[2][WIDE ? D / 4 : 1];
     float amax[2];

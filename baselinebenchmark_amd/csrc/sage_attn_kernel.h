@@ -92,12 +92,6 @@ __device__ inline float xchg32_sum(float x) {
   return lo + hi;
 }
 
-// Workgroup barrier that only orders LDS traffic: waits for this wavefront's outstanding LDS
-// operations, then s_barrier (global-memory traffic issued ahead stays in flight).
-__device__ inline void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // Nothing that reads or copies x comes before this place, nor after it the product that writes x.
 template <class T>
 __device__ __forceinline__ void pin_registers(T& x) { asm volatile("" : "+v"(x)); }
@@ -288,7 +282,8 @@ __global__ void __launch_bounds__(NW * 64, attn_is_small(NW) ? (attn_small_per_c
           r0 += 1 << rs;
           if (r0 >= a.nqt) return;   // (a grid larger than the tile count: nothing to do)
         }
-        // Inside a round (32 consecutive workgroups of the XCD: one per compute unit) the order alternates: lightest
+        // Inside a round (32 consecutive workgroups of the XCD: one per compute unit with 256 rows; with 128 rows, where two or three share
+        // one, the same 32, not measured apart) the order alternates: lightest
         // q-tile first in even rounds, heaviest first in odd ones.  The hardware hands out workgroups strictly in index
         // order and round-robin over the XCD's four shader engines, so a free compute unit waits until every earlier
         // workgroup has found a place in ITS engine.  A round that starts on all compute units at once with ascending

@@ -4,7 +4,8 @@
 //
 // With eight wavefronts a workgroup takes a compute unit for itself, and the 9 us that a q-tile spends on its addresses, raw rows,
 // quantisation and output run beside nothing; at 1000 keys that is half of its time.  Four wavefronts use half the registers and
-// 32 to 64 KB of LDS, so two workgroups (three at head_dim 64) share a compute unit and run those parts, and each other's matrix and
+// 32 to 64 KB of LDS, so two workgroups (three at head_dim 64: 168 registers, a few of them in scratch memory, see attn_small_per_cu) share a
+// compute unit and run those parts, and each other's matrix and
 // vector work, side by side without barriers between them.  A wavefront is raised over the others of its SIMD while it issues
 // matrix instructions (1 to 3 %).  The last tile is cut down to the 32-key groups that a wavefront sees, and only it is masked.
 // Whole calls, 256 rows -> 128: 96 packed prompts of 16..1024 rows, 32/8 heads, head_dim 128, causal, FP16 524 -> 446 us, FP8 462 -> 393; head_dim

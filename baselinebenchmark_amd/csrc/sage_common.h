@@ -160,6 +160,10 @@ __device__ inline void store16(bool cached, void* p, uint4 v) {
   else store_stream16(p, v);
 }
 
+// Workgroup barrier that only orders LDS traffic: waits for this wavefront's outstanding LDS
+// operations, then s_barrier (global-memory traffic issued ahead stays in flight).
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // ---------------------------------------------------------------------------------------------
 // Wavefront (64-lane) reductions with DPP inside rows of 16 lanes, then lane reads across rows.
 // The result is uniform across the wavefront.
