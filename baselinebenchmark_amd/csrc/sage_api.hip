@@ -257,8 +257,10 @@ struct MaskArg {
 //     200..2000 680 / 635, 30 of 1000..4000 1822 / 1840, FP8 1366 / 1302, 16 of 512..8000 1666 / 1661, full FP16 40 of 200..2000 988 / 972, FP8 30 of
 //     1000..4000 2124 / 2119;
 //   masks: one bias per head, 2 x 16 heads of 1000 rows, head_dim 64 69 / 49, 128 82 / 60, 1 x 4 of 6000 325 / 211, 363 / 232; documents, head_dim 64, 2
-//     x 16 of 1500 53 / 50, 4 x 32 123 / 110, FP8 128 1 x 32 of 2200 133 / 101; padding, head_dim 64, 1 x 32 of 2200 109 / 85, but, head_dim 128, FP16,
-//     in one round of the chip, 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), of 1000 52 / 48, and in three whole ones, 4 x 32 of 1500, 195 / 200.
+//     x 16 of 1500 53 / 50, 4 x 32 123 / 110, FP8 128 1 x 32 of 2200 133 / 101; padding, head_dim 64, 1 x 32 of 2200 109 / 85; boolean ones over FP16 P.V
+//     by rounds, as without a mask: head_dim 128, in one round 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), in two 67 of 1500 115 / 119, 42 of 3000 175 / 182, but 33
+//     of 2078 139 / 125; head_dim 64, in one round, padding 22 of 2078 63 / 68, 12 of 4200 107 / 115, 33 of 1500 60 / 60, one mask per head 22 of 2078 105 / 110, but
+//     documents 27 of 1500 48 / 46, 22 of 2078 59 / 58, and in two rounds padding 33 of 2078 105 / 82, one mask per head 175 / 145.
 enum MaskClass { kNoMask, kKeepMask, kBiasMask, kOtherMask };   // boolean (in bits, or contiguous keys), additive with contiguous keys, other strides
 struct TileRows { int B, Hq, Sq, Skv, D, pv, causal, blkk, kgroups; bool lse; MaskClass mask; bool packed; int total_q, total_k; };
 
@@ -292,8 +294,9 @@ bool small_tiles_pay(const TileRows& c) {
   }
   const int64_t heads = (int64_t)c.B * c.Hq, large = heads * ((c.Sq + kLargeTileRows - 1) / kLargeTileRows);
   if (c.mask != kNoMask) {
-    if (c.mask != kKeepMask || c.D == 64 || fp8 || large <= 128) return true;
-    return large <= 256 ? c.Skv <= 512 : c.Skv <= 1024 || large <= 512;
+    if (c.mask != kKeepMask || fp8 || large <= 128) return true;
+    if (c.D == 64) return large > 256 || c.Skv <= 1792;
+    return fewer_rounds_pay(kRoundCost128[0], 2, large, heads * ((c.Sq + kSmallTileRows - 1) / kSmallTileRows), c.Skv);
   }
   // FP8 P.V with LSE: the exact exponentials are the longer half, and nothing is lost by fetching a tile twice; full calls of head_dim 64 in
   // one round of the chip are the exception.

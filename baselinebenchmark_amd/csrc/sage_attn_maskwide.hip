@@ -10,7 +10,7 @@ hipError_t launch_mask(const AttnArgs& a, int grid, hipStream_t st) {
   if (a.k_interleave) return launch_one<D, 8, 128, PV, false, false, MASK, 3>(a, grid, st);
   if (a.blkk == 16) return launch_one<D, 8, 128, PV, false, false, MASK, 2>(a, grid, st);
   if (a.tile_rows == kSmallTileRows) return launch_one<D, 4, 128, PV, false, false, MASK, 1>(a, grid, st);
-  if constexpr (D == 128 && PV == 0 && MASK == 4) return launch_one<D, 8, 128, PV, false, false, MASK, 1>(a, grid, st);
+  if constexpr (PV == 0 && MASK == 4) return launch_one<D, 8, 128, PV, false, false, MASK, 1>(a, grid, st);
   else return hipErrorInvalidValue;   // (they take 128 rows at every size: small_tiles_pay)
 }
 template <int D, int PV>

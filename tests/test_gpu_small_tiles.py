@@ -197,3 +197,14 @@ PLAIN, FINE, INTERLEAVED = dict(BLKQ=128, BLKK=64), dict(BLKQ=128, BLKK=16), dic
 def test_calls_take_the_size_that_measured_faster(D, pv, causal, lse, scales, H, L, rows):
     q, k, v = (torch.zeros((1, H, L, D), device=DEV, dtype=torch.bfloat16) for _ in range(3))
     assert rows_of(lambda: sa.sageattn(q, k, v, is_causal=causal, pv_mode=pv, return_lse=lse, **scales))[1] == rows
+
+
+@pytest.mark.parametrize("D,pv,mask,H,L,rows", [
+    (64, "fp16", "keep", 24, 2078, 256), (64, "fp16", "keep", 24, 1500, 128), (64, "fp16", "keep", 33, 2078, 128), (64, "fp16", "bias", 24, 2078, 128),
+    (64, "fp8", "keep", 24, 2078, 128), (128, "fp16", "keep", 67, 1500, 256), (128, "fp16", "keep", 33, 2078, 128), (128, "fp16", "keep", 32, 1500, 256),
+    (128, "fp8", "keep", 67, 1500, 128),
+])
+def test_masked_calls_take_the_size_that_measured_faster(D, pv, mask, H, L, rows):
+    q, k, v = (torch.zeros((1, H, L, D), device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    m = torch.ones((1, 1, 1, L), device=DEV, dtype=torch.bool) if mask == "keep" else torch.zeros((1, 1, L, L), device=DEV)
+    assert rows_of(lambda: sa.sageattn(q, k, v, attn_mask=m, pv_mode=pv))[1] == rows
