@@ -258,7 +258,7 @@ struct MaskArg {
 //     1000..4000 2124 / 2119;
 //   masks: one bias per head, 2 x 16 heads of 1000 rows, head_dim 64 69 / 49, 128 82 / 60, 1 x 4 of 6000 325 / 211, 363 / 232; documents, head_dim 64, 2
 //     x 16 of 1500 53 / 50, 4 x 32 123 / 110, FP8 128 1 x 32 of 2200 133 / 101; padding, head_dim 64, 1 x 32 of 2200 109 / 85; boolean ones over FP16 P.V
-//     by rounds, as without a mask: head_dim 128, in one round 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), in two 67 of 1500 115 / 119, 42 of 3000 175 / 182, but 33
+//     by rounds, as without a mask: head_dim 128, in one round, 2 x 16 of 1500 70 / 75 (one mask per head 101 / 106), in two, 67 of 1500 115 / 119, 42 of 3000 175 / 182, but 33
 //     of 2078 139 / 125; head_dim 64, in one round, padding 22 of 2078 63 / 68, 12 of 4200 107 / 115, 33 of 1500 60 / 60, one mask per head 22 of 2078 105 / 110, but
 //     documents 27 of 1500 48 / 46, 22 of 2078 59 / 58, and in two rounds padding 33 of 2078 105 / 82, one mask per head 175 / 145.
 enum MaskClass { kNoMask, kKeepMask, kBiasMask, kOtherMask };   // boolean (in bits, or contiguous keys), additive with contiguous keys, other strides
@@ -311,7 +311,7 @@ bool small_tiles_pay(const TileRows& c) {
     return fewer_rounds_pay(cost, c.D == 64 ? 3 : 2, large, heads * ((c.Sq + kSmallTileRows - 1) / kSmallTileRows), c.Skv);
   }
   // Causal ones differ by themselves.  Up to five quarters of a round the small ones spread the longest tiles over compute units that have
-  // nothing else; in the second round 256 rows pair a long tile with a short one and come out even; beyond, the tiles' cost decides, at half
+  // nothing else; in the second round, 256 rows pair a long tile with a short one and come out even; beyond, the tiles' cost decides, at half
   // the keys.  256 / 128 rows, us: head_dim 128, FP16, 12 heads of 5600 rows 127 / 122, 32 of 3500 114 / 124, 75 of 1500 86 / 88, 100 of 1500
   // 109 / 104, 85 of 2300 159 / 162, 73 of 3500 258 / 274, FP8 12 of 5600 101 / 98, 73 of 3500 205 / 227, with K blocks of 16 100 of 2300 167 / 158; head_dim 64, FP16, 20 of 5600
   // 104 / 107, 47 of 5600 237 / 218, FP8 32 of 3000 53 / 55, 64 of 3000 95 / 92.
